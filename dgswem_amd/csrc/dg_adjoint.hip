@@ -395,11 +395,11 @@ struct AdjArgs {
     double* __restrict__ gnbar;          // [ne] accumulated cotangent of the element mean Manning n
     const uint8_t* __restrict__ wd;      // WDFLG during the stage, or nullptr (every element wet)
     // block-local staging, as in the forward stage kernel: tile t stages its elements and its halo
-    // hidx[hoff[t]..hoff[t+1]); snbl packs each side's local neighbour index (10 bits each)
-    const int* __restrict__ hoff;
+    // hidx[t*nh..t*nh+nh) (-1 past the tile's last); snbl packs each side's local neighbour index
+    // (10 bits each)
     const int* __restrict__ hidx;
     const int* __restrict__ snbl;
-    int ns;                              // staged elements per block (LDS row length)
+    int nh, ns;                          // halo entries per tile, staged elements per block (LDS row length)
 };
 
 // RHS cotangent of element `el` (its own stage contribution): sum_j b_j DT src_j.
@@ -468,10 +468,10 @@ __global__ void __launch_bounds__(NT, P == 1 ? 2 : 1) adj_stage_kernel(AdjArgs a
     }
     {
         // this tile's elements and its halo, all loads in flight together
-        const int h0 = a.hoff[tile], nh = a.hoff[tile + 1] - h0;
-        for (int j = tid; j < NT + nh; j += NT) {
-            const int g = j < NT ? tile * NT + j : a.hidx[h0 + j - NT];
-            if (g < ne) {
+        const int* hx = a.hidx + (size_t)tile * a.nh;
+        for (int j = tid; j < NT + a.nh; j += NT) {
+            const int g = j < NT ? tile * NT + j : hx[j - NT];
+            if (g >= 0 && g < ne) {
 #pragma unroll
                 for (int f = 0; f < 3 * DOF; f++) stg[f * ns + j] = a.u[(size_t)f * ne + g];
                 double L0[3][DOF];

@@ -134,12 +134,14 @@ struct Ctx {
     DevBuf<int> sinfo, snbr, nm, n2e_off, n2e;
     std::vector<int> h_sinfo, h_snbr;            // host copies (staging lists)
     bool has_cori_el = false;
+    bool mid = true;                             // G and the spherical factors allow llf_flux_nl2
     // block-local staging of the stage kernel, per block size: each block copies the states of its
     // own elements and of its halo (out-of-block internal neighbours) into LDS
     struct Staging {
         int ns = 0;                              // staged elements per block: block size + largest halo
         size_t lds = 0;                          // dynamic LDS bytes per block
-        DevBuf<int> hoff, hidx, snbl;            // halo offsets per tile, halo elements, packed local indices
+        int nh = 0;                              // halo entries per tile (the largest tile's)
+        DevBuf<int> hidx, snbl;                  // halo elements per tile (-1 past its last), packed local indices
     };
     std::map<int, Staging> stg;
     int max_lds = 65536;                         // LDS bytes per block the device allows
@@ -191,6 +193,7 @@ struct Ctx {
     DevBuf<uint8_t> wdsave;                      // wet/dry flags at the start of a gradient call
     // launch configuration
     int block = 256;
+    int split = -1;                              // stage_split_kernel: 1 yes, 0 no, -1 by the number of elements
     int dev = 0;                                 // device current at dg_gpu_init
     // adjoint: gauges, checkpoints, segment stage states, cotangents, parameter accumulators
     int ng = 0, ngu = 0;                         // gauges, distinct gauge elements
@@ -751,6 +754,8 @@ int upload_mesh(Ctx& c) {
                     }
                 }
             }
+        // llf_flux_nl2 needs NY^2+(NX*SF)^2 well inside the range of its square root
+        for (double f : sfe) if (!(f >= 0x1p-20 && f <= 0x1p+20)) c.mid = false;
         HIPCHK(c.sfs.upload(sfs.data(), sfs.size(), c.stream));
         HIPCHK(hipStreamSynchronize(c.stream));
     }
@@ -790,16 +795,33 @@ int init_ctx_common(Ctx& c, const dg_params* prm, bool manning) {
     for (int l = 0; l < 3; l++)
         for (int q = 0; q < c.T.negp; q++)
             if (c.T.phi_edge[l][q][0] != 1.0) return fail("basis tables: PHI_EDGE of mode 1 is not 1");
-    // the stage kernel forms the P1 bathymetry gradient once per element: the linear modes'
-    // derivative tables must be the same at every area point
+    // the stage kernel forms the linear modes' gradients and the P1 bathymetry gradient once per element:
+    // the derivative tables of these modes must be the same at every area point, with these values
     for (int q = 0; q < c.T.nagp; q++)
         if (c.T.phi_area[q][0] != 1.0) return fail("basis tables: PHI_AREA of mode 1 is not 1");
-    for (int q = 1; q < c.T.nagp; q++)
+    const double dr[3] = {0.0, 0.0, 1.0}, ds[3] = {0.0, 1.5, 0.5};
+    for (int q = 0; q < c.T.nagp; q++)
         for (int k = 0; k < 3; k++)
-            if (c.T.drphi[q][k] != c.T.drphi[0][k] || c.T.dsphi[q][k] != c.T.dsphi[0][k])
-                return fail("basis tables: derivatives of the linear modes vary between area points");
+            if (c.T.drphi[q][k] != dr[k] || c.T.dsphi[q][k] != ds[k])
+                return fail("basis tables: unexpected derivatives of the linear modes");
+    if (prm->p == 1)
+        for (int q = 0; q < 3; q++)
+            for (int k = 0; k < 3; k++)
+                if (c.T.phi_area[q][k] != P1Area::phi[q][k] || c.T.mw[q][k] != P1Area::mw[k] ||
+                    c.T.srfac[q][k] != P1Area::srfac[q][k])
+                    return fail("basis tables: unexpected p=1 area rule");
+    // p=1: the stage kernel fuses the edge traces' products and sums, which is exact where the edge values
+    // are 0 or powers of two
+    if (prm->p == 1)
+        for (int l = 0; l < 3; l++)
+            for (int q = 0; q < c.T.negp; q++)
+                for (int k = 0; k < c.T.dof; k++) {
+                    int ex;
+                    const double m = std::fabs(std::frexp(c.T.phi_edge[l][q][k], &ex));
+                    if (m != 0.0 && m != 0.5) return fail("basis tables: an edge value of a p=1 mode is not a power of two");
+                }
     c.dof = c.T.dof; c.nagp = c.T.nagp; c.negp = c.T.negp;
-    c.block = 128;
+    c.block = prm->p == 1 ? 128 : 64;
     {
         int dev = 0, lds = 0;
         HIPCHK(hipGetDevice(&dev));
@@ -819,6 +841,7 @@ int init_ctx_common(Ctx& c, const dg_params* prm, bool manning) {
     }
     Phys& P = c.phys;
     P.g = prm->g;
+    c.mid = P.g >= 0x1p-60 && P.g <= 0x1p+60;
     P.nleq = prm->nolicat == 0 ? 0.0 : 1.0;
     P.leq = prm->nolicat == 0 ? 1.0 : 0.0;
     P.nleqg = P.nleq * P.g;
@@ -1022,17 +1045,26 @@ int build_stage_tables(Ctx& c, int it, int n) {
     return 0;
 }
 
-// Static LDS bytes of stage_kernel<P, NT, ..., MET, ...> (its __shared__ arrays).
-size_t stage_static_lds(int dof, int negp, int nt, bool met) {
-    (void)met;
-    return (size_t)8 * (2 * 3 * dof * nt + 2 * 3 * negp * dof);
-}
+// Static LDS bytes of stage_kernel (its edge tables).
+size_t stage_static_lds(int dof, int negp) { return (size_t)8 * (2 * 3 * negp * dof); }
 
 // Dynamic LDS bytes of adj_stage_kernel: 6*dof staged rows of ns doubles.
 size_t adj_dynamic_lds(int dof, int ns) { return (size_t)8 * (6 * dof) * ns; }
 
-// Block size the stage kernel runs with: the chosen one for nonlinear runs, 64 for linearised runs.
-int stage_nt(const Ctx& c, int nt) { return c.prm.nolicat != 0 ? nt : 64; }
+// Whether the stage runs as four waves per 64 elements (stage_split_kernel): the nonlinear equations and, unless
+// the launch shape was chosen by dg_gpu_set_block or the autotuner, few elements.  Measured per launch, one lane
+// per element against four waves per 64 elements: p=1 17.9 and 13.0 us at 5k elements, 20.4 and 17.8 at 59k, 21.3
+// and 22.3 at 89k (storm basins 27.0 and 13.9, 32.0 and 22.8, 35.0 and 29.9; 35.4 and 38.5 at 129k); p=2 27.9 and
+// 18.8 at 5k, 34.6 and 31.6 at 59k, 35.7 and 42.2 at 89k (storm 42.3 and 21.1, 47.5 and 39.5, 52.4 and 52.9).
+constexpr int SPLIT_MAX1 = 80000, SPLIT_MAX2 = 64000;
+bool stage_split(const Ctx& c) {
+    if (c.prm.nolicat == 0) return false;
+    return c.split < 0 ? c.ne <= (c.prm.p == 1 ? SPLIT_MAX1 : SPLIT_MAX2) : c.split == 1;
+}
+
+// Elements per block the stage kernel runs with: the chosen number for nonlinear runs, 64 for linearised runs
+// and for stage_split_kernel.
+int stage_nt(const Ctx& c, int nt) { return c.prm.nolicat != 0 && !stage_split(c) ? nt : 64; }
 
 // Halo lists of the stage kernel's blocks of `nt` elements (tile t = elements [t*nt, t*nt+nt)):
 // the out-of-tile internal neighbours of each tile in ascending order, and per element the local
@@ -1073,16 +1105,33 @@ int ensure_staging(Ctx& c, int nt) {
     const int ns = nt + hmax;
     if (ns > 1023) return fail("stage kernel staging: halo too large for block size " + std::to_string(nt));
     const size_t dyn = ((size_t)8 * (3 * c.dof + 3) * ns + ns + 7) / 8 * 8;
-    if (dyn + stage_static_lds(c.dof, c.negp, nt, c.met) > (size_t)c.max_lds)
+    // (with 64 elements per block stage_split_kernel may run too, with its exchange rows)
+    const size_t stat = stage_static_lds(c.dof, c.negp) + (nt == SPLIT_NT ? (size_t)8 * split_rows(c.dof, c.nagp) * nt : 0);
+    if (dyn + stat > (size_t)c.max_lds)
         return fail("stage kernel staging: block size " + std::to_string(nt) + " needs more LDS than a block may use");
     Ctx::Staging& S = c.stg[nt];
     S.ns = ns;
+    S.nh = hmax;
     S.lds = dyn;
-    if (hidx.empty()) hidx.push_back(0);
-    HIPCHK(S.hoff.upload(hoff.data(), hoff.size(), c.stream));
-    HIPCHK(S.hidx.upload(hidx.data(), hidx.size(), c.stream));
+    // every tile's list at the same stride, so that a block reads its indices without a look-up
+    std::vector<int> pad(std::max<size_t>(1, (size_t)ntiles * hmax), -1);
+    for (int t = 0; t < ntiles; t++) std::copy(hidx.begin() + hoff[t], hidx.begin() + hoff[t + 1], pad.begin() + (size_t)t * hmax);
+    HIPCHK(S.hidx.upload(pad.data(), pad.size(), c.stream));
     HIPCHK(S.snbl.upload(snbl.data(), snbl.size(), c.stream));
     HIPCHK(hipStreamSynchronize(c.stream));
+    return 0;
+}
+
+template <int P, bool MET>
+int launch_stage_split(Ctx& c, const StageArgs& a, int grid, size_t lds, bool sph, bool fuse) {
+    const dim3 b(4 * SPLIT_NT);
+    if (sph) {
+        if (fuse) hipLaunchKernelGGL((stage_split_kernel<P, true, true, MET>), dim3(grid), b, lds, c.stream, a);
+        else hipLaunchKernelGGL((stage_split_kernel<P, true, false, MET>), dim3(grid), b, lds, c.stream, a);
+    } else {
+        if (fuse) hipLaunchKernelGGL((stage_split_kernel<P, false, true, MET>), dim3(grid), b, lds, c.stream, a);
+        else hipLaunchKernelGGL((stage_split_kernel<P, false, false, MET>), dim3(grid), b, lds, c.stream, a);
+    }
     return 0;
 }
 
@@ -1092,13 +1141,15 @@ int launch_stage_v(Ctx& c, const StageArgs& a0, bool sph, bool fuse) {
     auto it = c.stg.find(NT);
     if (it == c.stg.end()) return fail("internal: stage kernel staging not built for this block size");
     StageArgs a = a0;
-    a.hoff = it->second.hoff.p; a.hidx = it->second.hidx.p; a.snbl = it->second.snbl.p; a.ns = it->second.ns;
+    a.hidx = it->second.hidx.p; a.snbl = it->second.snbl.p; a.nh = it->second.nh; a.ns = it->second.ns;
     const size_t lds = it->second.lds;
     // every pointer the variant dereferences must be set (a missing one is an error, not a launch)
     if (MET && (!a.mt.row || !a.mt.cd || !a.mt.wm || !a.mt.wx || !a.mt.wy || !a.mt.prn || !a.fo.ramp))
         return fail("internal: NWS=8 stage launch without its forcing arguments");
-    if (!a.uin || !a.uout || !a.wd_in || !a.hoff || !a.hidx || !a.snbl)
+    if (!a.uin || !a.uout || !a.wd_in || !a.hidx || !a.snbl)
         return fail("internal: stage launch with a missing buffer");
+    if constexpr (NL && NT == SPLIT_NT)
+        if (stage_split(c)) return launch_stage_split<P, MET>(c, a, grid, lds, sph, fuse);
     if (sph) {
         if (fuse) hipLaunchKernelGGL((stage_kernel<P, NT, true, true, MET, NL>), dim3(grid), dim3(NT), lds, c.stream, a);
         else hipLaunchKernelGGL((stage_kernel<P, NT, true, false, MET, NL>), dim3(grid), dim3(NT), lds, c.stream, a);
@@ -1157,7 +1208,7 @@ bool valid_block(int p, int nt) {
 
 template <int P>
 int launch_stage_nt(Ctx& c, const StageArgs& a, bool sph, bool fuse, int nt) {
-    if (nt == 64) return launch_stage<P, 64>(c, a, sph, fuse);
+    if (stage_nt(c, nt) == 64) return launch_stage<P, 64>(c, a, sph, fuse);
     if constexpr (P == 1) {
         if (nt == 128) return launch_stage<P, 128>(c, a, sph, fuse);
         return launch_stage<P, 256>(c, a, sph, fuse);
@@ -1189,6 +1240,7 @@ StageArgs stage_args(Ctx& c, int irk, const int slot[], bool captured = false) {
     a.wd_active = c.wd_active;
     a.tip = c.tip ? c.tip2.p + (size_t)irk * c.np : nullptr;
     a.cmout = cmean_out(c);
+    a.mid = c.mid;
     return a;
 }
 
@@ -1328,6 +1380,7 @@ int launch_step_explicit(Ctx& c, double* const* st, double* const* wsave = nullp
         a.wd_active = c.wd_active;
         a.tip = c.tip ? c.tip2.p + (size_t)irk * c.np : nullptr;
         a.cmout = cmean_out(c);
+        a.mid = c.mid;
         if (fsave) HIPCHK(hipMemcpyAsync(fsave[irk], c.wd[c.wdcur].p, c.ne, hipMemcpyDeviceToDevice, c.stream));
         if (launch_stage_nt<P>(c, a, sph, fuse, c.block)) return 1;
         HIPCHK(hipGetLastError());
@@ -1404,7 +1457,7 @@ int launch_adj_nl(Ctx& c, const AdjArgs& a0) {
     auto it = c.stg.find(NT);
     if (it == c.stg.end()) return fail("internal: adjoint staging not built for this block size");
     AdjArgs a = a0;
-    a.hoff = it->second.hoff.p; a.hidx = it->second.hidx.p; a.snbl = it->second.snbl.p; a.ns = it->second.ns;
+    a.hidx = it->second.hidx.p; a.snbl = it->second.snbl.p; a.nh = it->second.nh; a.ns = it->second.ns;
     const size_t lds = adj_dynamic_lds(c.dof, it->second.ns);
     if (a.met && (!a.mt.cd || !a.mt.wm || !a.mt.wx || !a.mt.wy || !a.mt.prn || !a.fo.ramp))
         return fail("internal: NWS=8 adjoint launch without its forcing arguments");
@@ -2381,7 +2434,10 @@ int dg_gpu_autotune(int h, int* block) {
     StageArgs a = stage_args(*c, 0, slot);
     a.rout = nullptr;
     const bool sph = c->prm.ics == 2, fuse = c->prm.nolifa >= 2 && c->prm.slopeflag == 0;
-    const std::vector<int> cand = c->prm.p == 1 ? std::vector<int>{64, 128, 256} : std::vector<int>{64, 128};
+    // candidates: stage_kernel at every block size and, for the nonlinear equations, stage_split_kernel (0)
+    std::vector<int> cand = c->prm.p == 1 ? std::vector<int>{64, 128, 256} : std::vector<int>{64, 128};
+    if (c->prm.nolicat != 0) cand.push_back(0);
+    const int block0 = c->block, split0 = stage_split(*c) ? 1 : 0, keep = c->split;
     if (build_stage_tables(*c, c->next_it, 1)) return 1;
     if (launch_forcing(*c, false)) return 1;
     if (c->met) {
@@ -2393,8 +2449,10 @@ int dg_gpu_autotune(int h, int* block) {
     HIPCHK(hipEventCreate(&e0));
     if (hipEventCreate(&e1) != hipSuccess) { (void)hipEventDestroy(e0); return fail("hipEventCreate failed"); }
     float best = 1e30f;
-    int best_nt = c->block, rc = 0;
-    for (int nt : cand) {
+    int best_nt = c->block, best_split = split0, rc = 0;
+    for (int cd : cand) {
+        const int nt = cd ? cd : SPLIT_NT;
+        c->split = cd ? 0 : 1;
         if (ensure_staging(*c, stage_nt(*c, nt))) continue;   // does not fit: not a candidate
         float ms = 0.f;
         for (int rep = 0; rep < 2 && !rc; rep++) {   // the first pass warms caches and code
@@ -2411,15 +2469,14 @@ int dg_gpu_autotune(int h, int* block) {
             if (e != hipSuccess) rc = fail(std::string("autotune: ") + hipGetErrorString(e));
         }
         if (rc) break;
-        if (ms < best) { best = ms; best_nt = nt; }
+        if (ms < best) { best = ms; best_nt = nt; best_split = c->split; }
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    if (rc) return rc;
-    if (best_nt != c->block) {
-        c->block = best_nt;
-        c->drop_graphs();
-    }
+    if (rc) { c->split = keep; return rc; }
+    c->block = best_nt;
+    c->split = best_split;
+    if (best_nt != block0 || best_split != split0) c->drop_graphs();
     if (block) *block = best_nt;
     return 0;
 }
@@ -2430,8 +2487,10 @@ int dg_gpu_set_block(int h, int block) {
     if (!valid_block(c->prm.p, block))
         return fail("block size must be 64, 128 or, for p=1, 256 threads");
     HIPCHK(hipStreamSynchronize(c->stream));
-    if (ensure_staging(*c, stage_nt(*c, block))) return 1;
-    if (block != c->block) { c->block = block; c->drop_graphs(); }
+    if (ensure_staging(*c, c->prm.nolicat != 0 ? block : 64)) return 1;
+    if (block != c->block || stage_split(*c)) c->drop_graphs();
+    c->block = block;
+    c->split = 0;
     return 0;
 }
 

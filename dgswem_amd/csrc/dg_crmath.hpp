@@ -143,33 +143,51 @@ DG_CRM_FN double cr_cos(double x) {
     return (q == 1 || q == 2) ? -res : res;
 }
 
-// Correctly rounded x**y for y = 1/3 rounded to a double (0x1.5555555555555p-2), for positive x
-// in [2^-1000, 2^1000]: x**y = x**(1/3) * x**(-d) with d = 1/3 - y = 2^-54/3.  The cube root is
-// refined to double-double by one Newton step from the library's cbrt, and the second factor is
-// 1 - d*ln(x) to 2^-110.  The correction terms need only modest accuracy (the Newton quotient
-// 2^-45 relative, ln(x) 2^-20 absolute: their errors enter at 2^-97 and 2^-75 of the result), so
-// they are formed in single precision: on the device from the hardware's approximate reciprocal
-// and base-2 logarithm (about 1 ulp each), ln(x) as ln(2) * (exponent + log2(significand)).
-// Outside that range as pow: +0 for +-0, NaN for negative x; the library's cube root otherwise.
+// Correctly rounded x**y for y = 1/3 rounded to a double (0x1.5555555555555p-2), for positive finite x:
+// x = 2^3k m with m in [1/2, 4), x**y = 2^k * m**(1/3) * x**(-d) with d = 1/3 - y = 2^-54/3.  The cube
+// root of m is refined to double-double by one Newton step from c0, and the last factor is 1 - d*ln(x) to
+// 2^-105.  c0 is itself one Newton step from exp2(log2(m)/3) in single precision (good to about 2^-22), so
+// it is good to about 2^-42 and the result before its rounding to about 2^-83.  The correction terms need
+// only modest accuracy (the Newton quotient 2^-40 relative; ln(x) 2^-14 absolute at the largest exponents,
+// entering at 2^-68 of the result, 2^-74 for depths of water), so they start from single precision: on
+// the device from the hardware's approximate reciprocal and base-2 exponential and logarithm (about 1 ulp
+// each).  Other x as pow: +0 for +-0, NaN for negative x, +infinity and NaN kept.
 DG_CRM_FN double cr_pow_third(double x) {
-    const double c0 = std::cbrt(x);
-    if (!(x >= 0x1p-1000 && x <= 0x1p+1000)) return x < 0.0 ? (x - x) / (x - x) : (x == 0.0 ? 0.0 : c0);
+    if (!(x > 0.0 && x < __builtin_inf())) return x < 0.0 ? (x - x) / (x - x) : std::fabs(x);
+#if defined(__HIP_DEVICE_COMPILE__)
+    const int ex = __builtin_amdgcn_frexp_exp(x);
+#else
+    int ex;
+    (void)std::frexp(x, &ex);
+#endif
+    const int k = (ex * 21846) >> 16;                      // floor(ex/3) for |ex| < 2^14
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double m = __builtin_amdgcn_ldexp(x, -3 * k);
+    const float l2 = __builtin_amdgcn_logf((float)m);
+    const double y = (double)__builtin_amdgcn_exp2f(l2 * 0x1.555556p-2f);
+    const double y2 = y * y;
+    double r = (double)__builtin_amdgcn_rcpf((float)(3.0 * y2));
+#else
+    const double m = std::ldexp(x, -3 * k);
+    const float l2 = std::log2((float)m);
+    const double y = (double)std::exp2(l2 * 0x1.555556p-2f);
+    const double y2 = y * y;
+    double r = (double)(1.0f / (float)(3.0 * y2));
+#endif
+    const double eps = (double)(l2 + (float)(3 * k)) * (0.6931471805599453 * 0x1.5555555555555p-56);   // ln(x) * 2^-54 / 3
+    const double c0 = y - std::fma(y2, y, -m) * r;
     const dd s = two_prod(c0, c0);
     const dd t = two_prod(c0, s.hi);
-    const double e = (t.hi - x) + (t.lo + c0 * s.lo);     // c0^3 - x (t.hi - x is exact)
+    const double e = (t.hi - m) + (t.lo + c0 * s.lo);     // c0^3 - m (t.hi - m is exact)
     const double a = 3.0 * s.hi;
+    r = r * (2.0 - a * r);                                 // 1/a to 2^-40
+    const double d = e * r;                                // Newton: cbrt(m) = c0 - d
+    const double res = c0 + (-d - c0 * eps);
 #if defined(__HIP_DEVICE_COMPILE__)
-    const float ra = __builtin_amdgcn_rcpf((float)a);
-    const float l2 = (float)__builtin_amdgcn_frexp_exp(x) + __builtin_amdgcn_logf((float)__builtin_amdgcn_frexp_mant(x));
-    const double eps = (double)l2 * (0.6931471805599453 * 0x1.5555555555555p-56);   // ln(x) * 2^-54 / 3
+    return __builtin_amdgcn_ldexp(res, k);
 #else
-    const float ra = 1.0f / (float)a;
-    const double eps = (double)std::log((float)x) * 0x1.5555555555555p-56;         // ln(x) * 2^-54 / 3
+    return std::ldexp(res, k);
 #endif
-    double r = (double)ra;
-    r = r * (2.0 - a * r);                                 // 1/a to 2^-46
-    const double d = e * r;                                // Newton: cbrt(x) = c0 - d
-    return c0 + (-d - c0 * eps);
 }
 
 }  // namespace crm

@@ -40,6 +40,16 @@ struct DevTables {
     double psi[KMAXAGP][3];   // linear nodal basis at the area points (wind stress interpolation)
 };
 
+// The p=1 area rule's values (RefTables' to the last bit, checked at set-up), as constants for unrolled code:
+// basis values, M_INV*WAGP (the same at every point) and its products with the basis values.
+struct P1Area {
+    static constexpr double phi[3][3] = {{1.0, 1.0, 0.0}, {1.0, -0.5, 0x1.0000000000001p-1}, {1.0, -0.5, -0x1.0000000000001p-1}};
+    static constexpr double mw[3] = {0x1.5555555555555p-2, 0x1.5555555555555p-1, 2.0};
+    static constexpr double srfac[3][3] = {{0x1.5555555555555p-2, 0x1.5555555555555p-1, 0.0},
+                                           {0x1.5555555555555p-2, -0x1.5555555555555p-2, 0x1.0000000000001p+0},
+                                           {0x1.5555555555555p-2, -0x1.5555555555555p-2, -0x1.0000000000001p+0}};
+};
+
 // Physics switches and constants shared by every scenario of a batch
 // (src/dgswem.F:131-170 derivations).
 struct Phys {
@@ -260,6 +270,63 @@ __device__ __forceinline__ void llf_flux_nl(double ze_in, double ze_ex, double q
     f0 = a1 - 0.5 * em * (j1);
     f1 = a2 - 0.5 * em * (j2);
     f2 = a3 - 0.5 * em * (j3);
+}
+
+// 1/x for x in [2^-500, 2^500], correctly rounded: the Newton steps and the final correction of the
+// IEEE division without its scaling of extreme operands and its fix-up of zeros and infinities (7
+// instructions instead of 11).
+__device__ __forceinline__ double recip_mid(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+    r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+    return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+}
+
+// sqrt(x) for x in [2^-700, 2^700], correctly rounded: the Goldschmidt steps and two corrections of the
+// IEEE square root without its scaling of small operands and its selection of zeros and infinities
+// (10 instructions instead of 19).
+__device__ __forceinline__ double sqrt_mid(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, r, g);
+    h = __builtin_fma(h, r, h);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
+
+// High word of a depth, offset so that one unsigned comparison with DEPTH_SPAN tells whether it lies in
+// [2^-500, 2^500), where recip_mid and sqrt_mid apply (negative values, zero and NaN lie outside).
+constexpr uint32_t DEPTH_SPAN = 1000u << 20;
+__device__ __forceinline__ uint32_t depth_key(double h) { return (uint32_t)__double2hiint(h) - ((1023u - 500u) << 20); }
+
+// Twice llf_flux_nl's fluxes, the same bits, for depths ht in recip_mid's range and K = NY^2+(NX*SF)^2 such
+// that G*ht*K is in sqrt_mid's.  Where the operations differ from llf_flux_nl's:
+//   * multiplications by 0.5 are exact, so they move into the edge weight;
+//   * 0.5*z is exact, so 0.5*z + h is one fused operation;
+//   * c >= 0, so the largest of |un+c|, |un|, |un-c| is |un|+c (rounding is monotonic and symmetric).
+__device__ __forceinline__ void llf_flux_nl2(double ze_in, double ze_ex, double qx_in, double qx_ex, double qy_in,
+                                             double qy_ex, double hb_in, double hb_ex, double ht_in, double ht_ex,
+                                             double sf_in, double sf_ex, double K_in, double K_ex, double nx, double ny,
+                                             double G, double& f0, double& f1, double& f2) {
+    const double j1 = ze_ex - ze_in, j2 = qx_ex - qx_in, j3 = qy_ex - qy_in;
+    double fh = recip_mid(ht_in);
+    const double u_in = qx_in * fh, v_in = qy_in * fh;
+    double huu = qx_in * u_in, hvv = qy_in * v_in, huv = qx_in * v_in;
+    double gh2 = G * ze_in * __builtin_fma(0.5, ze_in, hb_in);
+    const double fx1_in = qx_in * sf_in, fx2_in = (huu + gh2) * sf_in, fy2_in = huv;
+    const double fx3_in = huv * sf_in, fy3_in = hvv + gh2;
+    fh = recip_mid(ht_ex);
+    const double u_ex = qx_ex * fh, v_ex = qy_ex * fh;
+    huu = qx_ex * u_ex; hvv = qy_ex * v_ex; huv = qx_ex * v_ex;
+    gh2 = G * ze_ex * __builtin_fma(0.5, ze_ex, hb_ex);
+    const double fx1_ex = qx_ex * sf_ex, fx2_ex = (huu + gh2) * sf_ex, fy2_ex = huv;
+    const double fx3_ex = huv * sf_ex, fy3_ex = hvv + gh2;
+    const double un_in = u_in * nx + v_in * ny, un_ex = u_ex * nx + v_ex * ny;
+    const double em = fmax(fabs(un_in) + sqrt_mid(G * ht_in * K_in), fabs(un_ex) + sqrt_mid(G * ht_ex * K_ex));
+    f0 = (fx1_in + fx1_ex) * nx + (qy_in + qy_ex) * ny - em * j1;
+    f1 = (fx2_in + fx2_ex) * nx + (fy2_in + fy2_ex) * ny - em * j2;
+    f2 = (fx3_in + fx3_ex) * nx + (fy3_in + fy3_ex) * ny - em * j3;
 }
 
 template <bool NL>

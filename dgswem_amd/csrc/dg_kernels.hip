@@ -6,7 +6,7 @@
 //                    (when the slope limiter is off) the element's wet/dry correction.  Internal
 //                    edge fluxes are evaluated by both neighbours with the same operands in the same
 //                    order, so both see bit-identical values and no scatter or atomics are needed.
-//   node_minmax      one thread per node: min/max of the updated cell means over incident elements
+//                    Small meshes run stage_split_kernel, four waves per 64 elements, instead.
 //   limit_wetdry     one thread per element: SLOPELIMITER5 on modes 2-3, then WETDRY
 // preceded once per step by tide_kernel (the tidal boundary terms of every stage) and, with NWS=8,
 // met_kernel (the Holland profile at the nodes); plus modal2nodal (one thread per node) on output
@@ -52,14 +52,15 @@ struct StageArgs {
     double* __restrict__ rout;           // RHS(IRK) kept for later stages, or nullptr
     int irk;                             // stage index
     // block-local staging: tile t (elements [t*NT, t*NT+NT)) stages its elements and its halo
-    // hidx[hoff[t]..hoff[t+1]) in LDS; snbl packs each side's local neighbour index (10 bits each)
-    const int* __restrict__ hoff;
+    // hidx[t*nh..t*nh+nh) (-1 past the tile's last) in LDS; snbl packs each side's local neighbour
+    // index (10 bits each)
     const int* __restrict__ hidx;
     const int* __restrict__ snbl;
-    int ns;                              // staged elements per block (LDS row length)
+    int nh, ns;                          // halo entries per tile, staged elements per block (LDS row length)
     int* __restrict__ wd_active;         // set to 1 when WETDRY changes an element, or nullptr
     const double* __restrict__ tip;      // TIP2 of this stage at the nodes (tidal potential), or nullptr
     double* __restrict__ cmout;          // copy of the output cell means [3][ne] for the limiter, or nullptr
+    int mid;                             // G and the spherical factors allow llf_flux_nl2 (depths permitting)
 };
 
 // ------------------------------------------------------------------------------------------
@@ -265,18 +266,485 @@ __device__ __forceinline__ double trace1(const double (&u)[DOF], const double* p
     return s;
 }
 
+// Element i of a row, addressed as the row's (uniform) base plus a 32-bit byte offset: the form in which
+// the base stays in scalar registers.  Batches hold fewer than 2^29 elements, so the offset fits.
+template <typename T>
+__device__ __forceinline__ T& at(T* row, int i) {
+    return *reinterpret_cast<T*>(reinterpret_cast<char*>(const_cast<std::remove_const_t<T>*>(row)) + (uint32_t)i * (uint32_t)sizeof(T));
+}
+
+// The same value, opaque to the optimiser: what is addressed by it is read where it is used and not
+// kept in registers over a loop.
+__device__ __forceinline__ int reread(int j) {
+    asm volatile("" : "+v"(j));
+    return j;
+}
+
+// s + u*ph with ph an edge value of a p=1 mode: 0 or a power of two (checked at set-up), so the product is
+// exact and one fused operation gives the two roundings' result.  At p=2 product and sum round apart.
+template <int DOF>
+__device__ __forceinline__ double edge_term(double s, double u, double ph) {
+    return DOF == 3 ? __builtin_fma(u, ph, s) : s + u * ph;
+}
+
+// The staged element j's traces (elevation, the two discharges, bathymetry) at an edge point with
+// basis values ph; PHI_EDGE of mode 1 is 1 (checked at set-up), so the sums start at mode 1.
+template <int DOF>
+__device__ __forceinline__ void edge_point(const double* stg, int ns, int j, const double* ph, double (&t)[4]) {
+#pragma unroll
+    for (int f = 0; f < 4; f++) {
+        t[f] = stg[f * DOF * ns + j];
+#pragma unroll
+        for (int k = 1; k < (f < 3 ? DOF : 3); k++) t[f] = edge_term<DOF>(t[f], stg[(f * DOF + k) * ns + j], ph[k]);
+    }
+}
+
+// The same at every point of an edge with the basis table tb, `rev`: the points in reverse.
+template <int DOF, int NEGP>
+__device__ __forceinline__ void edge_traces(const double* stg, int ns, int j, const double (*tb)[DOF], bool rev,
+                                            double (&t)[4][NEGP]) {
+    double V[3][DOF], hb[3];
+#pragma unroll
+    for (int f = 0; f < 3; f++)
+#pragma unroll
+        for (int k = 0; k < DOF; k++) V[f][k] = stg[(f * DOF + k) * ns + j];
+#pragma unroll
+    for (int m = 0; m < 3; m++) hb[m] = stg[(3 * DOF + m) * ns + j];
+#pragma unroll
+    for (int I = 0; I < NEGP; I++) {
+        const double* ph = tb[rev ? NEGP - 1 - I : I];
+#pragma unroll
+        for (int f = 0; f < 3; f++) {
+            t[f][I] = V[f][0];
+#pragma unroll
+            for (int k = 1; k < DOF; k++) t[f][I] = edge_term<DOF>(t[f][I], V[f][k], ph[k]);
+        }
+        t[3][I] = edge_term<DOF>(edge_term<DOF>(hb[0], hb[1], ph[1]), hb[2], ph[2]);
+    }
+}
+
+// The tile's edge basis and edge quadrature tables in LDS: they are indexed by each lane's own local
+// edge number, and read as divergent constant-memory loads they would put a memory latency into
+// every point.
+template <int DOF, int NEGP>
+struct EdgeTables {
+    double pe[3][NEGP][DOF], eq[3][NEGP][DOF];
+};
+
+template <int DOF, int NEGP>
+__device__ __forceinline__ void load_edge_tables(const DevTables& T, EdgeTables<DOF, NEGP>& t, int tid, int nt) {
+    for (int j = tid; j < 3 * NEGP * DOF; j += nt) {
+        const int l = j / (NEGP * DOF), g = (j / DOF) % NEGP, k = j % DOF;
+        t.pe[l][g][k] = T.phi_edge[l][g][k];
+        t.eq[l][g][k] = T.edgeq[l][g][k];
+    }
+}
+
+// One internal side (slot `slot`) of staged element `le`: its RHS terms, summed over the side's points
+// (INTERNAL_EDGE_HYDRO + add_internal_flux).  acc is set.
+template <int P, bool SPH, bool NL, int DRYU>
+__device__ __forceinline__ void internal_side(const StageArgs& a, const EdgeTables<(P + 1) * (P + 2) / 2, P + 2>& tb,
+                                              const double* stg, const uint8_t* stwd, int ne, int ec, int le, int slot,
+                                              int bits, int sl, int wd, double nx, double ny, double edfac,
+                                              double (&acc)[3][(P + 1) * (P + 2) / 2]) {
+    constexpr int DOF = (P + 1) * (P + 2) / 2, NEGP = P + 2;
+    const ElemData& E = a.ed;
+    const Phys& ph = a.ph;
+    const int ns = a.ns;
+    const int L = bits & 3, role = (bits >> 2) & 1, nled = (bits >> 5) & 3;
+    const int ln = (sl >> (10 * slot)) & 1023;
+    const int wdn = stwd[ln];
+#pragma unroll
+    for (int f = 0; f < 3; f++)
+#pragma unroll
+        for (int k = 0; k < DOF; k++) acc[f][k] = 0.0;
+    if (wd == 0 && wdn == 0) return;
+    // the edge's "in" (NEDEL(1)) and "ex" (NEDEL(2)) elements as staged rows and their local edge numbers
+    const int si0 = role ? ln : le, sx0 = role ? le : ln;
+    const int Li = role ? nled : L, Lx = role ? L : nled;
+    // the "in" side subtracts w*F and the "ex" side adds it; -(a*b) == (-a)*b exactly, so the sign
+    // goes on the edge factor once and one update serves both roles
+    const double edfs = role ? edfac : -edfac;
+    // spherical factors of both sides at every point, loaded together
+    double sfi[NEGP], sfx[NEGP];
+#pragma unroll
+    for (int I = 0; I < NEGP; I++) {
+        sfi[I] = SPH ? at(E.sfs + ((size_t)((role ? 3 : 0) + slot) * NEGP + I) * ne, ec) : 1.0;
+        sfx[I] = SPH ? at(E.sfs + ((size_t)((role ? 0 : 3) + slot) * NEGP + I) * ne, ec) : 1.0;
+    }
+    double F[3][NEGP];                   // twice the flux
+    bool mid = NL && a.mid;
+    {
+        // the traces of one side after the other, so that only one side's modes are held
+        double ti[4][NEGP], tx[4][NEGP];
+        edge_traces<DOF, NEGP>(stg, ns, si0, tb.pe[Li], false, ti);
+        edge_traces<DOF, NEGP>(stg, ns, sx0, tb.pe[Lx], true, tx);
+        if constexpr (NL) {
+            double Ki = 0.0, Kx = 0.0;
+            uint32_t key = 0;
+#pragma unroll
+            for (int I = 0; I < NEGP; I++) {
+                const double hi = ti[0][I] + ti[3][I], hx = tx[0][I] + tx[3][I];
+                key = max(key, max(depth_key(hi), depth_key(hx)));
+                if (SPH || I == 0) {
+                    const double ni = nx * sfi[I], ne_ = nx * sfx[I];
+                    Ki = ny * ny + ni * ni;
+                    Kx = ny * ny + ne_ * ne_;
+                }
+                llf_flux_nl2(ti[0][I], tx[0][I], ti[1][I], tx[1][I], ti[2][I], tx[2][I], ti[3][I], tx[3][I], hi, hx,
+                             sfi[I], sfx[I], Ki, Kx, nx, ny, ph.g, F[0][I], F[1][I], F[2][I]);
+            }
+            mid = mid && key < DEPTH_SPAN;
+        } else {
+#pragma unroll
+            for (int I = 0; I < NEGP; I++) {
+                llf<NL>(ph, ti[0][I], tx[0][I], ti[1][I], tx[1][I], ti[2][I], tx[2][I], ti[3][I], tx[3][I], sfi[I],
+                        sfx[I], nx, ny, ph.g, F[0][I], F[1][I], F[2][I]);
+#pragma unroll
+                for (int f = 0; f < 3; f++) F[f][I] = 2.0 * F[f][I];
+            }
+            mid = true;
+        }
+    }
+    if (!mid || wd == 0 || wdn == 0) {
+        // a depth outside llf_flux_nl2's range, or one side dry (few lanes, at the shoreline;
+        // src/internal_edge_hydro.F:212-302): 1 reflect into a dry "in" element, 2 zero-gravity flux for a
+        // dry "in", 3 reflect into a dry "ex", 4 zero-gravity flux for a dry "ex"; only what this element's
+        // side receives.  The traces are formed again from LDS: held over the fluxes above they would set
+        // the kernel's register count.
+        const int wd_in_el = role ? wdn : wd;
+#pragma unroll DRYU
+        for (int I = 0; I < NEGP; I++) {
+            double f0 = 0.0, f1 = 0.0, f2 = 0.0;
+            double si_ = 1.0, sx_ = 1.0;
+#pragma unroll
+            for (int j = 0; j < NEGP; j++)
+                if (j == I) { f0 = 0.5 * F[0][j]; f1 = 0.5 * F[1][j]; f2 = 0.5 * F[2][j]; si_ = sfi[j]; sx_ = sfx[j]; }
+            // the plain flux (where the range calls for it), then the dry-side case it selects
+            int mode = 0;
+#pragma unroll 1
+            for (int pass = mid ? 1 : 0; pass < 2; pass++) {
+                if (pass == 1) {
+                    if ((wd != 0 && wdn != 0) || !(fabs(f0) > 1.0e-8)) break;
+                    if (wd_in_el == 0) mode = (f0 > 0.0) ? 1 : (role ? 0 : 2);
+                    else mode = (f0 < 0.0) ? 3 : (role ? 4 : 0);
+                    if (mode == 0) break;
+                }
+                const double* pi_ = tb.pe[Li][I];
+                const double* px_ = tb.pe[Lx][NEGP - 1 - I];
+                const int si = reread(si0), sx = reread(sx0);
+                // reflection: the wet side's own state against its mirror image
+                const bool m1 = mode == 1, m3 = mode == 3;
+                double ti[4], te[4];
+                edge_point<DOF>(stg, ns, m1 ? sx : si, m1 ? px_ : pi_, ti);
+                edge_point<DOF>(stg, ns, m3 ? si : sx, m3 ? pi_ : px_, te);
+                const double sf_in = m1 ? sx_ : si_, sf_ex = m3 ? si_ : sx_;
+                if (m1 || m3) {
+                    const double tx = -ny, ty = nx;
+                    const double qn = ti[1] * nx + ti[2] * ny, qt = ti[1] * tx + ti[2] * ty;
+                    const double qnm = -qn, qtm = qt;
+                    const double den = (nx * ty - ny * tx);
+                    const double mqx = (ty * qnm - ny * qtm) / den;
+                    const double mqy = (-tx * qnm + nx * qtm) / den;
+                    ti[1] = m1 ? mqx : ti[1]; ti[2] = m1 ? mqy : ti[2];
+                    te[1] = m1 ? te[1] : mqx; te[2] = m1 ? te[2] : mqy;
+                }
+                double r0, r1, r2;
+                llf<NL>(ph, ti[0], te[0], ti[1], te[1], ti[2], te[2], ti[3], te[3], sf_in, sf_ex, nx, ny,
+                        mode == 2 || mode == 4 ? 0.0 : ph.g, r0, r1, r2);
+                // reflection: F0 and the wet side's momentum from the reflected flux, zero for the dry
+                // side; zero gravity: the momentum alone
+                const bool keep = m1 ? role != 0 : (m3 ? role == 0 : true);
+                f0 = mode == 2 || mode == 4 ? f0 : r0;
+                f1 = keep ? r1 : 0.0;
+                f2 = keep ? r2 : 0.0;
+            }
+#pragma unroll
+            for (int j = 0; j < NEGP; j++)
+                if (j == I) { F[0][j] = 2.0 * f0; F[1][j] = 2.0 * f1; F[2][j] = 2.0 * f2; }
+        }
+    }
+    const double edh = 0.5 * edfs;       // F is twice the flux
+#pragma unroll
+    for (int I = 0; I < NEGP; I++) {
+        const double* eq = tb.eq[L][role ? NEGP - 1 - I : I];
+#pragma unroll
+        for (int k = 0; k < DOF; k++) {
+            // the sums start from zero: 0 + x == x for every x but -0, so the first point's terms
+            // start them
+            const double ws = edh * eq[k];
+#pragma unroll
+            for (int f = 0; f < 3; f++) acc[f][k] = I == 0 ? ws * F[f][I] : acc[f][k] + ws * F[f][I];
+        }
+    }
+}
+
+// Number of an element's boundary sides: they are its first slots.
+__device__ __forceinline__ int boundary_slots(int info) {
+    return (((info >> 3) & 3) != SIDE_INTERNAL) + (((info >> 10) & 3) != SIDE_INTERNAL) + (((info >> 17) & 3) != SIDE_INTERNAL);
+}
+
+// The boundary sides (slots 0..nbd-1) of a wet element: their RHS terms accumulate point after point, as
+// the reference's boundary routines do.  acc is set.
+template <int P, bool SPH, bool NL>
+__device__ __forceinline__ void boundary_sides(const StageArgs& a, const DevTables& T,
+                                               const EdgeTables<(P + 1) * (P + 2) / 2, P + 2>& tb, const double* stg,
+                                               int ne, int ec, int le, int info, int nbd, double h0,
+                                               double (&acc)[3][(P + 1) * (P + 2) / 2]) {
+    constexpr int DOF = (P + 1) * (P + 2) / 2, NEGP = P + 2;
+    const ElemData& E = a.ed;
+    const Phys& ph = a.ph;
+#pragma unroll
+    for (int f = 0; f < 3; f++)
+#pragma unroll
+        for (int k = 0; k < DOF; k++) acc[f][k] = 0.0;
+#pragma unroll 1
+    for (int s = 0; s < nbd; s++) {
+        const int bits = side_bits(info, s);
+        const int L = bits & 3, role = (bits >> 2) & 1, kind = (bits >> 3) & 3;
+        const int nb = at(E.snbr + (size_t)s * ne, ec);
+        const double nx = at(E.geo + (size_t)(3 * s) * ne, ec), ny = at(E.geo + (size_t)(3 * s + 1) * ne, ec);
+        const double tx = -ny, ty = nx;
+        double xlen, AREAS;
+        side_xlen_areas(E, ne, ec, L, role, xlen, AREAS);
+#pragma unroll 1
+        for (int I = 0; I < NEGP; I++) {
+            const double* pv = tb.pe[L][I];
+            double t[4];
+            edge_point<DOF>(stg, a.ns, reread(le), pv, t);
+            const double ze_in = t[0], qx_in = t[1], qy_in = t[2], hb_in = t[3];
+            const double sf = SPH ? at(E.sfs + ((size_t)s * NEGP + I) * ne, ec) : 1.0;
+            // exterior values: a land side mirrors the normal flow, an ocean side takes the prescribed
+            // elevation, a flux side the prescribed normal flow
+            double ze_ex = ze_in, qx_ex = qx_in, qy_ex = qy_in;
+            if (kind == SIDE_LAND) {
+                const double qn_int = qx_in * nx + qy_in * ny, qt_int = qx_in * tx + qy_in * ty;
+                const double qn_ext = -qn_int, qt_ext = qt_int;
+                const double den = 1.0 / (nx * ty - ny * tx);
+                qx_ex = (ty * qn_ext - ny * qt_ext) * den;
+                qy_ex = (-tx * qn_ext + nx * qt_ext) * den;
+            } else if (kind == SIDE_OCEAN) {
+                ze_ex = 0.0;
+                const double xe = T.xegp[I];
+                // the constituents' endpoint terms EMO*RFF*COS(ARGJ-EFA) of this stage (tide_kernel)
+                for (int jj = 0; jj < a.fo.nbfr; jj++) {
+                    const size_t o = ((size_t)nb * a.fo.nbfr + jj) * 2;
+                    const double z1 = a.fo.tz[(size_t)a.irk * a.fo.tzn + o];
+                    const double z2 = a.fo.tz[(size_t)a.irk * a.fo.tzn + o + 1];
+                    ze_ex = ze_ex + (0.5 * (z1 + z2) + 0.5 * (z2 - z1) * xe);
+                }
+                if ((ze_ex * ph.ifnlfa + hb_in) <= 0) ze_ex = fabs(hb_in) + h0;
+            } else {
+                // the specified normal flux at this point (flow_kernel); the reference forms the
+                // exterior momentum after every constituent, so the last, full sum is what counts
+                const double qn_ext = a.fo.fz[(size_t)a.irk * a.fo.fzn + (size_t)nb * NEGP + I];
+                const double qt_ext = 0.0;
+                qx_ex = -(ty * qn_ext - ny * qt_ext) / (nx * ty - ny * tx);
+                qy_ex = -(-tx * qn_ext + nx * qt_ext) / (nx * ty - ny * tx);
+            }
+            double f0, f1, f2;
+            llf<NL>(ph, ze_in, ze_ex, qx_in, qx_ex, qy_in, qy_ex, hb_in, hb_in, sf, sf, nx, ny, ph.g, f0, f1, f2);
+#pragma unroll
+            for (int k = 0; k < DOF; k++) {
+                const double w = 2.0 * T.m_inv[k] / AREAS * xlen * pv[k] * T.wegp[I];
+                acc[0][k] = acc[0][k] - w * f0;
+                acc[1][k] = acc[1][k] - w * f1;
+                acc[2][k] = acc[2][k] - w * f2;
+            }
+        }
+    }
+}
+
+// What an element's area points share.
+struct VolumeTerms {
+    double drdx, dsdx, drdy, dsdy;       // Jacobian
+    double dpx1, dpy1, dpx2, dpy2;       // gradients of the linear modes
+    double dhbx, dhby;                   // gradient of the P1 bathymetry
+    double mw[8];                        // MET: vertex wind stresses (x, then y), pressure gradient
+    double tdx, tdy, tramp;              // tidal potential gradient and ramp
+    double hybf;                         // hybrid friction factor
+    double cori, nbar;                   // Coriolis, element-mean Manning n
+    double cf, fric, dtdph;              // the scenario's CF, uniform friction and 1/DT
+};
+
+template <int P, bool MET, bool NL>
+__device__ __forceinline__ void volume_terms(const StageArgs& a, const DevTables& T, int ne, int ec, int sid, int row,
+                                             double ze1, const double hb[3], VolumeTerms& v) {
+    const ElemData& E = a.ed;
+    const Phys& ph = a.ph;
+    const double drpsi[3] = {-1.0 / 2.0, 1.0 / 2.0, 0.0}, dspsi[3] = {-1.0 / 2.0, 0.0, 1.0 / 2.0};
+    // wind stress at the element's vertices and the pressure gradient sums (MET)
+    if (MET) {
+        // nodal WSX2/WSY2/PR2 of this stage (src/met_forcing.F:507-509) and the QP-independent sums
+        // PR2(Ni)*DPSIDX(i) of src/rhs_dg_hydro.F:117-122,366-372
+        const double ramp = a.fo.ramp[(size_t)sid * a.fo.rows + row];
+        double pdx = 0.0, pdy = 0.0;
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const int n = at(E.nm + (size_t)i * ne, ec);
+            const double cd = a.mt.cd[n], wm = a.mt.wm[n];
+            v.mw[i] = ramp * 0.001293 * cd * a.mt.wx[n] * wm;
+            v.mw[3 + i] = ramp * 0.001293 * cd * a.mt.wy[n] * wm;
+            const double pr = ramp * a.mt.prn[n];
+            const double dpsidx = drpsi[i] * v.drdx + dspsi[i] * v.dsdx;
+            const double dpsidy = drpsi[i] * v.drdy + dspsi[i] * v.dsdy;
+            if (i == 0) { pdx = pr * dpsidx; pdy = pr * dpsidy; }
+            else { pdx = pdx + pr * dpsidx; pdy = pdy + pr * dpsidy; }
+        }
+        v.mw[6] = pdx;
+        v.mw[7] = pdy;
+    }
+    // tidal potential (src/rhs_dg_hydro.F:117-122,378-386): the sums DPSIDX(i)*TIP2(Ni) are the same
+    // at every area point; RAMPDG multiplies them once more at each point
+    v.tdx = 0.0; v.tdy = 0.0; v.tramp = 0.0;
+    if (a.tip) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const double tv = a.tip[at(E.nm + (size_t)i * ne, ec)];
+            const double dpsidx = drpsi[i] * v.drdx + dspsi[i] * v.dsdx;
+            const double dpsidy = drpsi[i] * v.drdy + dspsi[i] * v.dsdy;
+            if (i == 0) { v.tdx = dpsidx * tv; v.tdy = dpsidy * tv; }
+            else { v.tdx = v.tdx + dpsidx * tv; v.tdy = v.tdy + dpsidy * tv; }
+        }
+        v.tramp = a.fo.ramp[(size_t)sid * a.fo.rows + row];
+    }
+    // hybrid friction factor (1 + (HBREAK/H_c)^FTHETA)^(FGAMMA/FTHETA) from the element-mean depth
+    // (src/rhs_dg_hydro.F:306-309): the same at every area point, evaluated once and only when the
+    // hybrid law is on
+    v.hybf = 1.0;
+    if (ph.ifhybf == 1) {
+        const double depth_c = hb[0] + ze1;
+        const double fh_nl_c = NL ? 1.0 / depth_c : 1.0 / (ph.nleq * depth_c + ph.leq);
+        v.hybf = pow(1.0 + pow(ph.hbreak * fh_nl_c, ph.ftheta), ph.fgamma / ph.ftheta);
+    }
+    // gradients of the linear modes, whose reference derivatives are (0, 0), (0, 3/2), (1, 1/2) at every
+    // area point (checked at set-up): products by 0, 1 and 1/2 are exact, so the fused sum rounds as the
+    // separate one; with them the P1 bathymetry's gradient
+    v.dpx1 = 1.5 * v.dsdx; v.dpy1 = 1.5 * v.dsdy;
+    v.dpx2 = __builtin_fma(0.5, v.dsdx, v.drdx); v.dpy2 = __builtin_fma(0.5, v.dsdy, v.drdy);
+    v.dhbx = hb[1] * v.dpx1 + hb[2] * v.dpx2;
+    v.dhby = hb[1] * v.dpy1 + hb[2] * v.dpy2;
+}
+
+// Fluxes and sources of a wet element at area point I (RHS_DG_HYDRO): q = fx fy gx gy hx hy sx sy.
+template <int P, bool MET, bool NL>
+__device__ __forceinline__ void area_point(const StageArgs& a, const DevTables& T, int I,
+                                           const VolumeTerms& v, double ze, double qx, double qy, double hbq, double sfq,
+                                           int wd, double (&q)[8]) {
+    const Phys& ph = a.ph;
+    const double depth = ze + hbq;
+    // with NL (NLEQ = 1, LEQ = 0) the constant factors fold exactly
+    const double f1 = NL ? 1.0 : ph.nleq + ph.leq * hbq;
+    const double fx = NL ? qx * sfq : qx * f1 * sfq, fy = NL ? qy : qy * f1;
+    const double fu = NL ? qx : ph.nleq * qx, fv = NL ? qy : ph.nleq * qy;
+    const double fg = ph.nleqg * ze * wd;
+    const double fh = NL ? 1.0 / depth : 1.0 / (ph.nleq * depth + ph.leq);
+    const double u = qx * fh, w = qy * fh;
+    const double huu = fu * u, hvv = fv * w, huv = fu * w;
+    const double gh2 = NL ? fg * (0.5 * ze + hbq) : fg * (0.5 * ze + hbq) + ph.fg_l * ze;
+    double fric = v.fric;
+    if (ph.load_manning) {
+        // DEPTH**(1.D0/3.D0) (src/rhs_dg_hydro.F:302), correctly rounded
+        fric = ph.g * (v.nbar * v.nbar) / crm::cr_pow_third(depth);
+        if (fric < v.cf) fric = v.cf;
+    }
+    double tau = fric;
+    if (ph.iflinbf == 0) {
+        const double umag = sqrt(u * u + w * w);
+        tau = tau * umag * fh;
+        if (ph.ifhybf == 1) tau = tau * v.hybf;
+        const double cap = 0.9 * v.dtdph;
+        if (cap < tau) tau = cap;
+    }
+    double sx = -(tau * qx) + fg * v.dhbx * sfq + v.cori * qy;
+    double sy = -(tau * qy) + fg * v.dhby - v.cori * qx;
+    if (MET) {
+        // wind stress and atmospheric pressure (src/rhs_dg_hydro.F:362-373)
+        const double* ps = T.psi[I];
+        const double wsx = v.mw[0] * ps[0] + v.mw[1] * ps[1] + v.mw[2] * ps[2];
+        const double wsy = v.mw[3] * ps[0] + v.mw[4] * ps[1] + v.mw[5] * ps[2];
+        const double fw = 1.0 / f1;
+        sx = sx + (NL ? wsx : fw * wsx) - ph.g * sfq * depth * v.mw[6];
+        sy = sy + (NL ? wsy : fw * wsy) - ph.g * depth * v.mw[7];
+    }
+    if (a.tip) {
+        sx = sx + v.tramp * ph.g * depth * sfq * v.tdx;
+        sy = sy + v.tramp * ph.g * depth * v.tdy;
+    }
+    q[0] = fx; q[1] = fy;
+    q[2] = (huu + gh2) * sfq; q[3] = huv;
+    q[4] = huv * sfq; q[5] = hvv + gh2;
+    q[6] = sx; q[7] = sy;
+}
+
+// The staged element le's values at area point I (PHI_AREA of mode 1 is 1, checked at set-up, so the sums
+// start at mode 1).  At p=1 the point's values are compile-time constants; mode 2's are powers of two, whose
+// products are exact, so product and sum fuse without a change, and mode 3's is zero at the first point.
+template <int P>
+__device__ __forceinline__ void area_values(const DevTables& T, const double* stg, int ns, int le, int I, double (&t)[4]) {
+    constexpr int DOF = (P + 1) * (P + 2) / 2;
+#pragma unroll
+    for (int f = 0; f < 4; f++) {
+        t[f] = stg[f * DOF * ns + le];
+        if constexpr (P == 1) {
+            const double p1 = I == 0 ? P1Area::phi[0][1] : P1Area::phi[1][1];
+            const double p2 = I == 1 ? P1Area::phi[1][2] : P1Area::phi[2][2];
+            t[f] = __builtin_fma(stg[(f * DOF + 1) * ns + le], p1, t[f]);
+            if (I > 0) t[f] = t[f] + stg[(f * DOF + 2) * ns + le] * p2;
+        } else {
+#pragma unroll
+            for (int k = 1; k < (f < 3 ? DOF : 3); k++) t[f] = t[f] + stg[(f * DOF + k) * ns + le] * T.phi_area[I][k];
+        }
+    }
+}
+
+// One element's state and vertex depths.
+template <int DOF>
+__device__ __forceinline__ void load_entry(const double* __restrict__ u, const double* __restrict__ dpv, int ne, int g,
+                                           double (&v)[3 * DOF + 3]) {
+#pragma unroll
+    for (int f = 0; f < 3 * DOF; f++) v[f] = at(u + (size_t)f * ne, g);
+#pragma unroll
+    for (int m = 0; m < 3; m++) v[3 * DOF + m] = at(dpv + (size_t)m * ne, g);
+}
+
+// Stages one element: its state v[0..3*DOF), the P1 bathymetry modes formed from its vertex depths
+// v[3*DOF..], its wet/dry flag.
+template <int DOF>
+__device__ __forceinline__ void stage_entry(double* stg, uint8_t* stwd, int ns, int j, const double (&v)[3 * DOF + 3],
+                                            uint8_t w) {
+    const double c13 = 1.0 / 3.0, c16 = 1.0 / 6.0;
+#pragma unroll
+    for (int f = 0; f < 3 * DOF; f++) stg[f * ns + j] = v[f];
+    const double d0 = v[3 * DOF], d1 = v[3 * DOF + 1], d2 = v[3 * DOF + 2];
+    stg[(3 * DOF) * ns + j] = c13 * (d0 + d1 + d2);
+    stg[(3 * DOF + 1) * ns + j] = -(c16 * (d0 + d1)) + c13 * d2;
+    stg[(3 * DOF + 2) * ns + j] = -(0.5 * d0) + 0.5 * d1;
+    stwd[j] = w;
+}
+
+// One lane per element.  What bounds it: FP64 instruction issue (about 2240 VALU instructions per element at p=1,
+// a wave each 4 cycles; the reciprocals and inverse square roots of the fluxes 16) and the latency of three phases
+// of loads (staging, quadrature, RK base), which the other waves on the SIMD have to cover.  So registers, which
+// set how many waves there are, matter as much as instructions:
+//   * the rare paths (dry sides, boundary sides) read the modes from LDS again at every point instead of holding
+//     them, the side sums live in registers instead of LDS, and one side's traces are formed after the other's:
+//     166 registers at p=1 (226 before), three waves per SIMD instead of two; 251 at p=2 (293 and accumulator
+//     registers before), two instead of one;
+//   * the spherical p=1 variants would spill at three waves (94 us against 78 us per launch on 16 storm basins,
+//     438k elements), so they keep two;
+//   * loads go out early: a tile's halo indices lie at a fixed stride (no look-up first), the next side's geometry
+//     is loaded while a side is evaluated, the quadrature's data before the sides and the RK base before the
+//     quadrature (which stood still for two thirds of its time when its loads waited behind the RK base).
+// Time per launch, 997,306 elements, p=1, limiter and wet/dry: 133 us before, 100 us with these and the shorter
+// arithmetic of llf_flux_nl2 and cr_pow_third (35.0M VALU instructions instead of 44.8M); 298,700 elements, p=2:
+// 121 us before, 86 us.
 template <int P, int NT, bool SPH, bool WDFUSED, bool MET, bool NL>
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(P == 1 ? 2 : 1))) stage_kernel(StageArgs a) {
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(P == 1 && !SPH ? 3 : 2))) stage_kernel(StageArgs a) {
     constexpr int DOF = (P + 1) * (P + 2) / 2;
     constexpr int NAGP = (P == 1) ? 3 : 6;
     constexpr int NEGP = P + 2;
-    // per-thread accumulators kept in LDS to bound register use: [0] boundary-edge part of the
-    // RHS (accumulated first, like the reference's boundary edge routines), [1] internal-edge
-    // slot sum (add_internal_flux)
-    __shared__ double acc_lds[2][3 * DOF][NT];
-    // edge basis and edge quadrature tables: indexed by each lane's own local edge number, so
-    // read from LDS (short latency) rather than as divergent constant-memory loads
-    __shared__ double tpe[3][NEGP][DOF], teq[3][NEGP][DOF];
+    __shared__ EdgeTables<DOF, NEGP> tb;
     // staged states: rows [field*DOF + mode] then the three bathymetry modes, ns entries each, then
     // the wet/dry flags (bytes)
     extern __shared__ double stg[];
@@ -287,278 +755,99 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(P == 1 
     const int tid = threadIdx.x;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     const int e = tile * NT + tid;
-    const double c13 = 1.0 / 3.0, c16 = 1.0 / 6.0;
     const int ns = a.ns;
     uint8_t* const stwd = reinterpret_cast<uint8_t*>(stg + (size_t)(3 * DOF + 3) * ns);
-    for (int j = tid; j < 3 * NEGP * DOF; j += NT) {
-        const int l = j / (NEGP * DOF), g = (j / DOF) % NEGP, k = j % DOF;
-        tpe[l][g][k] = T.phi_edge[l][g][k];
-        teq[l][g][k] = T.edgeq[l][g][k];
-    }
+    load_edge_tables<DOF, NEGP>(T, tb, tid, NT);
     // per-element loads that do not depend on the staged data, issued before the staging loads so
     // that the latencies overlap (lanes past the last element read element ne-1 and exit after
     // the barrier)
     const int ec = e < ne ? e : ne - 1;
-    double G[9];                         // per slot NX, NY, XLEN/AREAS
-#pragma unroll
-    for (int j = 0; j < 9; j++) G[j] = E.geo[(size_t)j * ne + ec];
-    const int info = E.sinfo[ec];
-    const int nb0 = E.snbr[ec], nb1 = E.snbr[(size_t)ne + ec], nb2 = E.snbr[2 * (size_t)ne + ec];
-    const int sl = a.snbl[ec];
-    const int sid = E.sid ? (int)E.sid[ec] : 0;
-    const Scen sc = E.scen[sid];
-    const double cori = E.cori_el ? E.cori_el[ec] : sc.cori;
-    const double nbar = ph.load_manning ? E.nbar[ec] : 0.0;
+    // the first side's NX, NY, XLEN/AREAS; each further side's are loaded while the one before it is
+    // evaluated
+    double nx = at(E.geo, ec), ny = E.geo[(size_t)ne + ec], edfac = at(E.geo + (size_t)2 * ne, ec);
+    const int info = at(E.sinfo, ec);
+    const int sl = at(a.snbl, ec);
     {
-        // this tile's elements and its halo, two entries per lane per pass with all their loads
-        // issued before any is used
-        const int h0 = a.hoff[tile], nh = a.hoff[tile + 1] - h0;
-        for (int j = tid; j < NT + nh; j += 2 * NT) {
-            const int j2 = j + NT;
-            const bool has2 = j2 < NT + nh;
-            int g = j < NT ? tile * NT + j : a.hidx[h0 + j - NT];
-            int g2 = has2 ? a.hidx[h0 + j2 - NT] : ne;
-            const bool ok = g < ne, ok2 = g2 < ne;
-            g = ok ? g : 0;
-            g2 = ok2 ? g2 : 0;
-            double v[3 * DOF + 3], v2[3 * DOF + 3];
-#pragma unroll
-            for (int f = 0; f < 3 * DOF; f++) { v[f] = a.uin[(size_t)f * ne + g]; v2[f] = a.uin[(size_t)f * ne + g2]; }
-#pragma unroll
-            for (int m = 0; m < 3; m++) { v[3 * DOF + m] = E.dpv[(size_t)m * ne + g]; v2[3 * DOF + m] = E.dpv[(size_t)m * ne + g2]; }
-            const uint8_t w = a.wd_in[g], w2 = a.wd_in[g2];
-            if (ok) {
-#pragma unroll
-                for (int f = 0; f < 3 * DOF; f++) stg[f * ns + j] = v[f];
-                const double d0 = v[3 * DOF], d1 = v[3 * DOF + 1], d2 = v[3 * DOF + 2];
-                stg[(3 * DOF) * ns + j] = c13 * (d0 + d1 + d2);
-                stg[(3 * DOF + 1) * ns + j] = -(c16 * (d0 + d1)) + c13 * d2;
-                stg[(3 * DOF + 2) * ns + j] = -(0.5 * d0) + 0.5 * d1;
-                stwd[j] = w;
-            }
-            if (ok2) {
-#pragma unroll
-                for (int f = 0; f < 3 * DOF; f++) stg[f * ns + j2] = v2[f];
-                const double d0 = v2[3 * DOF], d1 = v2[3 * DOF + 1], d2 = v2[3 * DOF + 2];
-                stg[(3 * DOF) * ns + j2] = c13 * (d0 + d1 + d2);
-                stg[(3 * DOF + 1) * ns + j2] = -(c16 * (d0 + d1)) + c13 * d2;
-                stg[(3 * DOF + 2) * ns + j2] = -(0.5 * d0) + 0.5 * d1;
-                stwd[j2] = w2;
-            }
+        // this tile's elements and its halo: the first halo entry's index, then the tile's own loads, then
+        // the halo's, before any is used (a halo past NT entries is staged after them)
+        const int* hx = a.hidx + (size_t)tile * a.nh;
+        const int nh = a.nh;
+        const int g = tid < nh ? hx[tid] : -1;
+        double v[3 * DOF + 3], v2[3 * DOF + 3];
+        load_entry<DOF>(a.uin, E.dpv, ne, ec, v);
+        const uint8_t w = at(a.wd_in, ec);
+        const int gc = g < 0 ? 0 : g;
+        load_entry<DOF>(a.uin, E.dpv, ne, gc, v2);
+        const uint8_t w2 = at(a.wd_in, gc);
+        stage_entry<DOF>(stg, stwd, ns, tid, v, w);
+        if (g >= 0) stage_entry<DOF>(stg, stwd, ns, NT + tid, v2, w2);
+#pragma unroll 1
+        for (int h = tid + NT; h < nh; h += NT) {
+            const int gh = hx[h];
+            if (gh < 0) break;
+            load_entry<DOF>(a.uin, E.dpv, ne, gh, v);
+            stage_entry<DOF>(stg, stwd, ns, NT + h, v, at(a.wd_in, gh));
         }
     }
     __syncthreads();
     if (e >= ne) return;
     const int row = table_step(a.fo) * a.fo.nrk + a.irk;
-
     const int wd = stwd[tid];
-#pragma unroll
-    for (int j = 0; j < 3 * DOF; j++) { acc_lds[0][j][tid] = 0.0; acc_lds[1][j][tid] = 0.0; }
+    const int sid = E.sid ? (int)at(E.sid, e) : 0;
 
-#pragma unroll 1
-    for (int slot = 0; slot < 3; slot++) {
-        const int bits = side_bits(info, slot);
-        const int L = bits & 3, role = (bits >> 2) & 1, kind = (bits >> 3) & 3, nled = (bits >> 5) & 3;
-        const int nb = slot == 0 ? nb0 : (slot == 1 ? nb1 : nb2);
-        // edge geometry in the reference's node order (the counter-clockwise order of NEDEL(1))
-        const double nx = slot == 0 ? G[0] : (slot == 1 ? G[3] : G[6]);
-        const double ny = slot == 0 ? G[1] : (slot == 1 ? G[4] : G[7]);
-        const double edfac = slot == 0 ? G[2] : (slot == 1 ? G[5] : G[8]);
-        const double tx = -ny, ty = nx;
-        if (kind == SIDE_INTERNAL) {
-            const int ln = (sl >> (10 * slot)) & 1023;
-            const int wdn = stwd[ln];
-            if (wd == 0 && wdn == 0) continue;
-            // the edge's "in" (NEDEL(1)) and "ex" (NEDEL(2)) elements as staged rows, their local
-            // edge numbers and wet/dry flags: the traces are formed in in/ex order directly
-            const int si = role ? ln : tid, sx = role ? tid : ln;
-            const int Li = role ? nled : L, Lx = role ? L : nled;
-            double Vi[3][DOF], Vx[3][DOF], hbi[3], hbx[3];
-#pragma unroll
-            for (int f = 0; f < 3; f++)
-#pragma unroll
-                for (int k = 0; k < DOF; k++) {
-                    Vi[f][k] = stg[(f * DOF + k) * ns + si];
-                    Vx[f][k] = stg[(f * DOF + k) * ns + sx];
-                }
-#pragma unroll
-            for (int m = 0; m < 3; m++) {
-                hbi[m] = stg[(3 * DOF + m) * ns + si];
-                hbx[m] = stg[(3 * DOF + m) * ns + sx];
-            }
-            const int wd_in_el = role ? wdn : wd, wd_ex_el = role ? wd : wdn;
-            // spherical factors of both sides at every point, loaded together
-            double sfi[NEGP], sfx[NEGP];
-#pragma unroll
-            for (int I = 0; I < NEGP; I++) {
-                sfi[I] = 1.0;
-                sfx[I] = 1.0;
-                if (SPH) {
-                    sfi[I] = E.sfs[((size_t)((role ? 3 : 0) + slot) * NEGP + I) * ne + e];
-                    sfx[I] = E.sfs[((size_t)((role ? 0 : 3) + slot) * NEGP + I) * ne + e];
-                }
-            }
-            // the "in" side subtracts w*F and the "ex" side adds it; -(a*b) == (-a)*b exactly, so
-            // the sign goes on the edge factor once and one update serves both roles
-            const double edfs = role ? edfac : -edfac;
-            double acc[3][DOF];
-#pragma unroll
-            for (int I = 0; I < NEGP; I++) {
-                const int gi = I, gx = NEGP - 1 - I;
-                const int gown = role ? gx : gi;
-                const double* pi_ = tpe[Li][gi];
-                const double* px_ = tpe[Lx][gx];
-                // PHI_EDGE mode 1 is 1 (checked at set-up), so the sum from zero starts at mode 1's
-                // coefficient with the same value
-                const double ze_in = trace1<DOF>(Vi[0], pi_), qx_in = trace1<DOF>(Vi[1], pi_), qy_in = trace1<DOF>(Vi[2], pi_);
-                const double ze_ex = trace1<DOF>(Vx[0], px_), qx_ex = trace1<DOF>(Vx[1], px_), qy_ex = trace1<DOF>(Vx[2], px_);
-                const double hb_in = trace1<3>(hbi, pi_), hb_ex = trace1<3>(hbx, px_);
-                const double sf_in = sfi[I], sf_ex = sfx[I];
-                double f0, f1, f2;
-                llf<NL>(ph, ze_in, ze_ex, qx_in, qx_ex, qy_in, qy_ex, hb_in, hb_ex, sf_in, sf_ex, nx, ny, ph.g, f0, f1, f2);
-                double fo = f0, gm = f1, hm = f2;
-                // dry-side treatment (src/internal_edge_hydro.F:212-302): 1 reflect into a dry
-                // "in" element, 2 zero-gravity flux for a dry "in", 3 reflect into a dry "ex",
-                // 4 zero-gravity flux for a dry "ex"; only what this element's side receives
-                int mode = 0;
-                if (fabs(f0) > 1.0e-8) {
-                    if (wd_in_el == 0) mode = (f0 > 0.0) ? 1 : (role ? 0 : 2);
-                    else if (wd_ex_el == 0) mode = (f0 < 0.0) ? 3 : (role ? 4 : 0);
-                }
-                if (mode) {
-                    double a_zi = ze_in, a_xi = qx_in, a_yi = qy_in, a_hi = hb_in, a_si = sf_in;
-                    double a_ze = ze_ex, a_xe = qx_ex, a_ye = qy_ex, a_he = hb_ex, a_se = sf_ex;
-                    double G = ph.g;
-                    if (mode == 1 || mode == 3) {
-                        const double sx = (mode == 1) ? qx_ex : qx_in, sy = (mode == 1) ? qy_ex : qy_in;
-                        const double qn = sx * nx + sy * ny, qt = sx * tx + sy * ty;
-                        const double qnm = -qn, qtm = qt;
-                        const double den = (nx * ty - ny * tx);
-                        const double mqx = (ty * qnm - ny * qtm) / den;
-                        const double mqy = (-tx * qnm + nx * qtm) / den;
-                        if (mode == 1) { a_zi = ze_ex; a_xi = mqx; a_yi = mqy; a_hi = hb_ex; a_si = sf_ex; }
-                        else { a_ze = ze_in; a_xe = mqx; a_ye = mqy; a_he = hb_in; a_se = sf_in; }
-                    } else {
-                        G = 0.0;
-                    }
-                    double r0, r1, r2;
-                    llf<NL>(ph, a_zi, a_ze, a_xi, a_xe, a_yi, a_ye, a_hi, a_he, a_si, a_se, nx, ny, G, r0, r1, r2);
-                    // mode 1: fo, ex momentum from the reflected flux, zero for the dry "in"
-                    // mode 3: fo, in momentum from the reflected flux, zero for the dry "ex"
-                    if (mode == 1) { fo = r0; gm = role ? r1 : 0.0; hm = role ? r2 : 0.0; }
-                    else if (mode == 3) { fo = r0; gm = role ? 0.0 : r1; hm = role ? 0.0 : r2; }
-                    else { gm = r1; hm = r2; }
-                }
-                // the slot sums start from zero: 0 + x == x for every x but -0, so the first
-                // point's terms start them
-                const double* eq = teq[L][gown];
-#pragma unroll
-                for (int k = 0; k < DOF; k++) {
-                    const double ws = edfs * eq[k];
-                    if (I == 0) {
-                        acc[0][k] = ws * fo; acc[1][k] = ws * gm; acc[2][k] = ws * hm;
-                    } else {
-                        acc[0][k] = acc[0][k] + ws * fo; acc[1][k] = acc[1][k] + ws * gm; acc[2][k] = acc[2][k] + ws * hm;
-                    }
-                }
-            }
-#pragma unroll
-            for (int f = 0; f < 3; f++)
-#pragma unroll
-                for (int k = 0; k < DOF; k++) acc_lds[1][f * DOF + k][tid] = acc_lds[1][f * DOF + k][tid] + acc[f][k];
-        } else {
-            if (wd == 0) continue;
-            double xlen, AREAS;
-            side_xlen_areas(E, ne, e, L, role, xlen, AREAS);
-            double U[3][DOF], hb[3];
-#pragma unroll
-            for (int f = 0; f < 3; f++)
-#pragma unroll
-                for (int k = 0; k < DOF; k++) U[f][k] = stg[(f * DOF + k) * ns + tid];
-#pragma unroll
-            for (int m = 0; m < 3; m++) hb[m] = stg[(3 * DOF + m) * ns + tid];
-#pragma unroll 1
-            for (int I = 0; I < NEGP; I++) {
-                const double* pv = tpe[L][I];
-                const double ze_in = trace<DOF>(U[0], pv), qx_in = trace<DOF>(U[1], pv), qy_in = trace<DOF>(U[2], pv);
-                const double hb_in = trace<3>(hb, pv);
-                const double sf = SPH ? E.sfs[((size_t)slot * NEGP + I) * ne + e] : 1.0;
-                double f0, f1, f2;
-                if (kind == SIDE_LAND) {
-                    const double qn_int = qx_in * nx + qy_in * ny, qt_int = qx_in * tx + qy_in * ty;
-                    const double qn_ext = -qn_int, qt_ext = qt_int;
-                    const double den = 1.0 / (nx * ty - ny * tx);
-                    const double qx_ex = (ty * qn_ext - ny * qt_ext) * den;
-                    const double qy_ex = (-tx * qn_ext + nx * qt_ext) * den;
-                    llf<NL>(ph, ze_in, ze_in, qx_in, qx_ex, qy_in, qy_ex, hb_in, hb_in, sf, sf, nx, ny, ph.g, f0, f1, f2);
-                } else if (kind == SIDE_OCEAN) {
-                    double ze_ex = 0.0;
-                    const double xe = T.xegp[I];
-                    // the constituents' endpoint terms EMO*RFF*COS(ARGJ-EFA) of this stage (tide_kernel)
-                    for (int jj = 0; jj < a.fo.nbfr; jj++) {
-                        const size_t o = ((size_t)nb * a.fo.nbfr + jj) * 2;
-                        const double z1 = a.fo.tz[(size_t)a.irk * a.fo.tzn + o];
-                        const double z2 = a.fo.tz[(size_t)a.irk * a.fo.tzn + o + 1];
-                        ze_ex = ze_ex + (0.5 * (z1 + z2) + 0.5 * (z2 - z1) * xe);
-                    }
-                    if ((ze_ex * ph.ifnlfa + hb_in) <= 0) ze_ex = fabs(hb_in) + sc.h0;
-                    llf<NL>(ph, ze_in, ze_ex, qx_in, qx_in, qy_in, qy_in, hb_in, hb_in, sf, sf, nx, ny, ph.g, f0, f1, f2);
-                } else {
-                    // the specified normal flux at this point (flow_kernel); the reference forms the
-                    // exterior momentum after every constituent, so the last, full sum is what counts
-                    const double qn_ext = a.fo.fz[(size_t)a.irk * a.fo.fzn + (size_t)nb * NEGP + I];
-                    const double qt_ext = 0.0;
-                    const double qx_ex = -(ty * qn_ext - ny * qt_ext) / (nx * ty - ny * tx);
-                    const double qy_ex = -(-tx * qn_ext + nx * qt_ext) / (nx * ty - ny * tx);
-                    llf<NL>(ph, ze_in, ze_in, qx_in, qx_ex, qy_in, qy_ex, hb_in, hb_in, sf, sf, nx, ny, ph.g, f0, f1, f2);
-                }
-#pragma unroll
-                for (int k = 0; k < DOF; k++) {
-                    const double w = 2.0 * T.m_inv[k] / AREAS * xlen * pv[k] * T.wegp[I];
-                    acc_lds[0][k][tid] = acc_lds[0][k][tid] - w * f0;
-                    acc_lds[0][DOF + k][tid] = acc_lds[0][DOF + k][tid] - w * f1;
-                    acc_lds[0][2 * DOF + k][tid] = acc_lds[0][2 * DOF + k][tid] - w * f2;
-                }
-            }
-        }
-    }
-    // the element's own state and bathymetry modes, staged
-    double U[3][DOF], hb[3];
-#pragma unroll
-    for (int f = 0; f < 3; f++)
-#pragma unroll
-        for (int k = 0; k < DOF; k++) U[f][k] = stg[(f * DOF + k) * ns + tid];
-#pragma unroll
-    for (int m = 0; m < 3; m++) hb[m] = stg[(3 * DOF + m) * ns + tid];
-    // add_internal_flux: RHS = RHS(boundary edges) + slot sum
+    // the Jacobian and Manning's n of the volume quadrature, loaded while the sides are evaluated
+    const double jac0 = at(E.geo + (size_t)9 * ne, e), jac1 = at(E.geo + (size_t)10 * ne, e);
+    const double jac2 = at(E.geo + (size_t)11 * ne, e), jac3 = at(E.geo + (size_t)12 * ne, e);
+    const double nbar0 = ph.load_manning ? at(E.nbar, e) : 0.0;
+    // ---- sides: the internal ones in slot order, then the boundary ones (a sum of the two, whose
+    // order of evaluation does not matter): RHS = RHS(boundary edges) + slot sum
     double R[3][DOF];
 #pragma unroll
     for (int f = 0; f < 3; f++)
 #pragma unroll
-        for (int k = 0; k < DOF; k++) R[f][k] = acc_lds[0][f * DOF + k][tid] + acc_lds[1][f * DOF + k][tid];
-
-    // loads of the volume quadrature and the RK update, issued together before the quadrature's
-    // arithmetic: the nodal wind and pressure (MET), the area-point spherical factors (SPH) and
-    // the first RK base state
-    double mcd[3], mwm[3], mwx[3], mwy[3], mpr[3];
-    if (MET) {
-#pragma unroll
-        for (int v = 0; v < 3; v++) {
-            const int n = E.nm[(size_t)v * ne + e];
-            mcd[v] = a.mt.cd[n]; mwm[v] = a.mt.wm[n]; mwx[v] = a.mt.wx[n]; mwy[v] = a.mt.wy[n]; mpr[v] = a.mt.prn[n];
+        for (int k = 0; k < DOF; k++) R[f][k] = 0.0;
+    const int nbd = boundary_slots(info);
+#pragma unroll 1
+    for (int slot = 0; slot < 3; slot++) {
+        double nx1 = nx, ny1 = ny, ed1 = edfac;
+        if (slot < 2) {
+            nx1 = at(E.geo + (size_t)(3 * slot + 3) * ne, e);
+            ny1 = at(E.geo + (size_t)(3 * slot + 4) * ne, e);
+            ed1 = at(E.geo + (size_t)(3 * slot + 5) * ne, e);
         }
-    }
-    double tipv[3] = {0.0, 0.0, 0.0};
-    if (a.tip) {
+        if (slot >= nbd) {
+            double acc[3][DOF];
+            internal_side<P, SPH, NL, 1>(a, tb, stg, stwd, ne, e, tid, slot, side_bits(info, slot), sl, wd, nx, ny, edfac, acc);
 #pragma unroll
-        for (int v = 0; v < 3; v++) tipv[v] = a.tip[E.nm[(size_t)v * ne + e]];
+            for (int f = 0; f < 3; f++)
+#pragma unroll
+                for (int k = 0; k < DOF; k++) R[f][k] = R[f][k] + acc[f][k];
+        }
+        nx = nx1; ny = ny1; edfac = ed1;
     }
+    if (nbd != 0 && wd != 0) {
+        double acc[3][DOF];
+        boundary_sides<P, SPH, NL>(a, T, tb, stg, ne, e, tid, info, nbd, E.scen[sid].h0, acc);
+#pragma unroll
+        for (int f = 0; f < 3; f++)
+#pragma unroll
+            for (int k = 0; k < DOF; k++) R[f][k] = acc[f][k] + R[f][k];
+    }
+
+    // the scenario's scalars, then the first RK base state, loaded before the volume quadrature's arithmetic
+    double dtdp, dtdph, cf, fric, rain;
+    VolumeTerms v;
+    if (E.sid) {
+        const Scen& sc = E.scen[sid];
+        dtdp = sc.dtdp; dtdph = sc.dtdph; cf = sc.cf; fric = sc.fric; rain = sc.rain; v.cori = sc.cori;
+    } else {
+        const Scen& sc = E.scen[0];
+        dtdp = sc.dtdp; dtdph = sc.dtdph; cf = sc.cf; fric = sc.fric; rain = sc.rain; v.cori = sc.cori;
+    }
+    if (E.cori_el) v.cori = at(E.cori_el, e);
     double sfqv[NAGP];
 #pragma unroll
-    for (int I = 0; I < NAGP; I++) sfqv[I] = SPH ? E.sfacq[(size_t)I * ne + e] : 1.0;
-    double jac[4];                       // DRDX, DSDX, DRDY, DSDY
-#pragma unroll
-    for (int j = 0; j < 4; j++) jac[j] = E.geo[(size_t)(9 + j) * ne + e];
+    for (int I = 0; I < NAGP; I++) sfqv[I] = SPH ? at(E.sfacq + (size_t)I * ne, e) : 1.0;
     const bool pre0 = a.nprev > 0 && a.aprev[0] != 0.0;
     double B0[3][DOF];
     if (pre0) {
@@ -566,141 +855,54 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(P == 1 
 #pragma unroll
         for (int f = 0; f < 3; f++)
 #pragma unroll
-            for (int k = 0; k < DOF; k++) B0[f][k] = up[(size_t)(f * DOF + k) * ne + e];
+            for (int k = 0; k < DOF; k++) B0[f][k] = at(up + (size_t)(f * DOF + k) * ne, e);
     }
-
     // ---- volume quadrature (RHS_DG_HYDRO)
-    if (sc.rain > 0.0) {
+    if (rain > 0.0) {
 #pragma unroll 1
         for (int I = 0; I < NAGP; I++)
 #pragma unroll
-            for (int k = 0; k < DOF; k++) R[0][k] = R[0][k] + T.srfac[I][k] * sc.rain;
+            for (int k = 0; k < DOF; k++) R[0][k] = R[0][k] + T.srfac[I][k] * rain;
     }
     if (wd != 0) {
-        const double drdx = jac[0], dsdx = jac[1], drdy = jac[2], dsdy = jac[3];
-        // wind stress at the element's vertices and the pressure gradient sums (MET)
-        double mw[8];
-        if (MET) {
-            // nodal WSX2/WSY2/PR2 of this stage (src/met_forcing.F:507-509) and the
-            // QP-independent sums PR2(Ni)*DPSIDX(i) of src/rhs_dg_hydro.F:117-122,366-372
-            const double ramp = a.fo.ramp[(size_t)sid * a.fo.rows + row];
-            const double drpsi[3] = {-1.0 / 2.0, 1.0 / 2.0, 0.0}, dspsi[3] = {-1.0 / 2.0, 0.0, 1.0 / 2.0};
-            double pdx = 0.0, pdy = 0.0;
-#pragma unroll
-            for (int v = 0; v < 3; v++) {
-                const double cd = mcd[v], wm = mwm[v];
-                mw[v] = ramp * 0.001293 * cd * mwx[v] * wm;
-                mw[3 + v] = ramp * 0.001293 * cd * mwy[v] * wm;
-                const double pr = ramp * mpr[v];
-                const double dpsidx = drpsi[v] * drdx + dspsi[v] * dsdx;
-                const double dpsidy = drpsi[v] * drdy + dspsi[v] * dsdy;
-                if (v == 0) { pdx = pr * dpsidx; pdy = pr * dpsidy; }
-                else { pdx = pdx + pr * dpsidx; pdy = pdy + pr * dpsidy; }
-            }
-            mw[6] = pdx;
-            mw[7] = pdy;
+        v.drdx = jac0; v.dsdx = jac1; v.drdy = jac2; v.dsdy = jac3; v.nbar = nbar0;
+        v.dtdph = dtdph; v.cf = cf; v.fric = fric;
+        {
+            const double hb[3] = {stg[3 * DOF * ns + tid], stg[(3 * DOF + 1) * ns + tid], stg[(3 * DOF + 2) * ns + tid]};
+            volume_terms<P, MET, NL>(a, T, ne, e, sid, row, stg[tid], hb, v);
         }
-        // tidal potential (src/rhs_dg_hydro.F:117-122,378-386): the sums DPSIDX(i)*TIP2(Ni) are
-        // the same at every area point; RAMPDG multiplies them once more at each point
-        double tdx = 0.0, tdy = 0.0, tramp = 0.0;
-        if (a.tip) {
-            const double drpsi[3] = {-1.0 / 2.0, 1.0 / 2.0, 0.0}, dspsi[3] = {-1.0 / 2.0, 0.0, 1.0 / 2.0};
-#pragma unroll
-            for (int v = 0; v < 3; v++) {
-                const double dpsidx = drpsi[v] * drdx + dspsi[v] * dsdx;
-                const double dpsidy = drpsi[v] * drdy + dspsi[v] * dsdy;
-                if (v == 0) { tdx = dpsidx * tipv[v]; tdy = dpsidy * tipv[v]; }
-                else { tdx = tdx + dpsidx * tipv[v]; tdy = tdy + dpsidy * tipv[v]; }
-            }
-            tramp = a.fo.ramp[(size_t)sid * a.fo.rows + row];
+        // p=1: the three area points unrolled, with the quadrature's constants in the code and the factors
+        // MW*DPSI formed once (the same at every point, checked at set-up); at p=2 the six points in a loop
+        double xf1[3], yf1[3];
+        if constexpr (P == 1) {
+            xf1[1] = P1Area::mw[1] * v.dpx1; yf1[1] = P1Area::mw[1] * v.dpy1;
+            xf1[2] = P1Area::mw[2] * v.dpx2; yf1[2] = P1Area::mw[2] * v.dpy2;
         }
-        // hybrid friction factor (1 + (HBREAK/H_c)^FTHETA)^(FGAMMA/FTHETA) from the element-mean
-        // depth (src/rhs_dg_hydro.F:306-309): the same at every area point, evaluated once and only
-        // when the hybrid law is on
-        double hybf = 1.0;
-        if (ph.ifhybf == 1) {
-            const double depth_c = hb[0] + U[0][0];
-            const double fh_nl_c = NL ? 1.0 / depth_c : 1.0 / (ph.nleq * depth_c + ph.leq);
-            hybf = pow(1.0 + pow(ph.hbreak * fh_nl_c, ph.ftheta), ph.fgamma / ph.ftheta);
-        }
-        // the P1 bathymetry's gradient: the linear modes' derivative tables are the same at every
-        // area point (checked at set-up), so the sums are those of every point
-        double dhbx = 0.0, dhby = 0.0;
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            const double dpxk = T.drphi[0][k] * drdx + T.dsphi[0][k] * dsdx;
-            const double dpyk = T.drphi[0][k] * drdy + T.dsphi[0][k] * dsdy;
-            dhbx = dhbx + hb[k] * dpxk;
-            dhby = dhby + hb[k] * dpyk;
-        }
-        // p=1: the three area points unrolled, so that their long dependent chains overlap (at p=2
-        // the six points unrolled run slower)
 #pragma unroll(P == 1 ? NAGP : 1)
         for (int I = 0; I < NAGP; I++) {
-            const double* pa = T.phi_area[I];
-            double ze = U[0][0], qx = U[1][0], qy = U[2][0];
+            double t[4], q[8];
+            area_values<P>(T, stg, ns, tid, I, t);
+            area_point<P, MET, NL>(a, T, I, v, t[0], t[1], t[2], t[3], sfqv[I], wd, q);
+            const double sr0 = P == 1 ? P1Area::srfac[I][0] : T.srfac[I][0];
+            R[1][0] = R[1][0] + sr0 * q[6];
+            R[2][0] = R[2][0] + sr0 * q[7];
 #pragma unroll
             for (int k = 1; k < DOF; k++) {
-                ze = ze + U[0][k] * pa[k];
-                qx = qx + U[1][k] * pa[k];
-                qy = qy + U[2][k] * pa[k];
-            }
-            // PHI_AREA of mode 1 is 1 (checked at set-up): the sum from zero starts at hb[0]
-            double hbq = hb[0];
-#pragma unroll
-            for (int k = 1; k < 3; k++) hbq = hbq + hb[k] * pa[k];
-            const double sfq = sfqv[I];
-            const double depth = ze + hbq;
-            // with NL (NLEQ = 1, LEQ = 0) the constant factors fold exactly
-            const double f1 = NL ? 1.0 : ph.nleq + ph.leq * hbq;
-            const double fx = NL ? qx * sfq : qx * f1 * sfq, fy = NL ? qy : qy * f1;
-            const double fu = NL ? qx : ph.nleq * qx, fv = NL ? qy : ph.nleq * qy;
-            const double fg = ph.nleqg * ze * wd;
-            const double fh = NL ? 1.0 / depth : 1.0 / (ph.nleq * depth + ph.leq);
-            const double u = qx * fh, v = qy * fh;
-            const double huu = fu * u, hvv = fv * v, huv = fu * v;
-            const double gh2 = NL ? fg * (0.5 * ze + hbq) : fg * (0.5 * ze + hbq) + ph.fg_l * ze;
-            const double gx = (huu + gh2) * sfq, gy = huv;
-            const double hx = huv * sfq, hy = hvv + gh2;
-            double fric = sc.fric;
-            if (ph.load_manning) {
-                // DEPTH**(1.D0/3.D0) (src/rhs_dg_hydro.F:302), correctly rounded
-                fric = ph.g * (nbar * nbar) / crm::cr_pow_third(depth);
-                if (fric < sc.cf) fric = sc.cf;
-            }
-            double tau = fric;
-            if (ph.iflinbf == 0) {
-                const double umag = sqrt(u * u + v * v);
-                tau = tau * umag * fh;
-                if (ph.ifhybf == 1) tau = tau * hybf;
-                const double cap = 0.9 * sc.dtdph;
-                if (cap < tau) tau = cap;
-            }
-            double sx = -(tau * qx) + fg * dhbx * sfq + cori * qy;
-            double sy = -(tau * qy) + fg * dhby - cori * qx;
-            if (MET) {
-                // wind stress and atmospheric pressure (src/rhs_dg_hydro.F:362-373)
-                const double* ps = T.psi[I];
-                const double wsx = mw[0] * ps[0] + mw[1] * ps[1] + mw[2] * ps[2];
-                const double wsy = mw[3] * ps[0] + mw[4] * ps[1] + mw[5] * ps[2];
-                const double fw = 1.0 / f1;
-                sx = sx + (NL ? wsx : fw * wsx) - ph.g * sfq * depth * mw[6];
-                sy = sy + (NL ? wsy : fw * wsy) - ph.g * depth * mw[7];
-            }
-            if (a.tip) {
-                sx = sx + tramp * ph.g * depth * sfq * tdx;
-                sy = sy + tramp * ph.g * depth * tdy;
-            }
-            R[1][0] = R[1][0] + T.srfac[I][0] * sx;
-            R[2][0] = R[2][0] + T.srfac[I][0] * sy;
-#pragma unroll
-            for (int k = 1; k < DOF; k++) {
-                const double dpxk = T.drphi[I][k] * drdx + T.dsphi[I][k] * dsdx;
-                const double dpyk = T.drphi[I][k] * drdy + T.dsphi[I][k] * dsdy;
-                const double xf = T.mw[I][k] * dpxk, yf = T.mw[I][k] * dpyk, sr = T.srfac[I][k];
-                R[0][k] = R[0][k] + xf * fx + yf * fy;
-                R[1][k] = R[1][k] + xf * gx + yf * gy + sr * sx;
-                R[2][k] = R[2][k] + xf * hx + yf * hy + sr * sy;
+                double xf, yf, sr;
+                if constexpr (P == 1) {
+                    xf = xf1[k]; yf = yf1[k]; sr = P1Area::srfac[I][k];
+                } else {
+                    const double dpxk = k == 1 ? v.dpx1 : (k == 2 ? v.dpx2 : T.drphi[I][k] * v.drdx + T.dsphi[I][k] * v.dsdx);
+                    const double dpyk = k == 1 ? v.dpy1 : (k == 2 ? v.dpy2 : T.drphi[I][k] * v.drdy + T.dsphi[I][k] * v.dsdy);
+                    xf = T.mw[I][k] * dpxk; yf = T.mw[I][k] * dpyk; sr = T.srfac[I][k];
+                }
+                R[0][k] = R[0][k] + xf * q[0] + yf * q[1];
+                R[1][k] = R[1][k] + xf * q[2] + yf * q[3];
+                R[2][k] = R[2][k] + xf * q[4] + yf * q[5];
+                if (P != 1 || I > 0 || k < 2) {     // p=1: SRFAC of mode 3 is zero at the first point
+                    R[1][k] = R[1][k] + sr * q[6];
+                    R[2][k] = R[2][k] + sr * q[7];
+                }
             }
         }
     }
@@ -709,17 +911,17 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(P == 1 
 #pragma unroll
         for (int f = 0; f < 3; f++)
 #pragma unroll
-            for (int k = 0; k < DOF; k++) a.rout[(size_t)(f * DOF + k) * ne + e] = R[f][k];
+            for (int k = 0; k < DOF; k++) at(a.rout + (size_t)(f * DOF + k) * ne, e) = R[f][k];
     }
     double W[3][DOF];
-    const double bcur = a.bcur * sc.dtdp;
+    const double bcur = a.bcur * dtdp;
 #pragma unroll
     for (int f = 0; f < 3; f++)
 #pragma unroll
         for (int k = 0; k < DOF; k++) W[f][k] = 0.0;
 #pragma unroll 1
     for (int i = 0; i < a.nprev; i++) {
-        const double ai = a.aprev[i], bi = a.bprev[i] * sc.dtdp;
+        const double ai = a.aprev[i], bi = a.bprev[i] * dtdp;
         if (i == 0 && pre0) {
 #pragma unroll
             for (int f = 0; f < 3; f++)
@@ -730,36 +932,275 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(P == 1 
 #pragma unroll
             for (int f = 0; f < 3; f++)
 #pragma unroll
-                for (int k = 0; k < DOF; k++) W[f][k] = W[f][k] + ai * up[(size_t)(f * DOF + k) * ne + e];
+                for (int k = 0; k < DOF; k++) W[f][k] = W[f][k] + ai * at(up + (size_t)(f * DOF + k) * ne, e);
         }
         if (bi != 0.0) {
             const double* rp = a.rprev[i];
 #pragma unroll
             for (int f = 0; f < 3; f++)
 #pragma unroll
-                for (int k = 0; k < DOF; k++) W[f][k] = W[f][k] + bi * rp[(size_t)(f * DOF + k) * ne + e];
+                for (int k = 0; k < DOF; k++) W[f][k] = W[f][k] + bi * at(rp + (size_t)(f * DOF + k) * ne, e);
         }
     }
 #pragma unroll
     for (int f = 0; f < 3; f++)
 #pragma unroll
-        for (int k = 0; k < DOF; k++) W[f][k] = W[f][k] + a.acur * U[f][k] + bcur * R[f][k];
+        for (int k = 0; k < DOF; k++) W[f][k] = W[f][k] + a.acur * stg[(f * DOF + k) * ns + tid] + bcur * R[f][k];
 
     if (WDFUSED) {
         const double D[3] = {E.dpv[e], E.dpv[(size_t)ne + e], E.dpv[2 * (size_t)ne + e]};
+        const double hb[3] = {stg[3 * DOF * ns + tid], stg[(3 * DOF + 1) * ns + tid], stg[(3 * DOF + 2) * ns + tid]};
+        const double h0 = E.scen[sid].h0;
         const double dpe_min = fmin(fmin(D[0], D[1]), D[2]);
-        if (a.wd_active && !wetdry_keeps<P>(T, W, D, wd, sc.h0)) a.wd_active[0] = 1;
-        const int nw = wetdry_element<P>(T, W, D, hb, dpe_min, wd, sc.h0);
-        a.wd_out[e] = (uint8_t)nw;
+        if (a.wd_active && !wetdry_keeps<P>(T, W, D, wd, h0)) a.wd_active[0] = 1;
+        const int nw = wetdry_element<P>(T, W, D, hb, dpe_min, wd, h0);
+        at(a.wd_out, e) = (uint8_t)nw;
     }
 #pragma unroll
     for (int f = 0; f < 3; f++)
 #pragma unroll
-        for (int k = 0; k < DOF; k++) a.uout[(size_t)(f * DOF + k) * ne + e] = W[f][k];
+        for (int k = 0; k < DOF; k++) at(a.uout + (size_t)(f * DOF + k) * ne, e) = W[f][k];
     if (a.cmout) {
 #pragma unroll
-        for (int f = 0; f < 3; f++) a.cmout[(size_t)f * ne + e] = W[f][0];
+        for (int f = 0; f < 3; f++) at(a.cmout + (size_t)f * ne, e) = W[f][0];
     }
+}
+
+// The same stage for meshes too small to fill the chip with one lane per element, where the time of a launch is
+// the serial chain of its slowest wave: a block of four waves works on 64 elements, lane l of every wave on
+// element l.  Wave c < 3
+//   1. stages field c of the tile and its halo (wave 3: the flags and the edge tables),
+//   2. evaluates side slot c if it is internal (wave 3: the boundary sides, one after the other),
+//   3. evaluates the area points c, c+3,
+//   4. sums field c's right-hand side in the reference's order from what the waves left in LDS, and updates
+//      field c.
+// Every value is formed by the operations of stage_kernel, so the results are the same bits.
+constexpr int SPLIT_NT = 64;             // elements per block
+constexpr int split_rows(int dof, int nagp) { return 4 * 3 * dof + 8 * nagp; }
+
+template <int P, bool SPH, bool WDFUSED, bool MET>
+__global__ void __launch_bounds__(4 * SPLIT_NT) __attribute__((amdgpu_waves_per_eu(2))) stage_split_kernel(StageArgs a) {
+    constexpr int DOF = (P + 1) * (P + 2) / 2;
+    constexpr int NAGP = (P == 1) ? 3 : 6;
+    constexpr int NEGP = P + 2;
+    constexpr int NT = SPLIT_NT;
+    __shared__ EdgeTables<DOF, NEGP> tb;
+    // exchange between an element's lanes: the sums of the side slots and of the boundary sides
+    // [wave*3*DOF + field*DOF + mode], then the area points' values [point*8 + quantity]; with WDFUSED last
+    // the updated modes
+    __shared__ double xch[split_rows(DOF, NAGP)][NT];
+    extern __shared__ double stg[];      // as in stage_kernel
+    const DevTables& T = tab<P>();
+    const ElemData& E = a.ed;
+    const Phys& ph = a.ph;
+    const int ne = E.ne;
+    const int c = __builtin_amdgcn_readfirstlane(threadIdx.x / NT), le = threadIdx.x % NT;
+    const int tile = xcd_tile(blockIdx.x, gridDim.x);
+    const int e = tile * NT + le;
+    const bool valid = e < ne;
+    const int ns = a.ns, nh = a.nh;
+    uint8_t* const stwd = reinterpret_cast<uint8_t*>(stg + (size_t)(3 * DOF + 3) * ns);
+    double* const vol = &xch[4 * 3 * DOF][0];
+    const int ec = valid ? e : ne - 1;   // lanes past the last element read element ne-1 and write nothing
+    const int* hx = a.hidx + (size_t)tile * nh;
+    const int g0 = le < nh ? hx[le] : -1;
+    const int info = at(E.sinfo, ec);
+    const int sl = at(a.snbl, ec);
+    const int sid = E.sid ? (int)at(E.sid, ec) : 0;
+    const int cs = c < 3 ? c : 0;
+    const double nx = at(E.geo + (size_t)(3 * cs) * ne, ec), ny = at(E.geo + (size_t)(3 * cs + 1) * ne, ec);
+    const double edfac = at(E.geo + (size_t)(3 * cs + 2) * ne, ec);
+    if (c < 3) {
+        const double c13 = 1.0 / 3.0, c16 = 1.0 / 6.0;
+        auto load = [&](int g, double (&v)[DOF + 3]) {
+#pragma unroll
+            for (int k = 0; k < DOF; k++) v[k] = at(a.uin + (size_t)(c * DOF + k) * ne, g);
+#pragma unroll
+            for (int m = 0; m < 3; m++) v[DOF + m] = at(E.dpv + (size_t)m * ne, g);
+        };
+        auto store = [&](int j, const double (&v)[DOF + 3]) {
+#pragma unroll
+            for (int k = 0; k < DOF; k++) stg[(c * DOF + k) * ns + j] = v[k];
+            const double d0 = v[DOF], d1 = v[DOF + 1], d2 = v[DOF + 2];
+            stg[(3 * DOF + c) * ns + j] = c == 0 ? c13 * (d0 + d1 + d2)
+                                                 : (c == 1 ? -(c16 * (d0 + d1)) + c13 * d2 : -(0.5 * d0) + 0.5 * d1);
+        };
+        double v[DOF + 3], v2[DOF + 3];
+        load(ec, v);
+        load(g0 < 0 ? 0 : g0, v2);
+        store(le, v);
+        if (g0 >= 0) store(NT + le, v2);
+#pragma unroll 1
+        for (int h = le + NT; h < nh; h += NT) {
+            const int g = hx[h];
+            if (g < 0) break;
+            load(g, v);
+            store(NT + h, v);
+        }
+    } else {
+        load_edge_tables<DOF, NEGP>(T, tb, le, NT);
+        const uint8_t w = at(a.wd_in, ec), w2 = at(a.wd_in, g0 < 0 ? 0 : g0);
+        stwd[le] = w;
+        if (g0 >= 0) stwd[NT + le] = w2;
+#pragma unroll 1
+        for (int h = le + NT; h < nh; h += NT) {
+            const int g = hx[h];
+            if (g < 0) break;
+            stwd[NT + h] = at(a.wd_in, g);
+        }
+    }
+    // loads of the volume quadrature and the RK update, under way while the sides are evaluated
+    const int row = table_step(a.fo) * a.fo.nrk + a.irk;
+    constexpr int NP = NAGP / 3;           // area points per wave: c and, at p=2, c + 3
+    VolumeTerms v;
+    v.drdx = at(E.geo + (size_t)9 * ne, ec); v.dsdx = at(E.geo + (size_t)10 * ne, ec);
+    v.drdy = at(E.geo + (size_t)11 * ne, ec); v.dsdy = at(E.geo + (size_t)12 * ne, ec);
+    v.nbar = ph.load_manning ? at(E.nbar, ec) : 0.0;
+    const Scen& sc = E.scen[sid];
+    const double dtdp = sc.dtdp, rain = sc.rain, h0 = sc.h0;
+    v.dtdph = sc.dtdph; v.cf = sc.cf; v.fric = sc.fric;
+    v.cori = E.cori_el ? at(E.cori_el, ec) : sc.cori;
+    double sfqv[NP];
+#pragma unroll
+    for (int j = 0; j < NP; j++) sfqv[j] = SPH ? at(E.sfacq + (size_t)(cs + 3 * j) * ne, ec) : 1.0;
+    const bool pre0 = a.nprev > 0 && a.aprev[0] != 0.0;
+    double B0[DOF];
+    if (pre0) {
+        const double* up = a.uprev[0];
+#pragma unroll
+        for (int k = 0; k < DOF; k++) B0[k] = at(up + (size_t)(cs * DOF + k) * ne, ec);
+    }
+    __syncthreads();
+    const int wd = valid ? stwd[le] : 0;
+    // ---- sides
+    const int nbd = boundary_slots(info);
+    {
+        double acc[3][DOF];
+        if (c < 3) {
+            // a boundary slot is the boundary wave's; its place in the exchange is not read
+            if (c >= nbd && valid)
+                internal_side<P, SPH, true, NEGP>(a, tb, stg, stwd, ne, ec, le, c, side_bits(info, c), sl, wd, nx, ny,
+                                                  edfac, acc);
+        } else if (nbd != 0 && wd != 0) {
+            boundary_sides<P, SPH, true>(a, T, tb, stg, ne, ec, le, info, nbd, h0, acc);
+        } else {
+#pragma unroll
+            for (int f = 0; f < 3; f++)
+#pragma unroll
+                for (int k = 0; k < DOF; k++) acc[f][k] = 0.0;
+        }
+        if (c == 3 || (c >= nbd && valid)) {
+#pragma unroll
+            for (int f = 0; f < 3; f++)
+#pragma unroll
+                for (int k = 0; k < DOF; k++) xch[(c * 3 + f) * DOF + k][le] = acc[f][k];
+        }
+    }
+    // ---- volume quadrature (RHS_DG_HYDRO) at this wave's area points
+    {
+        const double hb[3] = {stg[3 * DOF * ns + le], stg[(3 * DOF + 1) * ns + le], stg[(3 * DOF + 2) * ns + le]};
+        volume_terms<P, MET, true>(a, T, ne, ec, sid, row, stg[le], hb, v);
+    }
+    if (c < 3 && wd != 0) {
+#pragma unroll
+        for (int j = 0; j < NP; j++) {
+            double t[4], q[8];
+            area_values<P>(T, stg, ns, le, c + 3 * j, t);
+            area_point<P, MET, true>(a, T, c + 3 * j, v, t[0], t[1], t[2], t[3], sfqv[j], wd, q);
+#pragma unroll
+            for (int i = 0; i < 8; i++) vol[((c + 3 * j) * 8 + i) * NT + le] = q[i];
+        }
+    }
+    __syncthreads();
+    if (c == 3) {
+        if (WDFUSED) { __syncthreads(); }
+        return;
+    }
+    // ---- field c: add_internal_flux (RHS of the boundary edges + slot sum), then the volume terms, point after
+    // point
+    double R[DOF];
+#pragma unroll
+    for (int k = 0; k < DOF; k++) {
+        double s = 0.0;
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            if (i >= nbd) s = s + xch[(i * 3 + c) * DOF + k][le];
+        R[k] = xch[(9 + c) * DOF + k][le] + s;
+    }
+    if (c == 0 && rain > 0.0) {
+#pragma unroll 1
+        for (int I = 0; I < NAGP; I++)
+#pragma unroll
+            for (int k = 0; k < DOF; k++) R[k] = R[k] + T.srfac[I][k] * rain;
+    }
+    if (wd != 0) {
+#pragma unroll
+        for (int I = 0; I < NAGP; I++) {
+            const double fx = vol[(I * 8 + 2 * c) * NT + le], fy = vol[(I * 8 + 2 * c + 1) * NT + le];
+            const double s = vol[(I * 8 + 5 + c) * NT + le];            // source of field c > 0
+            if (c != 0) R[0] = R[0] + T.srfac[I][0] * s;
+#pragma unroll
+            for (int k = 1; k < DOF; k++) {
+                const double dpxk = k == 1 ? v.dpx1 : (k == 2 ? v.dpx2 : T.drphi[I][k] * v.drdx + T.dsphi[I][k] * v.dsdx);
+                const double dpyk = k == 1 ? v.dpy1 : (k == 2 ? v.dpy2 : T.drphi[I][k] * v.drdy + T.dsphi[I][k] * v.dsdy);
+                R[k] = R[k] + (T.mw[I][k] * dpxk) * fx + (T.mw[I][k] * dpyk) * fy;
+                if (c != 0) R[k] = R[k] + T.srfac[I][k] * s;
+            }
+        }
+    }
+    // ---- SSP-RK update U(IRK+1) = sum_I ATVD(IRK,I) U(I) + BTVD(IRK,I) DT RHS(I)
+    if (a.rout && valid) {
+#pragma unroll
+        for (int k = 0; k < DOF; k++) at(a.rout + (size_t)(c * DOF + k) * ne, e) = R[k];
+    }
+    double W[DOF];
+    const double bcur = a.bcur * dtdp;
+#pragma unroll
+    for (int k = 0; k < DOF; k++) W[k] = 0.0;
+#pragma unroll 1
+    for (int i = 0; i < a.nprev; i++) {
+        const double ai = a.aprev[i], bi = a.bprev[i] * dtdp;
+        if (i == 0 && pre0) {
+#pragma unroll
+            for (int k = 0; k < DOF; k++) W[k] = W[k] + ai * B0[k];
+        } else if (ai != 0.0) {
+            const double* up = a.uprev[i];
+#pragma unroll
+            for (int k = 0; k < DOF; k++) W[k] = W[k] + ai * at(up + (size_t)(c * DOF + k) * ne, ec);
+        }
+        if (bi != 0.0) {
+            const double* rp = a.rprev[i];
+#pragma unroll
+            for (int k = 0; k < DOF; k++) W[k] = W[k] + bi * at(rp + (size_t)(c * DOF + k) * ne, ec);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < DOF; k++) W[k] = W[k] + a.acur * stg[(c * DOF + k) * ns + le] + bcur * R[k];
+    if (WDFUSED) {
+        // WETDRY needs all three fields: each wave takes the others' from LDS and keeps its own (the rows
+        // are the boundary sums', of which wave c alone read field c's)
+#pragma unroll
+        for (int k = 0; k < DOF; k++) xch[(9 + c) * DOF + k][le] = W[k];
+        __syncthreads();
+        if (!valid) return;
+        double A[3][DOF];
+        const double hb[3] = {stg[3 * DOF * ns + le], stg[(3 * DOF + 1) * ns + le], stg[(3 * DOF + 2) * ns + le]};
+#pragma unroll
+        for (int f = 0; f < 3; f++)
+#pragma unroll
+            for (int k = 0; k < DOF; k++) A[f][k] = xch[(9 + f) * DOF + k][le];
+        const double D[3] = {at(E.dpv, e), at(E.dpv + (size_t)ne, e), at(E.dpv + (size_t)2 * ne, e)};
+        const double dpe_min = fmin(fmin(D[0], D[1]), D[2]);
+        if (c == 0 && a.wd_active && !wetdry_keeps<P>(T, A, D, wd, h0)) a.wd_active[0] = 1;
+        const int nw = wetdry_element<P>(T, A, D, hb, dpe_min, wd, h0);
+        if (c == 0) at(a.wd_out, e) = (uint8_t)nw;
+#pragma unroll
+        for (int k = 0; k < DOF; k++) W[k] = c == 0 ? A[0][k] : (c == 1 ? A[1][k] : A[2][k]);
+    }
+    if (!valid) return;
+#pragma unroll
+    for (int k = 0; k < DOF; k++) at(a.uout + (size_t)(c * DOF + k) * ne, e) = W[k];
+    if (a.cmout) at(a.cmout + (size_t)c * ne, e) = W[0];
 }
 
 // ------------------------------------------------------------------------------------------
