@@ -150,9 +150,9 @@ struct Ctx {
     // bounds read them there, never from the state it limits in place) and the per-tile node lists
     DevBuf<double> cmean;
     struct LimBufs {
-        DevBuf<int> vhoff, vhidx, qoff, qinc_off, elq;
-        DevBuf<uint16_t> qinc;
-        int nsl = 0, nql = 0;
+        DevBuf<int> vhidx, xoff, xq, elq;
+        DevBuf<uint16_t> qinc, xinc;
+        int nvh = 0, nql = 0, nx = 0;
     } lim;
     DevBuf<int> nodecode;
     // modal2nodal: node rows in the host's ELETAB order (default: the node->element CSR) and the
@@ -595,19 +595,21 @@ int upload_met(Ctx& c) {
     return 0;
 }
 
-// The slope limiter's tiles of LIM_NT elements (LimTiles): each tile's vertex halo (ascending),
-// its nodes in order of first appearance, every node's incident elements as staged rows in the
-// node->element order `n2e` (entries elem<<2 | vertex), and each element's tile-local nodes.
+// The slope limiter's tiles of LIM_NT elements (LimTiles): each tile's vertex halo (ascending), its nodes in order
+// of first appearance, every node's incident elements as staged rows in the node->element order `n2e` (entries
+// elem<<2 | vertex), and each element's tile-local nodes.
 int build_limtiles(Ctx& c, const std::vector<int>& nm, const std::vector<int>& off, const std::vector<int>& n2e) {
     const int ne = c.ne, nt = LIM_NT, ntiles = (ne + nt - 1) / nt;
-    std::vector<int> vhoff(ntiles + 1, 0), vhidx, qoff(ntiles + 1, 0), qinc_off(1, 0), elq(ne, 0), halo, nodes;
-    std::vector<uint16_t> qinc;
-    std::vector<int> qlocal(c.np, -1);
-    int nsl = nt, nql = 1;
+    std::vector<int> xoff(ntiles + 1, 0), xq, elq(ne, 0), voff(ntiles + 1, 0), vall, qoff(ntiles + 1, 0), nodes;
+    std::vector<uint16_t> qall, xinc;
+    std::vector<int> qlocal(c.np, -1), row(ne, -1);          // local numbers of the current tile's nodes, staged rows
+    vall.reserve((size_t)ne);
+    qall.reserve((size_t)ntiles * 8 * 48);
+    int nvh = 0, nql = 1;
     for (int t = 0; t < ntiles; t++) {
         const int b = t * nt, en = std::min(ne, b + nt);
+        const size_t v0 = vall.size();
         nodes.clear();
-        halo.clear();
         for (int e = b; e < en; e++) {
             int packed = 0;
             for (int v = 0; v < 3; v++) {
@@ -616,44 +618,54 @@ int build_limtiles(Ctx& c, const std::vector<int>& nm, const std::vector<int>& o
                 packed |= qlocal[n] << (10 * v);
             }
             elq[e] = packed;
+            row[e] = e - b;
         }
         for (int n : nodes)
             for (int j = off[n]; j < off[n + 1]; j++) {
                 const int g = n2e[j] >> 2;
-                if (g < b || g >= en) halo.push_back(g);
+                if (row[g] < 0) { row[g] = 0; vall.push_back(g); }
             }
-        std::sort(halo.begin(), halo.end());
-        halo.erase(std::unique(halo.begin(), halo.end()), halo.end());
-        if (nt + (int)halo.size() > 65535 || (int)nodes.size() > 1023)
+        std::sort(vall.begin() + v0, vall.end());
+        const int nh = (int)(vall.size() - v0);
+        if (nt + nh > 8191 || (int)nodes.size() > 1023)
             return fail("slope limiter tiles: a tile touches too many nodes or elements");
-        for (int n : nodes) {
-            for (int j = off[n]; j < off[n + 1]; j++) {
-                const int g = n2e[j] >> 2;
-                const int r = (g >= b && g < en) ? g - b
-                                                 : nt + (int)(std::lower_bound(halo.begin(), halo.end(), g) - halo.begin());
-                qinc.push_back((uint16_t)r);
+        for (int i = 0; i < nh; i++) row[vall[v0 + i]] = nt + i;
+        for (size_t q = 0; q < nodes.size(); q++) {
+            const int j0 = off[nodes[q]], j1 = off[nodes[q] + 1];
+            for (int i = 0; i < std::max(8, (j1 - j0 + 7) / 8 * 8); i++) {
+                const uint16_t r = (uint16_t)(8 * row[n2e[std::min(j0 + i, j1 - 1)] >> 2]);
+                if (i >= 8 && i % 8 == 0) xq.push_back((int)q);
+                (i < 8 ? qall : xinc).push_back(r);
             }
-            qinc_off.push_back((int)qinc.size());
-            qlocal[n] = -1;
+            qlocal[nodes[q]] = -1;
         }
-        nsl = std::max(nsl, nt + (int)halo.size());
+        for (int e = b; e < en; e++) row[e] = -1;
+        for (size_t i = v0; i < vall.size(); i++) row[vall[i]] = -1;
+        nvh = std::max(nvh, nh);
         nql = std::max(nql, (int)nodes.size());
-        vhidx.insert(vhidx.end(), halo.begin(), halo.end());
-        vhoff[t + 1] = (int)vhidx.size();
+        voff[t + 1] = (int)vall.size();
         qoff[t + 1] = qoff[t] + (int)nodes.size();
+        xoff[t + 1] = (int)xq.size();
     }
-    if ((size_t)8 * (3 * nsl + 6 * nql) > (size_t)c.max_lds)
+    if ((size_t)lim_lds(nvh, nql) > (size_t)c.max_lds)
         return fail("slope limiter tiles: a tile needs more LDS than a block may use");
-    if (vhidx.empty()) vhidx.push_back(0);
-    if (qinc.empty()) qinc.push_back(0);
+    // every tile's lists at the same stride
+    std::vector<int> vhidx(std::max<size_t>(1, (size_t)ntiles * nvh), -1);
+    std::vector<uint16_t> qinc((size_t)ntiles * nql * 8, 0);
+    for (int t = 0; t < ntiles; t++) {
+        std::copy(vall.begin() + voff[t], vall.begin() + voff[t + 1], vhidx.begin() + (size_t)t * nvh);
+        std::copy(qall.begin() + (size_t)8 * qoff[t], qall.begin() + (size_t)8 * qoff[t + 1], qinc.begin() + (size_t)8 * t * nql);
+    }
     Ctx::LimBufs& L = c.lim;
-    L.nsl = nsl;
+    L.nvh = nvh;
     L.nql = nql;
-    HIPCHK(L.vhoff.upload(vhoff.data(), vhoff.size(), c.stream));
+    L.nx = (int)xq.size();
+    if (xq.empty()) { xq.push_back(0); xinc.resize(8, 0); }
     HIPCHK(L.vhidx.upload(vhidx.data(), vhidx.size(), c.stream));
-    HIPCHK(L.qoff.upload(qoff.data(), qoff.size(), c.stream));
-    HIPCHK(L.qinc_off.upload(qinc_off.data(), qinc_off.size(), c.stream));
     HIPCHK(L.qinc.upload(qinc.data(), qinc.size(), c.stream));
+    HIPCHK(L.xoff.upload(xoff.data(), xoff.size(), c.stream));
+    HIPCHK(L.xq.upload(xq.data(), xq.size(), c.stream));
+    HIPCHK(L.xinc.upload(xinc.data(), xinc.size(), c.stream));
     HIPCHK(L.elq.upload(elq.data(), elq.size(), c.stream));
     HIPCHK(c.cmean.alloc((size_t)3 * ne));
     HIPCHK(hipStreamSynchronize(c.stream));
@@ -810,16 +822,18 @@ int init_ctx_common(Ctx& c, const dg_params* prm, bool manning) {
                 if (c.T.phi_area[q][k] != P1Area::phi[q][k] || c.T.mw[q][k] != P1Area::mw[k] ||
                     c.T.srfac[q][k] != P1Area::srfac[q][k])
                     return fail("basis tables: unexpected p=1 area rule");
+    // the limiter fuses the linear modes' corner values likewise
+    auto pow2 = [](double x) { int ex; const double m = std::fabs(std::frexp(x, &ex)); return m == 0.0 || m == 0.5; };
+    for (int q = 0; q < 3; q++)
+        for (int k = 0; k < 3; k++)
+            if (!pow2(c.T.phi_corner[q][k])) return fail("basis tables: a linear mode's corner value is not a power of two");
     // p=1: the stage kernel fuses the edge traces' products and sums, which is exact where the edge values
     // are 0 or powers of two
     if (prm->p == 1)
         for (int l = 0; l < 3; l++)
             for (int q = 0; q < c.T.negp; q++)
-                for (int k = 0; k < c.T.dof; k++) {
-                    int ex;
-                    const double m = std::fabs(std::frexp(c.T.phi_edge[l][q][k], &ex));
-                    if (m != 0.0 && m != 0.5) return fail("basis tables: an edge value of a p=1 mode is not a power of two");
-                }
+                for (int k = 0; k < c.T.dof; k++)
+                    if (!pow2(c.T.phi_edge[l][q][k])) return fail("basis tables: an edge value of a p=1 mode is not a power of two");
     c.dof = c.T.dof; c.nagp = c.T.nagp; c.negp = c.T.negp;
     c.block = prm->p == 1 ? 128 : 64;
     {
@@ -1073,33 +1087,31 @@ int stage_nt(const Ctx& c, int nt) { return c.prm.nolicat != 0 && !stage_split(c
 int ensure_staging(Ctx& c, int nt) {
     if (c.stg.count(nt)) return 0;
     const int ne = c.ne, ntiles = (ne + nt - 1) / nt;
-    std::vector<int> hoff(ntiles + 1, 0), hidx, snbl(ne, 0), halo;
+    std::vector<int> hoff(ntiles + 1, 0), hidx, snbl(ne, 0), row(ne, -1);   // row: staged rows of the current tile's halo
+    hidx.reserve((size_t)ne / 2);
     int hmax = 0;
     for (int t = 0; t < ntiles; t++) {
         const int b = t * nt, en = std::min(ne, b + nt);
-        halo.clear();
+        const size_t h0 = hidx.size();
         for (int e = b; e < en; e++)
             for (int sl = 0; sl < 3; sl++) {
                 if (((side_bits(c.h_sinfo[e], sl) >> 3) & 3) != SIDE_INTERNAL) continue;
                 const int nb = c.h_snbr[(size_t)sl * ne + e];
-                if (nb < b || nb >= en) halo.push_back(nb);
+                if ((nb < b || nb >= en) && row[nb] < 0) { row[nb] = 0; hidx.push_back(nb); }
             }
-        std::sort(halo.begin(), halo.end());
-        halo.erase(std::unique(halo.begin(), halo.end()), halo.end());
-        hmax = std::max(hmax, (int)halo.size());
+        std::sort(hidx.begin() + h0, hidx.end());
+        for (size_t i = h0; i < hidx.size(); i++) row[hidx[i]] = nt + (int)(i - h0);
+        hmax = std::max(hmax, (int)(hidx.size() - h0));
         for (int e = b; e < en; e++) {
             int packed = 0;
             for (int sl = 0; sl < 3; sl++) {
                 if (((side_bits(c.h_sinfo[e], sl) >> 3) & 3) != SIDE_INTERNAL) continue;
                 const int nb = c.h_snbr[(size_t)sl * ne + e];
-                int ln;
-                if (nb >= b && nb < en) ln = nb - b;
-                else ln = nt + (int)(std::lower_bound(halo.begin(), halo.end(), nb) - halo.begin());
-                packed |= ln << (10 * sl);
+                packed |= ((nb >= b && nb < en) ? nb - b : row[nb]) << (10 * sl);
             }
             snbl[e] = packed;
         }
-        hidx.insert(hidx.end(), halo.begin(), halo.end());
+        for (size_t i = h0; i < hidx.size(); i++) row[hidx[i]] = -1;
         hoff[t + 1] = (int)hidx.size();
     }
     const int ns = nt + hmax;
@@ -1244,29 +1256,32 @@ StageArgs stage_args(Ctx& c, int irk, const int slot[], bool captured = false) {
     return a;
 }
 
+LimTiles lim_tiles(const Ctx& c) {
+    const Ctx::LimBufs& L = c.lim;
+    return LimTiles{L.vhidx.p, L.qinc.p, L.xoff.p, L.xq.p, L.xinc.p, L.elq.p, L.nvh, L.nql, L.nx};
+}
+
 // SLOPELIMITER5 (+ WETDRY) on the stage output u, in place; with WETDRY the stage kernel has left
 // u's cell means in c.cmean.
 template <int P>
 int launch_limiter(Ctx& c, double* u, const ElemData& ed, bool capturing) {
     const int ne = c.ne;
-    const int ge = (ne + LIM_NT - 1) / LIM_NT;
     if (!c.lim.elq.p || !c.cmean.p) return fail("internal: slope limiter tiles not built");
     const bool wdon = c.prm.nolifa >= 2;
     const double* cm = wdon ? c.cmean.p : u;
     const size_t cms = wdon ? (size_t)ne : (size_t)c.dof * ne;
-    LimTiles lt{c.lim.vhoff.p, c.lim.vhidx.p, c.lim.qoff.p, c.lim.qinc_off.p, c.lim.qinc.p, c.lim.elq.p,
-                c.lim.nsl, c.lim.nql};
-    const size_t lds = (size_t)8 * (3 * lt.nsl + 6 * lt.nql);
+    const LimTiles lt = lim_tiles(c);
+    const dim3 grid((ne + LIM_NT - 1) / LIM_NT), block(3 * LIM_NT);
+    const size_t lds = lim_lds(lt.nvh, lt.nql);
+    const uint8_t* wd = c.wd[c.wdcur].p;
     int ev = prof_begin(c, K_LIMIT, capturing);
-    if (c.prm.nolifa >= 2) {
-        hipLaunchKernelGGL((limit_wetdry_kernel<P, true, false>), dim3(ge), dim3(LIM_NT), lds, c.stream, ed, u, cm,
-                           cms, lt, (const uint8_t*)c.wd[c.wdcur].p, c.wd[1 - c.wdcur].p, c.wd_active,
-                           (double*)nullptr, (double*)nullptr);
+    if (wdon) {
+        hipLaunchKernelGGL((limit_wetdry_kernel<P, true, false>), grid, block, lds, c.stream, ed, u, cm, cms, lt, wd,
+                           c.wd[1 - c.wdcur].p, c.wd_active, (double*)nullptr, (double*)nullptr);
         c.wdcur = 1 - c.wdcur;
     } else {
-        hipLaunchKernelGGL((limit_wetdry_kernel<P, false, false>), dim3(ge), dim3(LIM_NT), lds, c.stream, ed, u, cm,
-                           cms, lt, (const uint8_t*)c.wd[c.wdcur].p, c.wd[1 - c.wdcur].p, (int*)nullptr,
-                           (double*)nullptr, (double*)nullptr);
+        hipLaunchKernelGGL((limit_wetdry_kernel<P, false, false>), grid, block, lds, c.stream, ed, u, cm, cms, lt, wd,
+                           c.wd[1 - c.wdcur].p, (int*)nullptr, (double*)nullptr, (double*)nullptr);
     }
     prof_end(c, ev);
     HIPCHK(hipGetLastError());
@@ -1279,16 +1294,11 @@ int launch_limiter(Ctx& c, double* u, const ElemData& ed, bool capturing) {
 // limiter's output, gdp gains the vertex-depth terms.
 template <int P>
 int launch_wetdry_rev(Ctx& c, const double* wpre, const uint8_t* flags, double* cot) {
-    const int ne = c.ne;
-    const int ge = (ne + LIM_NT - 1) / LIM_NT;
     if (!c.lim.elq.p) return fail("internal: slope limiter tiles not built");
-    LimTiles lt{c.lim.vhoff.p, c.lim.vhidx.p, c.lim.qoff.p, c.lim.qinc_off.p, c.lim.qinc.p, c.lim.elq.p,
-                c.lim.nsl, c.lim.nql};
-    const size_t lds = (size_t)8 * (3 * lt.nsl + 6 * lt.nql);
-    const ElemData ed = elem_data(c);
-    hipLaunchKernelGGL((limit_wetdry_kernel<P, false, true>), dim3(ge), dim3(LIM_NT), lds, c.stream, ed,
-                       const_cast<double*>(wpre), wpre, (size_t)c.dof * ne, lt, flags, (uint8_t*)nullptr,
-                       (int*)nullptr, cot, c.gdp.p);
+    const LimTiles lt = lim_tiles(c);
+    hipLaunchKernelGGL((limit_wetdry_kernel<P, false, true>), dim3((c.ne + LIM_NT - 1) / LIM_NT), dim3(3 * LIM_NT),
+                       (size_t)lim_lds(lt.nvh, lt.nql), c.stream, elem_data(c), const_cast<double*>(wpre), wpre,
+                       (size_t)c.dof * c.ne, lt, flags, (uint8_t*)nullptr, (int*)nullptr, cot, c.gdp.p);
     HIPCHK(hipGetLastError());
     return 0;
 }

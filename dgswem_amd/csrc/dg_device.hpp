@@ -161,20 +161,22 @@ struct Met {
     double* __restrict__ prn;           // [np] surface pressure (m of water)
 };
 
-// Block-local node bounds of the slope limiter.  Tile t (elements [t*NT, t*NT+NT)) stages the
-// cell means of its own elements (rows 0..NT-1) and of its vertex halo -- the elements outside
-// the tile that share a node with it, vhidx[vhoff[t]..vhoff[t+1]) (rows NT..) -- and forms the
-// bounds of its nodes qnode[qoff[t]..qoff[t+1]) from their incident elements, listed in the
-// node->element order as staged rows qinc[qinc_off[q]..qinc_off[q+1]).  elq packs each element's
-// three tile-local node numbers (10 bits each).
+// Block-local node bounds of the slope limiter.  Tile t (elements [t*nt, t*nt+nt)) stages the
+// cell means of its own elements (rows 0..nt-1) and of its vertex halo -- the elements outside
+// the tile that share a node with it, vhidx[t*nvh..t*nvh+nvh), -1 past its last (rows nt..) -- and forms
+// the bounds of its nodes from their incident elements: node q's first eight as staged rows (times 8, the
+// byte offset) qinc[(t*nql+q)*8..+8), fewer repeated (min and max are idempotent), and further ones in the extra entries
+// xoff[t]..xoff[t+1) (xq: the node, xinc: eight rows).  elq packs each element's three tile-local node
+// numbers (10 bits each).
 struct LimTiles {
-    const int* __restrict__ vhoff;
     const int* __restrict__ vhidx;
-    const int* __restrict__ qoff;
-    const int* __restrict__ qinc_off;
     const uint16_t* __restrict__ qinc;
+    const int* __restrict__ xoff;
+    const int* __restrict__ xq;
+    const uint16_t* __restrict__ xinc;
     const int* __restrict__ elq;
-    int nsl, nql;                       // LDS rows: staged elements, nodes (largest tile)
+    int nvh, nql;                       // halo entries and nodes per tile (the largest tile's)
+    int nx;                             // extra entries of all tiles (none: xoff is not read)
 };
 
 // Local Lax-Friedrichs flux (src/numerical_flux.F:750-1022), operation order kept.

@@ -1336,28 +1336,100 @@ __global__ void __launch_bounds__(256) node_minmax_kernel(int np, int ne, const 
 }
 
 // ------------------------------------------------------------------------------------------
-// SLOPELIMITER5 (src/slopelimiter.F:3290-3676) then WETDRY (src/wetdry.F), one thread per element.
+// SLOPELIMITER5 (src/slopelimiter.F:3290-3676) then WETDRY (src/wetdry.F).
 // The node bounds of part 1 are formed per tile in LDS (LimTiles): the tile stages the updated cell
 // means of its elements and of its vertex halo, each node of the tile takes the min/max over its
-// incident elements in the node->element order (as node_minmax_kernel does, so the bounds are the
-// same bit for bit), and each element then limits its modes 2-3 against the bounds of its nodes.
+// incident elements, and each element then limits its modes 2-3 against the bounds of its nodes.
 // With WETDRY the cell means come from the stage kernel's copy `cmean` [3][ne] (field stride
 // cms = ne): WETDRY rewrites some cell means of u in place, which other tiles' halos must not see.
 // Without it they are read from u itself (cms = DOF*ne), whose cell means the limiter keeps.
-// Blocks of LIM_NT threads; the launch passes 8*(3*nsl + 6*nql) bytes of dynamic LDS.
 // ------------------------------------------------------------------------------------------
+// Three waves per 64 elements: wave c stages, bounds and limits field c, so its branches on c are uniform.  What
+// bounds it is memory (about 165 bytes per element at p=1) and, on small meshes, the chain of loads before the first
+// bound.  A third of the work per lane keeps three times the loads under way, and lists at fixed strides need no
+// look-up before them.  Tiles of 64 and of 256 elements take the same time on large meshes (the larger halo of the
+// small ones comes from the L2), and on small ones 64 use four times the compute units (7.4 against 9.0 us at 5k
+// elements).  The modes past the third are touched only where WETDRY changes the element.
+// Per launch, one lane per element and 256-element tiles before, now: 997,306 elements p=1 48.2 and 49.2 us, 298,700
+// elements p=2 27.6 and 20.5 us, 4,783 elements p=1 9.2 and 4.6 us.
+//
 // With WDADJ (the adjoint's reverse sweep; WETDRY false) the kernel writes nothing to u: each
-// element's limited modes, formed in registers exactly as the forward formed them, go to the
+// element's limited modes, formed exactly as the forward formed them, go to the
 // frozen-branch WETDRY reverse of that element (wetdry_adj_element), which turns the cotangent ub
 // of WETDRY's output into that of its input and adds the vertex-depth cotangents to gdp.
-constexpr int LIM_NT = 256;
+//
+// The launch passes lim_lds() bytes of dynamic LDS.
+constexpr int LIM_NT = 64;               // elements per tile
+constexpr int lim_lds(int nvh, int nql) {
+    return 8 * (3 * (LIM_NT + nvh) + 6 * nql > 9 * LIM_NT ? 3 * (LIM_NT + nvh) + 6 * nql : 9 * LIM_NT) + LIM_NT;
+}
+
+// x/3, correctly rounded: the rounded product with 1/3, its exact remainder and one correction (Markstein), in four
+// instructions instead of eleven; the fix-up keeps infinities and zeros as a division has them.
+__device__ __forceinline__ double div3(double x) {
+    const double q = x * (1.0 / 3.0);
+    return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-3.0, q, x), 1.0 / 3.0, q), 3.0, x);
+}
+
+// fmin and fmax as one instruction each: of the library's the compiler makes two where it cannot see that an operand
+// (one read from memory) is no signalling NaN, which no arithmetic here produces.
+__device__ __forceinline__ double min1(double a, double b) {
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ double max1(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// SLOPELIMITER5 of one field of one element: mean c0, linear modes w1 and w2 (in place), its nodes' bounds.
+// SIGNDIF is +-1, so products with it are exact: they become sign flips and fuse with the sums after them, and
+// DIF > 0 is a comparison of the vertex value with the mean.
+__device__ __forceinline__ void limit_field(const DevTables& T, double c0, double& w1, double& w2,
+                                            const double (&vmin)[3], const double (&vmax)[3]) {
+    double v[3];
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        // the linear modes' corner values are powers of two or zero (checked at set-up): exact products fuse
+        const double t = __builtin_fma(T.phi_corner[c][2], w2, __builtin_fma(T.phi_corner[c][1], w1, c0));
+        v[c] = max1(min1(t, vmax[c]), vmin[c]);
+    }
+#pragma unroll
+    for (int ll = 0; ll < 3; ll++) {
+        const double sumloc = div3(v[0] + v[1] + v[2]);
+        double sumdif = (sumloc - c0) * 3.0;
+        const int sgn = __double2hiint(sumdif) & 0x80000000;
+        const bool up = sgn == 0;
+        const double signdif = __hiloint2double(0x3ff00000 | sgn, 0);
+        bool d[3];
+#pragma unroll
+        for (int c = 0; c < 3; c++) d[c] = up ? v[c] > c0 : v[c] < c0;
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            // REDFAC = (SUMDIF*SIGNDIF)/DIV with DIV the positive differences not yet passed: at most 3 - k.
+            // x/1 and x/2 are x and x*0.5 exactly.
+            const double a = __hiloint2double(__double2hiint(sumdif) ^ sgn, __double2loint(sumdif));
+            double redfac = a;
+            if (k < 2) redfac = (k == 0 ? d[1] || d[2] : d[2]) ? a * 0.5 : a;
+            if (k == 0 && d[1] && d[2]) redfac = div3(a);
+            redfac = d[k] ? redfac : 0.0;
+            redfac = min1(redfac, up ? v[k] - vmin[k] : vmax[k] - v[k]);
+            sumdif = __builtin_fma(-redfac, signdif, sumdif);
+            v[k] = __builtin_fma(-redfac, signdif, v[k]);
+        }
+    }
+    w1 = -(1.0 / 6.0 * (v[0] + v[1])) + 1.0 / 3.0 * v[2];
+    w2 = -(0.5 * v[0]) + 0.5 * v[1];
+}
 
 template <int P>
 __device__ void wetdry_adj_element(const DevTables& T, const double (&U)[3][3], const double (&D)[3], int wdflg,
                                    double H0, int e, int ne, double* __restrict__ ub, double* __restrict__ gdp);
 
 template <int P, bool WETDRY, bool WDADJ>
-__global__ void __launch_bounds__(LIM_NT) limit_wetdry_kernel(ElemData E, double* __restrict__ u,
+__global__ void __launch_bounds__(3 * LIM_NT) __attribute__((amdgpu_waves_per_eu(4))) limit_wetdry_kernel(ElemData E, double* __restrict__ u,
                                                               const double* __restrict__ cmean, size_t cms,
                                                               LimTiles lt,
                                                               const uint8_t* __restrict__ wd_in,
@@ -1366,156 +1438,151 @@ __global__ void __launch_bounds__(LIM_NT) limit_wetdry_kernel(ElemData E, double
                                                               double* __restrict__ ub, double* __restrict__ gdp) {
     static_assert(!(WETDRY && WDADJ), "the WETDRY reverse starts from the limiter's output alone");
     constexpr int DOF = (P + 1) * (P + 2) / 2;
+    constexpr int NT = LIM_NT;
     const DevTables& T = tab<P>();
     const int ne = E.ne;
-    const int tid = threadIdx.x;
+    const int c = __builtin_amdgcn_readfirstlane(threadIdx.x / NT), le = threadIdx.x - c * NT;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
-    const int e = tile * LIM_NT + tid;
+    const int e = tile * NT + le;
+    const bool valid = e < ne;
     extern __shared__ double lds[];
-    const int nsl = lt.nsl, nql = lt.nql;
-    double* const cm = lds;                  // [3][nsl] staged cell means
-    double* const bnd = lds + 3 * nsl;       // [6][nql] zmin zmax qxmin qxmax qymin qymax
-    // the element's own loads first, so that their latency overlaps the staging below (lanes past
-    // the last element read element ne-1 and exit after the second barrier)
-    const int ec = e < ne ? e : ne - 1;
+    const int nsl = NT + lt.nvh, nql = lt.nql;
+    double* const cm = lds + c * nsl;                       // field c's staged cell means
+    double* const bnd = lds + 3 * nsl + 2 * c * nql;        // field c's node minima, maxima
+    // the first halo entry's and node's indices and the element's own loads, then the staging (lanes past the last
+    // element read element ne-1 and write nothing)
+    const int ec = valid ? e : ne - 1;
+    const int* vh = lt.vhidx + (size_t)tile * lt.nvh;
+    const uint4* qi = reinterpret_cast<const uint4*>(lt.qinc) + (size_t)tile * nql;
+    const int g = le < lt.nvh ? vh[le] : -1;
+    uint4 rq = le < nql ? qi[le] : make_uint4(0, 0, 0, 0);
+    const double* row = cmean + (size_t)c * cms;
+    const double c0 = at(row, ec);
+    double w1 = at(u + (size_t)(c * DOF + 1) * ne, ec), w2 = at(u + (size_t)(c * DOF + 2) * ne, ec);
+    const int lq = at(lt.elq, ec);
+    double D[3] = {0.0, 0.0, 0.0}, h0 = 0.0;
+    int wdi = 0;
+    if ((WETDRY || WDADJ) && c == 0) {
+#pragma unroll
+        for (int v = 0; v < 3; v++) D[v] = at(E.dpv + (size_t)v * ne, ec);
+        const int sid = E.sid ? (int)at(E.sid, ec) : 0;
+        h0 = E.scen[sid].h0;
+        wdi = at(wd_in, ec);
+    }
+    const double m = at(row, g < 0 ? 0 : g);
+    cm[le] = c0;
+    if (g >= 0) cm[NT + le] = m;
+#pragma unroll 1
+    for (int h = le + NT; h < lt.nvh; h += NT) {
+        const int gh = vh[h];
+        if (gh < 0) break;
+        cm[NT + h] = at(row, gh);
+    }
+    __syncthreads();
+    // the bounds of the tile's nodes
+    const char* const cmb = reinterpret_cast<const char*>(cm);
+    auto minmax8 = [&](const uint4& r, double& lo, double& hi) {
+        const uint32_t p[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const double a = *reinterpret_cast<const double*>(cmb + (p[i] & 0xffffu));
+            const double b = *reinterpret_cast<const double*>(cmb + (p[i] >> 16));
+            lo = min1(lo, min1(a, b));
+            hi = max1(hi, max1(a, b));
+        }
+    };
+    for (int q = le; q < nql; q += NT) {
+        if (q != le) rq = qi[q];
+        double lo = 99999., hi = -99999.;
+        minmax8(rq, lo, hi);
+        bnd[q] = lo;
+        bnd[nql + q] = hi;
+    }
+    if (lt.nx > 0) {
+        // nodes with more than eight elements: one lane of each field goes through the tile's extra entries
+        const int x0 = lt.xoff[tile], x1 = lt.xoff[tile + 1];
+        if (x1 > x0) {
+            __syncthreads();
+            if (le == 0)
+                for (int x = x0; x < x1; x++) {
+                    const int q = lt.xq[x];
+                    double lo = bnd[q], hi = bnd[nql + q];
+                    minmax8(reinterpret_cast<const uint4*>(lt.xinc)[x], lo, hi);
+                    bnd[q] = lo;
+                    bnd[nql + q] = hi;
+                }
+        }
+    }
+    __syncthreads();
+    {
+        const int q[3] = {lq & 1023, (lq >> 10) & 1023, (lq >> 20) & 1023};
+        double vmin[3], vmax[3];
+#pragma unroll
+        for (int i = 0; i < 3; i++) { vmin[i] = bnd[q[i]]; vmax[i] = bnd[nql + q[i]]; }
+        limit_field(T, c0, w1, w2, vmin, vmax);
+    }
+    if (!WETDRY && !WDADJ) {
+        if (!valid) return;
+        at(u + (size_t)(c * DOF + 1) * ne, e) = w1;
+        at(u + (size_t)(c * DOF + 2) * ne, e) = w2;
+        return;
+    }
+    // elements that WETDRY changes: the three lanes' values meet in LDS and the element's first lane goes on alone
+    uint8_t* const keep = reinterpret_cast<uint8_t*>(lds + max(3 * nsl + 6 * nql, 9 * NT));
+    bool mine = true;
+    if (c == 0) {
+        if (valid) {
+            const double U[3][DOF] = {{c0, w1, w2}};
+            mine = wetdry_keeps<P>(T, U, D, wdi, h0);
+        }
+        keep[le] = mine;
+    }
+    if (!__syncthreads_or(!mine)) {
+        if (WDADJ || !valid) return;
+        if (c == 0) at(wd_out, e) = 1;
+        at(u + (size_t)(c * DOF + 1) * ne, e) = w1;
+        at(u + (size_t)(c * DOF + 2) * ne, e) = w2;
+        return;
+    }
+    mine = keep[le];
+    double* const ex = lds;                                 // [field*3 + mode][NT]
+    if (!mine) {
+        ex[(c * 3) * NT + le] = c0;
+        ex[(c * 3 + 1) * NT + le] = w1;
+        ex[(c * 3 + 2) * NT + le] = w2;
+    } else if (WETDRY && valid) {
+        if (c == 0) at(wd_out, e) = 1;
+        at(u + (size_t)(c * DOF + 1) * ne, e) = w1;
+        at(u + (size_t)(c * DOF + 2) * ne, e) = w2;
+    }
+    __syncthreads();
+    if (mine || c != 0) return;
+    if (WDADJ) {
+        double U3[3][3];
+#pragma unroll
+        for (int f = 0; f < 3; f++)
+#pragma unroll
+            for (int k = 0; k < 3; k++) U3[f][k] = ex[(f * 3 + k) * NT + le];
+        wetdry_adj_element<P>(T, U3, D, wdi, h0, e, ne, ub, gdp);
+        return;
+    }
     double U[3][DOF];
 #pragma unroll
     for (int f = 0; f < 3; f++)
 #pragma unroll
-        for (int k = 1; k < DOF; k++) U[f][k] = u[(size_t)(f * DOF + k) * ne + ec];
-    const int lq = lt.elq[ec];
-    double D[3] = {0.0, 0.0, 0.0}, h0 = 0.0;
-    int wdi = 0;
-    if (WETDRY || WDADJ) {
-#pragma unroll
-        for (int v = 0; v < 3; v++) D[v] = E.dpv[(size_t)v * ne + ec];
-        const int sid = E.sid ? (int)E.sid[ec] : 0;
-        h0 = E.scen[sid].h0;
-        wdi = wd_in[ec];
-    }
-    {
-        // the tile's cell means and its vertex halo's, two entries per lane per pass with all their
-        // loads issued before any is stored
-        const int h0t = lt.vhoff[tile], nh = lt.vhoff[tile + 1] - h0t;
-        for (int j = tid; j < LIM_NT + nh; j += 2 * LIM_NT) {
-            const int j2 = j + LIM_NT;
-            const bool has2 = j2 < LIM_NT + nh;
-            int g = j < LIM_NT ? tile * LIM_NT + j : lt.vhidx[h0t + j - LIM_NT];
-            int g2 = has2 ? lt.vhidx[h0t + j2 - LIM_NT] : ne;
-            const bool ok = g < ne, ok2 = g2 < ne;
-            g = ok ? g : 0;
-            g2 = ok2 ? g2 : 0;
-            const double z = cmean[g], x = cmean[cms + g], y = cmean[2 * cms + g];
-            const double z2 = cmean[g2], x2 = cmean[cms + g2], y2 = cmean[2 * cms + g2];
-            if (ok) { cm[j] = z; cm[nsl + j] = x; cm[2 * nsl + j] = y; }
-            if (ok2) { cm[j2] = z2; cm[nsl + j2] = x2; cm[2 * nsl + j2] = y2; }
-        }
-    }
-    __syncthreads();
-    {
-        const int q0 = lt.qoff[tile], nq = lt.qoff[tile + 1] - q0;
-        for (int q = tid; q < nq; q += LIM_NT) {
-            double zmin = 99999., zmax = -99999., xmin = 99999., xmax = -99999., ymin = 99999., ymax = -99999.;
-            const int i1 = lt.qinc_off[q0 + q + 1];
-            // up to eight incidences per pass, their rows loaded together; past the node's last
-            // incidence the pass repeats it (min and max are idempotent, so a repeat changes nothing)
-            constexpr int B = 8;
-            for (int i = lt.qinc_off[q0 + q]; i < i1; i += B) {
-                int r[B];
-#pragma unroll
-                for (int b = 0; b < B; b++) r[b] = lt.qinc[min(i + b, i1 - 1)];
-#pragma unroll
-                for (int b = 0; b < B; b++) {
-                    const double z = cm[r[b]], x = cm[nsl + r[b]], y = cm[2 * nsl + r[b]];
-                    zmin = fmin(zmin, z); xmin = fmin(xmin, x); ymin = fmin(ymin, y);
-                    zmax = fmax(zmax, z); xmax = fmax(xmax, x); ymax = fmax(ymax, y);
-                }
-            }
-            bnd[q] = zmin; bnd[nql + q] = zmax; bnd[2 * nql + q] = xmin;
-            bnd[3 * nql + q] = xmax; bnd[4 * nql + q] = ymin; bnd[5 * nql + q] = ymax;
-        }
-    }
-    __syncthreads();
-    if (e >= ne) return;
-#pragma unroll
-    for (int f = 0; f < 3; f++) U[f][0] = cm[f * nsl + tid];
-    // the limiter keeps the cell means; wetting and drying changes them only for some elements,
-    // so a cell mean is written back only when its bits changed
-    const double c0in[3] = {U[0][0], U[1][0], U[2][0]};
-    double bmin[3][3], bmax[3][3];
-    {
-        const int q[3] = {lq & 1023, (lq >> 10) & 1023, (lq >> 20) & 1023};
-#pragma unroll
-        for (int iv = 0; iv < 3; iv++)
-#pragma unroll
-            for (int c = 0; c < 3; c++) {
-                bmin[iv][c] = bnd[(2 * iv) * nql + q[c]];
-                bmax[iv][c] = bnd[(2 * iv + 1) * nql + q[c]];
-            }
-    }
-    {
-#pragma unroll
-        for (int iv = 0; iv < 3; iv++) {
-            const double* vmin = bmin[iv];
-            const double* vmax = bmax[iv];
-            const double c0 = U[iv][0];
-            double v[3];
-#pragma unroll
-            for (int c = 0; c < 3; c++) {
-                double t = c0;
-#pragma unroll
-                for (int kk = 1; kk < 3; kk++) t = t + T.phi_corner[c][kk] * U[iv][kk];
-                v[c] = fmax(fmin(t, vmax[c]), vmin[c]);
-            }
-#pragma unroll
-            for (int ll = 0; ll < 3; ll++) {
-                const double sumloc = (v[0] + v[1] + v[2]) / 3.0;
-                double sumdif = (sumloc - c0) * 3.0;
-                const double signdif = copysign(1.0, sumdif);
-                double dif[3];
-#pragma unroll
-                for (int c = 0; c < 3; c++) dif[c] = (v[c] - c0) * signdif;
-                int kdp = (dif[0] > 0) + (dif[1] > 0) + (dif[2] > 0);
-#pragma unroll
-                for (int k = 0; k < 3; k++) {
-                    double redfac;
-                    if (dif[k] > 0) {
-                        // (sumdif*signdif)/DIV with DIV = kdp, which is 1, 2 or 3 here: x/1 and
-                        // x/2 are x and x*0.5 exactly, so only DIV = 3 needs a division
-                        const double a = sumdif * signdif;
-                        redfac = kdp == 1 ? a : (kdp == 2 ? a * 0.5 : a / 3.0);
-                        kdp = kdp - 1;
-                    } else {
-                        redfac = 0;
-                    }
-                    const double redmax = (signdif > 0) ? v[k] - vmin[k] : vmax[k] - v[k];
-                    redfac = fmin(redfac, redmax);
-                    sumdif = sumdif - redfac * signdif;
-                    v[k] = v[k] - redfac * signdif;
-                }
-            }
-            U[iv][1] = -(1.0 / 6.0 * (v[0] + v[1])) + 1.0 / 3.0 * v[2];
-            U[iv][2] = -(0.5 * v[0]) + 0.5 * v[1];
-        }
-    }
-    if (WDADJ) {
-        const double U3[3][3] = {{U[0][0], U[0][1], U[0][2]}, {U[1][0], U[1][1], U[1][2]}, {U[2][0], U[2][1], U[2][2]}};
-        wetdry_adj_element<P>(T, U3, D, wdi, h0, e, ne, ub, gdp);
-        return;
-    }
-    if (WETDRY) {
-        const double c13 = 1.0 / 3.0, c16 = 1.0 / 6.0;
-        const double hb[3] = {c13 * (D[0] + D[1] + D[2]), -(c16 * (D[0] + D[1])) + c13 * D[2], -(0.5 * D[0]) + 0.5 * D[1]};
-        const double dpe_min = fmin(fmin(D[0], D[1]), D[2]);
-        if (wd_active && !wetdry_keeps<P>(T, U, D, wdi, h0)) wd_active[0] = 1;
-        wd_out[e] = (uint8_t)wetdry_element<P>(T, U, D, hb, dpe_min, wdi, h0);
-    }
+        for (int k = 0; k < DOF; k++) U[f][k] = k < 3 ? ex[(f * 3 + k) * NT + le] : at(u + (size_t)(f * DOF + k) * ne, e);
+    const double c13 = 1.0 / 3.0, c16 = 1.0 / 6.0;
+    const double hb[3] = {c13 * (D[0] + D[1] + D[2]), -(c16 * (D[0] + D[1])) + c13 * D[2], -(0.5 * D[0]) + 0.5 * D[1]};
+    const double dpe_min = fmin(fmin(D[0], D[1]), D[2]);
+    if (wd_active) wd_active[0] = 1;
+    at(wd_out, e) = (uint8_t)wetdry_element<P>(T, U, D, hb, dpe_min, wdi, h0);
 #pragma unroll
     for (int f = 0; f < 3; f++) {
-        if (WETDRY && __double_as_longlong(U[f][0]) != __double_as_longlong(c0in[f]))
-            u[(size_t)(f * DOF) * ne + e] = U[f][0];
+        // wetting and drying changes the cell mean only of some elements: written back when its bits changed
+        if (__double_as_longlong(U[f][0]) != __double_as_longlong(ex[(f * 3) * NT + le]))
+            at(u + (size_t)(f * DOF) * ne, e) = U[f][0];
 #pragma unroll
-        for (int k = 1; k < DOF; k++) u[(size_t)(f * DOF + k) * ne + e] = U[f][k];
+        for (int k = 1; k < DOF; k++) at(u + (size_t)(f * DOF + k) * ne, e) = U[f][k];
     }
 }
 

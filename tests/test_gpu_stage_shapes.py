@@ -90,3 +90,40 @@ def test_depths_outside_the_short_flux(p, depth):
         ok = ~np.isnan(y)
         assert ok.any() or depth == 0.0
         np.testing.assert_array_equal(x[ok], y[ok])
+
+
+def fan(k, p):
+    """A closed disc of k sectors and three rings around one node: the centre node belongs to k elements (the
+    limiter's node lists hold eight per entry)."""
+    rings = 3
+    r = np.concatenate([[0.0], np.repeat(np.arange(1, rings + 1) * 1000.0, k)])
+    t = np.concatenate([[0.0], np.tile(np.arange(k) * 2.0 * np.pi / k, rings)])
+    nid = lambda i, j: 2 + (i - 1) * k + j % k
+    nm = [(1, nid(1, j), nid(1, j + 1)) for j in range(k)]
+    for i in range(1, rings):
+        for j in range(k):
+            nm += [(nid(i, j), nid(i + 1, j), nid(i + 1, j + 1)), (nid(i, j), nid(i + 1, j + 1), nid(i, j + 1))]
+    c = closed(1, 1, p, nolifa=2, slopeflag=5)
+    c.x, c.y = r * np.cos(t), r * np.sin(t)
+    c.nm = np.array(nm, dtype=np.int32)
+    n = len(c.x)
+    c.slam, c.sfea, c.sfac, c.corif = c.x / 6378206.4, c.y / 6378206.4, np.ones(n), np.zeros(n)
+    c.dp = 3.0 - 0.0015 * c.x
+    c.land_segs = [(0, np.array([nid(rings, j) for j in range(k + 1)], dtype=np.int32))]
+    c.params.dtdp = 0.5
+    return c
+
+
+@pytest.mark.parametrize("p", [1, 2])
+@pytest.mark.parametrize("k", [5, 8, 9, 17])
+def test_limiter_nodes_of_many_elements(k, p):
+    c = fan(k, p)
+    rng = np.random.default_rng(k)
+    ze, qx, qy, wd = wetdry_state(c, 1.0)
+    wet = wd == 1
+    ze[wet, 1:3] += rng.uniform(-0.3, 0.3, (wet.sum(), 2))
+    qx[wet, :3] += rng.uniform(-1.0, 1.0, (wet.sum(), 3))
+    o = Oracle(c, threads=1)
+    o.set_state(ze, qx, qy, wd)
+    o.step(20)
+    same(run(c, 20, (ze, qx, qy, wd)), o.state())
