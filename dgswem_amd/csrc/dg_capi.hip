@@ -126,6 +126,7 @@ struct Ctx {
     DevBuf<double> r[KMAXRK];
     bool keep_r[KMAXRK] = {};
     DevBuf<uint8_t> wd[2];
+    DevBuf<int> iflags;                          // WDFLG as the host's integers (dg_gpu_get_state, dg_gpu_set_state)
     int wdcur = 0;
     // mesh
     DevBuf<uint16_t> sid;
@@ -1649,6 +1650,20 @@ int adj_backward(Ctx& c, int it0, int nsteps, int interval, double weight) {
     return 0;
 }
 
+// The stage slot after the current one: free between steps (the next step's first stage writes it).
+double* spare_state(Ctx& c) { return c.u[(c.ucur + 1) % (c.rk.nrk + 1)].p; }
+
+// The current state to (OUT) or from the host's layout in `aos`.
+template <bool OUT>
+int launch_state_layout(Ctx& c, double* aos) {
+    const size_t n = (size_t)3 * c.dof * c.ne;
+    const dim3 grid((unsigned)((n + 255) / 256)), block(256);
+    if (c.prm.p == 1) hipLaunchKernelGGL((state_layout_kernel<3, OUT>), grid, block, 0, c.stream, c.ne, c.u[c.ucur].p, aos);
+    else hipLaunchKernelGGL((state_layout_kernel<6, OUT>), grid, block, 0, c.stream, c.ne, c.u[c.ucur].p, aos);
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
 int validate(const dg_params* p) {
     if (!p) return fail("null parameters");
     if (p->p < 1 || p->p > 2) return fail("p must be 1 or 2");
@@ -1945,18 +1960,18 @@ int dg_holland_storm_at(int nrec, const int* rec, const int* ref, int storm_numb
 int dg_gpu_set_state(int h, const double* ze, const double* qx, const double* qy, const int* wdflg) {
     Ctx* c = get(h);
     if (!c) return 1;
-    const int ne = c->ne, dof = c->dof;
-    std::vector<double> buf((size_t)3 * dof * ne);
+    const size_t n = (size_t)c->ne * c->dof;
     const double* src[3] = {ze, qx, qy};
+    double* aos = spare_state(*c);
     for (int f = 0; f < 3; f++)
-        for (int e = 0; e < ne; e++)
-            for (int k = 0; k < dof; k++) buf[((size_t)f * dof + k) * ne + e] = src[f][(size_t)e * dof + k];
-    HIPCHK(hipMemcpyAsync(c->u[c->ucur].p, buf.data(), buf.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    std::vector<uint8_t> w;
+        HIPCHK(hipMemcpyAsync(aos + f * n, src[f], n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    if (launch_state_layout<false>(*c, aos)) return 1;
     if (wdflg) {
-        w.resize(ne);
-        for (int e = 0; e < ne; e++) w[e] = wdflg[e] ? 1 : 0;
-        HIPCHK(hipMemcpyAsync(c->wd[c->wdcur].p, w.data(), ne, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(c->iflags.alloc(c->ne));
+        HIPCHK(hipMemcpyAsync(c->iflags.p, wdflg, (size_t)c->ne * sizeof(int), hipMemcpyHostToDevice, c->stream));
+        hipLaunchKernelGGL((flags_kernel<false>), dim3((c->ne + 255) / 256), dim3(256), 0, c->stream, c->ne,
+                           c->wd[c->wdcur].p, c->iflags.p);
+        HIPCHK(hipGetLastError());
     }
     HIPCHK(hipStreamSynchronize(c->stream));
     return 0;
@@ -1965,19 +1980,20 @@ int dg_gpu_set_state(int h, const double* ze, const double* qx, const double* qy
 int dg_gpu_get_state(int h, double* ze, double* qx, double* qy, int* wdflg) {
     Ctx* c = get(h);
     if (!c) return 1;
-    const int ne = c->ne, dof = c->dof;
-    std::vector<double> buf((size_t)3 * dof * ne);
-    HIPCHK(hipMemcpyAsync(buf.data(), c->u[c->ucur].p, buf.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    std::vector<uint8_t> w(ne);
-    HIPCHK(hipMemcpyAsync(w.data(), c->wd[c->wdcur].p, ne, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    const size_t n = (size_t)c->ne * c->dof;
     double* dst[3] = {ze, qx, qy};
-    for (int f = 0; f < 3; f++) {
-        if (!dst[f]) continue;
-        for (int e = 0; e < ne; e++)
-            for (int k = 0; k < dof; k++) dst[f][(size_t)e * dof + k] = buf[((size_t)f * dof + k) * ne + e];
+    double* aos = spare_state(*c);
+    if (launch_state_layout<true>(*c, aos)) return 1;
+    if (wdflg) {
+        HIPCHK(c->iflags.alloc(c->ne));
+        hipLaunchKernelGGL((flags_kernel<true>), dim3((c->ne + 255) / 256), dim3(256), 0, c->stream, c->ne,
+                           c->wd[c->wdcur].p, c->iflags.p);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(wdflg, c->iflags.p, (size_t)c->ne * sizeof(int), hipMemcpyDeviceToHost, c->stream));
     }
-    if (wdflg) for (int e = 0; e < ne; e++) wdflg[e] = w[e];
+    for (int f = 0; f < 3; f++)
+        if (dst[f]) HIPCHK(hipMemcpyAsync(dst[f], aos + f * n, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
     return 0;
 }
 
