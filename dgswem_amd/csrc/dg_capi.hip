@@ -165,12 +165,16 @@ struct Ctx {
     // forcing
     DevBuf<double> emo, efa, qnam, qnph, argj, rff, fargj, frff;
     DevBuf<int> step;                            // device step counter within the current tables
-    DevBuf<double> tz;                           // tidal terms of the current step [stage][needs][nbfr][2]
+    DevBuf<double> tz;                           // tidal terms [step of the batch][stage][needs][nbfr][2]
     DevBuf<uint16_t> osid;                       // scenario of each ocean edge (ensembles)
     int tzn = 0;                                 // tidal terms per stage
     int hstep = 0;                               // the same index for eager (uncaptured) launches
+    int tn = 0;                                  // steps in the current tables
+    // the forcing arrays (tz, fz, tip2 and the storm's node arrays) hold the steps fb0..fb0+fbn-1 of the
+    // current tables (fbn = 0: none), at most fbatch
+    int fbatch = 0, fb0 = 0, fbn = 0;
     int rows = 0;                                // table rows per scenario
-    // specified normal flux of the current step at every flux-edge point, and each flux edge's
+    // specified normal flux of the batch's steps at every flux-edge point, and each flux edge's
     // scenario (flow_kernel)
     DevBuf<double> fz;
     DevBuf<uint16_t> fsid;
@@ -307,18 +311,21 @@ ElemData elem_data(Ctx& c) {
     return E;
 }
 
-// Forcing-table arguments.  Captured launches read the step index from the device counter (graph
-// replays advance it); eager launches take it as an argument.
-Forcing forcing(Ctx& c, bool captured = false) {
+// Forcing-table arguments.  Captured launches are the step `cap` >= 0 of their graph and add the device
+// counter (which replays advance); eager launches (cap < 0) are the step c.hstep of the tables.
+int batch_step(const Ctx& c, int cap) { return cap >= 0 ? cap : c.hstep - c.fb0; }
+
+Forcing forcing(Ctx& c, int cap = -1) {
     Forcing F{};
     F.nbfr = c.nbfr; F.nffr = c.nffr; F.rows = c.rows; F.nrk = c.rk.nrk;
-    F.step = captured ? c.step.p : nullptr;
-    F.step_imm = c.hstep;
+    F.step = cap >= 0 ? c.step.p : nullptr;
+    F.step_imm = cap >= 0 ? cap : c.hstep;
     F.emo = c.emo.p; F.efa = c.efa.p; F.qnam = c.qnam.p; F.qnph = c.qnph.p;
     F.argj = c.argj.p; F.rff = c.rff.p; F.fargj = c.fargj.p; F.frff = c.frff.p;
     F.ramp = c.ramp.p;
-    F.tz = c.tz.p; F.tzn = c.tzn;
-    F.fz = c.fz.p; F.fzn = c.fzn;
+    const size_t row = (size_t)batch_step(c, cap) * c.rk.nrk;
+    F.tz = c.tz.p + row * c.tzn; F.tzn = c.tzn;
+    F.fz = c.fz.p + row * c.fzn; F.fzn = c.fzn;
     F.ets = c.eser ? c.ets.p : nullptr;
     F.qts = c.fser ? c.qts.p : nullptr;
     F.nfeds = c.foff[c.S];
@@ -336,13 +343,18 @@ Tip tip_args(Ctx& c) {
     return t;
 }
 
-Met met_args(Ctx& c) {
+const double* tip_stage(const Ctx& c, int irk, int cap = -1) {
+    return c.tip ? c.tip2.p + ((size_t)batch_step(c, cap) * c.rk.nrk + irk) * c.np : nullptr;
+}
+
+Met met_args(Ctx& c, int cap = -1) {
     Met m{};
     m.np = c.np; m.rows = kTableChunk;
     m.row = c.mrow.p;
     m.nsid = c.S > 1 ? c.nsid.p : nullptr;
     m.xc = c.mxc.p; m.yc = c.myc.p; m.cosy = c.mcosy.p; m.cor = c.mcor.p;
-    m.wx = c.mwx.p; m.wy = c.mwy.p; m.wm = c.mwm.p; m.cd = c.mcd.p; m.prn = c.mprn.p;
+    const size_t o = (size_t)batch_step(c, cap) * c.np;
+    m.wx = c.mwx.p + o; m.wy = c.mwy.p + o; m.wm = c.mwm.p + o; m.cd = c.mcd.p + o; m.prn = c.mprn.p + o;
     return m;
 }
 
@@ -504,6 +516,22 @@ Scen scen_of(const Member& m) {
     return s;
 }
 
+// The forcing arrays for the steps of one batch.  A batch is worth its size while its launches are bound by
+// latency and its arrays stay in the caches (8 MB); it covers at least a captured graph's steps.
+int alloc_batch(Ctx& c) {
+    const size_t nrk = c.rk.nrk, period = nrk + 1;
+    const size_t step = 8 * (nrk * ((size_t)c.tzn + c.fzn + (c.tip ? c.np : 0)) + (c.met ? 5 * (size_t)c.np : 0));
+    const size_t k = std::max(period, std::min<size_t>(64, ((size_t)8 << 20) / std::max<size_t>(step, 1)));
+    c.fbatch = (int)k;
+    c.fbn = 0;
+    if (c.tzn > 0) HIPCHK(c.tz.alloc(k * nrk * c.tzn));
+    if (c.fzn > 0) HIPCHK(c.fz.alloc(k * nrk * c.fzn));
+    if (c.tip) HIPCHK(c.tip2.alloc(k * nrk * c.np));
+    if (c.met)
+        for (DevBuf<double>* b : {&c.mwx, &c.mwy, &c.mwm, &c.mcd, &c.mprn}) HIPCHK(b->alloc(k * c.np));
+    return 0;
+}
+
 // Boundary forcing coefficients of all members, padded to the largest constituent counts, and
 // the per-stage tables, allocated once per context so that pointers captured in a graph stay valid.
 int upload_forcing(Ctx& c) {
@@ -541,7 +569,6 @@ int upload_forcing(Ctx& c) {
         for (int s = 0; s < c.S; s++)
             for (int L = c.ooff[s]; L < c.ooff[s + 1]; L++) os[L] = (uint16_t)s;
         HIPCHK(c.osid.upload(os.data(), os.size(), c.stream));
-        HIPCHK(c.tz.alloc((size_t)c.rk.nrk * c.tzn));
     }
     c.fzn = tot_f * c.negp;
     if (c.fzn > 0) {
@@ -549,8 +576,8 @@ int upload_forcing(Ctx& c) {
         for (int s = 0; s < c.S; s++)
             for (int L = c.foff[s]; L < c.foff[s + 1]; L++) fsd[L] = (uint16_t)s;
         HIPCHK(c.fsid.upload(fsd.data(), fsd.size(), c.stream));
-        HIPCHK(c.fz.alloc((size_t)c.rk.nrk * c.fzn));
     }
+    if (alloc_batch(c)) return 1;
     const size_t rows = (size_t)kTableChunk * c.rk.nrk;
     c.eser = c.fser = false;
     for (auto& m : c.mem) { c.eser = c.eser || m.eser; c.fser = c.fser || m.fser; }
@@ -590,7 +617,6 @@ int upload_met(Ctx& c) {
     HIPCHK(c.mcosy.upload(cy.data(), np, c.stream));
     HIPCHK(c.mcor.upload(co.data(), np, c.stream));
     if (c.S > 1) HIPCHK(c.nsid.upload(ns.data(), np, c.stream));
-    for (DevBuf<double>* b : {&c.mwx, &c.mwy, &c.mwm, &c.mcd, &c.mprn}) HIPCHK(b->alloc(np));
     HIPCHK(c.mrow.alloc((size_t)c.S * kTableChunk * MET_ROW));
     HIPCHK(hipStreamSynchronize(c.stream));
     return 0;
@@ -951,6 +977,8 @@ int series_seek(Member& m, Member::Series& S, bool elev, int it, int nrk) {
 // src/DG_hydro_timestep.F:79-200, src/ocean_edge_hydro.F:59-75, src/flow_edge_hydro.F:45-62,
 // src/tidal_potential.F:26-48).
 int build_stage_tables(Ctx& c, int it, int n) {
+    c.tn = n;
+    c.fbn = 0;
     if (c.nbfr == 0 && c.nffr == 0 && !c.met && !c.tip) return 0;
     if (n > kTableChunk) return fail("internal: table chunk overflow");
     const int nrk = c.rk.nrk, rows = c.rows;
@@ -1173,31 +1201,51 @@ int launch_stage_v(Ctx& c, const StageArgs& a0, bool sph, bool fuse) {
     return 0;
 }
 
-// The step's boundary and potential forcing for all stages, before the step's stage launches (the
-// forcing rows of the step must be in the tables): the open-boundary elevation terms (tide_kernel),
-// the specified normal flux (flow_kernel) and the tidal potential at the nodes (tip_kernel).
-int launch_forcing(Ctx& c, bool capturing) {
-    const Forcing F = forcing(c, capturing);
+// Boundary, potential and storm forcing of n steps from the step `first` (of the tables, or of the graph being
+// captured) into the forcing arrays: the open-boundary elevation terms (tide_kernel), the specified normal
+// flux (flow_kernel), the tidal potential at the nodes (tip_kernel) and the Holland profile (met_kernel).
+int launch_forcing(Ctx& c, int first, int n, bool capturing) {
+    c.fb0 = c.hstep = first;
+    c.fbn = n;
+    const int cap = capturing ? 0 : -1;
+    const Forcing F = forcing(c, cap);
+    const unsigned rows = (unsigned)(n * c.rk.nrk);
+    auto grid = [](int w, unsigned h) { return dim3((unsigned)((w + 255) / 256), h); };
     if (c.tzn > 0) {
-        const int n = c.rk.nrk * c.tzn;
-        hipLaunchKernelGGL(tide_kernel, dim3((n + 255) / 256), dim3(256), 0, c.stream, F,
+        hipLaunchKernelGGL(tide_kernel, grid(c.tzn, rows), dim3(256), 0, c.stream, F,
                            (const uint16_t*)(c.S > 1 ? c.osid.p : nullptr), c.tz.p);
         HIPCHK(hipGetLastError());
     }
     if (c.fzn > 0) {
-        const int n = c.rk.nrk * c.fzn;
         const uint16_t* fs = c.S > 1 ? c.fsid.p : nullptr;
         if (c.prm.p == 1)
-            hipLaunchKernelGGL(flow_kernel<1>, dim3((n + 255) / 256), dim3(256), 0, c.stream, F, fs, c.fz.p);
+            hipLaunchKernelGGL(flow_kernel<1>, grid(c.fzn, rows), dim3(256), 0, c.stream, F, fs, c.fz.p);
         else
-            hipLaunchKernelGGL(flow_kernel<2>, dim3((n + 255) / 256), dim3(256), 0, c.stream, F, fs, c.fz.p);
+            hipLaunchKernelGGL(flow_kernel<2>, grid(c.fzn, rows), dim3(256), 0, c.stream, F, fs, c.fz.p);
         HIPCHK(hipGetLastError());
     }
     if (c.tip) {
-        const int n = c.rk.nrk * c.np;
-        hipLaunchKernelGGL(tip_kernel, dim3((n + 255) / 256), dim3(256), 0, c.stream, tip_args(c), F);
+        hipLaunchKernelGGL(tip_kernel, grid(c.np, rows), dim3(256), 0, c.stream, tip_args(c), F);
         HIPCHK(hipGetLastError());
     }
+    if (c.met) {
+        int ev = prof_begin(c, K_MET, capturing);
+        hipLaunchKernelGGL(met_kernel, grid(c.np, (unsigned)n), dim3(256), 0, c.stream, met_args(c, cap), F);
+        prof_end(c, ev);
+        HIPCHK(hipGetLastError());
+    }
+    return 0;
+}
+
+// The forcing of the tables' step c.hstep is in the forcing arrays: they already hold it, or the batch of steps
+// from it on (back: up to it) is formed.
+int need_forcing(Ctx& c, bool back = false) {
+    const int k = c.hstep;
+    if (k >= c.fb0 && k < c.fb0 + c.fbn) return 0;
+    const int first = back ? std::max(0, k + 1 - c.fbatch) : k;
+    const int n = back ? k + 1 - first : std::min(c.fbatch, c.tn - k);
+    if (launch_forcing(c, first, n, false)) return 1;
+    c.hstep = k;
     return 0;
 }
 
@@ -1233,10 +1281,10 @@ int launch_stage_nt(Ctx& c, const StageArgs& a, bool sph, bool fuse, int nt) {
 // (WETDRY rewrites cell means in place).
 double* cmean_out(Ctx& c) { return c.prm.slopeflag != 0 && c.prm.nolifa >= 2 ? c.cmean.p : nullptr; }
 
-StageArgs stage_args(Ctx& c, int irk, const int slot[], bool captured = false) {
+StageArgs stage_args(Ctx& c, int irk, const int slot[], int cap = -1) {
     StageArgs a{};
-    a.ed = elem_data(c); a.ph = c.phys; a.fo = forcing(c, captured);
-    if (c.met) a.mt = met_args(c);
+    a.ed = elem_data(c); a.ph = c.phys; a.fo = forcing(c, cap);
+    if (c.met) a.mt = met_args(c, cap);
     a.uin = c.u[slot[irk]].p;
     a.uout = c.u[slot[irk + 1]].p;
     a.wd_in = c.wd[c.wdcur].p;
@@ -1251,7 +1299,7 @@ StageArgs stage_args(Ctx& c, int irk, const int slot[], bool captured = false) {
     a.rout = c.keep_r[irk] ? c.r[irk].p : nullptr;
     a.irk = irk;
     a.wd_active = c.wd_active;
-    a.tip = c.tip ? c.tip2.p + (size_t)irk * c.np : nullptr;
+    a.tip = tip_stage(c, irk, cap);
     a.cmout = cmean_out(c);
     a.mid = c.mid;
     return a;
@@ -1304,29 +1352,20 @@ int launch_wetdry_rev(Ctx& c, const double* wpre, const uint8_t* flags, double* 
     return 0;
 }
 
-// One time step: NRK stages (stage kernel, then node min/max + limiter/wet-dry when the slope
-// limiter is on) and the device step-counter increment.
+// One time step: NRK stages (stage kernel, then the limiter and wet/dry when the slope limiter is on).  A
+// captured step is step `cap` of its graph, whose forcing is already there; cap < 0: an eager step.
 template <int P>
-int launch_step(Ctx& c, bool capturing) {
-    if (launch_forcing(c, capturing)) return 1;
-    const int np = c.np;
-    const int B = 256;
-    const int gn = (np + B - 1) / B;
+int launch_step(Ctx& c, int cap) {
+    const bool capturing = cap >= 0;
     const bool wdon = c.prm.nolifa >= 2, lim = c.prm.slopeflag != 0, sph = c.prm.ics == 2;
     const int nrk = c.rk.nrk;
     // stage slots: slot(i) holds U(i+1); slot(0) = current stage-1 state
     int slot[KMAXRK + 1];
     for (int i = 0; i <= nrk; i++) slot[i] = (c.ucur + i) % (nrk + 1);
     if (c.prof && !capturing) c.prof_this = (c.prof_step++ % c.prof_every) == 0;
-    if (c.met) {
-        int ev = prof_begin(c, K_MET, capturing);
-        hipLaunchKernelGGL(met_kernel, dim3(gn), dim3(B), 0, c.stream, met_args(c),
-                           capturing ? (const int*)c.step.p : nullptr, c.hstep);
-        prof_end(c, ev);
-        HIPCHK(hipGetLastError());
-    }
+    if (!capturing && need_forcing(c)) return 1;
     for (int irk = 0; irk < nrk; irk++) {
-        StageArgs a = stage_args(c, irk, slot, capturing);
+        StageArgs a = stage_args(c, irk, slot, cap);
         for (int i = 0; i < irk; i++)
             if (a.bprev[i] != 0.0 && !c.keep_r[i]) return fail("internal: RHS of an earlier stage was not kept");
         const bool fuse = wdon && !lim;
@@ -1337,22 +1376,29 @@ int launch_step(Ctx& c, bool capturing) {
         if (fuse) c.wdcur = 1 - c.wdcur;
         if (lim && launch_limiter<P>(c, a.uout, a.ed, capturing)) return 1;
     }
-    if (capturing) {
-        hipLaunchKernelGGL(step_counter_kernel, dim3(1), dim3(1), 0, c.stream, c.step.p, 0, 0);
-        HIPCHK(hipGetLastError());
-    } else {
-        c.hstep++;
-    }
+    if (!capturing) c.hstep++;
     c.prof_this = true;
     c.ucur = slot[nrk];
     return 0;
 }
 
-int launch_steps(Ctx& c, int n, bool capturing) {
+int launch_steps(Ctx& c, int n) {
     for (int s = 0; s < n; s++) {
-        const int rc = c.prm.p == 1 ? launch_step<1>(c, capturing) : launch_step<2>(c, capturing);
+        const int rc = c.prm.p == 1 ? launch_step<1>(c, -1) : launch_step<2>(c, -1);
         if (rc) return rc;
     }
+    return 0;
+}
+
+// The launches of a graph of n steps: their forcing, the steps, and the device step counter moved past them.
+int capture_steps(Ctx& c, int n) {
+    if (launch_forcing(c, 0, n, true)) return 1;
+    for (int s = 0; s < n; s++) {
+        const int rc = c.prm.p == 1 ? launch_step<1>(c, s) : launch_step<2>(c, s);
+        if (rc) return rc;
+    }
+    hipLaunchKernelGGL(step_counter_kernel, dim3(1), dim3(1), 0, c.stream, c.step.p, 0, n);
+    HIPCHK(hipGetLastError());
     return 0;
 }
 
@@ -1366,11 +1412,7 @@ int launch_step_explicit(Ctx& c, double* const* st, double* const* wsave = nullp
     const bool sph = c.prm.ics == 2;
     const bool wdon = c.prm.nolifa >= 2, lim = c.prm.slopeflag != 0, fuse = wdon && !lim;
     const size_t ssz = (size_t)3 * c.dof * c.ne;
-    if (launch_forcing(c, false)) return 1;
-    if (c.met) {
-        hipLaunchKernelGGL(met_kernel, dim3((c.np + 255) / 256), dim3(256), 0, c.stream, met_args(c), nullptr, c.hstep);
-        HIPCHK(hipGetLastError());
-    }
+    if (need_forcing(c)) return 1;
     for (int irk = 0; irk < nrk; irk++) {
         StageArgs a{};
         a.ed = elem_data(c); a.ph = c.phys; a.fo = forcing(c);
@@ -1389,7 +1431,7 @@ int launch_step_explicit(Ctx& c, double* const* st, double* const* wsave = nullp
         a.rout = c.keep_r[irk] ? c.r[irk].p : nullptr;
         a.irk = irk;
         a.wd_active = c.wd_active;
-        a.tip = c.tip ? c.tip2.p + (size_t)irk * c.np : nullptr;
+        a.tip = tip_stage(c, irk);
         a.cmout = cmean_out(c);
         a.mid = c.mid;
         if (fsave) HIPCHK(hipMemcpyAsync(fsave[irk], c.wd[c.wdcur].p, c.ne, hipMemcpyDeviceToDevice, c.stream));
@@ -1422,7 +1464,7 @@ int run_chunk(Ctx& c, int n) {
         if (it == c.graphs.end()) {
             const int u0 = c.ucur, w0 = c.wdcur;
             HIPCHK(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal));
-            const int rc = launch_steps(c, period, true);
+            const int rc = capture_steps(c, period);
             hipGraph_t g = nullptr;
             const hipError_t ee = hipStreamEndCapture(c.stream, &g);
             if (rc) { if (g) (void)hipGraphDestroy(g); return rc; }
@@ -1438,8 +1480,9 @@ int run_chunk(Ctx& c, int n) {
         for (int r = 0; r < reps; r++) HIPCHK(hipGraphLaunch(it->second, c.stream));
         done = reps * period;
         c.hstep = done;
+        c.fbn = 0;                               // the replays used the forcing arrays
     }
-    return launch_steps(c, n - done, false);
+    return launch_steps(c, n - done);
 }
 
 // ---- discrete adjoint driver ------------------------------------------------------------
@@ -1519,7 +1562,7 @@ int adj_forward(Ctx& c, int it0, int nsteps, int interval, bool save) {
                     HIPCHK(hipMemcpyAsync(c.ckptwd.p + (size_t)(k / interval) * c.ne, c.wd[c.wdcur].p, c.ne,
                                           hipMemcpyDeviceToDevice, c.stream));
             }
-            if (launch_step<P>(c, false)) return 1;
+            if (launch_step<P>(c, -1)) return 1;
             hipLaunchKernelGGL((gauge_kernel<P>), dim3(gg), dim3(B), 0, c.stream, c.ng, c.ne, (const int*)c.gel.p,
                                (const double*)c.gphi.p, (const double*)c.u[c.ucur].p, c.geta.p + (size_t)k * c.ng);
             HIPCHK(hipGetLastError());
@@ -1603,12 +1646,7 @@ int adj_backward(Ctx& c, int it0, int nsteps, int interval, double weight) {
         }
         for (int k = k1; k > k0; k--) {
             c.hstep = k - k0 - 1;
-            if (launch_forcing(c, false)) return 1;   // the step's tidal terms for the adjoint stages
-            if (c.met) {   // the step's node forcing for the adjoint stages
-                hipLaunchKernelGGL(met_kernel, dim3((c.np + 255) / 256), dim3(256), 0, c.stream, met_args(c), nullptr,
-                                   c.hstep);
-                HIPCHK(hipGetLastError());
-            }
+            if (need_forcing(c, true)) return 1;   // the step's forcing for the adjoint stages
             ub[nrk] = lam;
             if (wdrev_on && wdrev(ub[nrk], wstage(k, nrk - 1), fstage(k, nrk - 1))) return 1;
             if (lim && limrev(ub[nrk], wstage(k, nrk - 1))) return 1;
@@ -1865,9 +1903,9 @@ int dg_gpu_set_tidal_potential(int h, int ntif, const double* tpk, const double*
         HIPCHK(c->tspha.upload(m.tspha.data(), m.tspha.size(), c->stream));
     }
     HIPCHK(c->tiprow.alloc((size_t)c->rows * ntif * 3));
-    HIPCHK(c->tip2.alloc((size_t)c->rk.nrk * np));
-    HIPCHK(hipStreamSynchronize(c->stream));
     c->tip = true;
+    if (alloc_batch(*c)) { c->tip = false; return 1; }
+    HIPCHK(hipStreamSynchronize(c->stream));
     return 0;
 }
 
@@ -2456,7 +2494,7 @@ int dg_gpu_autotune(int h, int* block) {
     const int nrk = c->rk.nrk;
     int slot[KMAXRK + 1];
     for (int i = 0; i <= nrk; i++) slot[i] = (c->ucur + i) % (nrk + 1);
-    c->hstep = 0;
+    c->hstep = c->fb0 = 0;
     StageArgs a = stage_args(*c, 0, slot);
     a.rout = nullptr;
     const bool sph = c->prm.ics == 2, fuse = c->prm.nolifa >= 2 && c->prm.slopeflag == 0;
@@ -2465,12 +2503,7 @@ int dg_gpu_autotune(int h, int* block) {
     if (c->prm.nolicat != 0) cand.push_back(0);
     const int block0 = c->block, split0 = stage_split(*c) ? 1 : 0, keep = c->split;
     if (build_stage_tables(*c, c->next_it, 1)) return 1;
-    if (launch_forcing(*c, false)) return 1;
-    if (c->met) {
-        hipLaunchKernelGGL(met_kernel, dim3((c->np + 255) / 256), dim3(256), 0, c->stream, met_args(*c),
-                           nullptr, 0);
-        HIPCHK(hipGetLastError());
-    }
+    if (launch_forcing(*c, 0, 1, false)) return 1;
     hipEvent_t e0, e1;
     HIPCHK(hipEventCreate(&e0));
     if (hipEventCreate(&e1) != hipSuccess) { (void)hipEventDestroy(e0); return fail("hipEventCreate failed"); }

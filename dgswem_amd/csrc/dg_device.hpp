@@ -96,9 +96,9 @@ struct ElemData {
 // that a captured graph of several steps can be replayed.
 struct Forcing {
     int nbfr, nffr, rows, nrk;
-    const int* __restrict__ step;       // device step counter within the current tables (graph
-                                        // replays), or nullptr: the step is step_imm
-    int step_imm;
+    const int* __restrict__ step;       // device counter of the tables' step at which a graph replay
+                                        // starts, or nullptr (eager launches)
+    int step_imm;                       // step within the replay, or within the tables
     const double* __restrict__ emo;     // [needs][nbfr][2]
     const double* __restrict__ efa;     // [needs][nbfr][2]
     const double* __restrict__ qnam;    // [nfeds][nffr][2]
@@ -109,7 +109,7 @@ struct Forcing {
     const double* __restrict__ frff;    // [nstage][nffr]
     const double* __restrict__ ramp;    // [scenario][row] RAMPDG of each stage (meteorological forcing)
     // tidal elevation terms EMO*RFF*COS(ARGJ-EFA) of the current step, [stage][needs][nbfr][2]
-    // (tzn = needs*nbfr*2 per stage), written by tide_kernel before the step's stages
+    // (tzn = needs*nbfr*2 per stage), written by tide_kernel for a batch of steps
     const double* __restrict__ tz;
     int tzn;
     // specified normal flux Q_N_EXT at every flux-edge quadrature point of the current step,
@@ -125,7 +125,7 @@ struct Forcing {
 };
 
 // Tidal potential (NTIP != 0): per-stage-row constituent terms and node data for tip_kernel, which
-// writes TIP2 of every stage at the nodes once per step.
+// writes TIP2 of every stage at the nodes for a batch of steps.
 struct Tip {
     int np, ntif;
     const double* __restrict__ row;      // [scenario*rows + row][ntif][3]: ARGT, TPMUL, SALTMUL
@@ -135,11 +135,11 @@ struct Tip {
     const double* __restrict__ s2sfea;   // [np] SIN(2*SFEA)
     const double* __restrict__ salt_amp; // [ntif][np], or nullptr (NTIP = 1: zero)
     const double* __restrict__ salt_pha; // [ntif][np] radians
-    double* __restrict__ tip2;           // [stage][np]
+    double* __restrict__ tip2;           // [step of the batch][stage][np]
 };
 
 // Step index within the current forcing tables.
-__device__ __forceinline__ int table_step(const Forcing& f) { return f.step ? *f.step : f.step_imm; }
+__device__ __forceinline__ int table_step(const Forcing& f) { return (f.step ? *f.step : 0) + f.step_imm; }
 
 
 // NWS=8 meteorological forcing at the nodes.  The node kernel evaluates the Holland profile once

@@ -8,8 +8,8 @@
 //                    order, so both see bit-identical values and no scatter or atomics are needed.
 //                    Small meshes run stage_split_kernel, four waves per 64 elements, instead.
 //   limit_wetdry     one thread per element: SLOPELIMITER5 on modes 2-3, then WETDRY
-// preceded once per step by tide_kernel (the tidal boundary terms of every stage) and, with NWS=8,
-// met_kernel (the Holland profile at the nodes); plus modal2nodal (one thread per node) on output
+// preceded once per batch of steps by tide_kernel (the tidal boundary terms of every stage) and, with
+// NWS=8, met_kernel (the Holland profile at the nodes); plus modal2nodal (one thread per node) on output
 // steps.
 //
 // Arithmetic follows the reference statement by statement (listed per kernel) and is compiled with
@@ -1204,16 +1204,21 @@ __global__ void __launch_bounds__(4 * SPLIT_NT) __attribute__((amdgpu_waves_per_
 }
 
 // ------------------------------------------------------------------------------------------
-// Tidal forcing of one step at the ocean boundary (src/ocean_edge_hydro.F:459-488): for every
-// stage, ocean edge, constituent and end node the term EMO*RFF*COS(ARGJ - EFA) that the edge's
-// elevation sums, with the cosine correctly rounded.  One thread per term; the stage kernels
-// read the stage's terms.
+// Tidal forcing of a batch of steps at the ocean boundary (src/ocean_edge_hydro.F:459-488): for
+// every stage, ocean edge, constituent and end node the term EMO*RFF*COS(ARGJ - EFA) that the edge's
+// elevation sums, with the cosine correctly rounded.  One thread per term, one block row per stage;
+// the stage kernels read the stage's terms.  A few hundred terms a stage: the launch is bound by the
+// latency of one cosine and takes as long for 64 steps as for one, so the boundary, potential and
+// storm forcing is formed for several steps at a time (launch_forcing).  100 steps of 4,972 p=1
+// elements 3.73 ms with a launch per step, 3.31 ms now; 30 of 59,600 p=2 elements under the
+// potential 3.3 and 2.6 ms; 60 of 16 storms in graphs 15.9 and 14.8 ms.
 // ------------------------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) tide_kernel(Forcing fo, const uint16_t* __restrict__ osid,
                                                    double* __restrict__ tz) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= fo.nrk * fo.tzn) return;
-    const int irk = i / fo.tzn, o = i - irk * fo.tzn;       // o = (edge*nbfr + jj)*2 + end
+    const int o = blockIdx.x * blockDim.x + threadIdx.x;    // (edge*nbfr + jj)*2 + end
+    if (o >= fo.tzn) return;
+    const int irk = blockIdx.y;                             // stage, counted over the steps of the batch
+    const size_t i = (size_t)irk * fo.tzn + o;
     const int jj = (o >> 1) % fo.nbfr, edge = (o >> 1) / fo.nbfr;
     const int sid = osid ? (int)osid[edge] : 0;
     const int row = table_step(fo) * fo.nrk + irk;
@@ -1226,7 +1231,7 @@ __global__ void __launch_bounds__(256) tide_kernel(Forcing fo, const uint16_t* _
 }
 
 // ------------------------------------------------------------------------------------------
-// Specified normal flux of one step (src/flow_edge_hydro.F:143-173): for every stage, flux edge
+// Specified normal flux of a batch of steps (src/flow_edge_hydro.F:143-173): for every stage, flux edge
 // and edge quadrature point Q_N_EXT = sum over constituents of QNAM_GP*RFF*COS(ARGJ - QNPH_GP),
 // with the cosine correctly rounded.  For NFFR = 0 the one term has ARGJ = 0, RFF = RAMPDG and the
 // end values of the time series (already ramped once, src/DG_hydro_timestep.F:188-195).
@@ -1236,9 +1241,10 @@ __global__ void __launch_bounds__(256) flow_kernel(Forcing fo, const uint16_t* _
                                                    double* __restrict__ fz) {
     constexpr int NEGP = P + 2;
     const DevTables& T = tab<P>();
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= fo.nrk * fo.fzn) return;
-    const int irk = i / fo.fzn, o = i - irk * fo.fzn;       // o = edge*NEGP + point
+    const int o = blockIdx.x * blockDim.x + threadIdx.x;    // edge*NEGP + point
+    if (o >= fo.fzn) return;
+    const int irk = blockIdx.y;                             // stage, counted over the steps of the batch
+    const size_t i = (size_t)irk * fo.fzn + o;
     const int edge = o / NEGP, I = o - edge * NEGP;
     const int sid = fsid ? (int)fsid[edge] : 0;
     const int row = table_step(fo) * fo.nrk + irk;
@@ -1266,31 +1272,32 @@ __global__ void __launch_bounds__(256) flow_kernel(Forcing fo, const uint16_t* _
 }
 
 // ------------------------------------------------------------------------------------------
-// TIDAL_POTENTIAL (src/tidal_potential.F:15-80) for every stage of one step: TIP2 at every node,
-// with the cosines of the time-dependent arguments correctly rounded (COS(SFEA)**2 and
-// SIN(2*SFEA) come from the host's libm).
+// TIDAL_POTENTIAL (src/tidal_potential.F:15-80) for every stage of a batch of steps: TIP2 at every
+// node, with the cosines of the time-dependent arguments correctly rounded (COS(SFEA)**2 and
+// SIN(2*SFEA) come from the host's libm).  Without self-attraction and load the second product is
+// SALTMUL*0*COS: adding SALTMUL*0 gives the same sum without the cosine (half of the kernel's work).
 // ------------------------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) tip_kernel(Tip tp, Forcing fo) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= fo.nrk * tp.np) return;
-    const int irk = i / tp.np, n = i - irk * tp.np;
+    const int n = blockIdx.x * blockDim.x + threadIdx.x;
+    if (n >= tp.np) return;
+    const int irk = blockIdx.y;                             // stage, counted over the steps of the batch
     const int row = table_step(fo) * fo.nrk + irk;
     const double* r = tp.row + (size_t)row * tp.ntif * 3;
     double tip = 0.0;
     for (int j = 0; j < tp.ntif; j++) {
         const double argt = r[3 * j], tpmul = r[3 * j + 1], saltmul = r[3 * j + 2];
-        const double sa = tp.salt_amp ? tp.salt_amp[(size_t)j * tp.np + n] : 0.0;
-        const double sp = tp.salt_pha ? tp.salt_pha[(size_t)j * tp.np + n] : 0.0;
         const int na = tp.na[j];
+        if (na != 1 && na != 2) continue;
+        double salt = saltmul * 0.0;
+        if (tp.salt_amp)
+            salt = saltmul * tp.salt_amp[(size_t)j * tp.np + n] * crm::cr_cos(argt - tp.salt_pha[(size_t)j * tp.np + n]);
         if (na == 1) {
             const double argtp = argt + 2.0 * tp.slam[n];
-            const double argsalt = argt - sp;
-            tip = tip + tpmul * tp.ccsfea[n] * crm::cr_cos(argtp) + saltmul * sa * crm::cr_cos(argsalt);
+            tip = tip + tpmul * tp.ccsfea[n] * crm::cr_cos(argtp) + salt;
         }
         if (na == 2) {
             const double argtp = argt + tp.slam[n];
-            const double argsalt = argt - sp;
-            tip = tip + tpmul * tp.s2sfea[n] * crm::cr_cos(argtp) + saltmul * sa * crm::cr_cos(argsalt);
+            tip = tip + tpmul * tp.s2sfea[n] * crm::cr_cos(argtp) + salt;
         }
     }
     tp.tip2[(size_t)irk * tp.np + n] = tip;
@@ -1650,14 +1657,16 @@ __global__ void __launch_bounds__(256) modal2nodal_kernel(int np, ElemData E, co
 
 // ------------------------------------------------------------------------------------------
 // NWS=8 node kernel: HollandGet's per-node profile (src/wind.F:2062-2131) and the wind speed and
-// Garratt drag of MET_FORCING (src/met_forcing.F:488-500, src/wind.F:135-141), at TIME_A of the
-// current step.  The stage's ramp is applied in the stage kernel.
+// Garratt drag of MET_FORCING (src/met_forcing.F:488-500, src/wind.F:135-141), at TIME_A of every
+// step of a batch.  The stage's ramp is applied in the stage kernel.
 // ------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) met_kernel(Met m, const int* __restrict__ step, int step_imm) {
+__global__ void __launch_bounds__(256) met_kernel(Met m, Forcing fo) {
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= m.np) return;
+    const int s = blockIdx.y;                               // step of the batch
+    const size_t o = (size_t)s * m.np + n;
     const int sid = m.nsid ? (int)m.nsid[n] : 0;
-    const double* r = m.row + ((size_t)sid * m.rows + (step ? *step : step_imm)) * MET_ROW;
+    const double* r = m.row + ((size_t)sid * m.rows + table_step(fo) + s) * MET_ROW;
     const double re = 6378206.4;
     const double deg2rad = 3.141592653589793 / 180.0;
     const double lat = r[MR_LAT], lon = r[MR_LON], spd = r[MR_SPD], B = r[MR_B];
@@ -1678,7 +1687,7 @@ __global__ void __launch_bounds__(256) met_kernel(Met m, const int* __restrict__
     const double wmag = sqrt(wx * wx + wy * wy);
     double cd = 0.001 * (0.75 + 0.067 * wmag);
     if (cd > 0.0035) cd = 0.0035;
-    m.wx[n] = wx; m.wy[n] = wy; m.wm[n] = wmag; m.cd[n] = cd; m.prn[n] = press;
+    m.wx[o] = wx; m.wy[o] = wy; m.wm[o] = wmag; m.cd[o] = cd; m.prn[o] = press;
 }
 
 // The state between the step's layout (soa: [field][mode][element]) and the host's (aos: [field][element][mode]), one
@@ -1708,7 +1717,7 @@ __global__ void __launch_bounds__(256) flags_kernel(int ne, uint8_t* __restrict_
 // Device step counter used by the forcing-table lookups of captured steps (a kernel, not a memset,
 // so that the sequence can be captured into a HIP graph).
 __global__ void step_counter_kernel(int* __restrict__ step, int set, int value) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) *step = set ? value : *step + 1;
+    if (threadIdx.x == 0 && blockIdx.x == 0) *step = set ? value : *step + value;
 }
 
 // Water volume per element: 0.5*AREAS*(ze_1 + hb_1), reduced per block.
