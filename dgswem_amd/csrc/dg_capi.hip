@@ -164,6 +164,7 @@ struct Ctx {
     bool has_etamax = false;
     // forcing
     DevBuf<double> emo, efa, qnam, qnph, argj, rff, fargj, frff;
+    DevBuf<double> tabrows;                      // packed table rows on their way into the tables
     DevBuf<int> step;                            // device step counter within the current tables
     DevBuf<double> tz;                           // tidal terms [step of the batch][stage][needs][nbfr][2]
     DevBuf<uint16_t> osid;                       // scenario of each ocean edge (ensembles)
@@ -981,15 +982,15 @@ int build_stage_tables(Ctx& c, int it, int n) {
     c.fbn = 0;
     if (c.nbfr == 0 && c.nffr == 0 && !c.met && !c.tip) return 0;
     if (n > kTableChunk) return fail("internal: table chunk overflow");
-    const int nrk = c.rk.nrk, rows = c.rows;
+    const int nrk = c.rk.nrk, rows = n * nrk;    // only the rows of these steps are formed and uploaded
     const int tot_f = c.foff[c.S];
     const bool ramped = c.met || c.tip;
-    std::vector<double> aj((size_t)c.S * rows * std::max(c.nbfr, 1), 0.0), rf(aj.size(), 0.0);
-    std::vector<double> fa((size_t)c.S * rows * std::max(c.nffr, 1), 0.0), fr(fa.size(), 0.0);
+    std::vector<double> aj((size_t)c.S * rows * c.nbfr, 0.0), rf(aj.size(), 0.0);
+    std::vector<double> fa((size_t)c.S * rows * c.nffr, 0.0), fr(fa.size(), 0.0);
     std::vector<double> rp, mr, et, qt, tr;
     if (ramped) rp.assign((size_t)c.S * rows, 0.0);
-    if (c.met) mr.assign((size_t)c.S * kTableChunk * MET_ROW, 0.0);
-    if (c.eser) et.assign((size_t)c.S * rows * std::max(c.tzn, 1), 0.0);
+    if (c.met) mr.assign((size_t)c.S * n * MET_ROW, 0.0);
+    if (c.eser) et.assign((size_t)c.S * rows * c.tzn, 0.0);
     if (c.fser) qt.assign((size_t)c.S * rows * tot_f * 2, 0.0);
     if (c.tip) tr.assign((size_t)c.S * rows * c.ntif * 3, 0.0);
     std::vector<double> eta_bc;
@@ -1005,7 +1006,7 @@ int build_stage_tables(Ctx& c, int it, int n) {
             const double time_a = itdt + m.prm.statim * 86400.0;
             const double timeh = itdt + (m.prm.statim - m.reftim) * 86400.0;
             // storm scalars at TIME_A (MET_FORCING is called with TIME_A at every stage)
-            if (c.met && !holland_row(m.track, time_a, m.prm.g, &mr[((size_t)sc * kTableChunk + s) * MET_ROW], err))
+            if (c.met && !holland_row(m.track, time_a, m.prm.g, &mr[((size_t)sc * n + s) * MET_ROW], err))
                 return fail(err);
             for (int irk = 0; irk < nrk; irk++) {
                 const size_t row = (size_t)sc * rows + (size_t)s * nrk + irk;
@@ -1069,21 +1070,44 @@ int build_stage_tables(Ctx& c, int it, int n) {
             if (m.fser) m.fs.it = IT;
         }
     }
-    // the previous chunk's launches may still read the tables
-    HIPCHK(hipStreamSynchronize(c.stream));
-    if (c.nbfr) {
-        HIPCHK(hipMemcpyAsync(c.argj.p, aj.data(), aj.size() * sizeof(double), hipMemcpyHostToDevice, c.stream));
-        HIPCHK(hipMemcpyAsync(c.rff.p, rf.data(), rf.size() * sizeof(double), hipMemcpyHostToDevice, c.stream));
+    // One list of all values, put into the tables by a kernel behind the launches that still read the old rows.
+    // Up to 4 * TABLE_ARGS values travel in launch arguments (about 3 us each, none of it waiting); beyond that
+    // one copy, which the host waits for because the list is its own, is the shorter way.  Calls of
+    // one step on 1,600 elements with their nodal values: 67 us a call when four whole tables were copied and
+    // waited for, 38 us now.
+    TableRows tr9{};
+    std::vector<double> list;
+    auto add = [&](DevBuf<double>& d, const std::vector<double>& v, size_t stride) {
+        if (v.empty()) return;
+        auto& t = tr9.t[tr9.n++];
+        t.dst = d.p; t.off = list.size(); t.w = v.size() / c.S; t.stride = stride;
+        list.insert(list.end(), v.begin(), v.end());
+    };
+    const size_t cap = c.rows;                   // table rows per scenario
+    add(c.argj, aj, cap * c.nbfr);
+    add(c.rff, rf, cap * c.nbfr);
+    add(c.fargj, fa, cap * c.nffr);
+    add(c.frff, fr, cap * c.nffr);
+    add(c.ramp, rp, cap);
+    add(c.mrow, mr, (size_t)kTableChunk * MET_ROW);
+    add(c.ets, et, cap * c.tzn);
+    add(c.qts, qt, cap * tot_f * 2);
+    add(c.tiprow, tr, cap * c.ntif * 3);
+    const size_t m = list.size();
+    if (m <= (size_t)4 * TABLE_ARGS) {
+        TableArgs v;
+        for (size_t f = 0; f < m; f += TABLE_ARGS) {
+            const int k = (int)std::min<size_t>(TABLE_ARGS, m - f);
+            std::copy_n(&list[f], k, v.v);
+            hipLaunchKernelGGL(table_args_kernel, dim3(1), dim3(TABLE_ARGS), 0, c.stream, tr9, v, f, k);
+            HIPCHK(hipGetLastError());
+        }
+        return 0;
     }
-    if (c.nffr) {
-        HIPCHK(hipMemcpyAsync(c.fargj.p, fa.data(), fa.size() * sizeof(double), hipMemcpyHostToDevice, c.stream));
-        HIPCHK(hipMemcpyAsync(c.frff.p, fr.data(), fr.size() * sizeof(double), hipMemcpyHostToDevice, c.stream));
-    }
-    if (ramped) HIPCHK(hipMemcpyAsync(c.ramp.p, rp.data(), rp.size() * sizeof(double), hipMemcpyHostToDevice, c.stream));
-    if (c.met) HIPCHK(hipMemcpyAsync(c.mrow.p, mr.data(), mr.size() * sizeof(double), hipMemcpyHostToDevice, c.stream));
-    if (c.eser) HIPCHK(hipMemcpyAsync(c.ets.p, et.data(), et.size() * sizeof(double), hipMemcpyHostToDevice, c.stream));
-    if (c.fser) HIPCHK(hipMemcpyAsync(c.qts.p, qt.data(), qt.size() * sizeof(double), hipMemcpyHostToDevice, c.stream));
-    if (c.tip) HIPCHK(hipMemcpyAsync(c.tiprow.p, tr.data(), tr.size() * sizeof(double), hipMemcpyHostToDevice, c.stream));
+    HIPCHK(c.tabrows.upload(list.data(), m, c.stream));
+    hipLaunchKernelGGL(table_rows_kernel, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, c.stream, tr9,
+                       (const double*)c.tabrows.p, m);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c.stream));
     return 0;
 }

@@ -1714,6 +1714,37 @@ __global__ void __launch_bounds__(256) flags_kernel(int ne, uint8_t* __restrict_
     else wd[e] = flags[e] ? 1 : 0;
 }
 
+// Rows of the forcing tables from one packed list of values: table t holds `w` values per scenario, taken from
+// list position `off` on and `stride` apart in the table (whose rows are laid out for the longest call).
+struct TableRows {
+    int n;
+    struct { double* dst; size_t off, w, stride; } t[9];
+};
+
+__device__ __forceinline__ void put_table_value(const TableRows& r, size_t i, double v) {
+    for (int t = r.n - 1; t >= 0; t--)
+        if (i >= r.t[t].off) {
+            const size_t j = i - r.t[t].off, sc = j / r.t[t].w;
+            r.t[t].dst[sc * r.t[t].stride + (j - sc * r.t[t].w)] = v;
+            return;
+        }
+}
+
+__global__ void __launch_bounds__(256) table_rows_kernel(TableRows r, const double* __restrict__ src, size_t n) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) put_table_value(r, i, src[i]);
+}
+
+// The same with the values in the launch's arguments: nothing to copy and nothing to wait for, which is what a
+// call of one step costs most (build_stage_tables).
+constexpr int TABLE_ARGS = 448;   // with TableRows within the 4 KB that a launch's arguments may take
+struct TableArgs { double v[TABLE_ARGS]; };
+
+__global__ void __launch_bounds__(TABLE_ARGS) table_args_kernel(TableRows r, TableArgs a, size_t first, int n) {
+    const int i = threadIdx.x;
+    if (i < n) put_table_value(r, first + i, a.v[i]);
+}
+
 // Device step counter used by the forcing-table lookups of captured steps (a kernel, not a memset,
 // so that the sequence can be captured into a HIP graph).
 __global__ void step_counter_kernel(int* __restrict__ step, int set, int value) {

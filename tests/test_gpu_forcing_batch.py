@@ -37,3 +37,27 @@ def test_batches(name, steps):
     for how in ("call", "graph"):
         for a, b in zip(run(how), ref):
             np.testing.assert_array_equal(a, b)
+
+
+# table rows of a call in launch arguments (one launch, several) and over a copy, with several scenarios
+@pytest.mark.parametrize("steps", [1, 9, 16, 17, 40])
+def test_table_rows_of_an_ensemble(steps):
+    cases = [mesh.storm_basin(n, seed=3 + n, p=1, nsteps=200) for n in (400, 700, 500)]
+    single = []
+    for c in cases:
+        g = gpu.GpuSolver(c)
+        for _ in range(steps):
+            g.step(1, sync=False)
+        single.append(g.state())
+        g.close()
+    for graph in (False, True):
+        members = [gpu.GpuSolver(c) for c in cases]
+        ens = gpu.Ensemble(members)
+        for m in members:
+            m.close()
+        ens.use_graph(graph)
+        ens.step(steps)
+        out = ens.state()
+        ens.close()
+        for k in range(4):
+            np.testing.assert_array_equal(out[k], np.concatenate([s[k] for s in single]))
