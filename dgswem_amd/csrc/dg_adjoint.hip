@@ -252,99 +252,53 @@ __device__ __forceinline__ void llf_flux_adj_side(const Phys& P, double zi, doub
     hbar = hb;
 }
 
-// The mass flux F0 of an internal edge at one point as the forward stage kernel forms it: its
-// traces in the forward's operation order (no contraction) and the LLF flux, so that the dry-side
-// case (src/internal_edge_hydro.F:212-302) is taken as the forward took it.
-template <int DOF, bool NL>
-__device__ __forceinline__ double edge_f0_exact(const Phys& ph, const double (&Vi)[3][DOF], const double (&Vx)[3][DOF],
-                                                const double (&hbi)[3], const double (&hbx)[3], const double* pi_,
-                                                const double* px_, double sfi, double sfx, double nx, double ny) {
-    const double ze_in = trace1<DOF>(Vi[0], pi_), qx_in = trace1<DOF>(Vi[1], pi_), qy_in = trace1<DOF>(Vi[2], pi_);
-    const double ze_ex = trace1<DOF>(Vx[0], px_), qx_ex = trace1<DOF>(Vx[1], px_), qy_ex = trace1<DOF>(Vx[2], px_);
-    const double hb_in = trace1<3>(hbi, pi_), hb_ex = trace1<3>(hbx, px_);
-    double f0, f1, f2;
-    llf<NL>(ph, ze_in, ze_ex, qx_in, qx_ex, qy_in, qy_ex, hb_in, hb_ex, sfi, sfx, nx, ny, ph.g, f0, f1, f2);
-    return f0;
-}
-
-// The P1 bathymetry modes of element g as the forward stage kernel stages them (no contraction).
-__device__ __forceinline__ void elem_hb_exact(const ElemData& E, int ne, int g, double hb[3]) {
+// The P1 bathymetry modes from the vertex depths as the forward stage kernel stages them (no contraction).
+__device__ __forceinline__ void hb_modes(double d0, double d1, double d2, double hb[3]) {
     const double c13 = 1.0 / 3.0, c16 = 1.0 / 6.0;
-    const double d0 = E.dpv[g], d1 = E.dpv[(size_t)ne + g], d2 = E.dpv[2 * (size_t)ne + g];
     hb[0] = c13 * (d0 + d1 + d2);
     hb[1] = -(c16 * (d0 + d1)) + c13 * d2;
     hb[2] = -(0.5 * d0) + 0.5 * d1;
 }
 
-// Side geometry as the forward forms it (no contraction).
-__device__ __forceinline__ void side_geometry_exact(const ElemData& E, int ne, int e, int L, int role, double& xlen,
-                                                    double& nx, double& ny) {
-    int va = (L + 1) % 3, vb = (L + 2) % 3;
-    if (role) { const int t = va; va = vb; vb = t; }
-    const double dy = E.yv[(size_t)vb * ne + e] - E.yv[(size_t)va * ne + e];
-    const double dx = E.xv[(size_t)vb * ne + e] - E.xv[(size_t)va * ne + e];
-    xlen = sqrt(dy * dy + dx * dx);
-    nx = dy / xlen;
-    ny = -dx / xlen;
-}
-
-template <bool NL>
-__device__ void dry_side_adj_cases(const Phys& ph, int cas, int role, double zi, double ze, double xi, double xe,
-                                   double yi, double ye, double hi, double he, double sfi, double sfx, double nx,
-                                   double ny, const double cin[3], const double cex[3], double& zb, double& xb,
-                                   double& yb, double& hbar);
-
 // Reverse of an internal edge point where one side is dry (src/internal_edge_hydro.F:212-302),
-// for this element's own side: the case is taken from the forward's mass flux F0 (recomputed as
-// the forward formed it); cin/cex are d(loss)/d(flux the "in"/"ex" side received).  Cases:
+// for this element's own side; i and x are the "in" and "ex" traces (elevation, discharges, bathymetry) as the
+// forward forms them, so that the case is taken from the forward's mass flux; cin/cex are d(loss)/d(flux the
+// "in"/"ex" side received).  Cases:
 // 1 reflect into a dry "in" (both sides take the reflected flux's F0, "ex" its momentum: a function
 // of the "ex" traces only), 2 zero-gravity momentum for a dry "in", 3 reflect into a dry "ex",
 // 4 zero-gravity momentum for a dry "ex", 0 the plain flux.  Outputs this side's trace cotangents.
-template <int P, bool NL>
-__device__ void dry_side_adj(const Phys& ph, const ElemData& E, int ne, int e, int nb, int L, int role, int nled,
-                             int gi, int gx, const double (&U)[3][(P + 1) * (P + 2) / 2],
-                             const double (&V)[3][(P + 1) * (P + 2) / 2], int wd, int wdn,
-                             double zi, double ze, double xi, double xe, double yi, double ye, double hi, double he,
-                             double sfi, double sfx, double nx, double ny, const double cin[3], const double cex[3],
-                             double& zb, double& xb, double& yb, double& hbar) {
-    constexpr int DOF = (P + 1) * (P + 2) / 2;
-    const DevTables& T = tab<P>();
-    int cas = 0;
-    {
-        // the forward's F0, operation by operation
-        double hbo[3], hbn[3], xlen_x, nx_x, ny_x;
-        elem_hb_exact(E, ne, e, hbo);
-        elem_hb_exact(E, ne, nb, hbn);
-        side_geometry_exact(E, ne, e, L, role, xlen_x, nx_x, ny_x);
-        const int Li = role ? nled : L, Lx = role ? L : nled;
-        const double f0 = role ? edge_f0_exact<DOF, NL>(ph, V, U, hbn, hbo, T.phi_edge[Li][gi], T.phi_edge[Lx][gx], sfi, sfx, nx_x, ny_x)
-                               : edge_f0_exact<DOF, NL>(ph, U, V, hbo, hbn, T.phi_edge[Li][gi], T.phi_edge[Lx][gx], sfi, sfx, nx_x, ny_x);
-        const int wd_in_el = role ? wdn : wd, wd_ex_el = role ? wd : wdn;
-        if (fabs(f0) > 1.0e-8) {
-            if (wd_in_el == 0) cas = f0 > 0.0 ? 1 : 2;
-            else if (wd_ex_el == 0) cas = f0 < 0.0 ? 3 : 4;
-        }
-    }
-    dry_side_adj_cases<NL>(ph, cas, role, zi, ze, xi, xe, yi, ye, hi, he, sfi, sfx, nx, ny, cin, cex, zb, xb, yb, hbar);
+template <bool NL>
+__device__ __forceinline__ int dry_side_case(const Phys& ph, int wd_in_el, int wd_ex_el, const double (&i)[4],
+                                             const double (&x)[4], double sfi, double sfx, double nx, double ny) {
+    double f0, f1, f2;
+    llf<NL>(ph, i[0], x[0], i[1], x[1], i[2], x[2], i[3], x[3], sfi, sfx, nx, ny, ph.g, f0, f1, f2);
+    if (!(fabs(f0) > 1.0e-8)) return 0;
+    if (wd_in_el == 0) return f0 > 0.0 ? 1 : 2;
+    if (wd_ex_el == 0) return f0 < 0.0 ? 3 : 4;
+    return 0;
 }
 
-// The derivative part of dry_side_adj, for case `cas`.
 template <bool NL>
-__device__ void dry_side_adj_cases(const Phys& ph, int cas, int role, double zi, double ze, double xi, double xe,
-                                   double yi, double ye, double hi, double he, double sfi, double sfx, double nx,
-                                   double ny, const double cin[3], const double cex[3], double& zb, double& xb,
-                                   double& yb, double& hbar) {
+__device__ __forceinline__ void dry_side_adj(const Phys& ph, int cas, int role, const double (&i)[4], const double (&x)[4],
+                                             double sfi, double sfx, double nx, double ny, const double (&cin)[3],
+                                             const double (&cex)[3], double& zb, double& xb, double& yb, double& hbar) {
 #pragma clang fp contract(fast)
+    const double zi = i[0], xi = i[1], yi = i[2], hi = i[3], ze = x[0], xe = x[1], ye = x[2], he = x[3];
     zb = xb = yb = hbar = 0.0;
     if (cas == 0 || cas == 2 || cas == 4) {
-        double fbn[3] = {cin[0] + cex[0], cin[1] + cex[1], cin[2] + cex[2]};
-        double fbg[3] = {0.0, 0.0, 0.0};
-        if (cas == 2) { fbn[1] = cex[1]; fbn[2] = cex[2]; fbg[1] = cin[1]; fbg[2] = cin[2]; }
-        if (cas == 4) { fbn[1] = cin[1]; fbn[2] = cin[2]; fbg[1] = cex[1]; fbg[2] = cex[2]; }
-        llf_flux_adj_side<NL>(ph, zi, ze, xi, xe, yi, ye, hi, he, sfi, sfx, nx, ny, ph.g, fbn, role, zb, xb, yb, hbar);
-        if (cas != 0) {
+        // the flux, and for cases 2 and 4 the zero-gravity momentum flux that replaces one side's
+#pragma unroll 1
+        for (int k = 0; k < (cas == 0 ? 1 : 2); k++) {
+            double fb[3] = {cin[0] + cex[0], cin[1] + cex[1], cin[2] + cex[2]};
+            if (cas != 0) {
+                const bool in = (cas == 2) == (k == 1);
+                fb[0] = k == 0 ? fb[0] : 0.0;
+                fb[1] = in ? cin[1] : cex[1];
+                fb[2] = in ? cin[2] : cex[2];
+            }
             double z2, x2, y2, h2;
-            llf_flux_adj_side<NL>(ph, zi, ze, xi, xe, yi, ye, hi, he, sfi, sfx, nx, ny, 0.0, fbg, role, z2, x2, y2, h2);
+            llf_flux_adj_side<NL>(ph, zi, ze, xi, xe, yi, ye, hi, he, sfi, sfx, nx, ny, k == 0 ? ph.g : 0.0, fb, role, z2, x2,
+                                  y2, h2);
             zb += z2; xb += x2; yb += y2; hbar += h2;
         }
         return;
@@ -402,207 +356,359 @@ struct AdjArgs {
     int nh, ns;                          // halo entries per tile, staged elements per block (LDS row length)
 };
 
-// RHS cotangent of element `el` (its own stage contribution): sum_j b_j DT src_j.
-template <int DOF>
-__device__ __forceinline__ void load_lambda(const AdjArgs& a, int ne, int el, double dtdp, double (&L)[3][DOF]) {
-#pragma unroll
-    for (int f = 0; f < 3; f++)
-#pragma unroll
-        for (int k = 0; k < DOF; k++) L[f][k] = 0.0;
-    for (int j = 0; j < a.nsrc; j++) {
-        const double b = a.bcoef[j] * dtdp;
-        if (b == 0.0) continue;
-        const double* s = a.src[j];
-#pragma unroll
-        for (int f = 0; f < 3; f++)
-#pragma unroll
-            for (int k = 0; k < DOF; k++) L[f][k] = L[f][k] + b * s[(size_t)(f * DOF + k) * ne + el];
-    }
-}
-
-// Element g's P1 bathymetry modes and AREAS (twice the area), from its vertex depths and
-// coordinates, with the products and sums of the reference's set-up (src/read_input.F:1408,
-// src/prep_DG.F:959-1163) and of the forward stage kernel.
-__device__ __forceinline__ void elem_hb_areas(const ElemData& E, int ne, int g, double hb[3], double& areas) {
+// The reverse of the LLF flux of an internal edge point for one side's own arguments: `o` the side's own traces
+// (elevation, discharges, bathymetry), `n` the neighbour's, fs the flux cotangent with the sign of (neighbour - own),
+// (mx, my) half the canonical normal with that sign.  The wave-speed bound is the first largest of the candidates
+// in the canonical order ("in" side first, so `in` decides a tie between the sides); bo and bn, -1 for the "ex" side
+// and NaN for the "in" side, make a NaN first candidate count on the "in" side only, as comparing one candidate
+// after the other does.
+template <bool NL>
+__device__ __forceinline__ void llf_adj_own(const Phys& P, const double (&o)[4], const double (&n)[4], double so, double sn,
+                                            double nx, double ny, double mx, double my, const double (&fs)[3], bool in,
+                                            double bo, double bn, double (&bar)[4]) {
 #pragma clang fp contract(fast)
-    const double c13 = 1.0 / 3.0, c16 = 1.0 / 6.0;
-    const double d0 = E.dpv[g], d1 = E.dpv[(size_t)ne + g], d2 = E.dpv[2 * (size_t)ne + g];
-    hb[0] = c13 * (d0 + d1 + d2);
-    hb[1] = -(c16 * (d0 + d1)) + c13 * d2;
-    hb[2] = -(0.5 * d0) + 0.5 * d1;
-    const double X0 = E.xv[g], X1 = E.xv[(size_t)ne + g], X2 = E.xv[2 * (size_t)ne + g];
-    const double Y0 = E.yv[g], Y1 = E.yv[(size_t)ne + g], Y2 = E.yv[2 * (size_t)ne + g];
-    areas = (X0 - X2) * (Y1 - Y2) + (X2 - X1) * (Y0 - Y2);
+    const double NLEQ = NL ? 1.0 : P.nleq, LEQ = NL ? 0.0 : P.leq, FG_L = NL ? 0.0 : P.fg_l;
+    const double NLEQG = P.g * NLEQ;
+    const double z = o[0], x = o[1], y = o[2], h = o[3];
+    double un, c, K, fh, u, v, m, un_n, c_n, m_n;
+    int q;                               // the own side's candidate: 0 un + c, 1 un, 2 un - c
+    {
+        const double ht = z * NLEQ + h;
+        fh = NL ? 1.0 / ht : 1.0 / (NLEQ * ht + LEQ);
+        u = x * fh;
+        v = y * fh;
+        un = (u * nx + v * ny) * NLEQ;
+        const double nxs = nx * so;
+        K = ny * ny + nxs * nxs;
+        c = sqrt(P.g * ht * K);
+        m = fmax(fabs(un + c), bo);
+        q = 0;
+        if (fabs(un) > m) { m = fabs(un); q = 1; }
+        if (fabs(un - c) > m) { m = fabs(un - c); q = 2; }
+    }
+    {
+        const double ht = n[0] * NLEQ + n[3];
+        const double f = NL ? 1.0 / ht : 1.0 / (NLEQ * ht + LEQ);
+        un_n = (n[1] * f * nx + n[2] * f * ny) * NLEQ;
+        const double nxs = nx * sn;
+        c_n = sqrt(P.g * ht * (ny * ny + nxs * nxs));
+        m_n = fmax(fabs(un_n + c_n), bn);
+        if (fabs(un_n) > m_n) m_n = fabs(un_n);
+        if (fabs(un_n - c_n) > m_n) m_n = fabs(un_n - c_n);
+    }
+    const bool mine = in ? !(m_n > m) : m > m_n;
+    const double em = mine ? m : m_n;
+    const double j1 = n[0] - z, j2 = n[1] - x, j3 = n[2] - y;
+    double emb, d1, d2, d3;              // cotangents of the bound and of the jumps (own minus neighbour)
+    if constexpr (NL) {
+        emb = -0.5 * (j1 * fs[0] + j2 * fs[1] + j3 * fs[2]);
+        d1 = 0.5 * em * fs[0];
+        d2 = 0.5 * em * fs[1];
+        d3 = 0.5 * em * fs[2];
+    } else {
+        const double nx2 = NLEQ + LEQ * nx * nx, ny2 = NLEQ + LEQ * ny * ny, nxy = nx * ny;
+        emb = -0.5 * j1 * fs[0] - 0.5 * (j2 * nx2 + LEQ * j3 * nxy) * fs[1] - 0.5 * (j3 * ny2 + LEQ * j2 * nxy) * fs[2];
+        d1 = 0.5 * em * fs[0];
+        d2 = 0.5 * em * (nx2 * fs[1] + LEQ * nxy * fs[2]);
+        d3 = 0.5 * em * (LEQ * nxy * fs[1] + ny2 * fs[2]);
+    }
+    double unb = 0.0, cb = 0.0;
+    if (mine) {
+        const double val = q == 0 ? un + c : (q == 1 ? un : un - c);
+        unb = val > 0.0 ? emb : (val < 0.0 ? -emb : 0.0);
+        cb = q == 0 ? unb : (q == 2 ? -unb : 0.0);
+    }
+    const double fx1b = mx * fs[0], fy1b = my * fs[0];
+    const double hvvb = my * fs[2];
+    const double huub = so * (mx * fs[1]);
+    const double gh2b = hvvb + huub;
+    const double huvb = so * (mx * fs[2]) + my * fs[1];
+    const double fnl = NL ? 1.0 : NLEQ + LEQ * h;
+    const double fu = NLEQ * x, fv = NLEQ * y, fg = NLEQG * z;
+    const double ub = fu * huub + nx * NLEQ * unb;
+    const double vb = fv * hvvb + fu * huvb + ny * NLEQ * unb;
+    double htb;
+    if constexpr (NL) htb = c > 0.0 ? 0.5 * c * fh * cb : 0.0;
+    else htb = c > 0.0 ? P.g * K / (2.0 * c) * cb : 0.0;
+    htb += -NLEQ * fh * fh * (x * ub + y * vb);
+    bar[0] = (NL ? 0.5 * fg : 0.5 * fg + FG_L) * gh2b + NLEQG * ((0.5 * z + h) * gh2b) + NLEQ * htb + d1;
+    bar[1] = fh * ub + NLEQ * (u * huub + v * huvb) + fnl * so * fx1b + d2;
+    bar[2] = fh * vb + NLEQ * (v * hvvb) + fnl * fy1b + d3;
+    bar[3] = fg * gh2b + htb;
+    if constexpr (!NL) bar[3] += LEQ * (x * so * fx1b + y * fy1b);
 }
 
+// Rows of the staged tile: state, bathymetry modes, scaled RHS cotangent of the modes, AREAS; and what a wave
+// leaves for the sums: the cotangents of the modes, of the bathymetry modes and of Manning's n.
+constexpr int ADJ_NT = 64;               // elements per block
+constexpr int adj_stage_rows(int dof) { return 6 * dof + 4; }
+constexpr int adj_sum_rows(int dof) { return 3 * dof + 4; }
+
+// Reverse of one stage.  A block of four waves works on 64 elements, lane l of every wave on element l.  Wave c < 3
+//   1. stages the state and the RHS cotangent of field c of the tile and its halo (wave 3: bathymetry, AREAS,
+//      flags and the edge table),
+//   2. reverses side slot c,
+//   3. reverses its share of the area points (wave 3 without a side has more of them),
+//   4. adds what the four waves have for field c and the later stages' cotangents (wave 3: the parameters).
+// The time of this kernel was its serial chain: one lane per element took three sides and the area points one after
+// the other with two waves per SIMD (p=1) or one (p=2: 504 registers), the sums read and written in LDS at every
+// point.  49,800 p=1 elements: 27.2 us before, 15.8 us now; four p=2 storm basins of 99,000 elements with their
+// flags 108.7 and 65 us.  Two waves per SIMD: with three the p=2 form spills (85 us).
+// The RHS cotangent is staged times M_INV, which leaves the plain basis values and derivatives as the
+// transposed quadrature's tables: the edge cotangent is a trace like the state's, and the area points' ones
+// are two sums per field.
 // QF: quadratic bottom friction without the hybrid factor (NOLIBF=1), fixed at compile time.
 // WD: the stage's wet/dry flags are read (a.wd) and dry elements and dry-side edge cases are
 // reversed; without it every element is wet and that code is compiled out (it would otherwise
 // raise the kernel's register use past what the all-wet runs need).
-template <int P, int NT, bool SPH, bool NL, bool QF, bool WD>
-__global__ void __launch_bounds__(NT, P == 1 ? 2 : 1) adj_stage_kernel(AdjArgs a) {
+template <int P, bool SPH, bool NL, bool QF, bool WD>
+__global__ void __launch_bounds__(4 * ADJ_NT) __attribute__((amdgpu_waves_per_eu(2))) adj_stage_kernel(AdjArgs a) {
 #pragma clang fp contract(fast)
     constexpr int DOF = (P + 1) * (P + 2) / 2;
     constexpr int NAGP = (P == 1) ? 3 : 6;
     constexpr int NEGP = P + 2;
-    __shared__ double ub_lds[3 * DOF][NT];     // cotangent of this element's modes
-    __shared__ double tpe[3][NEGP][DOF], teq[3][NEGP][DOF];   // edge tables (lane-divergent index)
-    // staged rows (ns entries each): state [3*DOF], RHS cotangent [3*DOF].  The bathymetry modes
-    // and AREAS are formed from the vertex depths and coordinates where they are needed: staging
-    // them too would take the p=2 block past a quarter of the CU's LDS.
-    extern __shared__ double stg[];
-    constexpr int RL = 3 * DOF;
+    constexpr int NC = P + 1;
+    constexpr int NT = ADJ_NT, RL = 3 * DOF, SR = adj_sum_rows(DOF);
+    // (lane-divergent index) edge basis at the points, and the basis functions along the edge as polynomials
+    // in the points' coordinate
+    __shared__ double tpe[3][NEGP][DOF], tpc[3][NC][DOF];
+    extern __shared__ double stg[];        // the staged rows (ns entries each), then the flags; last the waves' sums
     const DevTables& T = tab<P>();
     const ElemData& E = a.ed;
     const Phys& ph = a.ph;
-    const int ne = E.ne;
-    const int tid = threadIdx.x;
+    const int ne = E.ne, ns = a.ns, nh = a.nh;
+    const int c = __builtin_amdgcn_readfirstlane(threadIdx.x / NT), le = threadIdx.x % NT;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
-    const int e = tile * NT + tid;
-    const double c13 = 1.0 / 3.0, c16 = 1.0 / 6.0;
-    const int ns = a.ns;
-    for (int j = tid; j < 3 * NEGP * DOF; j += NT) {
-        const int l = j / (NEGP * DOF), g = (j / DOF) % NEGP, k = j % DOF;
-        tpe[l][g][k] = T.phi_edge[l][g][k];
-        teq[l][g][k] = T.edgeq[l][g][k];
-    }
+    const int e = tile * NT + le;
+    const bool valid = e < ne;
+    const int ec = valid ? e : ne - 1;     // lanes past the last element read element ne-1 and write nothing
+    uint8_t* const stwd = reinterpret_cast<uint8_t*>(stg + (size_t)adj_stage_rows(DOF) * ns);
+    const int* hx = a.hidx + (size_t)tile * nh;
+    const int sid = E.sid ? (int)E.sid[ec] : 0;
+    const Scen& sc = E.scen[sid];
     {
-        // this tile's elements and its halo, all loads in flight together
-        const int* hx = a.hidx + (size_t)tile * a.nh;
-        for (int j = tid; j < NT + a.nh; j += NT) {
-            const int g = j < NT ? tile * NT + j : hx[j - NT];
-            if (g >= 0 && g < ne) {
+        // two staged elements at a time: the tile's and the first halo's, then the halo's rest
+        auto load = [&](int g, double (&v)[2 * DOF]) {
+            if (c < 3) {
 #pragma unroll
-                for (int f = 0; f < 3 * DOF; f++) stg[f * ns + j] = a.u[(size_t)f * ne + g];
-                double L0[3][DOF];
-                const int sg = E.sid ? (int)E.sid[g] : 0;
-                load_lambda<DOF>(a, ne, g, E.scen[sg].dtdp, L0);
+                for (int k = 0; k < DOF; k++) v[k] = at(a.u + (size_t)(c * DOF + k) * ne, g);
 #pragma unroll
-                for (int f = 0; f < 3; f++)
+                for (int k = 0; k < DOF; k++) v[DOF + k] = 0.0;
+                const double dtdp = E.scen[E.sid ? (int)at(E.sid, g) : 0].dtdp;
+                for (int j = 0; j < a.nsrc; j++) {
+                    if (a.bcoef[j] == 0.0) continue;
+                    const double b = a.bcoef[j] * dtdp;
+                    const double* s = a.src[j];
 #pragma unroll
-                    for (int k = 0; k < DOF; k++) stg[(RL + f * DOF + k) * ns + j] = L0[f][k];
+                    for (int k = 0; k < DOF; k++) v[DOF + k] += b * at(s + (size_t)(c * DOF + k) * ne, g);
+                }
+            } else {
+#pragma unroll
+                for (int m = 0; m < 3; m++) v[m] = at(E.dpv + (size_t)m * ne, g);
+                const double X0 = at(E.xv, g), X1 = at(E.xv + ne, g), X2 = at(E.xv + 2 * (size_t)ne, g);
+                const double Y0 = at(E.yv, g), Y1 = at(E.yv + ne, g), Y2 = at(E.yv + 2 * (size_t)ne, g);
+                v[3] = (X0 - X2) * (Y1 - Y2) + (X2 - X1) * (Y0 - Y2);
+                if (WD) v[4] = __hiloint2double(0, at(a.wd, g));
             }
+        };
+        auto store = [&](int j, const double (&v)[2 * DOF]) {
+            if (c < 3) {
+#pragma unroll
+                for (int k = 0; k < DOF; k++) stg[(c * DOF + k) * ns + j] = v[k];
+#pragma unroll
+                for (int k = 0; k < DOF; k++) stg[(RL + 3 + c * DOF + k) * ns + j] = T.m_inv[k] * v[DOF + k];
+            } else {
+                double hb[3];
+                hb_modes(v[0], v[1], v[2], hb);
+#pragma unroll
+                for (int m = 0; m < 3; m++) stg[(RL + m) * ns + j] = hb[m];
+                stg[(2 * RL + 3) * ns + j] = v[3];
+                if (WD) stwd[j] = (uint8_t)__double2loint(v[4]);
+            }
+        };
+        const int g0 = le < nh ? hx[le] : -1;
+        double v[2 * DOF], v2[2 * DOF];
+        load(ec, v);
+        load(g0 < 0 ? 0 : g0, v2);
+        store(le, v);
+        if (g0 >= 0) store(NT + le, v2);
+#pragma unroll 1
+        for (int h = le + NT; h < nh; h += NT) {
+            const int g = hx[h];
+            if (g < 0) break;
+            load(g, v);
+            store(NT + h, v);
+        }
+        if (c == 3)
+            for (int j = le; j < 3 * NEGP * DOF; j += NT) {
+                const int l = j / (NEGP * DOF), g = (j / DOF) % NEGP, k = j % DOF;
+                tpe[l][g][k] = T.phi_edge[l][g][k];
+            }
+        if (c == 3 && le < 3 * DOF) {
+            const int l = le / DOF, k = le % DOF;
+            const double lo = T.phi_edge[l][0][k], hi = T.phi_edge[l][NEGP - 1][k];   // at -1 and 1
+            if (P == 1) {
+                tpc[l][0][k] = T.phi_edge[l][1][k];                                   // at 0
+            } else {
+                // even part: at 1 and at the inner points
+                const double a = 0.5 * (hi + lo), b = 0.5 * (T.phi_edge[l][1][k] + T.phi_edge[l][2][k]);
+                const double c2 = (a - b) / (1.0 - T.xegp[1] * T.xegp[1]);
+                tpc[l][NC - 1][k] = c2;
+                tpc[l][0][k] = a - c2;
+            }
+            tpc[l][1][k] = 0.5 * (hi - lo);
         }
     }
     __syncthreads();
-    if (e >= ne) return;
-    const int sid = E.sid ? (int)E.sid[e] : 0;
-    const Scen sc = E.scen[sid];
-    const int row = table_step(a.fo) * a.fo.nrk + a.irk;
-    const bool quad = QF || ph.iflinbf == 0;
-    const bool hybrid = !QF && ph.ifhybf == 1;
-
-    double U[3][DOF];
+    const int wd = WD ? (valid ? stwd[le] : 0) : (valid ? 1 : 0);
+    double ubar[3][DOF], hbb[3] = {0.0, 0.0, 0.0}, nbarb = 0.0;
 #pragma unroll
     for (int f = 0; f < 3; f++)
 #pragma unroll
-        for (int k = 0; k < DOF; k++) U[f][k] = stg[(f * DOF + k) * ns + tid];
-#define Lm(f, k) stg[(RL + (f) * DOF + (k)) * ns + tid]
-#pragma unroll
-    for (int j = 0; j < 3 * DOF; j++) ub_lds[j][tid] = 0.0;
-    double hbb[3] = {0.0, 0.0, 0.0};
-    double AREAS, hb[3];
-    elem_hb_areas(E, ne, e, hb, AREAS);
-    const int info = E.sinfo[e];
-    const int nb0 = E.snbr[e], nb1 = E.snbr[(size_t)ne + e], nb2 = E.snbr[2 * (size_t)ne + e];
-    const int sl = a.snbl[e];
-    const int wd = WD ? (int)a.wd[e] : 1;
-#pragma unroll 1
-    for (int slot = 0; slot < 3; slot++) {
-        const int bits = side_bits(info, slot);
+        for (int k = 0; k < DOF; k++) ubar[f][k] = 0.0;
+    // ---- side slot c
+    if (c < 3) {
+        const int bits = side_bits(at(E.sinfo, ec), c);
         const int L = bits & 3, role = (bits >> 2) & 1, kind = (bits >> 3) & 3, nled = (bits >> 5) & 3;
-        const int nb = slot == 0 ? nb0 : (slot == 1 ? nb1 : nb2);
-        int va = (L + 1) % 3, vb = (L + 2) % 3;
-        if (role) { const int t = va; va = vb; vb = t; }
-        const double dy = E.yv[(size_t)vb * ne + e] - E.yv[(size_t)va * ne + e];
-        const double dx = E.xv[(size_t)vb * ne + e] - E.xv[(size_t)va * ne + e];
-        const double xlen = sqrt(dy * dy + dx * dx);
-        const double nx = dy / xlen, ny = -dx / xlen;
-        const double tx = -ny, ty = nx;
+        const double nx = at(E.geo + (size_t)(3 * c) * ne, ec), ny = at(E.geo + (size_t)(3 * c + 1) * ne, ec);
+        const double edfac = at(E.geo + (size_t)(3 * c + 2) * ne, ec);
+        // cotangents of the own traces' polynomials
+        double tb[3][NC], hc[2] = {0.0, 0.0};
+#pragma unroll
+        for (int f = 0; f < 3; f++)
+#pragma unroll
+            for (int m = 0; m < NC; m++) tb[f][m] = 0.0;
+        auto add = [&](double zb, double xb, double yb, double hbar, double s) {
+            double p = 1.0;
+#pragma unroll
+            for (int m = 0; m < NC; m++) {
+                tb[0][m] += zb * p;
+                tb[1][m] += xb * p;
+                tb[2][m] += yb * p;
+                if (m < 2) hc[m] += hbar * p;
+                p = p * s;
+            }
+        };
+        // the traces of the staged element j's RHS cotangent at an edge point
+        auto cotangent = [&](int j, const double* ph_, double (&t)[3]) {
+#pragma unroll
+            for (int f = 0; f < 3; f++) {
+                t[f] = stg[(RL + 3 + f * DOF) * ns + j];
+#pragma unroll
+                for (int k = 1; k < DOF; k++) t[f] += stg[(RL + 3 + f * DOF + k) * ns + j] * ph_[k];
+            }
+        };
         if (kind == SIDE_INTERNAL) {
-            const int ln = (sl >> (10 * slot)) & 1023;
-            const int wdn = WD ? (int)a.wd[nb] : 1;
-            if (wd == 0 && wdn == 0) continue;          // the forward adds no flux between dry elements
-            double V[3][DOF], Ln[3][DOF];
+            const int ln = (at(a.snbl, ec) >> (10 * c)) & 1023;
+            const int wdn = WD ? stwd[ln] : 1;
+            // (the forward adds no flux between dry elements)
+            const double edfac_n = edfac * (stg[(2 * RL + 3) * ns + le] / stg[(2 * RL + 3) * ns + ln]);
+            if (valid && (!WD || (wd != 0 && wdn != 0))) {
+                const double mx = role ? -0.5 * nx : 0.5 * nx, my = role ? -0.5 * ny : 0.5 * ny;
+                const double nan = __builtin_nan("");
+                const double bo = role ? -1.0 : nan, bn = role ? nan : -1.0;
+                // the traces along the edge as polynomials in the own points' coordinate (the neighbour's runs the
+                // other way), formed once per side from the modes: at p=2 30 numbers stay instead of 78, and
+                // the tables of the points are the same for every lane
+                auto along = [&](int row, int j, int l, double sign, int n, double (&t)[NC]) {
 #pragma unroll
-            for (int f = 0; f < 3; f++)
-#pragma unroll
-                for (int k = 0; k < DOF; k++) {
-                    V[f][k] = stg[(f * DOF + k) * ns + ln];
-                    Ln[f][k] = stg[(RL + f * DOF + k) * ns + ln];
-                }
-            double hbn[3], areas_n;
-            elem_hb_areas(E, ne, nb, hbn, areas_n);
-            const double edfac = xlen / AREAS, edfac_n = xlen / areas_n;
-#pragma unroll 1
-            for (int I = 0; I < NEGP; I++) {
-                const int gi = I, gx = NEGP - 1 - I;
-                const int gown = role ? gx : gi, gnb = role ? gi : gx;
-                const double* po = tpe[L][gown];
-                const double* pn = tpe[nled][gnb];
-                const double zo = trace<DOF>(U[0], po), xo = trace<DOF>(U[1], po), yo = trace<DOF>(U[2], po);
-                const double zn = trace<DOF>(V[0], pn), xn = trace<DOF>(V[1], pn), yn = trace<DOF>(V[2], pn);
-                const double ho = trace<3>(hb, po), hn = trace<3>(hbn, pn);
-                double so = 1.0, sn = 1.0;
-                if (SPH) {
-                    so = E.sfaced[((size_t)L * NEGP + gown) * ne + e];
-                    sn = E.sfaced[((size_t)nled * NEGP + gnb) * ne + nb];
-                }
-                // flux cotangent: the "in" element's RHS took -w_in*F, the "ex" element's +w_ex*F
-                const double* eqo = teq[L][gown];
-                const double* eqn = teq[nled][gnb];
-                double fb[3], cin[3], cex[3];
-#pragma unroll
-                for (int f = 0; f < 3; f++) {
-                    double so_ = 0.0, sn_ = 0.0;
+                    for (int m = 0; m < NC; m++) t[m] = 0.0;
 #pragma unroll
                     for (int k = 0; k < DOF; k++) {
-                        so_ = so_ + edfac * eqo[k] * Lm(f, k);
-                        sn_ = sn_ + edfac_n * eqn[k] * Ln[f][k];
+                        if (k >= n) break;
+                        const double v = stg[(row + k) * ns + j];
+#pragma unroll
+                        for (int m = 0; m < NC; m++)
+                            if (n == DOF || m < 2) t[m] += v * tpc[l][m][k];
                     }
-                    fb[f] = role ? (so_ - sn_) : (sn_ - so_);
-                    cin[f] = role ? -sn_ : -so_;
-                    cex[f] = role ? so_ : sn_;
-                }
-                // canonical (in, ex) order; this element is side `role`
-                double zb, xb, yb, hbar;
-                if (wd != 0 && wdn != 0) {
-                    llf_flux_adj_side<NL>(ph, role ? zn : zo, role ? zo : zn, role ? xn : xo, role ? xo : xn,
-                                          role ? yn : yo, role ? yo : yn, role ? hn : ho, role ? ho : hn,
-                                          role ? sn : so, role ? so : sn, nx, ny, ph.g, fb, role, zb, xb, yb, hbar);
-                } else {
-                    dry_side_adj<P, NL>(ph, E, ne, e, nb, L, role, nled, gi, gx, U, V, wd, wdn,
-                                        role ? zn : zo, role ? zo : zn, role ? xn : xo, role ? xo : xn,
-                                        role ? yn : yo, role ? yo : yn, role ? hn : ho, role ? ho : hn,
-                                        role ? sn : so, role ? so : sn, nx, ny, cin, cex, zb, xb, yb, hbar);
+                    t[1] = sign * t[1];
+                };
+                double to[4][NC], tn[4][NC], fc[3][NC];
+#pragma unroll
+                for (int f = 0; f < 4; f++) {
+                    along(f * DOF, le, L, 1.0, f < 3 ? DOF : 3, to[f]);
+                    along(f * DOF, ln, nled, -1.0, f < 3 ? DOF : 3, tn[f]);
                 }
 #pragma unroll
-                for (int k = 0; k < DOF; k++) {
-                    ub_lds[k][tid] += zb * po[k];
-                    ub_lds[DOF + k][tid] += xb * po[k];
-                    ub_lds[2 * DOF + k][tid] += yb * po[k];
-                }
+                for (int f = 0; f < 3; f++) {
+                    double co[NC], cn[NC];
+                    along(RL + 3 + f * DOF, le, L, 1.0, DOF, co);
+                    along(RL + 3 + f * DOF, ln, nled, -1.0, DOF, cn);
 #pragma unroll
-                for (int k = 0; k < 3; k++) hbb[k] += hbar * po[k];
+                    for (int m = 0; m < NC; m++) fc[f][m] = 2.0 * (edfac_n * cn[m] - edfac * co[m]);
+                }
+                auto point = [&](const double (&t)[NC], double s, int n) {
+                    double v = t[n - 1];
+#pragma unroll
+                    for (int m = NC - 2; m >= 0; m--)
+                        if (m < n - 1) v = v * s + t[m];
+                    return v;
+                };
+#pragma unroll 1
+                for (int q = 0; q < NEGP; q++) {
+                    const double s = T.xegp[q], w = T.wegp[q];
+                    const double o[4] = {point(to[0], s, NC), point(to[1], s, NC), point(to[2], s, NC), point(to[3], s, 2)};
+                    const double n[4] = {point(tn[0], s, NC), point(tn[1], s, NC), point(tn[2], s, NC), point(tn[3], s, 2)};
+                    const double fq[3] = {w * point(fc[0], s, NC), w * point(fc[1], s, NC), w * point(fc[2], s, NC)};
+                    double so = 1.0, sn = 1.0;
+                    if (SPH) {
+                        const int I = role ? NEGP - 1 - q : q;
+                        so = E.sfs[(size_t)(c * NEGP + I) * ne + ec];
+                        sn = E.sfs[(size_t)((3 + c) * NEGP + I) * ne + ec];
+                    }
+                    double bar[4];
+                    llf_adj_own<NL>(ph, o, n, so, sn, nx, ny, mx, my, fq, role == 0, bo, bn, bar);
+                    add(bar[0], bar[1], bar[2], bar[3], s);
+                }
             }
-        } else {
-            if (wd == 0) continue;                      // the forward skips a dry element's boundary edges
+            if constexpr (WD)
+                if (valid && (wd != 0) != (wdn != 0)) {
+#pragma unroll 1
+                    for (int q = 0; q < NEGP; q++) {
+                        const int gi = role ? NEGP - 1 - q : q;
+                        const double* po = tpe[L][q];
+                        const double* pn = tpe[nled][NEGP - 1 - q];
+                        const int jo = reread(le), jn = reread(ln);
+                        double to[4], tn[4], co[3], cn[3];
+                        edge_point<DOF>(stg, ns, role ? jn : jo, role ? pn : po, to);   // the "in" side's
+                        edge_point<DOF>(stg, ns, role ? jo : jn, role ? po : pn, tn);   // the "ex" side's
+                        double so = 1.0, sn = 1.0;
+                        if (SPH) {
+                            so = E.sfs[(size_t)(c * NEGP + gi) * ne + ec];
+                            sn = E.sfs[(size_t)((3 + c) * NEGP + gi) * ne + ec];
+                        }
+                        // flux cotangents: the "in" element's RHS took -w_in*F, the "ex" element's +w_ex*F
+                        cotangent(jo, po, co);
+                        cotangent(jn, pn, cn);
+                        const double w = 2.0 * T.wegp[q];
+                        double cin[3], cex[3];
+#pragma unroll
+                        for (int f = 0; f < 3; f++) {
+                            cin[f] = role ? -(w * edfac_n * cn[f]) : -(w * edfac * co[f]);
+                            cex[f] = role ? w * edfac * co[f] : w * edfac_n * cn[f];
+                        }
+                        const double sfi = role ? sn : so, sfx = role ? so : sn;
+                        const int cas = dry_side_case<NL>(ph, role ? wdn : wd, role ? wd : wdn, to, tn, sfi, sfx, nx, ny);
+                        double zb, xb, yb, hbar;
+                        dry_side_adj<NL>(ph, cas, role, to, tn, sfi, sfx, nx, ny, cin, cex, zb, xb, yb, hbar);
+                        add(zb, xb, yb, hbar, T.xegp[q]);
+                    }
+                }
+        } else if (wd != 0) {                            // the forward skips a dry element's boundary edges
+            const double tx = -ny, ty = nx;
+            const int nb = at(E.snbr + (size_t)c * ne, ec);
 #pragma unroll 1
             for (int I = 0; I < NEGP; I++) {
                 const double* pv = tpe[L][I];
-                const double ze_in = trace<DOF>(U[0], pv), qx_in = trace<DOF>(U[1], pv), qy_in = trace<DOF>(U[2], pv);
-                const double hb_in = trace<3>(hb, pv);
-                const double sf = SPH ? E.sfaced[((size_t)L * NEGP + I) * ne + e] : 1.0;
+                const int jo = reread(le);
+                double t[4], co[3];
+                edge_point<DOF>(stg, ns, jo, pv, t);
+                cotangent(jo, pv, co);
+                const double ze_in = t[0], qx_in = t[1], qy_in = t[2], hb_in = t[3];
+                const double sf = SPH ? E.sfs[(size_t)(c * NEGP + I) * ne + ec] : 1.0;
                 // flux cotangent: RHS(K) -= w_K*F with w_K = 2 M_INV(K)/AREAS*XLEN*PHI*WEGP
-                double fb[3] = {0.0, 0.0, 0.0};
-                const double wq = 2.0 * xlen / AREAS * T.wegp[I];
-#pragma unroll
-                for (int k = 0; k < DOF; k++) {
-                    const double w = wq * T.m_inv[k] * pv[k];
-                    fb[0] = fb[0] - w * Lm(0, k);
-                    fb[1] = fb[1] - w * Lm(1, k);
-                    fb[2] = fb[2] - w * Lm(2, k);
-                }
+                const double wq = -2.0 * T.wegp[I] * edfac;
+                const double fb[3] = {wq * co[0], wq * co[1], wq * co[2]};
                 double bar[8];
                 double zb = 0.0, xb = 0.0, yb = 0.0, hbar = 0.0;
                 if (kind == SIDE_LAND) {
@@ -650,37 +756,45 @@ __global__ void __launch_bounds__(NT, P == 1 ? 2 : 1) adj_stage_kernel(AdjArgs a
                     yb = bar[4];
                     hbar = bar[6] + bar[7];
                 }
-#pragma unroll
-                for (int k = 0; k < DOF; k++) {
-                    ub_lds[k][tid] += zb * pv[k];
-                    ub_lds[DOF + k][tid] += xb * pv[k];
-                    ub_lds[2 * DOF + k][tid] += yb * pv[k];
-                }
-#pragma unroll
-                for (int k = 0; k < 3; k++) hbb[k] += hbar * pv[k];
+                add(zb, xb, yb, hbar, T.xegp[I]);
             }
         }
+#pragma unroll
+        for (int k = 0; k < DOF; k++)
+#pragma unroll
+            for (int m = 0; m < NC; m++) {
+                const double t = tpc[L][m][k];
+#pragma unroll
+                for (int f = 0; f < 3; f++) ubar[f][k] += tb[f][m] * t;
+                if (k < 3 && m < 2) hbb[k] += hc[m] * t;
+            }
     }
 
-    // ---- volume quadrature (wet elements only, as in the forward)
-    double nbarb = 0.0;
-    if (wd != 0) {
-        double drdx, dsdx, drdy, dsdy;
-        {
-            const double X0 = E.xv[e], X1 = E.xv[(size_t)ne + e], X2 = E.xv[2 * (size_t)ne + e];
-            const double Y0 = E.yv[e], Y1 = E.yv[(size_t)ne + e], Y2 = E.yv[2 * (size_t)ne + e];
-            double AREA = (X0 - X2) * (Y1 - Y2) + (X2 - X1) * (Y0 - Y2);
-            AREA = AREA * 0.5;
-            drdx = 1.0 / AREA * (Y2 - Y0);
-            dsdx = 1.0 / AREA * (Y0 - Y1);
-            drdy = 1.0 / AREA * (X0 - X2);
-            dsdy = 1.0 / AREA * (X1 - X0);
-        }
-        const double depth_c = hb[0] + U[0][0];
+    // ---- volume quadrature (wet elements only, as in the forward): points [i0, i1) of this wave
+    const int i0 = P == 1 || c == 3 ? 0 : 3 + c, i1 = c == 3 ? 3 : (P == 1 ? 0 : 4 + c);
+    if (i0 < i1 && wd != 0) {
+        double hb[3];
+#pragma unroll
+        for (int m = 0; m < 3; m++) hb[m] = stg[(RL + m) * ns + le];
+        const bool quad = QF || ph.iflinbf == 0;
+        const bool hybrid = !QF && ph.ifhybf == 1;
+        const int row = table_step(a.fo) * a.fo.nrk + a.irk;
+        const double drdx = at(E.geo + (size_t)9 * ne, ec), dsdx = at(E.geo + (size_t)10 * ne, ec);
+        const double drdy = at(E.geo + (size_t)11 * ne, ec), dsdy = at(E.geo + (size_t)12 * ne, ec);
+        const double depth_c = hb[0] + stg[le];
         const double fh_nl_c = NL ? 1.0 / depth_c : 1.0 / (ph.nleq * depth_c + ph.leq);
-        const double cori = E.cori_el ? E.cori_el[e] : sc.cori;
-        const double nbar = ph.load_manning ? E.nbar[e] : 0.0;
+        const double cori = E.cori_el ? at(E.cori_el, ec) : sc.cori;
+        const double nbar = ph.load_manning ? at(E.nbar, ec) : 0.0;
         double depth_cb = 0.0;
+        // the bathymetry's gradient (its modes are linear, so it is the same at every point) and its cotangent
+        double dpx[3], dpy[3], dhbx = 0.0, dhby = 0.0, dhbxb = 0.0, dhbyb = 0.0;
+#pragma unroll
+        for (int k = 1; k < 3; k++) {
+            dpx[k] = T.drphi[0][k] * drdx + T.dsphi[0][k] * dsdx;
+            dpy[k] = T.drphi[0][k] * drdy + T.dsphi[0][k] * dsdy;
+            dhbx = dhbx + hb[k] * dpx[k];
+            dhby = dhby + hb[k] * dpy[k];
+        }
         // NWS=8: the stage's vertex wind stresses and the pressure-gradient sums, as the forward
         // forms them; the pressure term -g*SFAC*H*dP/dx depends on the state through H
         double mw[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, pdx = 0.0, pdy = 0.0;
@@ -689,35 +803,31 @@ __global__ void __launch_bounds__(NT, P == 1 ? 2 : 1) adj_stage_kernel(AdjArgs a
             const double drpsi[3] = {-1.0 / 2.0, 1.0 / 2.0, 0.0}, dspsi[3] = {-1.0 / 2.0, 0.0, 1.0 / 2.0};
 #pragma unroll
             for (int v = 0; v < 3; v++) {
-                const int n = E.nm[(size_t)v * ne + e];
-                const double cd = a.mt.cd[n], wm = a.mt.wm[n];
-                mw[v] = ramp * 0.001293 * cd * a.mt.wx[n] * wm;
-                mw[3 + v] = ramp * 0.001293 * cd * a.mt.wy[n] * wm;
+                const int n = at(E.nm + (size_t)v * ne, ec);
+                if constexpr (!NL) {
+                    const double cd = a.mt.cd[n], wm = a.mt.wm[n];
+                    mw[v] = ramp * 0.001293 * cd * a.mt.wx[n] * wm;
+                    mw[3 + v] = ramp * 0.001293 * cd * a.mt.wy[n] * wm;
+                }
                 const double pr = ramp * a.mt.prn[n];
                 pdx += pr * (drpsi[v] * drdx + dspsi[v] * dsdx);
                 pdy += pr * (drpsi[v] * drdy + dspsi[v] * dsdy);
             }
         }
 #pragma unroll 1
-        for (int I = 0; I < NAGP; I++) {
+        for (int I = i0; I < i1; I++) {
             const double* pa = T.phi_area[I];
-            double ze = U[0][0], qx = U[1][0], qy = U[2][0];
+            // read where it is used: held over the points the modes would set the kernel's register count
+            const int jo = reread(le);
+            auto value = [&](int row) {
+                double t = stg[row * ns + jo];
 #pragma unroll
-            for (int k = 1; k < DOF; k++) {
-                ze = ze + U[0][k] * pa[k];
-                qx = qx + U[1][k] * pa[k];
-                qy = qy + U[2][k] * pa[k];
-            }
-            double hbq = 0.0, dhbx = 0.0, dhby = 0.0;
-#pragma unroll
-            for (int k = 0; k < 3; k++) {
-                const double dpxk = T.drphi[I][k] * drdx + T.dsphi[I][k] * dsdx;
-                const double dpyk = T.drphi[I][k] * drdy + T.dsphi[I][k] * dsdy;
-                hbq = hbq + hb[k] * pa[k];
-                dhbx = dhbx + hb[k] * dpxk;
-                dhby = dhby + hb[k] * dpyk;
-            }
-            const double sfq = SPH ? E.sfacq[(size_t)I * ne + e] : 1.0;
+                for (int k = 1; k < DOF; k++) t += stg[(row + k) * ns + jo] * pa[k];
+                return t;
+            };
+            const double ze = value(0), qx = value(DOF), qy = value(2 * DOF);
+            const double hbq = trace1<3>(hb, pa);
+            const double sfq = SPH ? at(E.sfacq + (size_t)I * ne, ec) : 1.0;
             const double depth = ze + hbq;
             const double f1 = NL ? 1.0 : ph.nleq + ph.leq * hbq;
             const double fu = NL ? qx : ph.nleq * qx, fv = NL ? qy : ph.nleq * qy;
@@ -746,19 +856,25 @@ __global__ void __launch_bounds__(NT, P == 1 ? 2 : 1) adj_stage_kernel(AdjArgs a
                 const double cap = 0.9 * sc.dtdph;
                 if (cap < tau) { tau = cap; capped = true; }
             }
-            // cotangents of the quadrature-point fluxes and sources from RHS(K)
-            double fxb = 0.0, fyb = 0.0, gxb = 0.0, gyb = 0.0, hxb = 0.0, hyb_ = 0.0;
-            double sxb = T.srfac[I][0] * Lm(1, 0), syb = T.srfac[I][0] * Lm(2, 0);
+            // cotangents of the quadrature-point fluxes and sources from RHS(K): XFAC = M_INV*WAGP*dphi/dx and
+            // SRFAC = M_INV*WAGP*PHI, with WAGP = 2*(M_INV(1)*WAGP)
+            const double wagp = 2.0 * T.mw[I][0];
+            double dr[3] = {0.0, 0.0, 0.0}, ds[3] = {0.0, 0.0, 0.0};
 #pragma unroll
             for (int k = 1; k < DOF; k++) {
-                const double dpxk = T.drphi[I][k] * drdx + T.dsphi[I][k] * dsdx;
-                const double dpyk = T.drphi[I][k] * drdy + T.dsphi[I][k] * dsdy;
-                const double xf = T.mw[I][k] * dpxk, yf = T.mw[I][k] * dpyk, sr = T.srfac[I][k];
-                fxb += xf * Lm(0, k); fyb += yf * Lm(0, k);
-                gxb += xf * Lm(1, k); gyb += yf * Lm(1, k); sxb += sr * Lm(1, k);
-                hxb += xf * Lm(2, k); hyb_ += yf * Lm(2, k); syb += sr * Lm(2, k);
+                const double r = wagp * T.drphi[I][k], s = wagp * T.dsphi[I][k];
+#pragma unroll
+                for (int f = 0; f < 3; f++) {
+                    const double l = stg[(RL + 3 + f * DOF + k) * ns + jo];
+                    dr[f] += r * l;
+                    ds[f] += s * l;
+                }
             }
-            double zeb = 0.0, qxb = 0.0, qyb = 0.0, hbqb = 0.0, dhbxb = 0.0, dhbyb = 0.0, depthb = 0.0;
+            const double fxb = drdx * dr[0] + dsdx * ds[0], fyb = drdy * dr[0] + dsdy * ds[0];
+            const double gxb = drdx * dr[1] + dsdx * ds[1], gyb = drdy * dr[1] + dsdy * ds[1];
+            const double hxb = drdx * dr[2] + dsdx * ds[2], hyb_ = drdy * dr[2] + dsdy * ds[2];
+            const double sxb = wagp * value(RL + 3 + DOF), syb = wagp * value(RL + 3 + 2 * DOF);
+            double zeb = 0.0, qxb = 0.0, qyb = 0.0, hbqb = 0.0, depthb = 0.0;
             // sx = -(tau*qx) + fg*dhbx*sfq + cori*qy ; sy = -(tau*qy) + fg*dhby - cori*qx
             double taub = -qx * sxb - qy * syb;
             double f1b_met = 0.0;
@@ -834,47 +950,63 @@ __global__ void __launch_bounds__(NT, P == 1 ? 2 : 1) adj_stage_kernel(AdjArgs a
             zeb += depthb;
             hbqb += depthb;
             // traces
-            ub_lds[0][tid] += zeb;
-            ub_lds[DOF][tid] += qxb;
-            ub_lds[2 * DOF][tid] += qyb;
 #pragma unroll
-            for (int k = 1; k < DOF; k++) {
-                ub_lds[k][tid] += zeb * pa[k];
-                ub_lds[DOF + k][tid] += qxb * pa[k];
-                ub_lds[2 * DOF + k][tid] += qyb * pa[k];
+            for (int k = 0; k < DOF; k++) {
+                ubar[0][k] += zeb * pa[k];
+                ubar[1][k] += qxb * pa[k];
+                ubar[2][k] += qyb * pa[k];
             }
 #pragma unroll
-            for (int k = 0; k < 3; k++) {
-                const double dpxk = T.drphi[I][k] * drdx + T.dsphi[I][k] * dsdx;
-                const double dpyk = T.drphi[I][k] * drdy + T.dsphi[I][k] * dsdy;
-                hbb[k] += hbqb * pa[k] + dhbxb * dpxk + dhbyb * dpyk;
-            }
+            for (int k = 0; k < 3; k++) hbb[k] += hbqb * pa[k];
         }
+#pragma unroll
+        for (int k = 1; k < 3; k++) hbb[k] += dhbxb * dpx[k] + dhbyb * dpy[k];
         // depth_c = hb[0] + U[0][0]
         hbb[0] += depth_cb;
-        ub_lds[0][tid] += depth_cb;
+        ubar[0][0] += depth_cb;
     }
-    // ---- cotangent of U(IRK): later stages' ATVD terms plus this stage's RHS reverse
-    for (int j = 0; j < a.nsrc; j++) {
-        const double ac = a.acoef[j];
-        if (ac == 0.0) continue;
-        const double* s = a.src[j];
+    // ---- the waves' sums; the staged rows are no longer needed
+    __syncthreads();
+    {
+        double* const x = stg + (size_t)c * SR * NT + le;
 #pragma unroll
-        for (int f = 0; f < 3 * DOF; f++) ub_lds[f][tid] += ac * s[(size_t)f * ne + e];
-    }
+        for (int f = 0; f < 3; f++)
 #pragma unroll
-    for (int f = 0; f < 3 * DOF; f++) a.out[(size_t)f * ne + e] = ub_lds[f][tid];
-    // parameters: element-mean Manning n and the vertex depths through the P1 bathymetry modes
-    if (a.gnbar) a.gnbar[e] += nbarb;
-    if (a.gdp) {
-        const double D0b = c13 * hbb[0] - c16 * hbb[1] - 0.5 * hbb[2];
-        const double D1b = c13 * hbb[0] - c16 * hbb[1] + 0.5 * hbb[2];
-        const double D2b = c13 * hbb[0] + c13 * hbb[1];
-        a.gdp[e] += D0b;
-        a.gdp[(size_t)ne + e] += D1b;
-        a.gdp[2 * (size_t)ne + e] += D2b;
+            for (int k = 0; k < DOF; k++) x[(f * DOF + k) * NT] = ubar[f][k];
+#pragma unroll
+        for (int k = 0; k < 3; k++) x[(RL + k) * NT] = hbb[k];
+        x[(RL + 3) * NT] = nbarb;
     }
-#undef Lm
+    __syncthreads();
+    if (!valid) return;
+    auto sum = [&](int r) {
+        const double* x = stg + (size_t)r * NT + le;
+        return x[0] + x[SR * NT] + x[2 * SR * NT] + x[3 * SR * NT];
+    };
+    if (c < 3) {
+        // cotangent of U(IRK): this stage's RHS reverse plus later stages' ATVD terms
+        double s[DOF];
+#pragma unroll
+        for (int k = 0; k < DOF; k++) s[k] = sum(c * DOF + k);
+        for (int j = 0; j < a.nsrc; j++) {
+            const double ac = a.acoef[j];
+            if (ac == 0.0) continue;
+#pragma unroll
+            for (int k = 0; k < DOF; k++) s[k] += ac * at(a.src[j] + (size_t)(c * DOF + k) * ne, e);
+        }
+#pragma unroll
+        for (int k = 0; k < DOF; k++) at(a.out + (size_t)(c * DOF + k) * ne, e) = s[k];
+    } else {
+        // parameters: element-mean Manning n and the vertex depths through the P1 bathymetry modes
+        const double c13 = 1.0 / 3.0, c16 = 1.0 / 6.0;
+        const double b0 = sum(RL), b1 = sum(RL + 1), b2 = sum(RL + 2);
+        if (a.gnbar) a.gnbar[e] += sum(RL + 3);
+        if (a.gdp) {
+            a.gdp[e] += c13 * b0 - c16 * b1 - 0.5 * b2;
+            a.gdp[(size_t)ne + e] += c13 * b0 - c16 * b1 + 0.5 * b2;
+            a.gdp[2 * (size_t)ne + e] += c13 * b0 + c13 * b1;
+        }
+    }
 }
 
 // ------------------------------------------------------------------------------------------

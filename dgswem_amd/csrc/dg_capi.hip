@@ -1115,8 +1115,10 @@ int build_stage_tables(Ctx& c, int it, int n) {
 // Static LDS bytes of stage_kernel (its edge tables).
 size_t stage_static_lds(int dof, int negp) { return (size_t)8 * (2 * 3 * negp * dof); }
 
-// Dynamic LDS bytes of adj_stage_kernel: 6*dof staged rows of ns doubles.
-size_t adj_dynamic_lds(int dof, int ns) { return (size_t)8 * (6 * dof) * ns; }
+// Dynamic LDS bytes of adj_stage_kernel: its staged rows and flags, later the four waves' sums.
+size_t adj_dynamic_lds(int dof, int ns) {
+    return std::max(((size_t)8 * adj_stage_rows(dof) * ns + ns + 7) / 8 * 8, (size_t)8 * 4 * adj_sum_rows(dof) * ADJ_NT);
+}
 
 // Whether the stage runs as four waves per 64 elements (stage_split_kernel): the nonlinear equations and, unless
 // the launch shape was chosen by dg_gpu_set_block or the autotuner, few elements.  Measured per launch, one lane
@@ -1517,22 +1519,23 @@ int adj_check(Ctx& c) {
     return 0;
 }
 
-template <int P, int NT, bool NL, bool WD>
+template <int P, bool NL, bool WD>
 int launch_adj_v(Ctx& c, const AdjArgs& a, int grid, size_t lds, bool qf) {
+    const dim3 b(4 * ADJ_NT);
     if (c.prm.ics == 2) {
-        if (qf) hipLaunchKernelGGL((adj_stage_kernel<P, NT, true, NL, NL, WD>), dim3(grid), dim3(NT), lds, c.stream, a);
-        else hipLaunchKernelGGL((adj_stage_kernel<P, NT, true, NL, false, WD>), dim3(grid), dim3(NT), lds, c.stream, a);
+        if (qf) hipLaunchKernelGGL((adj_stage_kernel<P, true, NL, NL, WD>), dim3(grid), b, lds, c.stream, a);
+        else hipLaunchKernelGGL((adj_stage_kernel<P, true, NL, false, WD>), dim3(grid), b, lds, c.stream, a);
     } else {
-        if (qf) hipLaunchKernelGGL((adj_stage_kernel<P, NT, false, NL, NL, WD>), dim3(grid), dim3(NT), lds, c.stream, a);
-        else hipLaunchKernelGGL((adj_stage_kernel<P, NT, false, NL, false, WD>), dim3(grid), dim3(NT), lds, c.stream, a);
+        if (qf) hipLaunchKernelGGL((adj_stage_kernel<P, false, NL, NL, WD>), dim3(grid), b, lds, c.stream, a);
+        else hipLaunchKernelGGL((adj_stage_kernel<P, false, NL, false, WD>), dim3(grid), b, lds, c.stream, a);
     }
     return 0;
 }
 
-template <int P, int NT, bool NL>
+template <int P, bool NL>
 int launch_adj_nl(Ctx& c, const AdjArgs& a0) {
-    const int grid = (c.ne + NT - 1) / NT;
-    auto it = c.stg.find(NT);
+    const int grid = (c.ne + ADJ_NT - 1) / ADJ_NT;
+    auto it = c.stg.find(ADJ_NT);
     if (it == c.stg.end()) return fail("internal: adjoint staging not built for this block size");
     AdjArgs a = a0;
     a.hidx = it->second.hidx.p; a.snbl = it->second.snbl.p; a.nh = it->second.nh; a.ns = it->second.ns;
@@ -1543,26 +1546,22 @@ int launch_adj_nl(Ctx& c, const AdjArgs& a0) {
     // NOLIBF=1 (quadratic friction, no hybrid factor) with the nonlinear equations: friction fixed
     // at compile time
     const bool qf = NL && c.phys.iflinbf == 0 && c.phys.ifhybf == 0;
-    if (a.wd) return launch_adj_v<P, NT, NL, true>(c, a, grid, lds, qf);
-    return launch_adj_v<P, NT, NL, false>(c, a, grid, lds, qf);
+    if (a.wd) return launch_adj_v<P, NL, true>(c, a, grid, lds, qf);
+    return launch_adj_v<P, NL, false>(c, a, grid, lds, qf);
 }
 
-template <int P, int NT>
+template <int P>
 int launch_adj(Ctx& c, const AdjArgs& a) {
-    if (c.prm.nolicat != 0) return launch_adj_nl<P, NT, true>(c, a);
-    return launch_adj_nl<P, NT, false>(c, a);
+    if (c.prm.nolicat != 0) return launch_adj_nl<P, true>(c, a);
+    return launch_adj_nl<P, false>(c, a);
 }
-
-// Block size of the adjoint stage kernel.
-int adj_nt(int p) { return p == 1 ? 128 : 64; }
 
 // The adjoint kernel's block-local staging: the forward's halo lists for its block size, with its
 // own row count (state and RHS cotangent per staged element).
 int ensure_adj_staging(Ctx& c) {
-    const int nt = adj_nt(c.prm.p);
-    if (ensure_staging(c, nt)) return 1;
-    const size_t stat = (size_t)8 * (3 * c.dof * nt + 2 * 3 * c.negp * c.dof);
-    if (adj_dynamic_lds(c.dof, c.stg[nt].ns) + stat > (size_t)c.max_lds)
+    if (ensure_staging(c, ADJ_NT)) return 1;
+    const size_t stat = (size_t)8 * (3 * (c.negp + c.prm.p + 1) * c.dof);
+    if (adj_dynamic_lds(c.dof, c.stg[ADJ_NT].ns) + stat > (size_t)c.max_lds)
         return fail("adjoint staging needs more LDS than a block may use");
     return 0;
 }
@@ -1691,10 +1690,7 @@ int adj_backward(Ctx& c, int it0, int nsteps, int interval, double weight) {
                 a.gdp = c.gdp.p;
                 a.gnbar = c.phys.load_manning ? c.gnb.p : nullptr;
                 a.wd = wdrev_on ? fstage(k, i) : nullptr;
-                int rc;
-                if constexpr (P == 1) rc = launch_adj<P, 128>(c, a);
-                else rc = launch_adj<P, 64>(c, a);
-                if (rc) return rc;
+                if (launch_adj<P>(c, a)) return 1;
                 HIPCHK(hipGetLastError());
                 // ub[i] is now the whole cotangent of U(i), the output of stage i-1
                 if (wdrev_on && i >= 1 && wdrev(ub[i], wstage(k, i - 1), fstage(k, i - 1))) return 1;

@@ -1,0 +1,33 @@
+"""The adjoint stage kernel at the edges of its tiles of 64 elements (one short, a full tile, one pair more, several
+tiles), at both orders, with ocean, land and flow sides, the nonlinear and the linearised equations: gradients against
+fourth-order central differences, with the tolerance of the gradient tests on larger meshes (the difference's
+truncation is O(1e-16), its rounding about 1e-13/1e-4)."""
+import numpy as np
+import pytest
+
+from dgswem_amd import adjoint, mesh
+from test_gpu_adjoint import TOL, central_fd, directions
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nx,ny", [(31, 1), (8, 4), (11, 3), (13, 8)])
+@pytest.mark.parametrize("p", [1, 2])
+@pytest.mark.parametrize("nonlinear", [1, 0])
+def test_tile_edges(nx, ny, p, nonlinear):
+    c = mesh.structured_basin(nx=nx, ny=ny, dx=900.0, dy=1100.0, depth=6.0, amp=0.3, p=p, dt=6.0 if p == 1 else 3.0,
+                              flow_side=True, flow_amp=0.5, cori=1.0e-4)
+    c.params.nolica = c.params.nolicat = nonlinear
+    c.params.cf = 1e-4
+    rng = np.random.default_rng(nx * 10 + p)
+    c.x = c.x + rng.uniform(-60.0, 60.0, c.np_)          # no two sides alike: no ties between wave speeds
+    c.y = c.y + rng.uniform(-60.0, 60.0, c.np_)
+    c.dp = c.dp * (1.0 + 0.2 * rng.uniform(-1.0, 1.0, c.np_))
+    prob = adjoint.twin_problem(c, nsteps=20, ng=7, seed=3)
+    J, gn, gdp = prob.gradient(c.manning, c.dp)
+    assert J > 0.0 and np.isfinite(gn).all() and np.isfinite(gdp).all()
+    for vn, vd in directions(c, 3, seed=8):
+        ad = float(gn @ vn + gdp @ vd)
+        fd = central_fd(prob, c, vn, vd)
+        print(f"adjoint {ad:.12e} fd {fd:.12e} rel {abs(fd - ad) / abs(ad):.2e}", flush=True)
+        assert abs(fd - ad) <= TOL * abs(ad)
