@@ -1339,7 +1339,8 @@ LimTiles lim_tiles(const Ctx& c) {
 // SLOPELIMITER5 (+ WETDRY) on the stage output u, in place; with WETDRY the stage kernel has left
 // u's cell means in c.cmean.
 template <int P>
-int launch_limiter(Ctx& c, double* u, const ElemData& ed, bool capturing) {
+int launch_limiter(Ctx& c, double* u, const ElemData& ed, bool capturing, const uint8_t* fin = nullptr,
+                   uint8_t* fout = nullptr) {
     const int ne = c.ne;
     if (!c.lim.elq.p || !c.cmean.p) return fail("internal: slope limiter tiles not built");
     const bool wdon = c.prm.nolifa >= 2;
@@ -1348,12 +1349,12 @@ int launch_limiter(Ctx& c, double* u, const ElemData& ed, bool capturing) {
     const LimTiles lt = lim_tiles(c);
     const dim3 grid((ne + LIM_NT - 1) / LIM_NT), block(3 * LIM_NT);
     const size_t lds = lim_lds(lt.nvh, lt.nql);
-    const uint8_t* wd = c.wd[c.wdcur].p;
+    const uint8_t* wd = fin ? fin : c.wd[c.wdcur].p;
     int ev = prof_begin(c, K_LIMIT, capturing);
     if (wdon) {
         hipLaunchKernelGGL((limit_wetdry_kernel<P, true, false>), grid, block, lds, c.stream, ed, u, cm, cms, lt, wd,
-                           c.wd[1 - c.wdcur].p, c.wd_active, (double*)nullptr, (double*)nullptr);
-        c.wdcur = 1 - c.wdcur;
+                           fout ? fout : c.wd[1 - c.wdcur].p, c.wd_active, (double*)nullptr, (double*)nullptr);
+        if (!fout) c.wdcur = 1 - c.wdcur;
     } else {
         hipLaunchKernelGGL((limit_wetdry_kernel<P, false, false>), grid, block, lds, c.stream, ed, u, cm, cms, lt, wd,
                            c.wd[1 - c.wdcur].p, (int*)nullptr, (double*)nullptr, (double*)nullptr);
@@ -1429,15 +1430,14 @@ int capture_steps(Ctx& c, int n) {
 }
 
 // One step with explicit state pointers: st[0] input, st[1..NRK-1] the intermediate stage states,
-// st[NRK] output.  With the slope limiter on, each stage's output before limiting is also copied to
-// wsave[irk] (when wsave is given) for the adjoint's frozen-limiter reverse, and the wet/dry flags
-// at the start of each stage to fsave[irk] (when given).
+// st[NRK] output.  With the slope limiter on, each stage's output before limiting is also written to
+// wsave[irk] (when wsave is given) for the adjoint's frozen-limiter reverse; fsave (when given) holds the wet/dry
+// flags at the start of stage irk in fsave[irk] and takes the step's last flags in fsave[NRK].
 template <int P>
 int launch_step_explicit(Ctx& c, double* const* st, double* const* wsave = nullptr, uint8_t* const* fsave = nullptr) {
     const int nrk = c.rk.nrk;
     const bool sph = c.prm.ics == 2;
     const bool wdon = c.prm.nolifa >= 2, lim = c.prm.slopeflag != 0, fuse = wdon && !lim;
-    const size_t ssz = (size_t)3 * c.dof * c.ne;
     if (need_forcing(c)) return 1;
     for (int irk = 0; irk < nrk; irk++) {
         StageArgs a{};
@@ -1445,8 +1445,9 @@ int launch_step_explicit(Ctx& c, double* const* st, double* const* wsave = nullp
         if (c.met) a.mt = met_args(c);
         a.uin = st[irk];
         a.uout = st[irk + 1];
-        a.wd_in = c.wd[c.wdcur].p;
-        a.wd_out = c.wd[1 - c.wdcur].p;
+        a.wd_in = fsave ? fsave[irk] : c.wd[c.wdcur].p;
+        a.wd_out = fsave ? fsave[irk + 1] : c.wd[1 - c.wdcur].p;
+        a.wout = wsave && lim ? wsave[irk] : nullptr;
         a.nprev = irk;
         for (int i = 0; i < irk; i++) {
             a.uprev[i] = st[i]; a.aprev[i] = c.rk.a[irk][i];
@@ -1460,16 +1461,11 @@ int launch_step_explicit(Ctx& c, double* const* st, double* const* wsave = nullp
         a.tip = tip_stage(c, irk);
         a.cmout = cmean_out(c);
         a.mid = c.mid;
-        if (fsave) HIPCHK(hipMemcpyAsync(fsave[irk], c.wd[c.wdcur].p, c.ne, hipMemcpyDeviceToDevice, c.stream));
         if (launch_stage_nt<P>(c, a, sph, fuse, c.block)) return 1;
         HIPCHK(hipGetLastError());
-        if (fuse) c.wdcur = 1 - c.wdcur;
-        if (lim) {
-            if (wsave)
-                HIPCHK(hipMemcpyAsync(wsave[irk], st[irk + 1], ssz * sizeof(double), hipMemcpyDeviceToDevice,
-                                      c.stream));
-            if (launch_limiter<P>(c, st[irk + 1], a.ed, false)) return 1;
-        }
+        if (fuse && !fsave) c.wdcur = 1 - c.wdcur;
+        if (lim && launch_limiter<P>(c, st[irk + 1], a.ed, false, fsave ? fsave[irk] : nullptr,
+                                     fsave ? fsave[irk + 1] : nullptr)) return 1;
     }
     c.hstep++;
     return 0;
@@ -1625,12 +1621,12 @@ int adj_backward(Ctx& c, int it0, int nsteps, int interval, double weight) {
     auto limrev = [&](double* cot, const double* wpre) -> int {
         hipLaunchKernelGGL((node_minmax_kernel<P>), dim3(gn), dim3(B), 0, c.stream, np, ne, (const int*)c.n2e_off.p,
                            (const int*)c.n2e.p, wpre, c.nmm.p);
-        hipLaunchKernelGGL((limiter_adj_kernel<P>), dim3(ge), dim3(B), 0, c.stream, np, ed, wpre,
+        hipLaunchKernelGGL((limiter_adj_kernel<P>), dim3(ge, 3), dim3(B), 0, c.stream, np, ed, wpre,
                            (const double*)c.nmm.p, cot, c.lnbc.p);
-        hipLaunchKernelGGL((limiter_adj_node_kernel<P>), dim3(gn), dim3(B), 0, c.stream, np, ne,
+        hipLaunchKernelGGL((limiter_adj_node_kernel<P>), dim3(gn, 3), dim3(B), 0, c.stream, np, ne,
                            (const int*)c.n2e_off.p, (const int*)c.n2e.p, wpre, (const double*)c.lnbc.p,
                            c.lgsum.p, c.larg.p);
-        hipLaunchKernelGGL((limiter_adj_gather_kernel<P>), dim3(ge), dim3(B), 0, c.stream, np, ed,
+        hipLaunchKernelGGL((limiter_adj_gather_kernel<P>), dim3(ge, 3), dim3(B), 0, c.stream, np, ed,
                            (const double*)c.lgsum.p, (const int*)c.larg.p, cot);
         HIPCHK(hipGetLastError());
         return 0;
@@ -1651,20 +1647,21 @@ int adj_backward(Ctx& c, int it0, int nsteps, int interval, double weight) {
         HIPCHK(hipMemcpyAsync(stage(k0 + 1, 0), c.ckpt.p + (size_t)sg * ssz, ssz * sizeof(double),
                               hipMemcpyDeviceToDevice, c.stream));
         if (wdrev_on)
-            HIPCHK(hipMemcpyAsync(c.wd[c.wdcur].p, c.ckptwd.p + (size_t)sg * ne, ne, hipMemcpyDeviceToDevice, c.stream));
+            HIPCHK(hipMemcpyAsync(fstage(k0 + 1, 0), c.ckptwd.p + (size_t)sg * ne, ne, hipMemcpyDeviceToDevice, c.stream));
         c.hstep = 0;
         for (int k = k0 + 1; k <= k1; k++) {
             // the last step runs for its intermediate stages, pre-limiter outputs and flags only
             if (k == k1 && !(nrk > 1 || lim)) break;
             double* st[KMAXRK + 1];
             double* ws[KMAXRK];
-            uint8_t* fs[KMAXRK];
+            uint8_t* fs[KMAXRK + 1];
             for (int i = 0; i < nrk; i++) {
                 st[i] = stage(k, i);
                 ws[i] = lim ? wstage(k, i) : nullptr;
                 fs[i] = wdrev_on ? fstage(k, i) : nullptr;
             }
             st[nrk] = k < k1 ? stage(k + 1, 0) : c.pout.p;   // the last step's output is unused
+            if (wdrev_on) fs[nrk] = k < k1 ? fstage(k + 1, 0) : c.wd[c.wdcur].p;
             if (launch_step_explicit<P>(c, st, lim ? ws : nullptr, wdrev_on ? fs : nullptr)) return 1;
         }
         for (int k = k1; k > k0; k--) {

@@ -60,6 +60,7 @@ struct StageArgs {
     int* __restrict__ wd_active;         // set to 1 when WETDRY changes an element, or nullptr
     const double* __restrict__ tip;      // TIP2 of this stage at the nodes (tidal potential), or nullptr
     double* __restrict__ cmout;          // copy of the output cell means [3][ne] for the limiter, or nullptr
+    double* __restrict__ wout;           // copy of the output before the limiter (adjoint), or nullptr
     int mid;                             // G and the spherical factors allow llf_flux_nl2 (depths permitting)
 };
 
@@ -960,6 +961,12 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(P == 1 
     for (int f = 0; f < 3; f++)
 #pragma unroll
         for (int k = 0; k < DOF; k++) at(a.uout + (size_t)(f * DOF + k) * ne, e) = W[f][k];
+    if (a.wout) {
+#pragma unroll
+        for (int f = 0; f < 3; f++)
+#pragma unroll
+            for (int k = 0; k < DOF; k++) at(a.wout + (size_t)(f * DOF + k) * ne, e) = W[f][k];
+    }
     if (a.cmout) {
 #pragma unroll
         for (int f = 0; f < 3; f++) at(a.cmout + (size_t)f * ne, e) = W[f][0];
@@ -1200,6 +1207,10 @@ __global__ void __launch_bounds__(4 * SPLIT_NT) __attribute__((amdgpu_waves_per_
     if (!valid) return;
 #pragma unroll
     for (int k = 0; k < DOF; k++) at(a.uout + (size_t)(c * DOF + k) * ne, e) = W[k];
+    if (a.wout) {
+#pragma unroll
+        for (int k = 0; k < DOF; k++) at(a.wout + (size_t)(c * DOF + k) * ne, e) = W[k];
+    }
     if (a.cmout) at(a.cmout + (size_t)c * ne, e) = W[0];
 }
 
