@@ -2085,7 +2085,7 @@ int dg_gpu_nodal_update(int h) {
     if (!c) return 1;
     const int np = c->np;
     ElemData E = elem_data(*c);
-    const int B = 256, gn = (np + B - 1) / B;
+    const int B = M2N_NT, gn = (np + B - 1) / B;
     const int* off = c->m2n_set ? c->m2n_off.p : c->n2e_off.p;
     const int* row = c->m2n_set ? c->m2n.p : c->n2e.p;
     double* em = c->has_etamax ? c->etamax.p : nullptr;
