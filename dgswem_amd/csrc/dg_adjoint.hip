@@ -778,7 +778,6 @@ __global__ void __launch_bounds__(4 * ADJ_NT) __attribute__((amdgpu_waves_per_eu
         for (int m = 0; m < 3; m++) hb[m] = stg[(RL + m) * ns + le];
         const bool quad = QF || ph.iflinbf == 0;
         const bool hybrid = !QF && ph.ifhybf == 1;
-        const int row = table_step(a.fo) * a.fo.nrk + a.irk;
         const double drdx = at(E.geo + (size_t)9 * ne, ec), dsdx = at(E.geo + (size_t)10 * ne, ec);
         const double drdy = at(E.geo + (size_t)11 * ne, ec), dsdy = at(E.geo + (size_t)12 * ne, ec);
         const double depth_c = hb[0] + stg[le];
@@ -799,17 +798,17 @@ __global__ void __launch_bounds__(4 * ADJ_NT) __attribute__((amdgpu_waves_per_eu
         // forms them; the pressure term -g*SFAC*H*dP/dx depends on the state through H
         double mw[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, pdx = 0.0, pdy = 0.0;
         if (a.met) {
-            const double ramp = a.fo.ramp[(size_t)sid * a.fo.rows + row];
+            const double4* st = a.mt.st + (size_t)a.irk * a.mt.np;
             const double drpsi[3] = {-1.0 / 2.0, 1.0 / 2.0, 0.0}, dspsi[3] = {-1.0 / 2.0, 0.0, 1.0 / 2.0};
 #pragma unroll
             for (int v = 0; v < 3; v++) {
                 const int n = at(E.nm + (size_t)v * ne, ec);
+                const double4 s = st[n];
                 if constexpr (!NL) {
-                    const double cd = a.mt.cd[n], wm = a.mt.wm[n];
-                    mw[v] = ramp * 0.001293 * cd * a.mt.wx[n] * wm;
-                    mw[3 + v] = ramp * 0.001293 * cd * a.mt.wy[n] * wm;
+                    mw[v] = s.x;
+                    mw[3 + v] = s.y;
                 }
-                const double pr = ramp * a.mt.prn[n];
+                const double pr = s.z;
                 pdx += pr * (drpsi[v] * drdx + dspsi[v] * dsdx);
                 pdy += pr * (drpsi[v] * drdy + dspsi[v] * dsdy);
             }

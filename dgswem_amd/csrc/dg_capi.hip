@@ -190,7 +190,8 @@ struct Ctx {
     DevBuf<int> tna;
     // NWS=8 meteorological forcing
     bool met = false;
-    DevBuf<double> ramp, mrow, mxc, myc, mcosy, mcor, mwx, mwy, mwm, mcd, mprn;
+    DevBuf<double> ramp, mrow, mxc, myc, mcosy, mcor;
+    DevBuf<double4> mst;
     DevBuf<uint16_t> nsid;
     int next_it = 1;                             // IT of the next step (for the autotuner's tables)
     // set while the adjoint's forward sweeps run: WETDRY raises it when it changes an element
@@ -354,8 +355,7 @@ Met met_args(Ctx& c, int cap = -1) {
     m.row = c.mrow.p;
     m.nsid = c.S > 1 ? c.nsid.p : nullptr;
     m.xc = c.mxc.p; m.yc = c.myc.p; m.cosy = c.mcosy.p; m.cor = c.mcor.p;
-    const size_t o = (size_t)batch_step(c, cap) * c.np;
-    m.wx = c.mwx.p + o; m.wy = c.mwy.p + o; m.wm = c.mwm.p + o; m.cd = c.mcd.p + o; m.prn = c.mprn.p + o;
+    m.st = c.mst.p + (size_t)batch_step(c, cap) * c.rk.nrk * c.np;
     return m;
 }
 
@@ -521,15 +521,14 @@ Scen scen_of(const Member& m) {
 // latency and its arrays stay in the caches (8 MB); it covers at least a captured graph's steps.
 int alloc_batch(Ctx& c) {
     const size_t nrk = c.rk.nrk, period = nrk + 1;
-    const size_t step = 8 * (nrk * ((size_t)c.tzn + c.fzn + (c.tip ? c.np : 0)) + (c.met ? 5 * (size_t)c.np : 0));
+    const size_t step = 8 * (nrk * ((size_t)c.tzn + c.fzn + (c.tip ? c.np : 0) + (c.met ? 4 * (size_t)c.np : 0)));
     const size_t k = std::max(period, std::min<size_t>(64, ((size_t)8 << 20) / std::max<size_t>(step, 1)));
     c.fbatch = (int)k;
     c.fbn = 0;
     if (c.tzn > 0) HIPCHK(c.tz.alloc(k * nrk * c.tzn));
     if (c.fzn > 0) HIPCHK(c.fz.alloc(k * nrk * c.fzn));
     if (c.tip) HIPCHK(c.tip2.alloc(k * nrk * c.np));
-    if (c.met)
-        for (DevBuf<double>* b : {&c.mwx, &c.mwy, &c.mwm, &c.mcd, &c.mprn}) HIPCHK(b->alloc(k * c.np));
+    if (c.met) HIPCHK(c.mst.alloc(k * nrk * c.np));
     return 0;
 }
 
@@ -1211,7 +1210,7 @@ int launch_stage_v(Ctx& c, const StageArgs& a0, bool sph, bool fuse) {
     a.hidx = it->second.hidx.p; a.snbl = it->second.snbl.p; a.nh = it->second.nh; a.ns = it->second.ns;
     const size_t lds = it->second.lds;
     // every pointer the variant dereferences must be set (a missing one is an error, not a launch)
-    if (MET && (!a.mt.row || !a.mt.cd || !a.mt.wm || !a.mt.wx || !a.mt.wy || !a.mt.prn || !a.fo.ramp))
+    if (MET && (!a.mt.row || !a.mt.st || !a.fo.ramp))
         return fail("internal: NWS=8 stage launch without its forcing arguments");
     if (!a.uin || !a.uout || !a.wd_in || !a.hidx || !a.snbl)
         return fail("internal: stage launch with a missing buffer");
@@ -1536,7 +1535,7 @@ int launch_adj_nl(Ctx& c, const AdjArgs& a0) {
     AdjArgs a = a0;
     a.hidx = it->second.hidx.p; a.snbl = it->second.snbl.p; a.nh = it->second.nh; a.ns = it->second.ns;
     const size_t lds = adj_dynamic_lds(c.dof, it->second.ns);
-    if (a.met && (!a.mt.cd || !a.mt.wm || !a.mt.wx || !a.mt.wy || !a.mt.prn || !a.fo.ramp))
+    if (a.met && !a.mt.st)
         return fail("internal: NWS=8 adjoint launch without its forcing arguments");
     if (!a.u || !a.out) return fail("internal: adjoint launch with a missing buffer");
     // NOLIBF=1 (quadratic friction, no hybrid factor) with the nonlinear equations: friction fixed

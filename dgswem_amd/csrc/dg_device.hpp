@@ -143,9 +143,9 @@ __device__ __forceinline__ int table_step(const Forcing& f) { return (f.step ? *
 
 
 // NWS=8 meteorological forcing at the nodes.  The node kernel evaluates the Holland profile once
-// per step at TIME_A (the reference evaluates it at every stage with the same TIME_A) and keeps the
-// ramp-free factors; the stage kernel forms WSX2 = RampMete*0.001293*Cd*Wx*|W| and
-// PR2 = RampMete*P with the stage's ramp, in the reference's operation order.
+// per step at TIME_A (the reference evaluates it at every stage with the same TIME_A) and forms
+// WSX2 = RampMete*0.001293*Cd*Wx*|W|, WSY2 and PR2 = RampMete*P with each stage's ramp, in the
+// reference's operation order.
 struct Met {
     int np, rows;                        // rows: steps per scenario in the storm table
     const double* __restrict__ row;     // [scenario][rows][MET_ROW] storm scalars per step
@@ -154,11 +154,7 @@ struct Met {
     const double* __restrict__ yc;      // [np] latitude (deg)
     const double* __restrict__ cosy;    // [np] cos(latitude)
     const double* __restrict__ cor;     // [np] 2 omega sin(latitude)
-    double* __restrict__ wx;            // [np] 10-m wind (m/s), x
-    double* __restrict__ wy;            // [np] y
-    double* __restrict__ wm;            // [np] |W|
-    double* __restrict__ cd;            // [np] drag coefficient
-    double* __restrict__ prn;           // [np] surface pressure (m of water)
+    double4* __restrict__ st;           // [step of the batch][stage][np] WSX2, WSY2, PR2 of the stage, unused
 };
 
 // Block-local node bounds of the slope limiter.  Tile t (elements [t*nt, t*nt+nt)) stages the

@@ -578,15 +578,14 @@ __device__ __forceinline__ void volume_terms(const StageArgs& a, const DevTables
     if (MET) {
         // nodal WSX2/WSY2/PR2 of this stage (src/met_forcing.F:507-509) and the QP-independent sums
         // PR2(Ni)*DPSIDX(i) of src/rhs_dg_hydro.F:117-122,366-372
-        const double ramp = a.fo.ramp[(size_t)sid * a.fo.rows + row];
+        const double4* st = a.mt.st + (size_t)a.irk * a.mt.np;
         double pdx = 0.0, pdy = 0.0;
 #pragma unroll
         for (int i = 0; i < 3; i++) {
-            const int n = at(E.nm + (size_t)i * ne, ec);
-            const double cd = a.mt.cd[n], wm = a.mt.wm[n];
-            v.mw[i] = ramp * 0.001293 * cd * a.mt.wx[n] * wm;
-            v.mw[3 + i] = ramp * 0.001293 * cd * a.mt.wy[n] * wm;
-            const double pr = ramp * a.mt.prn[n];
+            const double4 s = st[at(E.nm + (size_t)i * ne, ec)];
+            v.mw[i] = s.x;
+            v.mw[3 + i] = s.y;
+            const double pr = s.z;
             const double dpsidx = drpsi[i] * v.drdx + dspsi[i] * v.dsdx;
             const double dpsidy = drpsi[i] * v.drdy + dspsi[i] * v.dsdy;
             if (i == 0) { pdx = pr * dpsidx; pdy = pr * dpsidy; }
@@ -1710,7 +1709,6 @@ __global__ void __launch_bounds__(256) met_kernel(Met m, Forcing fo) {
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= m.np) return;
     const int s = blockIdx.y;                               // step of the batch
-    const size_t o = (size_t)s * m.np + n;
     const int sid = m.nsid ? (int)m.nsid[n] : 0;
     const double* r = m.row + ((size_t)sid * m.rows + table_step(fo) + s) * MET_ROW;
     const double re = 6378206.4;
@@ -1733,7 +1731,12 @@ __global__ void __launch_bounds__(256) met_kernel(Met m, Forcing fo) {
     const double wmag = sqrt(wx * wx + wy * wy);
     double cd = 0.001 * (0.75 + 0.067 * wmag);
     if (cd > 0.0035) cd = 0.0035;
-    m.wx[o] = wx; m.wy[o] = wy; m.wm[o] = wmag; m.cd[o] = cd; m.prn[o] = press;
+    const double* rp = fo.ramp + (size_t)sid * fo.rows + (size_t)(table_step(fo) + s) * fo.nrk;
+    for (int irk = 0; irk < fo.nrk; irk++) {
+        const double ramp = rp[irk];
+        m.st[((size_t)s * fo.nrk + irk) * m.np + n] =
+            make_double4(ramp * 0.001293 * cd * wx * wmag, ramp * 0.001293 * cd * wy * wmag, ramp * press, 0.0);
+    }
 }
 
 // The state between the step's layout (soa: [field][mode][element]) and the host's (aos: [field][element][mode]), one
