@@ -27,7 +27,7 @@ class MisfitProblem:
     nsteps: int
     data: np.ndarray                       # [nsteps, ng]
     weight: float = 1.0
-    interval: int = 0                      # checkpoint spacing (0: about sqrt(nsteps))
+    interval: int = 0                      # checkpoint spacing (0: all stages kept if they fit, else about sqrt(nsteps))
     state0: tuple = field(default=None)    # initial (ze, qx, qy, wdflg)
     it0: int = 0
 

@@ -1162,18 +1162,20 @@ __device__ void wetdry_adj_element(const DevTables& T, const double (&U)[3][3], 
     gdp[2 * (size_t)ne + e] += Db[2];
 }
 
-// Elevation at the gauges: eta_g = sum_K ZE(K, elem_g) * phi_K(gauge), written to out[g].
+// Elevation at the gauges: eta_g = sum_K ZE(K, elem_g) * phi_K(gauge), written to out[g]; blockIdx.y counts states
+// `stride` apart.
 template <int P>
 __global__ void gauge_kernel(int ng, int ne, const int* __restrict__ gel, const double* __restrict__ gphi,
-                             const double* __restrict__ u, double* __restrict__ out) {
+                             const double* __restrict__ u0, size_t stride, double* __restrict__ out) {
     constexpr int DOF = (P + 1) * (P + 2) / 2;
     const int g = blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= ng) return;
     const int e = gel[g];
+    const double* u = u0 + blockIdx.y * stride;
     double s = 0.0;
 #pragma unroll
     for (int k = 0; k < DOF; k++) s = s + u[(size_t)k * ne + e] * gphi[(size_t)g * DOF + k];
-    out[g] = s;
+    out[(size_t)blockIdx.y * ng + g] = s;
 }
 
 // Cotangent seed of the gauge misfit sum_g w (eta_g - d_g)^2 into lam.  One thread per gauge

@@ -320,8 +320,8 @@ class _Handle:
     def gradient(self, data, weight: float = 1.0, interval: int = 0):
         """Loss J = weight * sum_k sum_g (eta_g(U^k) - data[k-1, g])^2 over the next len(data)
         steps and its gradient with respect to the per-node Manning n and depth DP, by the
-        discrete adjoint with checkpoints every `interval` steps (0: about sqrt(N)).  The state
-        is left where it was."""
+        discrete adjoint with checkpoints every `interval` steps (0: every stage kept where
+        the device's memory allows, else about sqrt(N)).  The state is left where it was."""
         d = _f(data)
         n = d.shape[0]
         gn, gdp = np.empty(self.np_), np.empty(self.np_)

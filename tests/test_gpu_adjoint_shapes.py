@@ -31,3 +31,30 @@ def test_tile_edges(nx, ny, p, nonlinear):
         fd = central_fd(prob, c, vn, vd)
         print(f"adjoint {ad:.12e} fd {fd:.12e} rel {abs(fd - ad) / abs(ad):.2e}", flush=True)
         assert abs(fd - ad) <= TOL * abs(ad)
+
+
+# runs kept whole (no spacing given) against runs recomputed from checkpoints: over the ends of the forcing tables'
+# 2048 steps, and with limiter, wetting and drying
+@pytest.mark.parametrize("steps,interval", [(1, 1), (2047, 100), (2048, 100), (2049, 500), (4100, 999)])
+def test_kept_stages_equal_recomputed_ones(steps, interval):
+    c = mesh.structured_basin(nx=11, ny=3, dx=900.0, dy=1100.0, depth=6.0, amp=0.3, dt=6.0)
+    prob = adjoint.twin_problem(c, nsteps=steps, ng=7, seed=3)
+    ref = prob.solver.gradient(prob.data, prob.weight, interval)
+    prob.reset()
+    out = prob.solver.gradient(prob.data, prob.weight, 0)
+    for a, b in zip(out, ref):
+        np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("p", [1, 2])
+def test_kept_flags_equal_recomputed_ones(p):
+    c = mesh.delaunay_basin(n_elem=700, seed=34, p=p, lx=6.0e4, ly=3.6e4, depth_range=(2.0, 10.0), shelf=True,
+                            wetdry=True, slopeflag=5, nsteps=40, cf=1e-4)
+    prob = adjoint.twin_problem(c, nsteps=40, ng=9, seed=5, state0="cold")
+    outs = []
+    for interval in (0, 7, 0, 40):
+        prob.reset()
+        outs.append(prob.solver.gradient(prob.data, prob.weight, interval))
+    for o in outs[1:]:
+        for a, b in zip(outs[0], o):
+            np.testing.assert_array_equal(a, b)
