@@ -332,6 +332,29 @@ __device__ __forceinline__ void dry_side_adj(const Phys& ph, int cas, int role, 
     }
 }
 
+// Cotangent seed of the gauge misfit sum_g w (eta_g - d_g)^2 after a step.  ord lists the gauges grouped by element
+// (ascending gauge index within a group, group u at ord[off[u]..off[u+1])), so gauges sharing an element add up
+// in gauge order.
+struct GaugeSeed {
+    const int* __restrict__ idx;         // [ne] group of each element, or -1; nullptr: no seed
+    const int* __restrict__ off;
+    const int* __restrict__ ord;
+    const double* __restrict__ phi;      // [ng][dof]
+    const double* __restrict__ eta;      // the step's gauge elevations and data [ng]
+    const double* __restrict__ data;
+    double w;
+};
+
+template <int DOF>
+__device__ __forceinline__ void add_gauge_seed(const GaugeSeed& s, int u, double (&t)[DOF]) {
+    for (int j = s.off[u]; j < s.off[u + 1]; j++) {
+        const int g = s.ord[j];
+        const double r = 2.0 * s.w * (s.eta[g] - s.data[g]);
+#pragma unroll
+        for (int k = 0; k < DOF; k++) t[k] += r * s.phi[(size_t)g * DOF + k];
+    }
+}
+
 struct AdjArgs {
     ElemData ed;
     Phys ph;
@@ -354,6 +377,7 @@ struct AdjArgs {
     const int* __restrict__ hidx;
     const int* __restrict__ snbl;
     int nh, ns;                          // halo entries per tile, staged elements per block (LDS row length)
+    GaugeSeed seed;                      // of the step before (a step's first stage: out is that step's cotangent)
 };
 
 // The reverse of the LLF flux of an internal edge point for one side's own arguments: `o` the side's own traces
@@ -453,7 +477,11 @@ constexpr int adj_sum_rows(int dof) { return 3 * dof + 4; }
 // The time of this kernel was its serial chain: one lane per element took three sides and the area points one after
 // the other with two waves per SIMD (p=1) or one (p=2: 504 registers), the sums read and written in LDS at every
 // point.  49,800 p=1 elements: 27.2 us before, 15.8 us now; four p=2 storm basins of 99,000 elements with their
-// flags 108.7 and 65 us.  Two waves per SIMD: with three the p=2 form spills (85 us).
+// flags 108.7 and 65 us.  Three waves per SIMD where the registers allow (168: a 40-step gradient of 59,600 p=2
+// elements 5.69 ms with two, 5.43 ms with three; of four p=1 storms 6.14 and 5.75 ms); the p=2 form with flags would spill
+// (85 us) and runs with two, like the forms with the hybrid friction factor.
+// A step's first stage adds the misfit of the step before to the cotangent that it writes: as a launch of its own that
+// took 4.3 us a step.
 // The RHS cotangent is staged times M_INV, which leaves the plain basis values and derivatives as the
 // transposed quadrature's tables: the edge cotangent is a trace like the state's, and the area points' ones
 // are two sums per field.
@@ -462,7 +490,7 @@ constexpr int adj_sum_rows(int dof) { return 3 * dof + 4; }
 // reversed; without it every element is wet and that code is compiled out (it would otherwise
 // raise the kernel's register use past what the all-wet runs need).
 template <int P, bool SPH, bool NL, bool QF, bool WD>
-__global__ void __launch_bounds__(4 * ADJ_NT) __attribute__((amdgpu_waves_per_eu(2))) adj_stage_kernel(AdjArgs a) {
+__global__ void __launch_bounds__(4 * ADJ_NT) __attribute__((amdgpu_waves_per_eu(QF && !(P == 2 && WD) ? 3 : 2))) adj_stage_kernel(AdjArgs a) {
 #pragma clang fp contract(fast)
     constexpr int DOF = (P + 1) * (P + 2) / 2;
     constexpr int NAGP = (P == 1) ? 3 : 6;
@@ -993,6 +1021,10 @@ __global__ void __launch_bounds__(4 * ADJ_NT) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
             for (int k = 0; k < DOF; k++) s[k] += ac * at(a.src[j] + (size_t)(c * DOF + k) * ne, e);
         }
+        if (c == 0 && a.seed.idx) {
+            const int u = at(a.seed.idx, e);
+            if (u >= 0) add_gauge_seed<DOF>(a.seed, u, s);
+        }
 #pragma unroll
         for (int k = 0; k < DOF; k++) at(a.out + (size_t)(c * DOF + k) * ne, e) = s[k];
     } else {
@@ -1178,32 +1210,27 @@ __global__ void gauge_kernel(int ng, int ne, const int* __restrict__ gel, const 
     out[(size_t)blockIdx.y * ng + g] = s;
 }
 
-// Cotangent seed of the gauge misfit sum_g w (eta_g - d_g)^2 into lam.  One thread per gauge
-// element; gord lists the gauges grouped by element (ascending gauge index within a group, group u
-// at gord[goff[u]..goff[u+1])), so gauges sharing an element add up in gauge order.
+// The seed alone, one thread per gauge element: of the last step, whose cotangent no stage writes.
 template <int P>
-__global__ void __launch_bounds__(64) gauge_seed_kernel(int nu, int ne, const int* __restrict__ goff,
-                                                        const int* __restrict__ gord, const int* __restrict__ gel,
-                                                        const double* __restrict__ gphi,
-                                                        const double* __restrict__ eta,
-                                                        const double* __restrict__ data, double w,
+__global__ void __launch_bounds__(64) gauge_seed_kernel(int nu, int ne, GaugeSeed s, const int* __restrict__ gel,
                                                         double* __restrict__ lam) {
     constexpr int DOF = (P + 1) * (P + 2) / 2;
     const int u = blockIdx.x * blockDim.x + threadIdx.x;
     if (u >= nu) return;
-    const int j0 = goff[u], j1 = goff[u + 1];
-    const int e = gel[gord[j0]];
+    const int e = gel[s.ord[s.off[u]]];
     double t[DOF];
 #pragma unroll
     for (int k = 0; k < DOF; k++) t[k] = lam[(size_t)k * ne + e];
-    for (int j = j0; j < j1; j++) {
-        const int g = gord[j];
-        const double r = 2.0 * w * (eta[g] - data[g]);
-#pragma unroll
-        for (int k = 0; k < DOF; k++) t[k] += r * gphi[(size_t)g * DOF + k];
-    }
+    add_gauge_seed<DOF>(s, u, t);
 #pragma unroll
     for (int k = 0; k < DOF; k++) lam[(size_t)k * ne + e] = t[k];
+}
+
+// Group of each gauge element (the others hold -1).
+__global__ void __launch_bounds__(64) gauge_index_kernel(int nu, const int* __restrict__ off, const int* __restrict__ ord,
+                                                         const int* __restrict__ gel, int* __restrict__ idx) {
+    const int u = blockIdx.x * blockDim.x + threadIdx.x;
+    if (u < nu) idx[gel[ord[off[u]]]] = u;
 }
 
 // ------------------------------------------------------------------------------------------

@@ -204,7 +204,7 @@ struct Ctx {
     int dev = 0;                                 // device current at dg_gpu_init
     // adjoint: gauges, checkpoints, segment stage states, cotangents, parameter accumulators
     int ng = 0, ngu = 0;                         // gauges, distinct gauge elements
-    DevBuf<int> gel, goff, gord;
+    DevBuf<int> gel, goff, gord, gidx;
     DevBuf<double> gphi, geta, gdata, ckpt, seg, lam, gdp, gnb, pout;
     DevBuf<double> ubar[KMAXRK];
     // frozen-limiter reverse: pre-limiter stage outputs of a segment, vertex-bound cotangents,
@@ -1644,13 +1644,13 @@ int adj_backward(Ctx& c, int it0, int nsteps, int interval, bool keep, double we
     HIPCHK(hipMemsetAsync(c.gnb.p, 0, (size_t)ne * sizeof(double), c.stream));
     // seed: misfit at step N
     const int gs = (c.ngu + 63) / 64;
-    auto seed = [&](int k, double* l) {   // misfit of the state after step k (1-based)
-        hipLaunchKernelGGL((gauge_seed_kernel<P>), dim3(gs), dim3(64), 0, c.stream, c.ngu, ne, (const int*)c.goff.p,
-                           (const int*)c.gord.p, (const int*)c.gel.p, (const double*)c.gphi.p,
-                           (const double*)(c.geta.p + (size_t)(k - 1) * c.ng),
-                           (const double*)(c.gdata.p + (size_t)(k - 1) * c.ng), weight, l);
+    auto seed = [&](int k) {   // misfit of the state after step k (1-based)
+        return GaugeSeed{c.gidx.p, c.goff.p, c.gord.p, c.gphi.p, c.geta.p + (size_t)(k - 1) * c.ng,
+                         c.gdata.p + (size_t)(k - 1) * c.ng, weight};
     };
-    seed(nsteps, c.lam.p);
+    hipLaunchKernelGGL((gauge_seed_kernel<P>), dim3(gs), dim3(64), 0, c.stream, c.ngu, ne, seed(nsteps), (const int*)c.gel.p,
+                       c.lam.p);
+    HIPCHK(hipGetLastError());
     // frozen-limiter reverse of one stage: the cotangent `cot` of the limited stage output becomes
     // the cotangent of the pre-limiter output Wpre (node bounds from Wpre's cell means)
     const bool lim = c.prm.slopeflag != 0;
@@ -1734,6 +1734,7 @@ int adj_backward(Ctx& c, int it0, int nsteps, int interval, bool keep, double we
                 a.gdp = c.gdp.p;
                 a.gnbar = c.phys.load_manning ? c.gnb.p : nullptr;
                 a.wd = wdrev_on ? fstage(k, i) : nullptr;
+                if (i == 0 && k > 1) a.seed = seed(k - 1);
                 if (launch_adj<P>(c, a)) return 1;
                 HIPCHK(hipGetLastError());
                 // ub[i] is now the whole cotangent of U(i), the output of stage i-1
@@ -1741,7 +1742,6 @@ int adj_backward(Ctx& c, int it0, int nsteps, int interval, bool keep, double we
                 if (lim && i >= 1 && limrev(ub[i], wstage(k, i - 1))) return 1;
             }
             std::swap(lam, ub[0]);   // cotangent of U^(k-1)
-            if (k - 1 >= 1) seed(k - 1, lam);
         }
     }
     // keep the buffers' identities for the next call
@@ -2356,6 +2356,11 @@ int dg_adj_set_gauges(int h, int ng, const int* elem, const double* r, const dou
     HIPCHK(c->gord.upload(ord.data(), ng, c->stream));
     HIPCHK(c->goff.upload(off.data(), off.size(), c->stream));
     HIPCHK(c->gphi.upload(ph.data(), ph.size(), c->stream));
+    HIPCHK(c->gidx.alloc(c->ne));
+    HIPCHK(hipMemsetAsync(c->gidx.p, 0xff, (size_t)c->ne * sizeof(int), c->stream));
+    hipLaunchKernelGGL(gauge_index_kernel, dim3((c->ngu + 63) / 64), dim3(64), 0, c->stream, c->ngu, (const int*)c->goff.p,
+                       (const int*)c->gord.p, (const int*)c->gel.p, c->gidx.p);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c->stream));
     return 0;
 }
