@@ -31,3 +31,28 @@ def test_round_trip(nx, ny, p):
         np.testing.assert_array_equal(np.asarray(a).reshape(n, dof).view(np.int64), b.view(np.int64))
     np.testing.assert_array_equal(out[3], wd)
     g.close()
+
+
+# just under and over the size from which the state is read back in chunks (6 MiB), and more chunks than there are
+# slots for them; the elements of one size also by two threads at once, each with its own solver
+@pytest.mark.parametrize("nx,p", [(4139, 1), (4140, 1), (2125, 2), (2126, 2), (5000, 2)])
+def test_large_round_trip(nx, p):
+    from concurrent.futures import ThreadPoolExecutor
+    c = closed(nx, 10, p, nolifa=2)
+    n, dof = 20 * nx, 3 if p == 1 else 6
+
+    def trip(seed):
+        g = gpu.GpuSolver(c)
+        rng = np.random.default_rng(seed)
+        for _ in range(2):
+            st = [rng.standard_normal((n, dof)) for _ in range(3)]
+            wd = rng.integers(0, 2, n).astype(np.int32)
+            g.set_state(*st, wd)
+            for a, b in zip(g.state(), st + [wd]):
+                np.testing.assert_array_equal(np.asarray(a).reshape(b.shape), b)
+        g.close()
+
+    trip(1)
+    if nx == 5000:
+        with ThreadPoolExecutor(2) as ex:
+            list(ex.map(trip, (2, 3)))
