@@ -1239,14 +1239,17 @@ __global__ void __launch_bounds__(64) gauge_index_kernel(int nu, const int* __re
 // branch every clamp, every redistribution test and every min(redfac, redmax) took; given those,
 // the limiter is linear in (the element's linear modes, the node bounds) and its transpose maps
 // the cotangent of the limited modes (in ub, in place) to the cotangent of W's modes, plus the
-// cotangents of the vertex bounds (nbc: per field a record of two doubles [min|max] per element and
-// vertex, record 3e+v).  Modes >= 3 pass through.
-// One thread per element and field (blockIdx.y): with the three fields in one thread the launch was a serial chain
+// cotangents of the vertex bounds (nbc: a record of six doubles [field][min|max] per element and
+// vertex, record 3e+v, so that a node reads each incident element's six values from one place).
+// Modes >= 3 pass through.
+// A wave per field of 64 elements: with the three fields in one thread the launch was a serial chain
 // with three divisions by three and nine by a count of one to three for each (now div3, a product with 0.5 or
-// nothing, the same values).  99,000 elements: 15.7 us before, 11.1 us now.
+// nothing, the same values).  99,000 elements: 15.7 us before, 12.0 us now; 800,000 73 and 60 us.  (With a record per field the
+// node pass took 127 us at 800,000 elements instead of 75.)
 // ------------------------------------------------------------------------------------------
+constexpr int LADJ_NT = 64;              // elements per block
 template <int P>
-__global__ void __launch_bounds__(256) limiter_adj_kernel(int np, ElemData E, const double* __restrict__ W,
+__global__ void __launch_bounds__(3 * LADJ_NT) limiter_adj_kernel(int np, ElemData E, const double* __restrict__ W,
                                                           const double* __restrict__ mm, double* __restrict__ ub,
                                                           double* __restrict__ nbc) {
     // no contraction: the recorded branches must be those of the forward limiter, operation by
@@ -1254,8 +1257,12 @@ __global__ void __launch_bounds__(256) limiter_adj_kernel(int np, ElemData E, co
     constexpr int DOF = (P + 1) * (P + 2) / 2;
     const DevTables& T = tab<P>();
     const int ne = E.ne;
-    const int e = blockIdx.x * 256 + threadIdx.x, iv = blockIdx.y;
-    if (e >= ne) return;
+    // the block's bound-cotangent records, written out together: its elements hold one contiguous range of them
+    __shared__ double rec[LADJ_NT * 18];
+    const int iv = __builtin_amdgcn_readfirstlane(threadIdx.x / LADJ_NT), le = threadIdx.x % LADJ_NT;
+    const int e0 = blockIdx.x * LADJ_NT;
+    const bool valid = e0 + le < ne;
+    const int e = valid ? e0 + le : ne - 1;     // lanes past the last element read element ne-1 and write nothing
     // x over the number of positive differences (one to three): exactly x and x*0.5 for one and two
     auto by_count = [](double x, int n) { return n == 3 ? div3(x) : (n == 2 ? x * 0.5 : x); };
     const double* mn = mm + (size_t)(2 * iv) * np;
@@ -1347,83 +1354,103 @@ __global__ void __launch_bounds__(256) limiter_adj_kernel(int np, ElemData E, co
             vminb[c] += vb[c];
         }
     }
-    at(b, e) = c0b;
-    at(b + ne, e) = w1b;
-    at(b + 2 * (size_t)ne, e) = w2b;
-    double2* const r = reinterpret_cast<double2*>(nbc) + ((size_t)iv * ne + e) * 3;
+    if (valid) {
+        at(b, e) = c0b;
+        at(b + ne, e) = w1b;
+        at(b + 2 * (size_t)ne, e) = w2b;
 #pragma unroll
-    for (int c = 0; c < 3; c++) r[c] = make_double2(vminb[c], vmaxb[c]);
+        for (int c = 0; c < 3; c++) {
+            rec[le * 18 + c * 6 + iv * 2] = vminb[c];
+            rec[le * 18 + c * 6 + iv * 2 + 1] = vmaxb[c];
+        }
+    }
+    __syncthreads();
+    const int n = min(LADJ_NT, ne - e0) * 18;
+    double* dst = nbc + (size_t)e0 * 18;
+    for (int k = threadIdx.x; k < n; k += 3 * LADJ_NT) dst[k] = rec[k];
 }
 
 // Per node: the sums of the incident elements' vertex-bound cotangents, and the element whose
 // cell mean attains each bound (the first in the node's element list on ties; -1 when the
-// +-99999 starting bound stands).  gsum, arg: per field a record [min|max] per node.  One thread per node and field
-// (blockIdx.y); up to eight incidences per pass, their loads under way together, taken in list order.
+// +-99999 starting bound stands).  gsum, arg: a record [field][min|max] of six per node.  The three
+// fields go through the node's list together: every incident element's cell means and its bound
+// cotangent record (nbc) are loaded in one pass, and each field's sums still run in list order.
 template <int P>
 __global__ void __launch_bounds__(256) limiter_adj_node_kernel(int np, int ne, const int* __restrict__ off,
                                                                const int* __restrict__ n2e,
                                                                const double* __restrict__ W,
                                                                const double* __restrict__ nbc,
                                                                double* __restrict__ gsum, int* __restrict__ arg) {
-    constexpr int DOF = (P + 1) * (P + 2) / 2, B = 8;
-    const int n = blockIdx.x * 256 + threadIdx.x, f = blockIdx.y;
+    constexpr int DOF = (P + 1) * (P + 2) / 2;
+    const int n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= np) return;
-    const double* w = W + (size_t)(f * DOF) * ne;
-    const double2* rec = reinterpret_cast<const double2*>(nbc) + (size_t)f * 3 * ne;
-    double lo = 99999., hi = -99999., slo = 0.0, shi = 0.0;
-    int alo = -1, ahi = -1;
+    double lo[3], hi[3], slo[3], shi[3];
+    int alo[3], ahi[3];
+#pragma unroll
+    for (int f = 0; f < 3; f++) {
+        lo[f] = 99999.; hi[f] = -99999.; slo[f] = 0.0; shi[f] = 0.0;
+        alo[f] = -1; ahi[f] = -1;
+    }
     const int j1 = off[n + 1];
-    for (int j = off[n]; j < j1; j += B) {
-        int ent[B];
+    for (int j = off[n]; j < j1; j++) {
+        const int ent = n2e[j];
+        const int e = ent >> 2, v = ent & 3;
+        const double2* rec = reinterpret_cast<const double2*>(nbc + ((size_t)e * 3 + v) * 6);
+        double c[3];
+        double2 b[3];
 #pragma unroll
-        for (int q = 0; q < B; q++) ent[q] = n2e[min(j + q, j1 - 1)];
-        double c[B];
-        double2 b[B];
-#pragma unroll
-        for (int q = 0; q < B; q++) {
-            c[q] = w[ent[q] >> 2];
-            b[q] = rec[(size_t)(ent[q] >> 2) * 3 + (ent[q] & 3)];
+        for (int f = 0; f < 3; f++) {
+            c[f] = W[(size_t)(f * DOF) * ne + e];
+            b[f] = rec[f];
         }
 #pragma unroll
-        for (int q = 0; q < B; q++) {
-            if (j + q >= j1) break;
-            if (c[q] < lo) { lo = c[q]; alo = ent[q] >> 2; }
-            if (c[q] > hi) { hi = c[q]; ahi = ent[q] >> 2; }
-            slo += b[q].x;
-            shi += b[q].y;
+        for (int f = 0; f < 3; f++) {
+            if (c[f] < lo[f]) { lo[f] = c[f]; alo[f] = e; }
+            if (c[f] > hi[f]) { hi[f] = c[f]; ahi[f] = e; }
+            slo[f] += b[f].x;
+            shi[f] += b[f].y;
         }
     }
-    reinterpret_cast<double2*>(gsum)[(size_t)f * np + n] = make_double2(slo, shi);
-    reinterpret_cast<int2*>(arg)[(size_t)f * np + n] = make_int2(alo, ahi);
+    double2* g = reinterpret_cast<double2*>(gsum + (size_t)n * 6);
+    int2* a = reinterpret_cast<int2*>(arg + (size_t)n * 6);
+#pragma unroll
+    for (int f = 0; f < 3; f++) {
+        g[f] = make_double2(slo[f], shi[f]);
+        a[f] = make_int2(alo[f], ahi[f]);
+    }
 }
 
-// Per element and field (blockIdx.y): the bound cotangents of the nodes where this element's cell mean is the bound.
+// Per element: the bound cotangents of the nodes where this element's cell mean is the bound.
 template <int P>
 __global__ void __launch_bounds__(256) limiter_adj_gather_kernel(int np, ElemData E, const double* __restrict__ gsum,
                                                                  const int* __restrict__ arg, double* __restrict__ ub) {
     constexpr int DOF = (P + 1) * (P + 2) / 2;
     const int ne = E.ne;
-    const int e = blockIdx.x * 256 + threadIdx.x, f = blockIdx.y;
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= ne) return;
-    const int2* ar = reinterpret_cast<const int2*>(arg) + (size_t)f * np;
-    const double2* gs = reinterpret_cast<const double2*>(gsum) + (size_t)f * np;
-    // every node's bound owners and cotangent sums together (a sum that is not this element's adds zero, which
-    // leaves the running sum as it is)
-    int2 a[3];
-    double2 g[3];
+    // the node indices, then every node's bound owners and cotangent sums together (a sum that is
+    // not this element's adds zero, which leaves the running sum as it is)
+    int2 a[3][3];
+    double2 g[3][3];
 #pragma unroll
     for (int v = 0; v < 3; v++) {
-        const int n = at(E.nm + (size_t)v * ne, e);
-        a[v] = ar[n];
-        g[v] = gs[n];
-    }
-    double add = 0.0;
+        const int n = E.nm[(size_t)v * ne + e];
 #pragma unroll
-    for (int v = 0; v < 3; v++) {
-        add += a[v].x == e ? g[v].x : 0.0;
-        add += a[v].y == e ? g[v].y : 0.0;
+        for (int f = 0; f < 3; f++) {
+            a[v][f] = reinterpret_cast<const int2*>(arg + (size_t)n * 6)[f];
+            g[v][f] = reinterpret_cast<const double2*>(gsum + (size_t)n * 6)[f];
+        }
     }
-    at(ub + (size_t)(f * DOF) * ne, e) += add;
+#pragma unroll
+    for (int f = 0; f < 3; f++) {
+        double add = 0.0;
+#pragma unroll
+        for (int v = 0; v < 3; v++) {
+            add += a[v][f].x == e ? g[v][f].x : 0.0;
+            add += a[v][f].y == e ? g[v][f].y : 0.0;
+        }
+        ub[(size_t)(f * DOF) * ne + e] += add;
+    }
 }
 
 // Node gradients from the element accumulators: dJ/dDP(n) = sum over incident elements of the

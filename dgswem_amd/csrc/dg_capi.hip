@@ -1695,12 +1695,12 @@ int adj_backward(Ctx& c, int it0, int nsteps, int interval, bool keep, double we
     auto limrev = [&](double* cot, const double* wpre) -> int {
         hipLaunchKernelGGL((node_minmax_kernel<P>), dim3(gn), dim3(B), 0, c.stream, np, ne, (const int*)c.n2e_off.p,
                            (const int*)c.n2e.p, wpre, c.nmm.p);
-        hipLaunchKernelGGL((limiter_adj_kernel<P>), dim3(ge, 3), dim3(B), 0, c.stream, np, ed, wpre,
+        hipLaunchKernelGGL((limiter_adj_kernel<P>), dim3((ne + LADJ_NT - 1) / LADJ_NT), dim3(3 * LADJ_NT), 0, c.stream, np, ed, wpre,
                            (const double*)c.nmm.p, cot, c.lnbc.p);
-        hipLaunchKernelGGL((limiter_adj_node_kernel<P>), dim3(gn, 3), dim3(B), 0, c.stream, np, ne,
+        hipLaunchKernelGGL((limiter_adj_node_kernel<P>), dim3(gn), dim3(B), 0, c.stream, np, ne,
                            (const int*)c.n2e_off.p, (const int*)c.n2e.p, wpre, (const double*)c.lnbc.p,
                            c.lgsum.p, c.larg.p);
-        hipLaunchKernelGGL((limiter_adj_gather_kernel<P>), dim3(ge, 3), dim3(B), 0, c.stream, np, ed,
+        hipLaunchKernelGGL((limiter_adj_gather_kernel<P>), dim3(ge), dim3(B), 0, c.stream, np, ed,
                            (const double*)c.lgsum.p, (const int*)c.larg.p, cot);
         HIPCHK(hipGetLastError());
         return 0;

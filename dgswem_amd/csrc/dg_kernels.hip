@@ -1741,7 +1741,7 @@ __global__ void __launch_bounds__(256) met_kernel(Met m, Forcing fo) {
 
 // The state between the step's layout (soa: [field][mode][element]) and the host's (aos: [field][element][mode]), one
 // value per thread in the host's order, so that the copy to or from the caller's arrays is a plain one.  Transposing
-// on the host took longer than the copy: reading back 298,700 p=2 elements (43 MB) 14.4 ms before, 4.2 ms now, of
+// on the host took longer than the copy: reading back 298,700 p=2 elements (43 MB) 14.4 ms before, 4.2 ms then, of
 // which the kernel takes 0.03 ms (setting it 13.2 and 1.6 ms).
 template <int DOF, bool OUT>
 __global__ void __launch_bounds__(256) state_layout_kernel(int ne, double* __restrict__ soa, double* __restrict__ aos) {
