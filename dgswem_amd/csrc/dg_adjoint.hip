@@ -17,7 +17,7 @@
 // and staying wet): the forward sweeps flag any element WETDRY changes, and the gradient call then
 // fails.
 //
-// Kernel layout follows the forward stage kernel: one thread per element, gathers only.  The
+// Kernel layout follows the forward's small-mesh stage kernel: four waves per 64 elements, gathers only.  The
 // cotangent of an internal edge flux is the sum of what both neighbours' RHS cotangents ask of it;
 // each element forms that sum from its own and its neighbour's cotangents and keeps the part of
 // the flux derivative that belongs to its own trace, so no scatter or atomics are needed.

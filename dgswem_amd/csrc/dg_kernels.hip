@@ -7,7 +7,7 @@
 //                    edge fluxes are evaluated by both neighbours with the same operands in the same
 //                    order, so both see bit-identical values and no scatter or atomics are needed.
 //                    Small meshes run stage_split_kernel, four waves per 64 elements, instead.
-//   limit_wetdry     one thread per element: SLOPELIMITER5 on modes 2-3, then WETDRY
+//   limit_wetdry     a wave per field of 64 elements: SLOPELIMITER5 on modes 2-3, then WETDRY
 // preceded once per batch of steps by tide_kernel (the tidal boundary terms of every stage) and, with
 // NWS=8, met_kernel (the Holland profile at the nodes); plus modal2nodal (one thread per node) on output
 // steps.

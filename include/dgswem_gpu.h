@@ -186,7 +186,7 @@ int dg_gpu_mass_noalloc(int handle, double* mass);
  * long run with little event overhead); enable=0 switches timing off.  dg_gpu_kernel_stats
  * returns the summed milliseconds and
  * launch count of kernel `kernel_id` (0 stage kernel, 1 node min/max, 2 limiter+wet/dry,
- * 3 modal2nodal, 4 NWS=8 node forcing) since the last reset.  No counterpart in the reference
+ * 3 modal2nodal, 4 NWS=8 node forcing, a launch of which covers several steps) since the last reset.  No counterpart in the reference
  * (it has no timers). */
 int dg_gpu_profile(int handle, int enable);
 int dg_gpu_kernel_stats(int handle, int kernel_id, double* total_ms, long long* launches,
@@ -275,13 +275,13 @@ int dg_ens_layout(int handle, int* nmembers, int* elem_offsets, int* node_offset
  * only the eager remainder of each call. */
 int dg_gpu_use_graph(int handle, int enable);
 
-/* Time the stage kernel at each supported launch shape (see dg_gpu_set_block) on the handle's
- * current state and keep the fastest; writes it to *block.  Touches only scratch stage buffers:
+/* Time the stage kernel at each supported launch shape (see dg_gpu_set_block), and its form with four waves
+ * per 64 elements (reported as 64), on the handle's current state and keep the fastest; writes it to *block.  Touches only scratch stage buffers:
  * the state is unchanged. */
 int dg_gpu_autotune(int handle, int* block);
 
-/* Set the stage-kernel block size explicitly (one thread per element): 64, 128 or (p=1) 256.
- * All sizes give bit-identical results. */
+/* Set the stage-kernel block size explicitly (one thread per element): 64, 128 or (p=1) 256.  Otherwise small
+ * meshes run four waves per 64 elements.  All shapes give bit-identical results. */
 int dg_gpu_set_block(int handle, int block);
 
 /* Message of the last failure on this thread ("" if none). */
