@@ -11,9 +11,9 @@
 //
 // Both work in double-double arithmetic (a value as an unevaluated sum hi + lo) built from exact
 // error-free transformations (fma-based products, two-sums) and round once at the end; the
-// result is correctly rounded unless the exact value lies within about 2^-100 (relative) of a
-// midpoint between two doubles.  Everything here must be compiled without floating-point
-// contraction.
+// result is correctly rounded unless the exact value lies closer to a midpoint between two doubles
+// than the value before that rounding is good to, relative: 2^-90 for the cosine, 2^-78 for the power.
+// Everything here must be compiled without floating-point contraction.
 //
 // Usable from host and device code (the host build is what the CPU tests check against the C
 // library).
@@ -145,13 +145,14 @@ DG_CRM_FN double cr_cos(double x) {
 
 // Correctly rounded x**y for y = 1/3 rounded to a double (0x1.5555555555555p-2), for positive finite x:
 // x = 2^3k m with m in [1/2, 4), x**y = 2^k * m**(1/3) * x**(-d) with d = 1/3 - y = 2^-54/3.  The cube
-// root of m is refined to double-double by one Newton step from c0, and the last factor is 1 - d*ln(x) to
-// 2^-105.  c0 is itself one Newton step from exp2(log2(m)/3) in single precision (good to about 2^-22), so
-// it is good to about 2^-42 and the result before its rounding to about 2^-83.  The correction terms need
-// only modest accuracy (the Newton quotient 2^-40 relative; ln(x) 2^-14 absolute at the largest exponents,
-// entering at 2^-68 of the result, 2^-74 for depths of water), so they start from single precision: on
-// the device from the hardware's approximate reciprocal and base-2 exponential and logarithm (about 1 ulp
-// each).  Other x as pow: +0 for +-0, NaN for negative x, +infinity and NaN kept.
+// root of m is refined to double-double by one Newton step from c0, and the last factor is 1 - d*ln(x).  c0 is
+// itself one Newton step from exp2(log2(m)/3) in single precision (good to about 2^-22), so it is good to about
+// 2^-42.  The correction terms need only modest accuracy (the Newton quotient 2^-40 relative; log2(m) 2^-23
+// absolute, while the exponent's share of ln(x) is added to it in double precision), so they start from single
+// precision: on the device from the hardware's approximate reciprocal and base-2 exponential and logarithm (about 1
+// ulp each).  The result before its rounding is good to 2^-78 at every exponent (the largest error of 16 million
+// arguments against quadruple precision was 2^-78.8).  Other x as pow: +0 for +-0, NaN for negative x, +infinity
+// and NaN kept.
 DG_CRM_FN double cr_pow_third(double x) {
     if (!(x > 0.0 && x < __builtin_inf())) return x < 0.0 ? (x - x) / (x - x) : std::fabs(x);
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -160,7 +161,7 @@ DG_CRM_FN double cr_pow_third(double x) {
     int ex;
     (void)std::frexp(x, &ex);
 #endif
-    const int k = (ex * 21846) >> 16;                      // floor(ex/3) for |ex| < 2^14
+    const int k = (ex * 21845 + 10922) >> 16;              // floor(ex/3) for every exponent of a double
 #if defined(__HIP_DEVICE_COMPILE__)
     const double m = __builtin_amdgcn_ldexp(x, -3 * k);
     const float l2 = __builtin_amdgcn_logf((float)m);
@@ -174,7 +175,7 @@ DG_CRM_FN double cr_pow_third(double x) {
     const double y2 = y * y;
     double r = (double)(1.0f / (float)(3.0 * y2));
 #endif
-    const double eps = (double)(l2 + (float)(3 * k)) * (0.6931471805599453 * 0x1.5555555555555p-56);   // ln(x) * 2^-54 / 3
+    const double eps = ((double)(3 * k) + (double)l2) * (0.6931471805599453 * 0x1.5555555555555p-56);   // ln(x) * 2^-54 / 3
     const double c0 = y - std::fma(y2, y, -m) * r;
     const dd s = two_prod(c0, c0);
     const dd t = two_prod(c0, s.hi);
