@@ -113,11 +113,12 @@ struct Member {
     } es, fs;
 };
 
-// Page-locked chunks for reading results back (read_back), allocated at the first large one.
+// Page-locked memory for reading results back (read_back), allocated at the first large result and again at the first
+// that calls for more.
 constexpr int RB_SLOTS = 6;
-constexpr size_t RB_CHUNK = (size_t)2 << 20;
 struct HostChunks {
     char* p = nullptr;
+    size_t cap = 0;
     hipEvent_t ev[RB_SLOTS] = {};
     bool ok = true;                      // false: not to be had, not tried again
     HostChunks() = default;
@@ -127,14 +128,18 @@ struct HostChunks {
         for (hipEvent_t e : ev) if (e) (void)hipEventDestroy(e);
         if (p) (void)hipHostFree(p);
     }
-    bool ensure(int dev) {               // dev: the stream's device, whose the events have to be
-        if (p || !ok) return ok;
+    bool ensure(int dev, size_t bytes) { // dev: the stream's device, whose the events have to be
+        if (!ok || cap >= bytes) return ok;
         int cur = dev;
         ok = hipGetDevice(&cur) == hipSuccess && (cur == dev || hipSetDevice(dev) == hipSuccess);
-        ok = ok && hipHostMalloc((void**)&p, RB_SLOTS * RB_CHUNK, hipHostMallocDefault) == hipSuccess;
-        for (hipEvent_t& e : ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        cap = 0;
+        ok = ok && hipHostMalloc((void**)&p, bytes, hipHostMallocDefault) == hipSuccess;
+        for (hipEvent_t& e : ev) ok = ok && (e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess);
         if (cur != dev) (void)hipSetDevice(cur);
-        if (!ok) (void)hipGetLastError();
+        if (ok) cap = bytes;
+        else (void)hipGetLastError();
         return ok;
     }
 };
@@ -1785,28 +1790,34 @@ int adj_backward(Ctx& c, int it0, int nsteps, int interval, bool keep, double we
 // Device arrays to the caller's memory, on the context's stream; complete on return.  A large copy into pageable
 // memory ran at 10 GB/s, most of it the host's copy out of the runtime's buffer with the page faults of an array that
 // was just allocated.  From RB_MIN on it goes through page-locked chunks instead, which up to four threads copy out
-// while the next ones arrive.  State of 298,700 p=2 elements (43 MB) 4.2 ms before, 1.8 ms now (two threads 2.1, six
-// 1.9); of 119,200 p=1 elements (9 MB) 1.9 and 0.9 ms.
+// while the next ones arrive.  A handle's first such result pays for the page-locking, about 0.1 ms a MiB where the
+// runtime has none to give again, so up to RB_LARGE four chunks of 1 MiB have to do: state of 118,933 p=1 and of 59,318
+// p=2 elements (9 MB) 1.2 to 1.7 ms with plain copies and a transposition on the host; 1.1 to 1.7 ms at first (1.8 to 2.2
+// with the chunks of larger results) and 0.35 ms then (0.33).  Beyond it six of 2 MiB: 298,579 p=2 elements (43 MB) 14 ms,
+// now 3 to 4 ms at first and 1.2 ms then (1.5 with the smaller chunks; two threads were slower than four, six no
+// faster).
 struct Piece { void* dst; const void* src; size_t n; };
-constexpr size_t RB_MIN = (size_t)6 << 20;
+constexpr size_t RB_MIN = (size_t)6 << 20, RB_LARGE = (size_t)16 << 20;
 int read_back(Ctx& c, const std::vector<Piece>& pieces) {
     size_t total = 0;
     for (auto& p : pieces) total += p.n;
-    if (total < RB_MIN || !c.chunks.ensure(c.dev)) {
+    const int slots = total < RB_LARGE ? 4 : RB_SLOTS;
+    const size_t chunk = (size_t)(total < RB_LARGE ? 1 : 2) << 20;
+    if (total < RB_MIN || !c.chunks.ensure(c.dev, slots * chunk)) {
         for (auto& p : pieces) HIPCHK(hipMemcpyAsync(p.dst, p.src, p.n, hipMemcpyDeviceToHost, c.stream));
         HIPCHK(hipStreamSynchronize(c.stream));
         return 0;
     }
     std::vector<Piece> ch;
     for (auto& p : pieces)
-        for (size_t o = 0; o < p.n; o += RB_CHUNK)
-            ch.push_back({(char*)p.dst + o, (const char*)p.src + o, std::min(RB_CHUNK, p.n - o)});
+        for (size_t o = 0; o < p.n; o += chunk)
+            ch.push_back({(char*)p.dst + o, (const char*)p.src + o, std::min(chunk, p.n - o)});
     const int n = (int)ch.size();
     std::vector<std::atomic<char>> done(n);
     for (auto& d : done) d.store(0);
     std::atomic<int> ready{0}, next{0};
     std::atomic<bool> stop{false};
-    auto slot = [&](int k) { return c.chunks.p + (size_t)(k % RB_SLOTS) * RB_CHUNK; };
+    auto slot = [&](int k) { return c.chunks.p + (size_t)(k % slots) * chunk; };
     auto copy = [&](int k) {
         std::memcpy(ch[k].dst, slot(k), ch[k].n);
         done[k].store(1, std::memory_order_release);
@@ -1824,9 +1835,9 @@ int read_back(Ctx& c, const std::vector<Piece>& pieces) {
     int issued = 0;
     auto issue = [&]() {
         while (err == hipSuccess && issued < n &&
-               (issued < RB_SLOTS || done[issued - RB_SLOTS].load(std::memory_order_acquire))) {
+               (issued < slots || done[issued - slots].load(std::memory_order_acquire))) {
             err = hipMemcpyAsync(slot(issued), ch[issued].src, ch[issued].n, hipMemcpyDeviceToHost, c.stream);
-            if (err == hipSuccess) err = hipEventRecord(c.chunks.ev[issued % RB_SLOTS], c.stream);
+            if (err == hipSuccess) err = hipEventRecord(c.chunks.ev[issued % slots], c.stream);
             issued++;
         }
     };
@@ -1847,7 +1858,7 @@ int read_back(Ctx& c, const std::vector<Piece>& pieces) {
         issue();
         if (err != hipSuccess) break;
         if (k == issued) { std::this_thread::yield(); continue; }   // every chunk is still being copied out
-        err = hipEventSynchronize(c.chunks.ev[k % RB_SLOTS]);
+        err = hipEventSynchronize(c.chunks.ev[k % slots]);
         if (err != hipSuccess) break;
         if (th.empty()) copy(k);
         else ready.store(k + 1, std::memory_order_release);
