@@ -234,8 +234,7 @@ struct Ctx {
     DevBuf<int> wdact;
     DevBuf<uint8_t> wdsave;                      // wet/dry flags at the start of a gradient call
     // launch configuration
-    int block = 256;
-    int split = -1;                              // stage_split_kernel: 1 yes, 0 no, -1 by the number of elements
+    int block = 0;                               // elements per block of the stage kernel, 0: by the rule (stage_block)
     int dev = 0;                                 // device current at dg_gpu_init
     // adjoint: gauges, checkpoints, segment stage states, cotangents, parameter accumulators
     int ng = 0, ngu = 0;                         // gauges, distinct gauge elements
@@ -897,7 +896,6 @@ int init_ctx_common(Ctx& c, const dg_params* prm, bool manning) {
                 for (int k = 0; k < c.T.dof; k++)
                     if (!pow2(c.T.phi_edge[l][q][k])) return fail("basis tables: an edge value of a p=1 mode is not a power of two");
     c.dof = c.T.dof; c.nagp = c.T.nagp; c.negp = c.T.negp;
-    c.block = prm->p == 1 ? 128 : 64;
     {
         int dev = 0, lds = 0;
         HIPCHK(hipGetDevice(&dev));
@@ -1154,20 +1152,21 @@ size_t adj_dynamic_lds(int dof, int ns) {
     return std::max(((size_t)8 * adj_stage_rows(dof) * ns + ns + 7) / 8 * 8, (size_t)8 * 4 * adj_sum_rows(dof) * ADJ_NT);
 }
 
-// Whether the stage runs as four waves per 64 elements (stage_split_kernel): the nonlinear equations and, unless
-// the launch shape was chosen by dg_gpu_set_block or the autotuner, few elements.  Measured per launch, one lane
-// per element against four waves per 64 elements: p=1 17.9 and 13.0 us at 5k elements, 20.4 and 17.8 at 59k, 21.3
-// and 22.3 at 89k (storm basins 27.0 and 13.9, 32.0 and 22.8, 35.0 and 29.9; 35.4 and 38.5 at 129k); p=2 27.9 and
-// 18.8 at 5k, 34.6 and 31.6 at 59k, 35.7 and 42.2 at 89k (storm 42.3 and 21.1, 47.5 and 39.5, 52.4 and 52.9).
+// Whether blocks of 64 elements run as four waves each (stage_split_kernel): the nonlinear equations and few
+// elements.  Measured per launch, one lane per element against four waves per 64 elements: p=1 17.9 and 13.0 us at 5k
+// elements, 20.4 and 17.8 at 59k, 21.3 and 22.3 at 89k (storm basins 27.0 and 13.9, 32.0 and 22.8, 35.0 and 29.9; 35.4 and
+// 38.5 at 129k); p=2 27.9 and 18.8 at 5k, 34.6 and 31.6 at 59k, 35.7 and 42.2 at 89k (storm 42.3 and 21.1, 47.5 and
+// 39.5, 52.4 and 52.9).
 constexpr int SPLIT_MAX1 = 80000, SPLIT_MAX2 = 64000;
-bool stage_split(const Ctx& c) {
-    if (c.prm.nolicat == 0) return false;
-    return c.split < 0 ? c.ne <= (c.prm.p == 1 ? SPLIT_MAX1 : SPLIT_MAX2) : c.split == 1;
-}
+bool stage_split(const Ctx& c) { return c.prm.nolicat != 0 && c.ne <= (c.prm.p == 1 ? SPLIT_MAX1 : SPLIT_MAX2); }
 
-// Elements per block the stage kernel runs with: the chosen number for nonlinear runs, 64 for linearised runs
-// and for stage_split_kernel.
-int stage_nt(const Ctx& c, int nt) { return c.prm.nolicat != 0 && !stage_split(c) ? nt : 64; }
+// Elements per block the stage kernel runs with: 64 for linearised runs; the number chosen by dg_gpu_set_block or the
+// autotuner; otherwise 64 where stage_split_kernel runs, else one lane per element in blocks of 128 (p=1) or 64.
+// The number alone says how the stage runs, so that one that the autotuner reported can be set again.
+int stage_block(const Ctx& c) {
+    if (c.prm.nolicat == 0) return 64;
+    return c.block ? c.block : (stage_split(c) || c.prm.p != 1 ? SPLIT_NT : 128);
+}
 
 // Halo lists of the stage kernel's blocks of `nt` elements (tile t = elements [t*nt, t*nt+nt)):
 // the out-of-tile internal neighbours of each tile in ascending order, and per element the local
@@ -1329,7 +1328,7 @@ bool valid_block(int p, int nt) {
 
 template <int P>
 int launch_stage_nt(Ctx& c, const StageArgs& a, bool sph, bool fuse, int nt) {
-    if (stage_nt(c, nt) == 64) return launch_stage<P, 64>(c, a, sph, fuse);
+    if (nt == 64 || c.prm.nolicat == 0) return launch_stage<P, 64>(c, a, sph, fuse);
     if constexpr (P == 1) {
         if (nt == 128) return launch_stage<P, 128>(c, a, sph, fuse);
         return launch_stage<P, 256>(c, a, sph, fuse);
@@ -1431,7 +1430,7 @@ int launch_step(Ctx& c, int cap) {
             if (a.bprev[i] != 0.0 && !c.keep_r[i]) return fail("internal: RHS of an earlier stage was not kept");
         const bool fuse = wdon && !lim;
         int ev = prof_begin(c, K_STAGE, capturing);
-        if (launch_stage_nt<P>(c, a, sph, fuse, c.block)) return 1;
+        if (launch_stage_nt<P>(c, a, sph, fuse, stage_block(c))) return 1;
         prof_end(c, ev);
         HIPCHK(hipGetLastError());
         if (fuse) c.wdcur = 1 - c.wdcur;
@@ -1495,7 +1494,7 @@ int launch_step_explicit(Ctx& c, double* const* st, double* const* wsave = nullp
         a.tip = tip_stage(c, irk);
         a.cmout = cmean_out(c);
         a.mid = c.mid;
-        if (launch_stage_nt<P>(c, a, sph, fuse, c.block)) return 1;
+        if (launch_stage_nt<P>(c, a, sph, fuse, stage_block(c))) return 1;
         HIPCHK(hipGetLastError());
         if (fuse && !fsave) c.wdcur = 1 - c.wdcur;
         if (lim && launch_limiter<P>(c, st[irk + 1], a.ed, false, fsave ? fsave[irk] : nullptr,
@@ -2227,7 +2226,7 @@ int dg_gpu_step(int h, int it, int nsteps) {
         if (m.prm.nws == 8 && !m.met) return fail("NWS=8 forcing not set (dg_gpu_set_holland)");
         if (m.prm.ntip != 0 && m.ntif == 0) return fail("tidal potential not set (dg_gpu_set_tidal_potential)");
     }
-    if (ensure_staging(*c, stage_nt(*c, c->block))) return 1;
+    if (ensure_staging(*c, stage_block(*c))) return 1;
     for (int s0 = 0; s0 < nsteps; s0 += kTableChunk) {
         const int n = std::min(kTableChunk, nsteps - s0);
         if (build_stage_tables(*c, it + s0, n)) return 1;
@@ -2489,7 +2488,7 @@ int dg_adj_gauges(int h, int it, int nsteps, double* eta) {
     if (!c) return 1;
     if (c->ng == 0) return fail("no gauges set (dg_adj_set_gauges)");
     if (nsteps <= 0) return 0;
-    if (ensure_staging(*c, stage_nt(*c, c->block))) return 1;
+    if (ensure_staging(*c, stage_block(*c))) return 1;
     HIPCHK(c->geta.alloc((size_t)nsteps * c->ng));
     const int rc = c->prm.p == 1 ? adj_forward<1>(*c, it, nsteps, 1, false) : adj_forward<2>(*c, it, nsteps, 1, false);
     if (rc) return rc;
@@ -2505,7 +2504,7 @@ int dg_adj_gradient(int h, int it, int nsteps, const double* data, double weight
     if (!c) return 1;
     if (adj_check(*c)) return 1;
     if (nsteps <= 0) return fail("nsteps must be positive");
-    if (ensure_staging(*c, stage_nt(*c, c->block)) || ensure_adj_staging(*c)) return 1;
+    if (ensure_staging(*c, stage_block(*c)) || ensure_adj_staging(*c)) return 1;
     const int nrk = c->rk.nrk, ne = c->ne, np = c->np;
     const size_t ssz = (size_t)3 * c->dof * ne;
     const bool lim = c->prm.slopeflag != 0;
@@ -2710,21 +2709,17 @@ int dg_gpu_autotune(int h, int* block) {
     StageArgs a = stage_args(*c, 0, slot);
     a.rout = nullptr;
     const bool sph = c->prm.ics == 2, fuse = c->prm.nolifa >= 2 && c->prm.slopeflag == 0;
-    // candidates: stage_kernel at every block size and, for the nonlinear equations, stage_split_kernel (0)
-    std::vector<int> cand = c->prm.p == 1 ? std::vector<int>{64, 128, 256} : std::vector<int>{64, 128};
-    if (c->prm.nolicat != 0) cand.push_back(0);
-    const int block0 = c->block, split0 = stage_split(*c) ? 1 : 0, keep = c->split;
+    const std::vector<int> cand = c->prm.p == 1 ? std::vector<int>{64, 128, 256} : std::vector<int>{64, 128};
+    const int block0 = stage_block(*c);
     if (build_stage_tables(*c, c->next_it, 1)) return 1;
     if (launch_forcing(*c, 0, 1, false)) return 1;
     hipEvent_t e0, e1;
     HIPCHK(hipEventCreate(&e0));
     if (hipEventCreate(&e1) != hipSuccess) { (void)hipEventDestroy(e0); return fail("hipEventCreate failed"); }
     float best = 1e30f;
-    int best_nt = c->block, best_split = split0, rc = 0;
-    for (int cd : cand) {
-        const int nt = cd ? cd : SPLIT_NT;
-        c->split = cd ? 0 : 1;
-        if (ensure_staging(*c, stage_nt(*c, nt))) continue;   // does not fit: not a candidate
+    int best_nt = block0, rc = 0;
+    for (int nt : cand) {
+        if (ensure_staging(*c, c->prm.nolicat != 0 ? nt : 64)) continue;   // does not fit: not a candidate
         float ms = 0.f;
         for (int rep = 0; rep < 2 && !rc; rep++) {   // the first pass warms caches and code
             if (hipEventRecord(e0, c->stream) != hipSuccess) { rc = fail("hipEventRecord failed"); break; }
@@ -2740,14 +2735,13 @@ int dg_gpu_autotune(int h, int* block) {
             if (e != hipSuccess) rc = fail(std::string("autotune: ") + hipGetErrorString(e));
         }
         if (rc) break;
-        if (ms < best) { best = ms; best_nt = nt; best_split = c->split; }
+        if (ms < best) { best = ms; best_nt = nt; }
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    if (rc) { c->split = keep; return rc; }
+    if (rc) return rc;
     c->block = best_nt;
-    c->split = best_split;
-    if (best_nt != block0 || best_split != split0) c->drop_graphs();
+    if (stage_block(*c) != block0) c->drop_graphs();
     if (block) *block = best_nt;
     return 0;
 }
@@ -2759,9 +2753,9 @@ int dg_gpu_set_block(int h, int block) {
         return fail("block size must be 64, 128 or, for p=1, 256 threads");
     HIPCHK(hipStreamSynchronize(c->stream));
     if (ensure_staging(*c, c->prm.nolicat != 0 ? block : 64)) return 1;
-    if (block != c->block || stage_split(*c)) c->drop_graphs();
+    const int block0 = stage_block(*c);
     c->block = block;
-    c->split = 0;
+    if (stage_block(*c) != block0) c->drop_graphs();
     return 0;
 }
 

@@ -275,13 +275,14 @@ int dg_ens_layout(int handle, int* nmembers, int* elem_offsets, int* node_offset
  * only the eager remainder of each call. */
 int dg_gpu_use_graph(int handle, int enable);
 
-/* Time the stage kernel at each supported launch shape (see dg_gpu_set_block), and its form with four waves
- * per 64 elements (reported as 64), on the handle's current state and keep the fastest; writes it to *block.  Touches only scratch stage buffers:
- * the state is unchanged. */
+/* Time the stage kernel at each supported launch shape (see dg_gpu_set_block) on the handle's current
+ * state and keep the fastest; writes it to *block, for dg_gpu_set_block to choose again.  Touches only scratch
+ * stage buffers: the state is unchanged. */
 int dg_gpu_autotune(int handle, int* block);
 
-/* Set the stage-kernel block size explicitly (one thread per element): 64, 128 or (p=1) 256.  Otherwise small
- * meshes run four waves per 64 elements.  All shapes give bit-identical results. */
+/* Set the stage kernel's elements per block explicitly: 64, 128 or (p=1) 256, one thread per element; with 64,
+ * meshes small enough for it run four waves per 64 elements, which is also what they run when nothing is
+ * chosen.  All shapes give bit-identical results. */
 int dg_gpu_set_block(int handle, int block);
 
 /* Message of the last failure on this thread ("" if none). */
