@@ -1153,12 +1153,22 @@ size_t adj_dynamic_lds(int dof, int ns) {
 }
 
 // Whether blocks of 64 elements run as four waves each (stage_split_kernel): the nonlinear equations and few
-// elements.  Measured per launch, one lane per element against four waves per 64 elements: p=1 17.9 and 13.0 us at 5k
-// elements, 20.4 and 17.8 at 59k, 21.3 and 22.3 at 89k (storm basins 27.0 and 13.9, 32.0 and 22.8, 35.0 and 29.9; 35.4 and
-// 38.5 at 129k); p=2 27.9 and 18.8 at 5k, 34.6 and 31.6 at 59k, 35.7 and 42.2 at 89k (storm 42.3 and 21.1, 47.5 and
-// 39.5, 52.4 and 52.9).
-constexpr int SPLIT_MAX1 = 80000, SPLIT_MAX2 = 64000;
-bool stage_split(const Ctx& c) { return c.prm.nolicat != 0 && c.ne <= (c.prm.p == 1 ? SPLIT_MAX1 : SPLIT_MAX2); }
+// elements.  How many depends on how much of a launch is serial (a storm's gathers, its shoreline) and how much is
+// throughput, which the four waves lose: each variant's limit lies between the largest mesh measured on which they were
+// the faster and the smallest on which they were not.  Per launch, four waves per 64 elements against one lane per
+// element (us):
+//   p=1             20.3 and 21.3 at 81,369 elements, 22.1 and 21.1 at 89,340 (13.0 and 17.9 at 5k)
+//   p=1 spherical   20.4 and 20.4 at 61,972, 23.9 and 22.1 at 66,187
+//   p=1 storm       29.2 and 33.5 at 93,850, 30.8 and 30.8 at 99,015 (13.9 and 27.0 at 5k)
+//   p=2             31.0 and 31.4 at 63,445, 36.2 and 35.0 at 67,198 (18.8 and 27.9 at 5k)
+//   p=2 spherical   32.4 and 32.5 at 56,276, 34.2 and 32.4 at 59,314
+//   p=2 storm       47.5 and 48.5 at 81,369, 51.3 and 49.9 at 89,340 (21.1 and 42.3 at 5k)
+int split_max(const Ctx& c) {
+    if (c.met) return c.prm.p == 1 ? 96000 : 85000;
+    if (c.prm.ics == 2) return c.prm.p == 1 ? 64000 : 58000;
+    return c.prm.p == 1 ? 85000 : 64000;
+}
+bool stage_split(const Ctx& c) { return c.prm.nolicat != 0 && c.ne <= split_max(c); }
 
 // Elements per block the stage kernel runs with: 64 for linearised runs; the number chosen by dg_gpu_set_block or the
 // autotuner; otherwise 64 where stage_split_kernel runs, else one lane per element in blocks of 128 (p=1) or 64.
