@@ -261,7 +261,9 @@ struct Ctx {
     double ktime[K_COUNT] = {};
     long long kcount[K_COUNT] = {};
     std::vector<std::pair<hipEvent_t, hipEvent_t>> evpool;
-    std::vector<std::pair<int, int>> pending;    // (kernel id, event pair index)
+    // launches timed and not yet added: kernel id, event pair, sampled steps of those it covers, their share of its time
+    struct Timed { int kid, ev, count; double share; };
+    std::vector<Timed> pending;
     void drop_graphs() {
         for (auto& g : graphs) (void)hipGraphExecDestroy(g.second);
         graphs.clear();
@@ -303,8 +305,8 @@ DevTables to_dev(const RefTables& t) {
 }
 
 // ---- profiling helpers (no events are recorded into a captured graph)
-int prof_begin(Ctx& c, int kid, bool capturing) {
-    if (!c.prof || capturing || !c.prof_this) return -1;
+int prof_begin(Ctx& c, int kid, bool capturing, int count = 1, double share = 1.0) {
+    if (!c.prof || capturing || count == 0 || !(c.prof_this || kid == K_MET)) return -1;
     const int idx = (int)c.pending.size();
     if (idx >= (int)c.evpool.size()) {
         hipEvent_t a, b;
@@ -312,7 +314,7 @@ int prof_begin(Ctx& c, int kid, bool capturing) {
         c.evpool.push_back({a, b});
     }
     (void)hipEventRecord(c.evpool[idx].first, c.stream);
-    c.pending.push_back({kid, idx});
+    c.pending.push_back({kid, idx, count, share});
     return idx;
 }
 void prof_end(Ctx& c, int idx) {
@@ -323,9 +325,9 @@ int prof_flush(Ctx& c) {
     HIPCHK(hipStreamSynchronize(c.stream));
     for (auto& pr : c.pending) {
         float ms = 0.f;
-        HIPCHK(hipEventElapsedTime(&ms, c.evpool[pr.second].first, c.evpool[pr.second].second));
-        c.ktime[pr.first] += ms;
-        c.kcount[pr.first] += 1;
+        HIPCHK(hipEventElapsedTime(&ms, c.evpool[pr.ev].first, c.evpool[pr.ev].second));
+        c.ktime[pr.kid] += pr.share * ms;
+        c.kcount[pr.kid] += pr.count;
     }
     c.pending.clear();
     return 0;
@@ -1272,8 +1274,9 @@ int launch_stage_v(Ctx& c, const StageArgs& a0, bool sph, bool fuse) {
 
 // Boundary, potential and storm forcing of n steps from the step `first` (of the tables, or of the graph being
 // captured) into the forcing arrays: the open-boundary elevation terms (tide_kernel), the specified normal
-// flux (flow_kernel), the tidal potential at the nodes (tip_kernel) and the Holland profile (met_kernel).
-int launch_forcing(Ctx& c, int first, int n, bool capturing) {
+// flux (flow_kernel), the tidal potential at the nodes (tip_kernel) and the Holland profile (met_kernel), which is
+// timed for the `sampled` steps among them.
+int launch_forcing(Ctx& c, int first, int n, bool capturing, int sampled = 0) {
     c.fb0 = c.hstep = first;
     c.fbn = n;
     const int cap = capturing ? 0 : -1;
@@ -1298,7 +1301,7 @@ int launch_forcing(Ctx& c, int first, int n, bool capturing) {
         HIPCHK(hipGetLastError());
     }
     if (c.met) {
-        int ev = prof_begin(c, K_MET, capturing);
+        int ev = prof_begin(c, K_MET, capturing, sampled, (double)sampled / n);
         hipLaunchKernelGGL(met_kernel, grid(c.np, (unsigned)n), dim3(256), 0, c.stream, met_args(c, cap), F);
         prof_end(c, ev);
         HIPCHK(hipGetLastError());
@@ -1313,7 +1316,11 @@ int need_forcing(Ctx& c, bool back = false) {
     if (k >= c.fb0 && k < c.fb0 + c.fbn) return 0;
     const int first = back ? std::max(0, k + 1 - c.fbatch) : k;
     const int n = back ? k + 1 - first : std::min(c.fbatch, c.tn - k);
-    if (launch_forcing(c, first, n, false)) return 1;
+    // the profiler's steps of the batch: the current one is prof_step - 1
+    int sampled = 0;
+    if (c.prof)
+        for (int s = 0; s < n; s++) sampled += (c.prof_step - 1 + s) % c.prof_every == 0;
+    if (launch_forcing(c, first, n, false, sampled)) return 1;
     c.hstep = k;
     return 0;
 }

@@ -186,7 +186,8 @@ int dg_gpu_mass_noalloc(int handle, double* mass);
  * long run with little event overhead); enable=0 switches timing off.  dg_gpu_kernel_stats
  * returns the summed milliseconds and
  * launch count of kernel `kernel_id` (0 stage kernel, 1 node min/max, 2 limiter+wet/dry,
- * 3 modal2nodal, 4 NWS=8 node forcing, a launch of which covers several steps) since the last reset.  No counterpart in the reference
+ * 3 modal2nodal, 4 NWS=8 node forcing, whose launches cover several steps: each timed step counts as one, with
+ * its share of the time) since the last reset.  No counterpart in the reference
  * (it has no timers). */
 int dg_gpu_profile(int handle, int enable);
 int dg_gpu_kernel_stats(int handle, int kernel_id, double* total_ms, long long* launches,
