@@ -1042,7 +1042,7 @@ __global__ void __launch_bounds__(4 * ADJ_NT) __attribute__((amdgpu_waves_per_eu
 
 // ------------------------------------------------------------------------------------------
 // WETDRY (src/wetdry.F:58-548) of element e reversed with its branches frozen: from the state it
-// was applied to (U: the limited stage output's modes 1-3, formed by limit_wetdry_kernel's adjoint
+// was applied to (U: the limited stage output's modes 1-3, formed by limit_wide_kernel's adjoint
 // variant), the vertex depths D and the element's flag before it, the element retakes the
 // forward's decisions operation by operation (no contraction, so that they are the forward's) --
 // which vertices are dry, the branch, the vertices' depth order, the two fmax(H0, .) choices, the

@@ -1386,28 +1386,40 @@ LimTiles lim_tiles(const Ctx& c) {
     return LimTiles{L.vhidx.p, L.qinc.p, L.xoff.p, L.xq.p, L.xinc.p, L.elq.p, L.nvh, L.nql, L.nx};
 }
 
+// Elements from which on the limiter runs as limit_wide_kernel (a wave per tile) instead of limit_wetdry_kernel (a wave
+// per field and tile).  Per launch, the latter and the former (us): with WETDRY p=1 15.4 and 15.6 at 199,027 elements,
+// 20.5 and 19.6 at 298,563; p=2 9.9 and 10.3 at 79,119, 12.0 and 11.1 at 99,015.  The limiter alone gains less from it: p=1 30.4
+// and 30.7 at 696,907, 35.5 and 33.9 at 796,320; p=2 24.6 and 24.8 at 498,722, 29.2 and 28.8 at 597,806.
+constexpr int lim_wide(int p, bool wetdry) { return wetdry ? (p == 1 ? 250000 : 90000) : (p == 1 ? 750000 : 550000); }
+
 // SLOPELIMITER5 (+ WETDRY) on the stage output u, in place; with WETDRY the stage kernel has left
 // u's cell means in c.cmean.
 template <int P>
-int launch_limiter(Ctx& c, double* u, const ElemData& ed, bool capturing, const uint8_t* fin = nullptr,
-                   uint8_t* fout = nullptr) {
-    const int ne = c.ne;
+int launch_limiter(Ctx& c, double* u, bool capturing, const uint8_t* fin = nullptr, uint8_t* fout = nullptr) {
     if (!c.lim.elq.p || !c.cmean.p) return fail("internal: slope limiter tiles not built");
     const bool wdon = c.prm.nolifa >= 2;
-    const double* cm = wdon ? c.cmean.p : u;
-    const size_t cms = wdon ? (size_t)ne : (size_t)c.dof * ne;
-    const LimTiles lt = lim_tiles(c);
-    const dim3 grid((ne + LIM_NT - 1) / LIM_NT), block(3 * LIM_NT);
-    const size_t lds = lim_lds(lt.nvh, lt.nql);
     const uint8_t* wd = fin ? fin : c.wd[c.wdcur].p;
+    uint8_t* wd_out = fout ? fout : c.wd[1 - c.wdcur].p;
+    const double* cm = wdon ? c.cmean.p : u;
+    const size_t cms = wdon ? (size_t)c.ne : (size_t)c.dof * c.ne;
+    const ElemData ed = elem_data(c);
+    const LimTiles lt = lim_tiles(c);
+    const dim3 grid((c.ne + LIM_NT - 1) / LIM_NT);
+    const size_t lds = lim_lds(lt.nvh, lt.nql);
+    const bool wide = c.ne >= lim_wide(P, wdon);
+    double* const none = nullptr;
     int ev = prof_begin(c, K_LIMIT, capturing);
     if (wdon) {
-        hipLaunchKernelGGL((limit_wetdry_kernel<P, true, false>), grid, block, lds, c.stream, ed, u, cm, cms, lt, wd,
-                           fout ? fout : c.wd[1 - c.wdcur].p, c.wd_active, (double*)nullptr, (double*)nullptr);
+        if (wide) hipLaunchKernelGGL((limit_wide_kernel<P, true, false>), grid, dim3(LIM_NT), lds, c.stream, ed, u, cm, cms, lt, wd,
+                                     wd_out, c.wd_active, none, none);
+        else hipLaunchKernelGGL((limit_wetdry_kernel<P, true>), grid, dim3(3 * LIM_NT), lds, c.stream, ed, u, cm, cms, lt, wd,
+                                wd_out, c.wd_active);
         if (!fout) c.wdcur = 1 - c.wdcur;
     } else {
-        hipLaunchKernelGGL((limit_wetdry_kernel<P, false, false>), grid, block, lds, c.stream, ed, u, cm, cms, lt, wd,
-                           c.wd[1 - c.wdcur].p, (int*)nullptr, (double*)nullptr, (double*)nullptr);
+        if (wide) hipLaunchKernelGGL((limit_wide_kernel<P, false, false>), grid, dim3(LIM_NT), lds, c.stream, ed, u, cm, cms, lt, wd,
+                                     wd_out, (int*)nullptr, none, none);
+        else hipLaunchKernelGGL((limit_wetdry_kernel<P, false>), grid, dim3(3 * LIM_NT), lds, c.stream, ed, u, cm, cms, lt, wd,
+                                wd_out, (int*)nullptr);
     }
     prof_end(c, ev);
     HIPCHK(hipGetLastError());
@@ -1422,7 +1434,7 @@ template <int P>
 int launch_wetdry_rev(Ctx& c, const double* wpre, const uint8_t* flags, double* cot) {
     if (!c.lim.elq.p) return fail("internal: slope limiter tiles not built");
     const LimTiles lt = lim_tiles(c);
-    hipLaunchKernelGGL((limit_wetdry_kernel<P, false, true>), dim3((c.ne + LIM_NT - 1) / LIM_NT), dim3(3 * LIM_NT),
+    hipLaunchKernelGGL((limit_wide_kernel<P, false, true>), dim3((c.ne + LIM_NT - 1) / LIM_NT), dim3(LIM_NT),
                        (size_t)lim_lds(lt.nvh, lt.nql), c.stream, elem_data(c), const_cast<double*>(wpre), wpre,
                        (size_t)c.dof * c.ne, lt, flags, (uint8_t*)nullptr, (int*)nullptr, cot, c.gdp.p);
     HIPCHK(hipGetLastError());
@@ -1451,7 +1463,7 @@ int launch_step(Ctx& c, int cap) {
         prof_end(c, ev);
         HIPCHK(hipGetLastError());
         if (fuse) c.wdcur = 1 - c.wdcur;
-        if (lim && launch_limiter<P>(c, a.uout, a.ed, capturing)) return 1;
+        if (lim && launch_limiter<P>(c, a.uout, capturing)) return 1;
     }
     if (!capturing) c.hstep++;
     c.prof_this = true;
@@ -1514,7 +1526,7 @@ int launch_step_explicit(Ctx& c, double* const* st, double* const* wsave = nullp
         if (launch_stage_nt<P>(c, a, sph, fuse, stage_block(c))) return 1;
         HIPCHK(hipGetLastError());
         if (fuse && !fsave) c.wdcur = 1 - c.wdcur;
-        if (lim && launch_limiter<P>(c, st[irk + 1], a.ed, false, fsave ? fsave[irk] : nullptr,
+        if (lim && launch_limiter<P>(c, st[irk + 1], false, fsave ? fsave[irk] : nullptr,
                                      fsave ? fsave[irk + 1] : nullptr)) return 1;
     }
     c.hstep++;

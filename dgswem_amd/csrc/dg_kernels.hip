@@ -7,7 +7,8 @@
 //                    edge fluxes are evaluated by both neighbours with the same operands in the same
 //                    order, so both see bit-identical values and no scatter or atomics are needed.
 //                    Small meshes run stage_split_kernel, four waves per 64 elements, instead.
-//   limit_wetdry     a wave per field of 64 elements: SLOPELIMITER5 on modes 2-3, then WETDRY
+//   limit_wetdry     SLOPELIMITER5 on modes 2-3, then WETDRY: a wave per field of 64 elements, on large meshes
+//                    (limit_wide) a wave for all three
 // preceded once per batch of steps by tide_kernel (the tidal boundary terms of every stage) and, with
 // NWS=8, met_kernel (the Holland profile at the nodes); plus modal2nodal (one thread per node) on output
 // steps.
@@ -1361,21 +1362,29 @@ __global__ void __launch_bounds__(256) node_minmax_kernel(int np, int ne, const 
 // cms = ne): WETDRY rewrites some cell means of u in place, which other tiles' halos must not see.
 // Without it they are read from u itself (cms = DOF*ne), whose cell means the limiter keeps.
 // ------------------------------------------------------------------------------------------
-// Three waves per 64 elements: wave c stages, bounds and limits field c, so its branches on c are uniform.  What
-// bounds it is memory (about 165 bytes per element at p=1) and, on small meshes, the chain of loads before the first
-// bound.  A third of the work per lane keeps three times the loads under way, and lists at fixed strides need no
-// look-up before them.  Tiles of 64 and of 256 elements take the same time on large meshes (the larger halo of the
-// small ones comes from the L2), and on small ones 64 use four times the compute units (7.4 against 9.0 us at 5k
-// elements).  The modes past the third are touched only where WETDRY changes the element.
-// Per launch, one lane per element and 256-element tiles before, now: 997,306 elements p=1 48.2 and 49.2 us, 298,700
-// elements p=2 27.6 and 20.5 us, 4,783 elements p=1 9.2 and 4.6 us.
+// limit_wetdry_kernel: three waves per 64 elements; wave c stages, bounds and limits field c, so its branches on c are
+// uniform.  What bounds it on small meshes is the chain of loads before the first bound: a third of the work per lane
+// keeps three times the loads under way, and lists at fixed strides need no look-up before them.  Tiles of 64 use four
+// times the compute units of tiles of 256 there (7.4 against 9.0 us at 5k elements).  The modes past the third are
+// touched only where WETDRY changes the element.
+// Per launch, one lane per element and 256-element tiles before, now: 4,783 elements p=1 9.2 and 4.6 us, 99,015 elements
+// p=2 16.3 and 12.0 us.
+//
+// limit_wide_kernel: a wave per tile, a lane for the three fields of an element.  On large meshes the chip is full
+// either way, and what the three waves do three times (the lists, the addresses, the exchange before WETDRY) is time: 1103
+// VALU instructions per element, 943 here, for the same bytes (165 per element at p=1).  lim_wide says from how many
+// elements on it is the faster form.  Per launch, one lane per element and 256-element tiles before, three waves per
+// tile, a wave per tile (us):
+//   limiter and WETDRY  p=1  46.6, 52.6, 43.0 at 997,306 elements; 32.3, 31.4, 27.5 at 597,806; 22.0, 19.9, 19.5 at 298,563
+//                       p=2  48.6, 39.2, 30.2 at 597,806; 26.7, 21.7, 19.9 at 298,579
+//   WETDRY's reverse    p=2  29.9, 48.9, 24.5 at 792,120; 8.8, 9.2, 6.8 at 84,370; 7.2, 5.1, 4.7 at 4,783
 //
 // With WDADJ (the adjoint's reverse sweep; WETDRY false) the kernel writes nothing to u: each
 // element's limited modes, formed exactly as the forward formed them, go to the
 // frozen-branch WETDRY reverse of that element (wetdry_adj_element), which turns the cotangent ub
 // of WETDRY's output into that of its input and adds the vertex-depth cotangents to gdp.
 //
-// The launch passes lim_lds() bytes of dynamic LDS.
+// The launches pass lim_lds() bytes of dynamic LDS.
 constexpr int LIM_NT = 64;               // elements per tile
 constexpr int lim_lds(int nvh, int nql) {
     return 8 * (3 * (LIM_NT + nvh) + 6 * nql > 9 * LIM_NT ? 3 * (LIM_NT + nvh) + 6 * nql : 9 * LIM_NT) + LIM_NT;
@@ -1445,15 +1454,51 @@ template <int P>
 __device__ void wetdry_adj_element(const DevTables& T, const double (&U)[3][3], const double (&D)[3], int wdflg,
                                    double H0, int e, int ne, double* __restrict__ ub, double* __restrict__ gdp);
 
-template <int P, bool WETDRY, bool WDADJ>
+// Minimum and maximum of the staged means at eight byte offsets.
+__device__ __forceinline__ void minmax8(const char* cm, const uint4& r, double& lo, double& hi) {
+    const uint32_t p[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const double a = *reinterpret_cast<const double*>(cm + (p[i] & 0xffffu));
+        const double b = *reinterpret_cast<const double*>(cm + (p[i] >> 16));
+        lo = min1(lo, min1(a, b));
+        hi = max1(hi, max1(a, b));
+    }
+}
+
+// WETDRY of an element that it changes, from its limited modes L (mean and linear modes of each field); the modes
+// past the third are read here.
+template <int P>
+__device__ __forceinline__ void wetdry_limited(const DevTables& T, const double (&L)[3][3], const double (&D)[3], int wdi,
+                                               double h0, double* __restrict__ u, int e, int ne,
+                                               uint8_t* __restrict__ wd_out, int* __restrict__ wd_active) {
+    constexpr int DOF = (P + 1) * (P + 2) / 2;
+    double U[3][DOF];
+#pragma unroll
+    for (int f = 0; f < 3; f++)
+#pragma unroll
+        for (int k = 0; k < DOF; k++) U[f][k] = k < 3 ? L[f][k] : at(u + (size_t)(f * DOF + k) * ne, e);
+    const double c13 = 1.0 / 3.0, c16 = 1.0 / 6.0;
+    const double hb[3] = {c13 * (D[0] + D[1] + D[2]), -(c16 * (D[0] + D[1])) + c13 * D[2], -(0.5 * D[0]) + 0.5 * D[1]};
+    const double dpe_min = fmin(fmin(D[0], D[1]), D[2]);
+    if (wd_active) wd_active[0] = 1;
+    at(wd_out, e) = (uint8_t)wetdry_element<P>(T, U, D, hb, dpe_min, wdi, h0);
+#pragma unroll
+    for (int f = 0; f < 3; f++) {
+        // wetting and drying changes the cell mean only of some elements: written back when its bits changed
+        if (__double_as_longlong(U[f][0]) != __double_as_longlong(L[f][0])) at(u + (size_t)(f * DOF) * ne, e) = U[f][0];
+#pragma unroll
+        for (int k = 1; k < DOF; k++) at(u + (size_t)(f * DOF + k) * ne, e) = U[f][k];
+    }
+}
+
+template <int P, bool WETDRY>
 __global__ void __launch_bounds__(3 * LIM_NT) __attribute__((amdgpu_waves_per_eu(4))) limit_wetdry_kernel(ElemData E, double* __restrict__ u,
                                                               const double* __restrict__ cmean, size_t cms,
                                                               LimTiles lt,
                                                               const uint8_t* __restrict__ wd_in,
                                                               uint8_t* __restrict__ wd_out,
-                                                              int* __restrict__ wd_active,
-                                                              double* __restrict__ ub, double* __restrict__ gdp) {
-    static_assert(!(WETDRY && WDADJ), "the WETDRY reverse starts from the limiter's output alone");
+                                                              int* __restrict__ wd_active) {
     constexpr int DOF = (P + 1) * (P + 2) / 2;
     constexpr int NT = LIM_NT;
     const DevTables& T = tab<P>();
@@ -1479,7 +1524,7 @@ __global__ void __launch_bounds__(3 * LIM_NT) __attribute__((amdgpu_waves_per_eu
     const int lq = at(lt.elq, ec);
     double D[3] = {0.0, 0.0, 0.0}, h0 = 0.0;
     int wdi = 0;
-    if ((WETDRY || WDADJ) && c == 0) {
+    if (WETDRY && c == 0) {
 #pragma unroll
         for (int v = 0; v < 3; v++) D[v] = at(E.dpv + (size_t)v * ne, ec);
         const int sid = E.sid ? (int)at(E.sid, ec) : 0;
@@ -1498,20 +1543,10 @@ __global__ void __launch_bounds__(3 * LIM_NT) __attribute__((amdgpu_waves_per_eu
     __syncthreads();
     // the bounds of the tile's nodes
     const char* const cmb = reinterpret_cast<const char*>(cm);
-    auto minmax8 = [&](const uint4& r, double& lo, double& hi) {
-        const uint32_t p[4] = {r.x, r.y, r.z, r.w};
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const double a = *reinterpret_cast<const double*>(cmb + (p[i] & 0xffffu));
-            const double b = *reinterpret_cast<const double*>(cmb + (p[i] >> 16));
-            lo = min1(lo, min1(a, b));
-            hi = max1(hi, max1(a, b));
-        }
-    };
     for (int q = le; q < nql; q += NT) {
         if (q != le) rq = qi[q];
         double lo = 99999., hi = -99999.;
-        minmax8(rq, lo, hi);
+        minmax8(cmb, rq, lo, hi);
         bnd[q] = lo;
         bnd[nql + q] = hi;
     }
@@ -1524,7 +1559,7 @@ __global__ void __launch_bounds__(3 * LIM_NT) __attribute__((amdgpu_waves_per_eu
                 for (int x = x0; x < x1; x++) {
                     const int q = lt.xq[x];
                     double lo = bnd[q], hi = bnd[nql + q];
-                    minmax8(reinterpret_cast<const uint4*>(lt.xinc)[x], lo, hi);
+                    minmax8(cmb, reinterpret_cast<const uint4*>(lt.xinc)[x], lo, hi);
                     bnd[q] = lo;
                     bnd[nql + q] = hi;
                 }
@@ -1538,7 +1573,7 @@ __global__ void __launch_bounds__(3 * LIM_NT) __attribute__((amdgpu_waves_per_eu
         for (int i = 0; i < 3; i++) { vmin[i] = bnd[q[i]]; vmax[i] = bnd[nql + q[i]]; }
         limit_field(T, c0, w1, w2, vmin, vmax);
     }
-    if (!WETDRY && !WDADJ) {
+    if (!WETDRY) {
         if (!valid) return;
         at(u + (size_t)(c * DOF + 1) * ne, e) = w1;
         at(u + (size_t)(c * DOF + 2) * ne, e) = w2;
@@ -1555,7 +1590,7 @@ __global__ void __launch_bounds__(3 * LIM_NT) __attribute__((amdgpu_waves_per_eu
         keep[le] = mine;
     }
     if (!__syncthreads_or(!mine)) {
-        if (WDADJ || !valid) return;
+        if (!valid) return;
         if (c == 0) at(wd_out, e) = 1;
         at(u + (size_t)(c * DOF + 1) * ne, e) = w1;
         at(u + (size_t)(c * DOF + 2) * ne, e) = w2;
@@ -1567,39 +1602,129 @@ __global__ void __launch_bounds__(3 * LIM_NT) __attribute__((amdgpu_waves_per_eu
         ex[(c * 3) * NT + le] = c0;
         ex[(c * 3 + 1) * NT + le] = w1;
         ex[(c * 3 + 2) * NT + le] = w2;
-    } else if (WETDRY && valid) {
+    } else if (valid) {
         if (c == 0) at(wd_out, e) = 1;
         at(u + (size_t)(c * DOF + 1) * ne, e) = w1;
         at(u + (size_t)(c * DOF + 2) * ne, e) = w2;
     }
     __syncthreads();
     if (mine || c != 0) return;
-    if (WDADJ) {
-        double U3[3][3];
-#pragma unroll
-        for (int f = 0; f < 3; f++)
-#pragma unroll
-            for (int k = 0; k < 3; k++) U3[f][k] = ex[(f * 3 + k) * NT + le];
-        wetdry_adj_element<P>(T, U3, D, wdi, h0, e, ne, ub, gdp);
-        return;
-    }
-    double U[3][DOF];
+    double U3[3][3];
 #pragma unroll
     for (int f = 0; f < 3; f++)
 #pragma unroll
-        for (int k = 0; k < DOF; k++) U[f][k] = k < 3 ? ex[(f * 3 + k) * NT + le] : at(u + (size_t)(f * DOF + k) * ne, e);
-    const double c13 = 1.0 / 3.0, c16 = 1.0 / 6.0;
-    const double hb[3] = {c13 * (D[0] + D[1] + D[2]), -(c16 * (D[0] + D[1])) + c13 * D[2], -(0.5 * D[0]) + 0.5 * D[1]};
-    const double dpe_min = fmin(fmin(D[0], D[1]), D[2]);
-    if (wd_active) wd_active[0] = 1;
-    at(wd_out, e) = (uint8_t)wetdry_element<P>(T, U, D, hb, dpe_min, wdi, h0);
+        for (int k = 0; k < 3; k++) U3[f][k] = ex[(f * 3 + k) * NT + le];
+    wetdry_limited<P>(T, U3, D, wdi, h0, u, e, ne, wd_out, wd_active);
+}
+
+template <int P, bool WETDRY, bool WDADJ>
+__global__ void __launch_bounds__(LIM_NT) limit_wide_kernel(ElemData E, double* __restrict__ u, const double* __restrict__ cmean,
+                                                            size_t cms, LimTiles lt, const uint8_t* __restrict__ wd_in,
+                                                            uint8_t* __restrict__ wd_out, int* __restrict__ wd_active,
+                                                            double* __restrict__ ub, double* __restrict__ gdp) {
+    static_assert(!(WETDRY && WDADJ), "the WETDRY reverse starts from the limiter's output alone");
+    constexpr int DOF = (P + 1) * (P + 2) / 2;
+    constexpr int NT = LIM_NT;
+    const DevTables& T = tab<P>();
+    const int ne = E.ne;
+    const int le = threadIdx.x;
+    const int tile = xcd_tile(blockIdx.x, gridDim.x);
+    const int e = tile * NT + le;
+    const bool valid = e < ne;
+    extern __shared__ double lds[];
+    const int nsl = NT + lt.nvh, nql = lt.nql;
+    double* const cm = lds;                                 // [field][nsl] staged cell means
+    double* const bnd = lds + 3 * nsl;                      // [field][min, max][nql] node bounds
+    const int ec = valid ? e : ne - 1;                      // lanes past the last element read element ne-1 and write nothing
+    const int* vh = lt.vhidx + (size_t)tile * lt.nvh;
+    const uint4* qi = reinterpret_cast<const uint4*>(lt.qinc) + (size_t)tile * nql;
+    const int g = le < lt.nvh ? vh[le] : -1;
+    uint4 rq = le < nql ? qi[le] : make_uint4(0, 0, 0, 0);
+    double c0[3], w1[3], w2[3], m[3];
 #pragma unroll
     for (int f = 0; f < 3; f++) {
-        // wetting and drying changes the cell mean only of some elements: written back when its bits changed
-        if (__double_as_longlong(U[f][0]) != __double_as_longlong(ex[(f * 3) * NT + le]))
-            at(u + (size_t)(f * DOF) * ne, e) = U[f][0];
+        c0[f] = at(cmean + (size_t)f * cms, ec);
+        w1[f] = at(u + (size_t)(f * DOF + 1) * ne, ec);
+        w2[f] = at(u + (size_t)(f * DOF + 2) * ne, ec);
+    }
+    const int lq = at(lt.elq, ec);
+    double D[3] = {0.0, 0.0, 0.0}, h0 = 0.0;
+    int wdi = 0;
+    if (WETDRY || WDADJ) {
 #pragma unroll
-        for (int k = 1; k < DOF; k++) at(u + (size_t)(f * DOF + k) * ne, e) = U[f][k];
+        for (int v = 0; v < 3; v++) D[v] = at(E.dpv + (size_t)v * ne, ec);
+        const int sid = E.sid ? (int)at(E.sid, ec) : 0;
+        h0 = E.scen[sid].h0;
+        wdi = at(wd_in, ec);
+    }
+#pragma unroll
+    for (int f = 0; f < 3; f++) m[f] = at(cmean + (size_t)f * cms, g < 0 ? 0 : g);
+#pragma unroll
+    for (int f = 0; f < 3; f++) {
+        cm[f * nsl + le] = c0[f];
+        if (g >= 0) cm[f * nsl + NT + le] = m[f];
+    }
+#pragma unroll 1
+    for (int h = le + NT; h < lt.nvh; h += NT) {
+        const int gh = vh[h];
+        if (gh < 0) break;
+#pragma unroll
+        for (int f = 0; f < 3; f++) cm[f * nsl + NT + h] = at(cmean + (size_t)f * cms, gh);
+    }
+    __syncthreads();
+    const char* const cmb = reinterpret_cast<const char*>(cm);
+    for (int q = le; q < nql; q += NT) {
+        if (q != le) rq = qi[q];
+#pragma unroll
+        for (int f = 0; f < 3; f++) {
+            double lo = 99999., hi = -99999.;
+            minmax8(cmb + (size_t)8 * f * nsl, rq, lo, hi);
+            bnd[2 * f * nql + q] = lo;
+            bnd[(2 * f + 1) * nql + q] = hi;
+        }
+    }
+    if (lt.nx > 0) {
+        const int x0 = lt.xoff[tile], x1 = lt.xoff[tile + 1];
+        if (x1 > x0) {
+            // nodes with more than eight elements: a lane of each field goes through the tile's extra entries
+            __syncthreads();
+            if (le < 3)
+                for (int x = x0; x < x1; x++) {
+                    const int q = lt.xq[x];
+                    double lo = bnd[2 * le * nql + q], hi = bnd[(2 * le + 1) * nql + q];
+                    minmax8(cmb + (size_t)8 * le * nsl, reinterpret_cast<const uint4*>(lt.xinc)[x], lo, hi);
+                    bnd[2 * le * nql + q] = lo;
+                    bnd[(2 * le + 1) * nql + q] = hi;
+                }
+        }
+    }
+    __syncthreads();
+    {
+        const int q[3] = {lq & 1023, (lq >> 10) & 1023, (lq >> 20) & 1023};
+#pragma unroll
+        for (int f = 0; f < 3; f++) {
+            double vmin[3], vmax[3];
+#pragma unroll
+            for (int i = 0; i < 3; i++) { vmin[i] = bnd[2 * f * nql + q[i]]; vmax[i] = bnd[(2 * f + 1) * nql + q[i]]; }
+            limit_field(T, c0[f], w1[f], w2[f], vmin, vmax);
+        }
+    }
+    if (!valid) return;
+    if (WETDRY || WDADJ) {
+        const double K[3][DOF] = {{c0[0], w1[0], w2[0]}};
+        if (!wetdry_keeps<P>(T, K, D, wdi, h0)) {
+            const double L[3][3] = {{c0[0], w1[0], w2[0]}, {c0[1], w1[1], w2[1]}, {c0[2], w1[2], w2[2]}};
+            if constexpr (WDADJ) wetdry_adj_element<P>(T, L, D, wdi, h0, e, ne, ub, gdp);
+            else wetdry_limited<P>(T, L, D, wdi, h0, u, e, ne, wd_out, wd_active);
+            return;
+        }
+        if (WDADJ) return;
+        at(wd_out, e) = 1;
+    }
+#pragma unroll
+    for (int f = 0; f < 3; f++) {
+        at(u + (size_t)(f * DOF + 1) * ne, e) = w1[f];
+        at(u + (size_t)(f * DOF + 2) * ne, e) = w2[f];
     }
 }
 
