@@ -61,6 +61,11 @@ struct DevBuf {
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
     ~DevBuf() { if (p) (void)hipFree(p); }
+    void release() {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+        n = cap = 0;
+    }
     hipError_t alloc(size_t count) {
         n = count;
         if (p && count <= cap) return hipSuccess;
@@ -143,6 +148,9 @@ struct HostChunks {
         return ok;
     }
 };
+
+// Device bytes in which all handles of the process keep the stages of their gradients (dg_adj_gradient).
+std::atomic<size_t> g_kept{0};
 
 struct Ctx {
     std::vector<Member> mem;
@@ -248,6 +256,7 @@ struct Ctx {
     // active wetting/drying under the limiter: the flags at each checkpoint and at the start of every
     // stage of a segment
     DevBuf<uint8_t> ckptwd, segwd;
+    size_t kept = 0;                             // this handle's share of g_kept
     bool adj_wd = false;      // WETDRY after the limiter: flags kept at the checkpoints
     bool adj_wdrev = false;   // ... and WETDRY changed an element in the forward sweep: reversed
     // graphs of one slot-rotation period, keyed by (ucur, wdcur) at capture
@@ -270,6 +279,7 @@ struct Ctx {
     }
     ~Ctx() {
         if (stream) (void)hipStreamSynchronize(stream);
+        g_kept -= kept;
         drop_graphs();
         for (auto& e : evpool) { (void)hipEventDestroy(e.first); (void)hipEventDestroy(e.second); }
         if (stream) (void)hipStreamDestroy(stream);
@@ -2541,45 +2551,53 @@ int dg_adj_gradient(int h, int it, int nsteps, const double* data, double weight
     // per checkpoint and per stage)
     c->adj_wd = c->prm.nolifa >= 2 && lim;
     c->adj_wdrev = false;
-    // Without a spacing from the caller every stage of the run is kept if that takes no more than a sixteenth of the
-    // device's memory and half of what is free (buffers that are already this large are used as they are), and
-    // the reverse sweep recomputes nothing; otherwise checkpoints about sqrt(N) steps apart.  The gradients are the
-    // same bits.  80 steps of 49,800 p=1 elements (0.6 GB) 7.6 ms with the recomputation, 5.5 ms without; 30 steps of
-    // four p=2 storm basins of 99,000 elements (1.7 GB) 15.7 and 11.9 ms.
-    bool keep = false;
-    if (interval <= 0) {
-        const size_t n = (size_t)nsteps * nrk;
-        keep = c->seg.p && c->seg.cap >= n * ssz && (!lim || (c->wseg.p && c->wseg.cap >= n * ssz)) &&
-               (!c->adj_wd || (c->segwd.p && c->segwd.cap >= n * ne));
-        size_t avail = 0, total = 0;
-        if (!keep && hipMemGetInfo(&avail, &total) == hipSuccess) {
-            const size_t need = n * (ssz * sizeof(double) * (lim ? 2 : 1) + (c->adj_wd ? ne : 0));
-            keep = need <= total / 16 && need <= avail / 2;
-        }
-        if (keep && (c->seg.alloc(n * ssz) != hipSuccess || (lim && c->wseg.alloc(n * ssz) != hipSuccess) ||
-                     (c->adj_wd && c->segwd.alloc(n * ne) != hipSuccess))) {
-            (void)hipGetLastError();
-            keep = false;
-        }
-        interval = keep ? kTableChunk : std::max(1, (int)std::lround(std::sqrt((double)nsteps)));
-    }
-    interval = std::min(interval, nsteps);
-    const int ncp = keep ? 1 : (nsteps + interval - 1) / interval;
     HIPCHK(c->geta.alloc((size_t)nsteps * c->ng));
     HIPCHK(c->gdata.upload(data, (size_t)nsteps * c->ng, c->stream));
-    HIPCHK(c->ckpt.alloc((size_t)ncp * ssz));
-    if (!keep) HIPCHK(c->seg.alloc((size_t)interval * nrk * ssz));
     HIPCHK(c->lam.alloc(ssz));
     for (int i = 0; i < nrk; i++) HIPCHK(c->ubar[i].alloc(ssz));
     HIPCHK(c->gdp.alloc((size_t)3 * ne));
     HIPCHK(c->gnb.alloc(ne));
     HIPCHK(c->pout.alloc(std::max(ssz, (size_t)2 * np)));
     if (lim) {
-        if (!keep) HIPCHK(c->wseg.alloc((size_t)interval * nrk * ssz));
         HIPCHK(c->lnbc.alloc((size_t)18 * ne));
         HIPCHK(c->lgsum.alloc((size_t)6 * np));
         HIPCHK(c->larg.alloc((size_t)6 * np));
     }
+    // Without a spacing from the caller every stage of the run is kept, if that takes no more than half of the memory
+    // that is free and all handles of the process together keep no more than a sixteenth of the device's (buffers that
+    // are already this large are used as they are), and the reverse sweep recomputes nothing; otherwise checkpoints
+    // about sqrt(N) steps apart.  The gradients are the same bits.  80 steps of 49,800 p=1 elements (0.6 GB) 7.6 ms with
+    // the recomputation, 5.5 ms without; 30 steps of four p=2 storm basins of 99,000 elements (1.7 GB) 15.7 and 11.9 ms.
+    bool keep = false;
+    if (interval <= 0) {
+        const size_t n = (size_t)nsteps * nrk;
+        keep = c->seg.p && c->seg.cap >= n * ssz && (!lim || (c->wseg.p && c->wseg.cap >= n * ssz)) &&
+               (!c->adj_wd || (c->segwd.p && c->segwd.cap >= n * ne));
+        const size_t need = n * (ssz * sizeof(double) * (lim ? 2 : 1) + (c->adj_wd ? ne : 0));
+        size_t avail = 0, total = 0;
+        if (!keep && hipMemGetInfo(&avail, &total) == hipSuccess && need <= avail / 2) {
+            size_t all = g_kept.load();
+            do keep = all - c->kept + need <= total / 16;
+            while (keep && !g_kept.compare_exchange_weak(all, all - c->kept + need));
+            if (keep) c->kept = need;
+            if (keep && (c->seg.alloc(n * ssz) != hipSuccess || (lim && c->wseg.alloc(n * ssz) != hipSuccess) ||
+                         (c->adj_wd && c->segwd.alloc(n * ne) != hipSuccess))) {
+                (void)hipGetLastError();
+                c->seg.release();
+                c->wseg.release();
+                c->segwd.release();
+                g_kept -= c->kept;
+                c->kept = 0;
+                keep = false;
+            }
+        }
+        interval = keep ? kTableChunk : std::max(1, (int)std::lround(std::sqrt((double)nsteps)));
+    }
+    interval = std::min(interval, nsteps);
+    const int ncp = keep ? 1 : (nsteps + interval - 1) / interval;
+    HIPCHK(c->ckpt.alloc((size_t)ncp * ssz));
+    if (!keep) HIPCHK(c->seg.alloc((size_t)interval * nrk * ssz));
+    if (!keep && lim) HIPCHK(c->wseg.alloc((size_t)interval * nrk * ssz));
     if (c->adj_wd && !keep) HIPCHK(c->ckptwd.alloc((size_t)ncp * ne));
     // the state and wet/dry flags at entry: every exit path puts them back (the sweeps rotate the
     // stage slots and flip the flag buffers)

@@ -233,8 +233,9 @@ int dg_adj_gauges(int handle, int it, int nsteps, double* eta);
 /* Loss J = weight * sum_{k<nsteps} sum_g (eta_g after step it+k - data[k][g])^2 from the current
  * state, and its gradient with respect to the per-node Manning n and depth DP, by the discrete
  * adjoint of the stage RHS and the SSP-RK stages.  States are checkpointed every `interval` steps
- * and each segment is recomputed once on the way back; 0: every stage's state is kept and nothing is recomputed
- * where that takes at most 1/16 of the device's memory and half of what is free, else a checkpoint every
+ * and each segment is recomputed once on the way back; 0: every stage's state is kept and nothing is
+ * recomputed where that takes at most half of the memory that is free and all handles of the process
+ * together keep at most 1/16 of the device's until they are closed, else a checkpoint every
  * round(sqrt(nsteps)) steps.  The gradient does not depend on the choice.  The slope
  * limiter (SLOPELIMITER5) is differentiated with its active set frozen as the forward run
  * recomputes it (the selected node bounds, the redistribution counts and signs are those of the
