@@ -170,6 +170,8 @@ struct Ctx {
     DevBuf<uint8_t> wd[2];
     HostChunks chunks;
     DevBuf<int> iflags;                          // WDFLG as the host's integers (dg_gpu_get_state, dg_gpu_set_state)
+    DevBuf<double> pack;                         // a small state in the host's layout, the flags behind it
+    std::vector<double> h_pack;
     int wdcur = 0;
     // mesh
     DevBuf<uint16_t> sid;
@@ -1911,15 +1913,31 @@ int read_back(Ctx& c, const std::vector<Piece>& pieces) {
 // The stage slot after the current one: free between steps (the next step's first stage writes it).
 double* spare_state(Ctx& c) { return c.u[(c.ucur + 1) % (c.rk.nrk + 1)].p; }
 
-// The current state to (OUT) or from the host's layout in `aos`.
+// The current state to (OUT) or from the host's layout in `aos`, and with `flags` WDFLG.
 template <bool OUT>
-int launch_state_layout(Ctx& c, double* aos) {
+int launch_state_layout(Ctx& c, double* aos, int* flags) {
     const size_t n = (size_t)3 * c.dof * c.ne;
     const dim3 grid((unsigned)((n + 255) / 256)), block(256);
-    if (c.prm.p == 1) hipLaunchKernelGGL((state_layout_kernel<3, OUT>), grid, block, 0, c.stream, c.ne, c.u[c.ucur].p, aos);
-    else hipLaunchKernelGGL((state_layout_kernel<6, OUT>), grid, block, 0, c.stream, c.ne, c.u[c.ucur].p, aos);
+    double* const u = c.u[c.ucur].p;
+    uint8_t* const wd = c.wd[c.wdcur].p;
+    if (c.prm.p == 1) hipLaunchKernelGGL((state_layout_kernel<3, OUT>), grid, block, 0, c.stream, c.ne, u, aos, wd, flags);
+    else hipLaunchKernelGGL((state_layout_kernel<6, OUT>), grid, block, 0, c.stream, c.ne, u, aos, wd, flags);
     HIPCHK(hipGetLastError());
     return 0;
+}
+
+// A copy costs about 10 us however small it is, so a state of up to PACK_MAX bytes travels whole, in one copy to or from
+// a host buffer; a larger one in a copy per array, without the host's pass over it.  Whole and per array, reading with
+// the flags (us): 200 p=1 elements 36 and 74, 4,200 44 and 64, 10,000 (0.8 MB) 71 and 83, 20,000 139 and 116; p=2 6,080
+// (0.9 MB) 79 and 89, 10,000 139 and 114.  (Transposed on the host, in two copies: 47, 68, 113, 231; 110 and 233.)
+// Setting up to SET_MAX bytes without flags is shortest with the host's transposition and no kernel: 200 p=2 elements 16 us
+// against 26, 3,000 p=1 31 and 34, 4,200 (0.3 MB) 39 and 38.
+constexpr size_t PACK_MAX = (size_t)1 << 20, SET_MAX = (size_t)256 << 10;
+bool pack_state(Ctx& c, size_t n) {
+    const size_t words = 3 * n + ((size_t)c.ne + 1) / 2;
+    if (words * sizeof(double) > PACK_MAX || c.pack.alloc(words) != hipSuccess) return false;
+    c.h_pack.resize(words);
+    return true;
 }
 
 int validate(const dg_params* p) {
@@ -2218,19 +2236,35 @@ int dg_holland_storm_at(int nrec, const int* rec, const int* ref, int storm_numb
 int dg_gpu_set_state(int h, const double* ze, const double* qx, const double* qy, const int* wdflg) {
     Ctx* c = get(h);
     if (!c) return 1;
-    const size_t n = (size_t)c->ne * c->dof;
+    const size_t n = (size_t)c->ne * c->dof, nf = (size_t)c->ne * sizeof(int);
     const double* src[3] = {ze, qx, qy};
+    const bool packed = pack_state(*c, n);
+    if (packed && !wdflg && 3 * n * sizeof(double) <= SET_MAX) {
+        const size_t ne = c->ne, dof = c->dof;
+        for (size_t f = 0; f < 3; f++)
+            for (size_t e = 0; e < ne; e++)
+                for (size_t k = 0; k < dof; k++) c->h_pack[(f * dof + k) * ne + e] = src[f][e * dof + k];
+        HIPCHK(hipMemcpyAsync(c->u[c->ucur].p, c->h_pack.data(), 3 * n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        return 0;
+    }
+    if (packed) {
+        int* const flags = (int*)(c->pack.p + 3 * n);
+        for (int f = 0; f < 3; f++) std::memcpy(&c->h_pack[f * n], src[f], n * sizeof(double));
+        if (wdflg) std::memcpy(&c->h_pack[3 * n], wdflg, nf);
+        HIPCHK(hipMemcpyAsync(c->pack.p, c->h_pack.data(), 3 * n * sizeof(double) + (wdflg ? nf : 0), hipMemcpyHostToDevice, c->stream));
+        if (launch_state_layout<false>(*c, c->pack.p, wdflg ? flags : nullptr)) return 1;
+        HIPCHK(hipStreamSynchronize(c->stream));
+        return 0;
+    }
     double* aos = spare_state(*c);
     for (int f = 0; f < 3; f++)
         HIPCHK(hipMemcpyAsync(aos + f * n, src[f], n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    if (launch_state_layout<false>(*c, aos)) return 1;
     if (wdflg) {
         HIPCHK(c->iflags.alloc(c->ne));
-        HIPCHK(hipMemcpyAsync(c->iflags.p, wdflg, (size_t)c->ne * sizeof(int), hipMemcpyHostToDevice, c->stream));
-        hipLaunchKernelGGL((flags_kernel<false>), dim3((c->ne + 255) / 256), dim3(256), 0, c->stream, c->ne,
-                           c->wd[c->wdcur].p, c->iflags.p);
-        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(c->iflags.p, wdflg, nf, hipMemcpyHostToDevice, c->stream));
     }
+    if (launch_state_layout<false>(*c, aos, wdflg ? c->iflags.p : nullptr)) return 1;
     HIPCHK(hipStreamSynchronize(c->stream));
     return 0;
 }
@@ -2238,20 +2272,24 @@ int dg_gpu_set_state(int h, const double* ze, const double* qx, const double* qy
 int dg_gpu_get_state(int h, double* ze, double* qx, double* qy, int* wdflg) {
     Ctx* c = get(h);
     if (!c) return 1;
-    const size_t n = (size_t)c->ne * c->dof;
+    const size_t n = (size_t)c->ne * c->dof, nf = (size_t)c->ne * sizeof(int);
     double* dst[3] = {ze, qx, qy};
-    double* aos = spare_state(*c);
-    if (launch_state_layout<true>(*c, aos)) return 1;
-    if (wdflg) {
-        HIPCHK(c->iflags.alloc(c->ne));
-        hipLaunchKernelGGL((flags_kernel<true>), dim3((c->ne + 255) / 256), dim3(256), 0, c->stream, c->ne,
-                           c->wd[c->wdcur].p, c->iflags.p);
-        HIPCHK(hipGetLastError());
+    if (pack_state(*c, n)) {
+        if (launch_state_layout<true>(*c, c->pack.p, (int*)(c->pack.p + 3 * n))) return 1;
+        HIPCHK(hipMemcpyAsync(c->h_pack.data(), c->pack.p, 3 * n * sizeof(double) + (wdflg ? nf : 0), hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        for (int f = 0; f < 3; f++)
+            if (dst[f]) std::memcpy(dst[f], &c->h_pack[f * n], n * sizeof(double));
+        if (wdflg) std::memcpy(wdflg, &c->h_pack[3 * n], nf);
+        return 0;
     }
+    double* aos = spare_state(*c);
+    if (wdflg) HIPCHK(c->iflags.alloc(c->ne));
+    if (launch_state_layout<true>(*c, aos, wdflg ? c->iflags.p : nullptr)) return 1;
     std::vector<Piece> pieces;
     for (int f = 0; f < 3; f++)
         if (dst[f]) pieces.push_back({dst[f], aos + f * n, n * sizeof(double)});
-    if (wdflg) pieces.push_back({wdflg, c->iflags.p, (size_t)c->ne * sizeof(int)});
+    if (wdflg) pieces.push_back({wdflg, c->iflags.p, nf});
     return read_back(*c, pieces);
 }
 

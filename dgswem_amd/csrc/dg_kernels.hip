@@ -1865,27 +1865,23 @@ __global__ void __launch_bounds__(256) met_kernel(Met m, Forcing fo) {
 }
 
 // The state between the step's layout (soa: [field][mode][element]) and the host's (aos: [field][element][mode]), one
-// value per thread in the host's order, so that the copy to or from the caller's arrays is a plain one.  Transposing
-// on the host took longer than the copy: reading back 298,700 p=2 elements (43 MB) 14.4 ms before, 4.2 ms then, of
-// which the kernel takes 0.03 ms (setting it 13.2 and 1.6 ms).
+// value per thread in the host's order, so that the copy to or from the caller's arrays is a plain one; with `flags`
+// WDFLG between bytes and the host's integers too.  Transposing on the host took longer than the copy: reading back
+// 298,700 p=2 elements (43 MB) 14.4 ms before, 4.2 ms then, of which the kernel takes 0.03 ms (setting it 13.2 and 1.6 ms).
 template <int DOF, bool OUT>
-__global__ void __launch_bounds__(256) state_layout_kernel(int ne, double* __restrict__ soa, double* __restrict__ aos) {
+__global__ void __launch_bounds__(256) state_layout_kernel(int ne, double* __restrict__ soa, double* __restrict__ aos,
+                                                           uint8_t* __restrict__ wd, int* __restrict__ flags) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, n = (size_t)ne * DOF;
     if (i >= 3 * n) return;
+    if (flags && i < (size_t)ne) {
+        if (OUT) flags[i] = wd[i];
+        else wd[i] = flags[i] ? 1 : 0;
+    }
     const int f = (int)(i / n);
     const size_t j = i - f * n, e = j / DOF, k = j - e * DOF;
     double* const s = soa + ((size_t)f * DOF + k) * ne + e;
     if (OUT) aos[i] = *s;
     else *s = aos[i];
-}
-
-// WDFLG between bytes and the host's integers.
-template <bool OUT>
-__global__ void __launch_bounds__(256) flags_kernel(int ne, uint8_t* __restrict__ wd, int* __restrict__ flags) {
-    const int e = blockIdx.x * 256 + threadIdx.x;
-    if (e >= ne) return;
-    if (OUT) flags[e] = wd[e];
-    else wd[e] = flags[e] ? 1 : 0;
 }
 
 // Rows of the forcing tables from one packed list of values: table t holds `w` values per scenario, taken from
