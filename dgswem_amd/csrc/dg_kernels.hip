@@ -732,8 +732,8 @@ __device__ __forceinline__ void stage_entry(double* stg, uint8_t* stwd, int ns, 
 //     them, the side sums live in registers instead of LDS, and one side's traces are formed after the other's:
 //     166 registers at p=1 (226 before), three waves per SIMD instead of two; 251 at p=2 (293 and accumulator
 //     registers before), two instead of one;
-//   * the spherical p=1 variants would spill at three waves (94 us against 78 us per launch on 16 storm basins,
-//     438k elements), so they keep two;
+//   * the spherical and the linearised p=1 variants would spill at three waves (16 storm basins of 438k elements 94 us
+//     against 78 us per launch; linearised 796,320 elements 125 and 99 us, 118,933 31 and 26 us), so they keep two;
 //   * loads go out early: a tile's halo indices lie at a fixed stride (no look-up first), the next side's geometry
 //     is loaded while a side is evaluated, the quadrature's data before the sides and the RK base before the
 //     quadrature (which stood still for two thirds of its time when its loads waited behind the RK base).
@@ -741,7 +741,7 @@ __device__ __forceinline__ void stage_entry(double* stg, uint8_t* stwd, int ns, 
 // arithmetic of llf_flux_nl2 and cr_pow_third (35.0M VALU instructions instead of 44.8M); 298,700 elements, p=2:
 // 121 us before, 86 us.
 template <int P, int NT, bool SPH, bool WDFUSED, bool MET, bool NL>
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(P == 1 && !SPH ? 3 : 2))) stage_kernel(StageArgs a) {
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(P == 1 && !SPH && NL ? 3 : 2))) stage_kernel(StageArgs a) {
     constexpr int DOF = (P + 1) * (P + 2) / 2;
     constexpr int NAGP = (P == 1) ? 3 : 6;
     constexpr int NEGP = P + 2;
