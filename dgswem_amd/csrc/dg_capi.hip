@@ -120,11 +120,11 @@ struct Member {
 
 // Page-locked memory for reading results back (read_back), allocated at the first large result and again at the first
 // that calls for more.
-constexpr int RB_SLOTS = 6;
+constexpr int RB_SLOTS = 3;
 struct HostChunks {
     char* p = nullptr;
     size_t cap = 0;
-    hipEvent_t ev[RB_SLOTS] = {};
+    hipEvent_t ev[RB_SLOTS + 1] = {};    // of each chunk, and of the work before the result
     bool ok = true;                      // false: not to be had, not tried again
     HostChunks() = default;
     HostChunks(const HostChunks&) = delete;
@@ -1169,18 +1169,18 @@ size_t adj_dynamic_lds(int dof, int ns) {
 // Whether blocks of 64 elements run as four waves each (stage_split_kernel): the nonlinear equations and few
 // elements.  How many depends on how much of a launch is serial (a storm's gathers, its shoreline) and how much is
 // throughput, which the four waves lose: each variant's limit lies between the largest mesh measured on which they were
-// the faster and the smallest on which they were not.  Per launch, four waves per 64 elements against one lane per
-// element (us):
-//   p=1             20.3 and 21.3 at 81,369 elements, 22.1 and 21.1 at 89,340 (13.0 and 17.9 at 5k)
-//   p=1 spherical   20.4 and 20.4 at 61,972, 23.9 and 22.1 at 66,187
-//   p=1 storm       29.2 and 33.5 at 93,850, 30.8 and 30.8 at 99,015 (13.9 and 27.0 at 5k)
-//   p=2             31.0 and 31.4 at 63,445, 36.2 and 35.0 at 67,198 (18.8 and 27.9 at 5k)
-//   p=2 spherical   32.4 and 32.5 at 56,276, 34.2 and 32.4 at 59,314
-//   p=2 storm       47.5 and 48.5 at 81,369, 51.3 and 49.9 at 89,340 (21.1 and 42.3 at 5k)
+// the faster and the smallest on which they were not.  A time step with four waves per 64 elements and with one lane per
+// element (us, two stages and the limiters, back to back; launches timed one by one favour the latter by 2 to 4 %):
+//   p=1             34.2 and 35.9 at 81,369 elements, 37.0 and 36.3 at 85,090 (a stage 13.0 and 17.9 at 5k)
+//   p=1 spherical   42.0 and 44.8 at 61,972, 48.9 and 44.9 at 66,187
+//   p=1 storm       76.4 and 83.5 at 93,850, 78.2 and 79.0 at 99,015 (a stage 13.9 and 27.0 at 5k)
+//   p=2             70.4 and 70.9 at 64,038, 86.2 and 81.7 at 66,187 (a stage 18.8 and 27.9 at 5k)
+//   p=2 spherical   66.2 and 67.5 at 59,318, 71.0 and 67.5 at 61,972
+//   p=2 storm       116.4 and 118.8 at 89,340 (a stage 53.0 and 50.3 at 93,850; 21.1 and 42.3 at 5k)
 int split_max(const Ctx& c) {
-    if (c.met) return c.prm.p == 1 ? 96000 : 85000;
-    if (c.prm.ics == 2) return c.prm.p == 1 ? 64000 : 58000;
-    return c.prm.p == 1 ? 85000 : 64000;
+    if (c.met) return c.prm.p == 1 ? 96000 : 90000;
+    if (c.prm.ics == 2) return c.prm.p == 1 ? 64000 : 60500;
+    return c.prm.p == 1 ? 83000 : 64000;
 }
 bool stage_split(const Ctx& c) { return c.prm.nolicat != 0 && c.ne <= split_max(c); }
 
@@ -1829,62 +1829,76 @@ int adj_backward(Ctx& c, int it0, int nsteps, int interval, bool keep, double we
 
 // Device arrays to the caller's memory, on the context's stream; complete on return.  A large copy into pageable
 // memory ran at 10 GB/s, most of it the host's copy out of the runtime's buffer with the page faults of an array that
-// was just allocated.  From RB_MIN on it goes through page-locked chunks instead, which up to four threads copy out
-// while the next ones arrive.  A handle's first such result pays for the page-locking, about 0.1 ms a MiB where the
-// runtime has none to give again, so up to RB_LARGE four chunks of 1 MiB have to do: state of 118,933 p=1 and of 59,318
-// p=2 elements (9 MB) 1.2 to 1.7 ms with plain copies and a transposition on the host; 1.1 to 1.7 ms at first (1.8 to 2.2
-// with the chunks of larger results) and 0.35 ms then (0.33).  Beyond it six of 2 MiB: 298,579 p=2 elements (43 MB) 14 ms,
-// now 3 to 4 ms at first and 1.2 ms then (1.5 with the smaller chunks; two threads were slower than four, six no
-// faster).
+// was just allocated.  From RB_MIN on it goes through page-locked chunks instead, which up to four threads copy out, a
+// part each at a time, while the next ones arrive.  A handle's first such result pays for the page-locking, about 0.1 ms a
+// MiB where the runtime has none to give again, so the chunks are few: two up to RB_LARGE, three beyond it.  State of
+// 118,933 p=1 and of 59,318 p=2 elements (9 MB) 1.2 to 1.7 ms with plain copies and a transposition on the host, now 1.0 ms
+// at first (1.8 with six chunks, each copied by one thread) and 0.35 then; of 298,579 p=2 elements (43 MB) 14 ms, now 2.3
+// to 3 ms at first (3.2 to 3.9) and 1.2 then (two threads were slower than four, six no faster).
 struct Piece { void* dst; const void* src; size_t n; };
-constexpr size_t RB_MIN = (size_t)6 << 20, RB_LARGE = (size_t)16 << 20;
-int read_back(Ctx& c, const std::vector<Piece>& pieces) {
+constexpr size_t RB_MIN = (size_t)6 << 20, RB_LARGE = (size_t)16 << 20, RB_CHUNK = (size_t)2 << 20, RB_PART = (size_t)256 << 10;
+int rb_slots(size_t total) { return total < RB_MIN ? 0 : (total < RB_LARGE ? 2 : RB_SLOTS); }
+
+// Before the kernels that form a result of `total` bytes are launched: marks the end of the work queued until then.
+// False where the result will not go through the chunks.
+bool mark_queue(Ctx& c, size_t total) {
+    const int slots = rb_slots(total);
+    return slots > 0 && c.chunks.ensure(c.dev, slots * RB_CHUNK) && hipEventRecord(c.chunks.ev[RB_SLOTS], c.stream) == hipSuccess;
+}
+
+int read_back(Ctx& c, const std::vector<Piece>& pieces, bool marked) {
     size_t total = 0;
     for (auto& p : pieces) total += p.n;
-    const int slots = total < RB_LARGE ? 4 : RB_SLOTS;
-    const size_t chunk = (size_t)(total < RB_LARGE ? 1 : 2) << 20;
-    if (total < RB_MIN || !c.chunks.ensure(c.dev, slots * chunk)) {
+    const int slots = rb_slots(total);
+    if (!marked) {
         for (auto& p : pieces) HIPCHK(hipMemcpyAsync(p.dst, p.src, p.n, hipMemcpyDeviceToHost, c.stream));
         HIPCHK(hipStreamSynchronize(c.stream));
         return 0;
     }
+    // the chunks, and the parts of them that a thread copies at a time
+    struct Part { int k; size_t off, n; };
     std::vector<Piece> ch;
+    std::vector<Part> part;
     for (auto& p : pieces)
-        for (size_t o = 0; o < p.n; o += chunk)
-            ch.push_back({(char*)p.dst + o, (const char*)p.src + o, std::min(chunk, p.n - o)});
-    const int n = (int)ch.size();
-    std::vector<std::atomic<char>> done(n);
-    for (auto& d : done) d.store(0);
+        for (size_t o = 0; o < p.n; o += RB_CHUNK) {
+            const size_t n = std::min(RB_CHUNK, p.n - o);
+            for (size_t f = 0; f < n; f += RB_PART) part.push_back({(int)ch.size(), f, std::min(RB_PART, n - f)});
+            ch.push_back({(char*)p.dst + o, (const char*)p.src + o, n});
+        }
+    const int n = (int)ch.size(), np = (int)part.size();
+    std::vector<std::atomic<int>> left(n);               // parts of a chunk still to be copied out
+    for (int k = 0; k < n; k++) left[k].store((int)((ch[k].n + RB_PART - 1) / RB_PART));
     std::atomic<int> ready{0}, next{0};
     std::atomic<bool> stop{false};
-    auto slot = [&](int k) { return c.chunks.p + (size_t)(k % slots) * chunk; };
-    auto copy = [&](int k) {
-        std::memcpy(ch[k].dst, slot(k), ch[k].n);
-        done[k].store(1, std::memory_order_release);
+    auto slot = [&](int k) { return c.chunks.p + (size_t)(k % slots) * RB_CHUNK; };
+    auto copy = [&](const Part& p) {
+        std::memcpy((char*)ch[p.k].dst + p.off, slot(p.k) + p.off, p.n);
+        left[p.k].fetch_sub(1, std::memory_order_release);
     };
     auto work = [&]() {
-        for (int k; (k = next.fetch_add(1)) < n;) {
-            while (ready.load(std::memory_order_acquire) <= k) {
+        for (int j; (j = next.fetch_add(1)) < np;) {
+            while (ready.load(std::memory_order_acquire) <= part[j].k) {
                 if (stop.load()) return;
                 std::this_thread::yield();
             }
-            copy(k);
+            copy(part[j]);
         }
     };
     hipError_t err = hipSuccess;
-    int issued = 0;
+    int issued = 0, own = 0;
     auto issue = [&]() {
         while (err == hipSuccess && issued < n &&
-               (issued < slots || done[issued - slots].load(std::memory_order_acquire))) {
+               (issued < slots || left[issued - slots].load(std::memory_order_acquire) == 0)) {
             err = hipMemcpyAsync(slot(issued), ch[issued].src, ch[issued].n, hipMemcpyDeviceToHost, c.stream);
             if (err == hipSuccess) err = hipEventRecord(c.chunks.ev[issued % slots], c.stream);
             issued++;
         }
     };
-    // The threads start when the first chunk is there: before it lies all the work that is still queued, through which
-    // they would spin (a call behind 0.12 s of steps took 0.58 s of the host's cores, now 0.12).
+    // The threads start when the work queued before the result is done, while the first chunk is on its way: started
+    // at once they spin through that work (a call behind 0.12 s of steps took 0.58 s of the host's cores, now 0.12),
+    // started with the first chunk they are late (50 us of 0.35 ms).
     issue();
-    if (err == hipSuccess) err = hipEventSynchronize(c.chunks.ev[0]);
+    if (err == hipSuccess) err = hipEventSynchronize(c.chunks.ev[RB_SLOTS]);
     std::vector<std::thread> th;
     if (err == hipSuccess) {
         try {
@@ -1900,9 +1914,8 @@ int read_back(Ctx& c, const std::vector<Piece>& pieces) {
         if (k == issued) { std::this_thread::yield(); continue; }   // every chunk is still being copied out
         err = hipEventSynchronize(c.chunks.ev[k % slots]);
         if (err != hipSuccess) break;
-        if (th.empty()) copy(k);
-        else ready.store(k + 1, std::memory_order_release);
-        k++;
+        ready.store(++k, std::memory_order_release);
+        while (th.empty() && own < np && part[own].k < k) copy(part[own++]);
     }
     stop.store(err != hipSuccess);
     for (auto& t : th) t.join();
@@ -2285,12 +2298,15 @@ int dg_gpu_get_state(int h, double* ze, double* qx, double* qy, int* wdflg) {
     }
     double* aos = spare_state(*c);
     if (wdflg) HIPCHK(c->iflags.alloc(c->ne));
+    size_t total = wdflg ? nf : 0;
+    for (double* d : dst) total += d ? n * sizeof(double) : 0;
+    const bool marked = mark_queue(*c, total);
     if (launch_state_layout<true>(*c, aos, wdflg ? c->iflags.p : nullptr)) return 1;
     std::vector<Piece> pieces;
     for (int f = 0; f < 3; f++)
         if (dst[f]) pieces.push_back({dst[f], aos + f * n, n * sizeof(double)});
     if (wdflg) pieces.push_back({wdflg, c->iflags.p, nf});
-    return read_back(*c, pieces);
+    return read_back(*c, pieces, marked);
 }
 
 int dg_gpu_step(int h, int it, int nsteps) {
@@ -2355,7 +2371,9 @@ int dg_gpu_get_nodal(int h, double* eta2, double* uu2, double* vv2, int* nodecod
         if (dst[k]) pieces.push_back({dst[k], c->outbuf.p + k * np, np * sizeof(double)});
     if (nodecode) pieces.push_back({nodecode, c->nodecode.p, np * sizeof(int)});
     if (etamax) pieces.push_back({etamax, c->etamax.p, np * sizeof(double)});
-    if (read_back(*c, pieces)) return 1;
+    size_t total = 0;
+    for (auto& p : pieces) total += p.n;
+    if (read_back(*c, pieces, mark_queue(*c, total))) return 1;
     if (c->prof && prof_flush(*c)) return 1;
     return 0;
 }

@@ -1,5 +1,5 @@
-"""Results read back through page-locked chunks around the size from which there are more and larger ones (16 MiB),
-and a handle whose results fall on both sides of it in turn."""
+"""Results read back through page-locked chunks around the size from which there are more of them (16 MiB), and a handle
+whose results fall on both sides of it in turn."""
 import numpy as np
 import pytest
 
@@ -15,7 +15,7 @@ def random_state(n, seed):
 
 
 @pytest.mark.parametrize("nx", [11037, 11038])       # 76 bytes an element: just under and over
-def test_around_the_larger_chunks(nx):
+def test_around_the_larger_size(nx):
     c = closed(nx, 10, 1, nolifa=2)
     g = gpu.GpuSolver(c)
     for seed in (1, 2):
