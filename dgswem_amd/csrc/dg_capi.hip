@@ -120,7 +120,7 @@ struct Member {
 
 // Page-locked memory for reading results back (read_back), allocated at the first large result and again at the first
 // that calls for more.
-constexpr int RB_SLOTS = 3;
+constexpr int RB_SLOTS = 4;
 struct HostChunks {
     char* p = nullptr;
     size_t cap = 0;
@@ -1831,13 +1831,14 @@ int adj_backward(Ctx& c, int it0, int nsteps, int interval, bool keep, double we
 // memory ran at 10 GB/s, most of it the host's copy out of the runtime's buffer with the page faults of an array that
 // was just allocated.  From RB_MIN on it goes through page-locked chunks instead, which up to four threads copy out, a
 // part each at a time, while the next ones arrive.  A handle's first such result pays for the page-locking, about 0.1 ms a
-// MiB where the runtime has none to give again, so the chunks are few: two up to RB_LARGE, three beyond it.  State of
-// 118,933 p=1 and of 59,318 p=2 elements (9 MB) 1.2 to 1.7 ms with plain copies and a transposition on the host, now 1.0 ms
-// at first (1.8 with six chunks, each copied by one thread) and 0.35 then; of 298,579 p=2 elements (43 MB) 14 ms, now 2.3
-// to 3 ms at first (3.2 to 3.9) and 1.2 then (two threads were slower than four, six no faster).
+// MiB where the runtime has none to give again, so the chunks are few: three up to RB_LARGE, four beyond it (with one
+// fewer a new handle's first pass took 1 to 3 % longer).  State of 118,933 p=1 and of 59,318 p=2 elements (9 MB) 1.2 to
+// 1.7 ms with plain copies and a transposition on the host, now 1.4 ms at first (1.8 with six chunks, each copied by one
+// thread) and 0.33 then; of 298,579 p=2 elements (43 MB) 14 ms, now 3 ms at first (3.2 to 3.9) and 1.2 then (two threads
+// were slower than four, six no faster).
 struct Piece { void* dst; const void* src; size_t n; };
 constexpr size_t RB_MIN = (size_t)6 << 20, RB_LARGE = (size_t)16 << 20, RB_CHUNK = (size_t)2 << 20, RB_PART = (size_t)256 << 10;
-int rb_slots(size_t total) { return total < RB_MIN ? 0 : (total < RB_LARGE ? 2 : RB_SLOTS); }
+int rb_slots(size_t total) { return total < RB_MIN ? 0 : (total < RB_LARGE ? 3 : RB_SLOTS); }
 
 // Before the kernels that form a result of `total` bytes are launched: marks the end of the work queued until then.
 // False where the result will not go through the chunks.
