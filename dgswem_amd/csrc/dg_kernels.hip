@@ -724,7 +724,7 @@ __device__ __forceinline__ void stage_entry(double* stg, uint8_t* stwd, int ns, 
     stwd[j] = w;
 }
 
-// One lane per element.  What bounds it: FP64 instruction issue (about 2240 VALU instructions per element at p=1,
+// One lane per element.  What bounds it: FP64 instruction issue (2130 VALU instructions per element at p=1,
 // a wave each 4 cycles; the reciprocals and inverse square roots of the fluxes 16) and the latency of three phases
 // of loads (staging, quadrature, RK base), which the other waves on the SIMD have to cover.  So registers, which
 // set how many waves there are, matter as much as instructions:
@@ -737,8 +737,8 @@ __device__ __forceinline__ void stage_entry(double* stg, uint8_t* stwd, int ns, 
 //   * loads go out early: a tile's halo indices lie at a fixed stride (no look-up first), the next side's geometry
 //     is loaded while a side is evaluated, the quadrature's data before the sides and the RK base before the
 //     quadrature (which stood still for two thirds of its time when its loads waited behind the RK base).
-// Time per launch, 997,306 elements, p=1, limiter and wet/dry: 133 us before, 100 us with these and the shorter
-// arithmetic of llf_flux_nl2 and cr_pow_third (35.0M VALU instructions instead of 44.8M); 298,700 elements, p=2:
+// Time per launch, 997,306 elements, p=1, limiter and wet/dry: 129 us before, 91 us with these and the shorter
+// arithmetic of llf_flux_nl2 and cr_pow_third (33.2M VALU instructions instead of 44.1M); 298,579 elements, p=2:
 // 121 us before, 86 us.
 template <int P, int NT, bool SPH, bool WDFUSED, bool MET, bool NL>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(P == 1 && !SPH && NL ? 3 : 2))) stage_kernel(StageArgs a) {
@@ -1372,7 +1372,7 @@ __global__ void __launch_bounds__(256) node_minmax_kernel(int np, int ne, const 
 //
 // limit_wide_kernel: a wave per tile, a lane for the three fields of an element.  On large meshes the chip is full
 // either way, and what the three waves do three times (the lists, the addresses, the exchange before WETDRY) is time: 1103
-// VALU instructions per element, 943 here, for the same bytes (165 per element at p=1).  lim_wide says from how many
+// VALU instructions per element, 943 here, for the same bytes (174 per element at p=1).  lim_wide says from how many
 // elements on it is the faster form.  Per launch, one lane per element and 256-element tiles before, three waves per
 // tile, a wave per tile (us):
 //   limiter and WETDRY  p=1  46.6, 52.6, 43.0 at 997,306 elements; 32.3, 31.4, 27.5 at 597,806; 22.0, 19.9, 19.5 at 298,563
